@@ -98,7 +98,7 @@ hipError_t launch_spectra(const mi_particle* d_p, int64_t n, const mi_cube_desc&
 
 // Device FP64 setup (mi_prepare.hip): workspace layout and launcher.
 struct PrepLayout {
-    size_t keep, off, temp, temp_bytes, total;
+    size_t look, ticket, sums, total;
 };
 hipError_t prep_layout(int64_t n, PrepLayout* L);
 hipError_t prepare_particles(const double* xyz, const double* vxyz, const double* mHI,

@@ -12,11 +12,12 @@
 // Everything is FP64; the records carry the same integer/fraction splits as
 // the host packer.
 //
-// Two passes over the particles (keep flags, then the records at their scan
-// offsets) recompute the setup instead of storing it: the arithmetic is far
-// cheaper than 48 more bytes per particle of HBM traffic.
+// One pass over the particles: every work group sets up PREP_SPAN of them,
+// packs the records it keeps in LDS, finds its place in the output by a
+// decoupled look-back over the groups before it, and copies its records there.
 #include <hip/hip_runtime.h>
-#include <rocprim/device/device_scan.hpp>
+
+#include <cmath>
 
 #include "../../include/martini_mi355x.h"
 #include "mi_device.h"
@@ -50,12 +51,16 @@ __device__ inline void matvec(const double* m, const double* v, double* out) {
     out[2] = m[6] * v[0] + m[7] * v[1] + m[8] * v[2];
 }
 
-__device__ inline double pymod360(double x) { return x - 360.0 * floor(x / 360.0); }
+// The cube centre's sines and cosines, formed once on the host.
+struct Centre {
+    double sin_a0, cos_a0, sin_d0, cos_d0;
+};
 
 __device__ Setup setup_particle(int64_t i, const double* __restrict__ xyz,
                                 const double* __restrict__ vxyz, const double* __restrict__ mHI,
                                 const double* __restrict__ hsm, const double* __restrict__ T,
-                                const double* __restrict__ edges, const mi_observation& o) {
+                                const double* __restrict__ edges, const mi_observation& o,
+                                const Centre& c) {
     Setup S;
     S.flags = 0;
     // source frame: the source's rotation, then the observed frame
@@ -75,20 +80,27 @@ __device__ Setup setup_particle(int64_t i, const double* __restrict__ xyz,
     }
     const double dist = sqrt(pos[0] * pos[0] + pos[1] * pos[1] + pos[2] * pos[2]);
     const double vlos = (pos[0] * vel[0] + pos[1] * vel[1] + pos[2] * vel[2]) / dist;
-    const double ra_deg = pymod360(atan2(pos[1], pos[0]) * DEG_PER_RAD);
-    const double dec_deg = atan2(pos[2], hypot(pos[0], pos[1])) * DEG_PER_RAD;
 
-    // TAN projection about the cube centre, RA to the left
-    const double a0 = o.cube_ra_deg * RAD_PER_DEG, d0 = o.cube_dec_deg * RAD_PER_DEG;
-    const double ar = ra_deg * RAD_PER_DEG, dr = dec_deg * RAD_PER_DEG;
-    const double cos_d = cos(dr), sin_d = sin(dr);
-    const double cos_da = cos(ar - a0);
-    const double den = sin_d * sin(d0) + cos_d * cos(d0) * cos_da;
+    // TAN projection about the cube centre, RA to the left.  With the position
+    // (X, Y, Z) = dist (cos dec cos ra, cos dec sin ra, sin dec), the angles'
+    // products are ratios of linear forms in it: no inverse trigonometry, and
+    // no rounding of a right ascension near 360 degrees.
+    double X = pos[0], Y = pos[1], Z = pos[2];
+    if (!(dist < INFINITY)) {  // the direction that atan2 gives infinite components
+        X = isinf(X) ? copysign(1.0, X) : X - X;
+        Y = isinf(Y) ? copysign(1.0, Y) : Y - Y;
+        Z = isinf(Z) ? copysign(1.0, Z) : Z - Z;
+    } else if (dist == 0.0) {  // the observer: right ascension and declination zero
+        X = 1.0;
+    }
+    const double across = Y * c.cos_a0 - X * c.sin_a0;  // cos dec sin(ra - a0)
+    const double along = X * c.cos_a0 + Y * c.sin_a0;   // cos dec cos(ra - a0)
+    const double den = Z * c.sin_d0 + along * c.cos_d0;
     const double nan = __builtin_nan("");
     double x = nan, y = nan;
     if (den > 0.0) {
-        const double xi = cos_d * sin(ar - a0) / den * DEG_PER_RAD;
-        const double eta = (sin_d * cos(d0) - cos_d * sin(d0) * cos_da) / den * DEG_PER_RAD;
+        const double xi = across / den * DEG_PER_RAD;
+        const double eta = (Z * c.cos_d0 - along * c.sin_d0) / den * DEG_PER_RAD;
         x = o.crpix[0] - 1.0 + xi / o.cdelt[0];
         y = o.crpix[1] - 1.0 + eta / o.cdelt[1];
     }
@@ -175,7 +187,7 @@ __device__ Setup setup_particle(int64_t i, const double* __restrict__ xyz,
     const double k0 = floor(uu);
     const double fu = uu - k0;
     const double ade = fabs(o.de_ms);
-    const double amp = m * pow(dist, -2.0) / (ade / 1e3) / MHI_TO_JY * o.out_scale;
+    const double amp = m * (1.0 / (dist * dist)) / (ade / 1e3) / MHI_TO_JY * o.out_scale;
     double c_lo, c_hi, s = 0.0;
     if (o.spectrum == MI_SPECTRUM_GAUSS) {
         s = ade / (1.4142135623730951 * sigma * 1e3);
@@ -212,69 +224,188 @@ __device__ Setup setup_particle(int64_t i, const double* __restrict__ xyz,
     return S;
 }
 
-__global__ void k_prep_init(unsigned long long* counts) {
-    if (threadIdx.x < 4) counts[threadIdx.x] = 0ull;
+// A work group takes PREP_R rounds of PREP_T particles: 512 of them share one
+// look-back word and one ticket (requests to one cache line from all eight XCDs
+// are served one after another, about 11 ns each), and their records take
+// 24 KB of LDS, so six groups fit a CU.
+constexpr int PREP_T = 256;
+constexpr int PREP_R = 2;
+constexpr int PREP_SPAN = PREP_T * PREP_R;
+
+__host__ __device__ inline int64_t prep_groups(int64_t n) { return (n + PREP_SPAN - 1) / PREP_SPAN; }
+
+// A group's look-back word: state in the top bits, records kept in the low 32
+// (of the group alone, or of all groups up to it).
+constexpr unsigned long long LB_GROUP = 1ull << 62, LB_ALL = 2ull << 62;
+constexpr unsigned long long LB_STATE = 3ull << 62;
+
+// What a group adds to the totals (besides its records).
+struct PrepSums {
+    unsigned long long pairs, px, flags;
+};
+
+__global__ void k_prep_init(unsigned long long* __restrict__ counts,
+                            unsigned long long* __restrict__ look, uint32_t* __restrict__ ticket,
+                            int64_t groups) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < groups) look[i] = 0ull;
+    if (i < 4) counts[i] = 0ull;
+    if (i == 0 && ticket) *ticket = 0u;
 }
 
-__global__ void k_prep_flags(const double* __restrict__ xyz, const double* __restrict__ vxyz,
-                             const double* __restrict__ mHI, const double* __restrict__ hsm,
-                             const double* __restrict__ T, const double* __restrict__ edges,
-                             int64_t n, mi_observation o, uint32_t* __restrict__ keep) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    keep[i] = setup_particle(i, xyz, vxyz, mHI, hsm, T, edges, o).keep ? 1u : 0u;
-}
-
-__global__ void k_prep_write(const double* __restrict__ xyz, const double* __restrict__ vxyz,
-                             const double* __restrict__ mHI, const double* __restrict__ hsm,
-                             const double* __restrict__ T, const double* __restrict__ edges,
-                             int64_t n, mi_observation o, Grid g, const uint32_t* __restrict__ keep,
-                             const uint32_t* __restrict__ off, mi_particle* __restrict__ out,
-                             unsigned long long* __restrict__ counts) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long pairs = 0, px = 0;
-    uint32_t flags = 0;
-    if (i < n && keep[i]) {
-        const Setup S = setup_particle(i, xyz, vxyz, mHI, hsm, T, edges, o);
-        out[off[i]] = S.rec;
-        int a, b, c, d, e, f;
-        pairs = cells_of(S.rec, g, a, b, c, d, e, f);
-        flags = S.flags;
-        px = S.mask_px;
-    }
-    // one atomic per wave (integer sums: order-independent)
+__device__ inline unsigned long long wave_sum(unsigned long long v) {
 #pragma unroll
-    for (int dd = 32; dd > 0; dd >>= 1) {
-        pairs += __shfl_xor(pairs, dd, 64);
-        px += __shfl_xor(px, dd, 64);
-        flags |= __shfl_xor(flags, dd, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        if (pairs) atomicAdd(&counts[1], pairs);
-        if (flags) atomicOr(&counts[2], (unsigned long long)flags);
-        if (px) atomicAdd(&counts[3], px);
-    }
-    if (i == n - 1) atomicAdd(&counts[0], (unsigned long long)off[i] + keep[i]);
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+    return v;
 }
 
-// Workspace: keep flags and their exclusive scan (uint32[n] each), then the
-// scan's temporary storage.
+// Bound by the FP64 setup of a particle and by HBM (72 bytes read, 48 written).
+// Two passes (flags, scan, then the setup again with the records written at
+// their offsets and up to four atomics per wave on one cache line) took 387 +
+// 38 us for 1e6 particles, most of it in those atomics; this one takes 63 us
+// (1.9 TB/s), and the whole call with its counters read back 482 -> 117 us.
+// Groups of 256 particles make it 127 us, of 1024 117 us; held to 128 registers
+// (four waves per SIMD instead of three) it spills and takes 130 us.
+// Groups are numbered by a ticket, so every group that a look-back waits for
+// holds a lower ticket: it is running or done, and publishes its own count
+// before it waits for anything.
+__global__ __launch_bounds__(PREP_T) void k_prepare(
+    const double* __restrict__ xyz, const double* __restrict__ vxyz,
+    const double* __restrict__ mHI, const double* __restrict__ hsm, const double* __restrict__ T,
+    const double* __restrict__ edges, int64_t n, mi_observation o, Centre ctr,
+    Grid g, mi_particle* __restrict__ out, unsigned long long* __restrict__ counts,
+    unsigned long long* __restrict__ look, uint32_t* __restrict__ ticket,
+    PrepSums* __restrict__ sums) {
+    __shared__ uint4 recs[PREP_SPAN * 3];  // the kept records, packed
+    __shared__ uint32_t s_group, s_base, wcnt[PREP_R][PREP_T / 64];
+    __shared__ PrepSums wsum[PREP_T / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (t == 0)
+        s_group = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int64_t group = s_group;
+    unsigned long long pairs = 0, px = 0;
+    uint32_t flags = 0, kept = 0;
+#pragma unroll 1
+    for (int r = 0; r < PREP_R; ++r) {
+        const int64_t i = group * PREP_SPAN + r * PREP_T + t;
+        Setup S;
+        S.keep = false;
+        if (i < n) S = setup_particle(i, xyz, vxyz, mHI, hsm, T, edges, o, ctr);
+        const uint64_t mask = __ballot(S.keep);
+        if (lane == 0) wcnt[r][wave] = (uint32_t)__builtin_popcountll(mask);
+        __syncthreads();
+        uint32_t at = kept + (uint32_t)__builtin_popcountll(mask & ((1ull << lane) - 1ull));
+#pragma unroll
+        for (int w = 0; w < PREP_T / 64; ++w) {
+            at += w < wave ? wcnt[r][w] : 0u;
+            kept += wcnt[r][w];
+        }
+        if (S.keep) {
+            int a, b, c, d, e, f;
+            pairs += cells_of(S.rec, g, a, b, c, d, e, f);
+            flags |= S.flags;
+            px += S.mask_px;
+            uint4 words[3];
+            __builtin_memcpy(words, &S.rec, sizeof(words));
+#pragma unroll
+            for (int q = 0; q < 3; ++q) recs[at * 3 + q] = words[q];
+        }
+    }
+    if (t == 0)
+        __hip_atomic_store(&look[group], (group == 0 ? LB_ALL : LB_GROUP) | kept, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    pairs = wave_sum(pairs);
+    px = wave_sum(px);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) flags |= __shfl_xor(flags, d, 64);
+    if (lane == 0) wsum[wave] = PrepSums{pairs, px, flags};
+    if (wave == 0) {
+        // records kept by the groups before this one: 64 words at a time, back
+        // to the nearest group that already knows its total
+        uint32_t base = 0;
+        for (int64_t j = group - 1; j >= 0; j -= 64) {
+            unsigned long long v;
+            uint64_t all, need;
+            do {
+                v = j - lane >= 0 ? __hip_atomic_load(&look[j - lane], __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT)
+                                  : LB_ALL;
+                all = __ballot((v & LB_STATE) == LB_ALL);
+                need = all ? (all & (0ull - all)) * 2ull - 1ull : ~0ull;  // up to the nearest total
+            } while ((__ballot((v & LB_STATE) != 0ull) & need) != need);
+            uint32_t x = (need >> lane) & 1ull ? (uint32_t)v : 0u;
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
+            base += x;
+            if (all) break;
+        }
+        if (lane == 0) {
+            s_base = base;
+            if (group > 0)
+                __hip_atomic_store(&look[group], LB_ALL | (base + kept), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            if (group == prep_groups(n) - 1) counts[0] = (unsigned long long)base + kept;
+        }
+    }
+    __syncthreads();
+    if (t == 0) {
+        PrepSums s = wsum[0];
+#pragma unroll
+        for (int w = 1; w < PREP_T / 64; ++w) {
+            s.pairs += wsum[w].pairs;
+            s.px += wsum[w].px;
+            s.flags |= wsum[w].flags;
+        }
+        sums[group] = s;
+    }
+    uint4* dst = reinterpret_cast<uint4*>(out + s_base);
+    for (uint32_t e = t; e < kept * 3u; e += PREP_T) dst[e] = recs[e];
+}
 
+// The groups' sums into counts[1..3] (integers: any order gives the same).
+constexpr int PREP_SUM_T = 1024;
+
+__global__ __launch_bounds__(PREP_SUM_T) void k_prep_totals(const PrepSums* __restrict__ sums,
+                                                            int64_t groups,
+                                                            unsigned long long* __restrict__ counts) {
+    __shared__ PrepSums w[PREP_SUM_T / 64];
+    PrepSums s{0, 0, 0};
+    for (int64_t i = threadIdx.x; i < groups; i += PREP_SUM_T) {
+        s.pairs += sums[i].pairs;
+        s.px += sums[i].px;
+        s.flags |= sums[i].flags;
+    }
+    s.pairs = wave_sum(s.pairs);
+    s.px = wave_sum(s.px);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) s.flags |= __shfl_xor(s.flags, d, 64);
+    if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < PREP_SUM_T / 64; ++k) {
+            s.pairs += w[k].pairs;
+            s.px += w[k].px;
+            s.flags |= w[k].flags;
+        }
+        counts[1] = s.pairs;
+        counts[2] = s.flags;
+        counts[3] = s.px;
+    }
+}
+
+// Workspace: the groups' look-back words, the ticket, the groups' sums.
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 hipError_t prep_layout(int64_t n, PrepLayout* L) {
-    size_t tb = 0;
-    hipError_t e = rocprim::exclusive_scan(nullptr, tb, (const uint32_t*)nullptr, (uint32_t*)nullptr,
-                                           0u, (size_t)(n > 0 ? n : 1), rocprim::plus<uint32_t>(), 0);
-    if (e != hipSuccess) return e;
+    const size_t groups = (size_t)(n > 0 ? prep_groups(n) : 1);
     size_t o = 0;
-    L->keep = o;
-    o += align256(sizeof(uint32_t) * (size_t)(n > 0 ? n : 1));
-    L->off = o;
-    o += align256(sizeof(uint32_t) * (size_t)(n > 0 ? n : 1));
-    L->temp = o;
-    L->temp_bytes = tb;
-    o += align256(tb);
+    L->look = o;
+    o += align256(sizeof(unsigned long long) * groups);
+    L->ticket = o;
+    o += align256(sizeof(uint32_t));
+    L->sums = o;
+    o += align256(sizeof(PrepSums) * groups);
     L->total = o;
     return hipSuccess;
 }
@@ -284,20 +415,21 @@ hipError_t prepare_particles(const double* xyz, const double* vxyz, const double
                              const mi_observation& o, const Grid& g, mi_particle* out,
                              unsigned long long* counts, char* ws, const PrepLayout& L,
                              hipStream_t s) {
-    hipLaunchKernelGGL(k_prep_init, dim3(1), dim3(64), 0, s, counts);
-    if (n == 0) return hipGetLastError();
-    const int T_ = 256;
-    const unsigned blocks = (unsigned)((n + T_ - 1) / T_);
-    uint32_t* keep = (uint32_t*)(ws + L.keep);
-    uint32_t* off = (uint32_t*)(ws + L.off);
-    hipLaunchKernelGGL(k_prep_flags, dim3(blocks), dim3(T_), 0, s, xyz, vxyz, mHI, hsm, T, edges,
-                       n, o, keep);
-    size_t tb = L.temp_bytes;
-    hipError_t e = rocprim::exclusive_scan(ws + L.temp, tb, keep, off, 0u, (size_t)n,
-                                           rocprim::plus<uint32_t>(), s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_prep_write, dim3(blocks), dim3(T_), 0, s, xyz, vxyz, mHI, hsm, T, edges,
-                       n, o, g, keep, off, out, counts);
+    const int64_t groups = n > 0 ? prep_groups(n) : 0;
+    auto* look = (unsigned long long*)(ws + L.look);
+    auto* ticket = (uint32_t*)(ws + L.ticket);
+    auto* sums = (PrepSums*)(ws + L.sums);
+    if (groups == 0) {  // no workspace needed
+        hipLaunchKernelGGL(k_prep_init, dim3(1), dim3(256), 0, s, counts, look, nullptr, groups);
+        return hipGetLastError();
+    }
+    const double a0 = o.cube_ra_deg * RAD_PER_DEG, d0 = o.cube_dec_deg * RAD_PER_DEG;
+    const Centre ctr{sin(a0), cos(a0), sin(d0), cos(d0)};
+    hipLaunchKernelGGL(k_prep_init, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, counts,
+                       look, ticket, groups);
+    hipLaunchKernelGGL(k_prepare, dim3((unsigned)groups), dim3(PREP_T), 0, s, xyz, vxyz, mHI, hsm,
+                       T, edges, n, o, ctr, g, out, counts, look, ticket, sums);
+    hipLaunchKernelGGL(k_prep_totals, dim3(1), dim3(PREP_SUM_T), 0, s, sums, groups, counts);
     return hipGetLastError();
 }
 

@@ -115,3 +115,71 @@ def test_prepared_records_insert_like_host_records():
     diff = np.abs(dev_cube - host_cube).max() / np.abs(host_cube).max()
     print(f"device-setup cube vs host-setup cube: {diff:.3e}")
     assert diff <= 1e-6
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 511, 512, 513, 65 * 512 + 3])
+@pytest.mark.parametrize("massless", ["none", "some", "all"])
+def test_prepare_is_the_sum_of_its_parts(n, massless):
+    """The look-back over work groups of 512 particles: one call gives the
+    records and counts of separate calls on slices of at most 512 (one group
+    each), back to back, byte for byte, for groups that keep all, some (in
+    whole groups too) or none of their particles."""
+    import torch
+
+    w, _, make_k, make_s = _case("pruned_cube")
+    _, dc, k, s = synthetic.build(w, 16, kernel=make_k(), spectrum=make_s())
+    obs, _ = observation(distance=w.distance, datacube=dc, sph_kernel=k, spectral_model=s,
+                         rotation=w.rotation, h=0.7)
+    a = w.arrays(n)
+    m = a.mHI.copy()
+    if massless == "all":
+        m[:] = 0.0
+    elif massless == "some":
+        m[np.arange(n) % 7 < 3] = 0.0
+        m[(np.arange(n) // 512) % 3 == 1] = 0.0
+
+    def run(sl):
+        src = DeviceSource(a.xyz[sl], a.vxyz[sl], m[sl], a.hsm[sl], a.T[sl])
+        out, counts = prepare(src, obs)
+        counts = counts.cpu()
+        return out[: int(counts[0]) * 48].cpu(), counts
+
+    rec, counts = run(slice(0, n))
+    parts = [run(slice(b, min(b + 512, n))) for b in range(0, n, 512)]
+    assert torch.equal(rec, torch.cat([p[0] for p in parts]))
+    total = torch.stack([p[1] for p in parts]).sum(0)
+    assert torch.equal(counts[[0, 1, 3]], total[[0, 1, 3]])
+    if massless == "all":
+        assert counts.tolist() == [0, 0, 0, 0]
+
+
+def test_prepare_directions_match_host():
+    """Keep flags and sky pixels where the direction is degenerate: the
+    observer itself, the far hemisphere, infinite and NaN positions."""
+    inf, nan, D = np.inf, np.nan, 3000.0  # kpc
+    xyz = np.array([[0, 0, 0], [-D, 0, 0], [-2 * D, 1, 1], [inf, 0, 0], [0, inf, 0], [0, 0, -inf],
+                    [inf, 1, inf], [-inf, 2, 0], [nan, 0, 0], [0, 0, nan], [1, 2, 3]], float)
+    w = dataclasses.replace(synthetic.WORKLOADS["disc1e4_64px"], n=len(xyz))
+    n = len(xyz)
+    from martini_amd import DataCube, SPHSource
+
+    for ra, dec in ((0.0, 0.0), (30.0, -20.0)):
+        kw = dict(n_px_x=33, n_px_y=20, n_channels=16, px_size=16.0, channel_width=8.0,
+                  spectral_centre=w.vsys, ra=ra, dec=dec)
+        src = SPHSource(distance=w.distance, h=0.7, T_g=np.full(n, 1e4), mHI_g=np.full(n, 1e4),
+                        xyz_g=xyz, vxyz_g=np.zeros((n, 3)), hsm_g=np.full(n, 0.5))
+        with np.errstate(all="ignore"):
+            m = Martini(source=src, datacube=DataCube(**kw), sph_kernel=CubicSplineKernel(),
+                        spectral_model=GaussianSpectrum(sigma="thermal"), quiet=True)
+            from martini_amd import _pack
+
+            hrec, _ = _pack.pack_particles(m.source, m.sph_kernel, m.spectral_model, m.datacube)
+        obs, _ = observation(distance=w.distance, datacube=DataCube(**kw),
+                             sph_kernel=CubicSplineKernel(),
+                             spectral_model=GaussianSpectrum(sigma="thermal"))
+        out, counts = prepare(DeviceSource(xyz, np.zeros((n, 3)), np.full(n, 1e4), np.full(n, 0.5),
+                                           np.full(n, 1e4)), obs)
+        drec = out[: int(counts.cpu()[0]) * 48].cpu().numpy().view(_lib.PARTICLE_DTYPE)
+        assert drec.size == hrec.size
+        for f in ("ix", "iy", "c_lo", "c_hi"):
+            assert np.array_equal(drec[f], hrec[f]), (f, drec[f], hrec[f])
