@@ -192,6 +192,46 @@ def test_cube_to_fits_kernel(cube_bits, bitpix, shape, pad):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cube_bits,bitpix", [(32, -32), (32, -64), (64, -64), (64, -32)])
+@pytest.mark.parametrize("shape,offset", [((64, 3, 64), 0), ((68, 9, 100), 0), ((68, 9, 100), 1),
+                                          ((66, 1, 6), 0), ((130, 2, 65), 0), ((65, 70, 132), 0),
+                                          ((256, 300, 256), 0)])
+def test_cube_to_fits_alignment(cube_bits, bitpix, shape, offset):
+    """Rows that allow 16-byte loads, stores, both or neither (odd sides, or a
+    cube and an output one value off alignment), with signed zeros,
+    infinities and NaN, byte for byte against numpy; the range of a cube
+    without NaN exactly, with infinities as its extremes."""
+    import torch
+
+    from martini_amd import _lib
+
+    nx, ny, nc = shape
+    dt = np.float32 if cube_bits == 32 else np.float64
+    rng = np.random.default_rng(nx + 3 * ny + 7 * nc)
+    full = rng.normal(size=(nx, ny, nc)).astype(dt)
+    full.flat[:: max(1, full.size // 50)] = -0.0
+    full.flat[full.size // 2] = np.inf
+    full.flat[full.size // 3] = -np.inf
+    for nan in (False, True):
+        if nan:
+            full.flat[full.size // 5] = np.nan
+        buf = torch.zeros(full.size + offset, dtype=torch.float32 if cube_bits == 32 else torch.float64,
+                          device="cuda")
+        buf[offset:] = torch.from_numpy(full.ravel()).cuda()
+        size = -bitpix // 8
+        out = torch.zeros((full.size + offset) * size, dtype=torch.uint8, device="cuda")
+        d_range = torch.empty(2, dtype=torch.float64, device="cuda")
+        _lib.cube_to_fits(buf[offset:], nx, ny, nc, 0, 0, bitpix, out[offset * size:], d_range)
+        ref = np.ascontiguousarray(full.T).astype(">f4" if bitpix == -32 else ">f8")
+        got = np.frombuffer(out[offset * size:].cpu().numpy().tobytes(), ref.dtype).reshape(ref.shape)
+        finite = ~np.isnan(ref)
+        assert np.array_equal(np.isnan(got), ~finite)
+        assert got[finite].tobytes() == ref[finite].tobytes()
+        if not nan:
+            assert d_range.cpu().tolist() == [-np.inf, np.inf]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [None, np.float32, np.float64])
 def test_write_fits_data_and_dtype(tmp_path, dtype):
     """The written data unit is the unpadded cube transposed (the
