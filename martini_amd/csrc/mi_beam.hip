@@ -5,17 +5,19 @@
 //
 //   out[i, j, c] = sum_{a < kx, b < ky} K[a, b] * in[i + kx/2 - a, j + ky/2 - b, c]
 //
-// The cube is [nx][ny][nc], channels contiguous, so a thread carries a vector
-// of 4 channels through all taps.  A work group computes a 16 x 16 pixel x
-// 4-channel output tile; the beam image is taken in blocks of H rows x W
-// columns whose input halo ((16 + H - 1) x (16 + W - 1) pixels x 4 channels)
-// and taps (H x W) fit in LDS, so any beam size runs with the same code.
-// Direct summation in a fixed order (deterministic): FP32 along each row
-// segment of a block, FP64 across them.  A separable beam (a circular or
-// axis-aligned Gaussian's image is the outer product of two vectors) is
-// convolved by the caller as two such passes, a kx x 1 and a 1 x ky image;
-// those one-dimensional images take k_convolve_line, which reads each pixel's
-// channels contiguously.
+// The cube is [nx][ny][nc], channels contiguous.  Three kernels:
+//   k_convolve_line   one-dimensional images.  A separable beam (a circular or
+//                     axis-aligned Gaussian's image is the outer product of two
+//                     vectors) is convolved by the caller as two such passes, a
+//                     kx x 1 and a 1 x ky image;
+//   k_convolve_image  other images, where the cube fills the chip with its tiles;
+//   k_convolve_beam   other images on small cubes: a 16 x 16 pixel x 4-channel
+//                     output tile per work group, the beam image in blocks of H
+//                     rows x W columns whose input halo ((16 + H - 1) x (16 + W - 1)
+//                     pixels x 4 channels) and taps (H x W) fit in LDS.
+// Any beam size runs with each.  Direct summation in a fixed order
+// (deterministic): FP64, or FP32 along each row segment of a block and FP64
+// across them.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -24,6 +26,183 @@
 #include "mi_internal.h"
 
 namespace mi {
+
+// Rotated (non-separable) images: k_convolve_image.  A wave computes one output
+// row of a tile, 16 R pixels along y by 16 channels: lane = (pixel group of R,
+// quad of channels), so a tap is the same for the whole wave (a scalar
+// operand) and each 16-byte LDS read of an input pixel feeds R outputs from a
+// window of registers.  The IMG_X waves of a work group share the input rows,
+// which pass through LDS one at a time (two buffers, one barrier a row, the
+// next row's loads in flight): input row m feeds output row i through image
+// row i + kx/2 - m.  Each segment of an image row (up to IMG_MAX_W taps) is
+// summed in FP32 and added to FP64 totals, image rows in order: the FP32
+// rounding grows with the segment, not with kx * ky.
+// Bound by FP32 multiply-adds and the LDS reads beside them (27 x 27 taps on
+// 282 x 282 x 128: 0.19 ms of multiply-adds without packed FP32, 0.28 ms
+// measured; 0.31 with four outputs per lane and its 64-column tiles, 0.34 with
+// two, 0.36 with eight rows per group).  k_convolve_beam, with one LDS read of a
+// pixel and one of a tap for four multiply-adds, takes 0.60 ms there.
+constexpr int IMG_X = 4;          // output rows (waves) per work group
+constexpr int IMG_T = 64 * IMG_X;
+constexpr int IMG_C = 16;         // channels per work group
+constexpr int IMG_MAX_W = 128;    // image columns per segment
+constexpr int IMG_GROUPS = 256;   // work groups from which this kernel is taken
+
+// LDS slots of 64 bytes (one pixel's 16 channels) in a row buffer of px pixels.
+// The pixel groups of a wave lie R pixels apart: with an even R one spare slot
+// after every fourth pixel lets them read from different banks.  Four pixels
+// lie in front, which the register window may run into (and not use).
+template <int R>
+__host__ __device__ inline int img_slot(int px) { return R % 2 ? px : px + (px >> 2); }
+template <int R>
+__host__ __device__ inline int img_row_slots(int px) { return img_slot<R>(px + 4) + 1; }
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int R, bool VEC>
+__global__ __launch_bounds__(IMG_T) void k_convolve_image(const float* __restrict__ in,
+                                                          float* __restrict__ out, int nx, int ny,
+                                                          int nc, const float* __restrict__ K,
+                                                          int kx, int ky) {
+    extern __shared__ float4 rows[];  // two row buffers
+    constexpr int TY = 16 * R;
+    const int tiles_y = (ny + TY - 1) / TY;
+    const int x0 = (blockIdx.x / tiles_y) * IMG_X, y0 = (blockIdx.x % tiles_y) * TY;
+    const int c0 = blockIdx.y * IMG_C;
+    const int t = threadIdx.x, lane = t & 63;
+    const int i = x0 + __builtin_amdgcn_readfirstlane(t >> 6);  // this wave's output row
+    const int quad = lane & 3, yg = lane >> 2;
+    const int hx = kx / 2, hy = ky / 2;
+    const int wmax = ky < IMG_MAX_W ? ky : IMG_MAX_W;
+    const int buf = img_row_slots<R>(TY - 1 + wmax) * 4;  // float4s per row buffer
+    double tot[R][4];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) tot[r][c] = 0.0;
+
+    // Input rows reaching the tile, from the last (image row 0 first) to the first.
+    const int m_hi = min(nx - 1, x0 + IMG_X - 1 + hx), m_lo = max(0, x0 + hx - (kx - 1));
+    constexpr int PF = ((TY - 1 + IMG_MAX_W) * 4 + IMG_T - 1) / IMG_T;  // float4s per thread and row
+    for (int b0 = 0; b0 < ky; b0 += IMG_MAX_W) {
+        const int W = min(IMG_MAX_W, ky - b0);
+        const int ry0 = y0 + hy - b0 - (W - 1);  // input column of row pixel 0
+        const int n4 = (TY - 1 + W) * 4;
+        float4 pf[PF];
+        auto load = [&](int m) {
+#pragma unroll
+            for (int q = 0; q < PF; ++q) {
+                const int e = t + q * IMG_T, j = ry0 + (e >> 2), c = c0 + (e & 3) * 4;
+                pf[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (e >= n4 || j < 0 || j >= ny) continue;
+                const float* src = in + ((size_t)m * ny + j) * nc + c;
+                if (VEC) {
+                    if (c < nc) pf[q] = *reinterpret_cast<const float4*>(src);
+                } else {
+                    if (c < nc) pf[q].x = src[0];
+                    if (c + 1 < nc) pf[q].y = src[1];
+                    if (c + 2 < nc) pf[q].z = src[2];
+                    if (c + 3 < nc) pf[q].w = src[3];
+                }
+            }
+        };
+        __syncthreads();  // the last segment's rows are no longer read
+        int cur = 0;
+        load(m_hi);
+        for (int m = m_hi; m >= m_lo; --m) {
+            float4* row = rows + cur * buf;
+#pragma unroll
+            for (int q = 0; q < PF; ++q) {
+                const int e = t + q * IMG_T;
+                if (e < n4) row[img_slot<R>((e >> 2) + 4) * 4 + (e & 3)] = pf[q];
+            }
+            __syncthreads();  // the other buffer's readers are past the barrier before this one
+            if (m > m_lo) load(m - 1);
+            cur ^= 1;
+            const int a = i + hx - m;  // image row
+            if (a < 0 || a >= kx) continue;  // the same for the wave
+            const float* __restrict__ kr = K + (size_t)a * ky + b0;
+            // Tap b of the segment reads pixel yg R + r + (W - 1 - b) for output r;
+            // slot s of the window holds pixel p + s, p = yg R + W - 1 - b.
+            auto at = [&](int p) { return row[img_slot<R>(p + 4) * 4 + quad]; };
+            f32x4 acc[R], win[R];
+            auto get = [&](int p) {
+                const float4 v = at(p);
+                return f32x4{v.x, v.y, v.z, v.w};
+            };
+            int p = yg * R + W - 1;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+                win[r] = get(p + r);
+            }
+            auto step = [&](float k, int s) {  // tap with the window turned by s
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const f32x4 v = win[(r + R - s) % R];
+                    acc[r].x = fmaf(k, v.x, acc[r].x);
+                    acc[r].y = fmaf(k, v.y, acc[r].y);
+                    acc[r].z = fmaf(k, v.z, acc[r].z);
+                    acc[r].w = fmaf(k, v.w, acc[r].w);
+                }
+            };
+            int b = 0;
+            for (; b + R < W; b += R, p -= R) {
+                f32x4 next[R];
+#pragma unroll
+                for (int s = 0; s < R; ++s) next[s] = get(p - 1 - s);
+#pragma unroll
+                for (int s = 0; s < R; ++s) {
+                    step(kr[b + s], s);
+                    win[R - 1 - s] = next[s];
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < R; ++s) {  // the last 1 .. R taps
+                if (b + s >= W) break;
+                step(kr[b + s], s);
+                if (s + 1 < R) win[R - 1 - s] = get(p - 1 - s);
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) tot[r][c] += (double)acc[r][c];
+        }
+    }
+    const int c = c0 + quad * 4;
+    if (i >= nx || c >= nc) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int j = y0 + yg * R + r;
+        if (j >= ny) continue;
+        float* dst = out + ((size_t)i * ny + j) * nc + c;
+        if (VEC) {
+            *reinterpret_cast<float4*>(dst) = make_float4((float)tot[r][0], (float)tot[r][1],
+                                                          (float)tot[r][2], (float)tot[r][3]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c + q < nc) dst[q] = (float)tot[r][q];
+        }
+    }
+}
+
+template <int R>
+static hipError_t convolve_image(const float* in, float* out, int nx, int ny, int nc,
+                                 const float* K, int kx, int ky, hipStream_t s) {
+    const dim3 grid((unsigned)(((nx + IMG_X - 1) / IMG_X) * ((ny + 16 * R - 1) / (16 * R))),
+                    (unsigned)((nc + IMG_C - 1) / IMG_C));
+    const size_t lds = 2 * 64 * (size_t)img_row_slots<R>(16 * R - 1 + (ky < IMG_MAX_W ? ky : IMG_MAX_W));
+    const bool vec = nc % 4 == 0 &&
+                     ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    if (vec)
+        hipLaunchKernelGGL((k_convolve_image<R, true>), grid, dim3(IMG_T), lds, s, in, out, nx, ny,
+                           nc, K, kx, ky);
+    else
+        hipLaunchKernelGGL((k_convolve_image<R, false>), grid, dim3(IMG_T), lds, s, in, out, nx,
+                           ny, nc, K, kx, ky);
+    return hipGetLastError();
+}
 
 constexpr int BT = 16;               // output tile edge (pixels)
 constexpr int BEAM_LDS = 56 * 1024;  // bytes of LDS for one block's halo and taps
@@ -120,106 +299,189 @@ __global__ __launch_bounds__(256) void k_convolve_beam(const float* __restrict__
     }
 }
 
-// One-dimensional pass over a [O][L][E] view of the cube (E contiguous, in
-// units of V: float4 or float), along L:
+// One-dimensional pass over a [O][L][E] view of the cube (E contiguous), along L:
 //
 //   out[o][l][e] = sum_{a < k} K[a] * in[o][l + k/2 - a][e],  zero outside [0, L).
 //
 // A kx x 1 image is the pass along x (O = 1, L = nx, E = ny * nc), a 1 x ky
-// image the pass along y (O = nx, L = ny, E = nc).  The 64 lanes of a wave
-// take 64 consecutive elements of E (one 1 KB row of float4s per load), and
-// each wave LINE_R consecutive outputs along L: it walks the LINE_R + k - 1
-// input rows once, adding each to the outputs whose taps reach it, so an
-// input row is loaded (LINE_R + k - 1) / LINE_R times per wave instead of k.
-// The taps are held in LDS as FP64 and every sum is formed in FP64 in a fixed
-// order (deterministic; FP32 rounding only at the output).
-constexpr int LINE_R = 8;        // outputs per wave along the axis
-constexpr int LINE_WAVES = 4;    // waves per work group (consecutive strips along L)
-constexpr int LINE_MAX_K = 4096; // taps held in LDS (32 KB); longer images take k_convolve_beam
-constexpr int LINE_G = 4;        // input rows loaded together
+// image the pass along y (O = nx, L = ny, E = nc).  It is a contraction with a
+// banded matrix of taps, and runs on the FP64 matrix units: a wave takes
+// LINE_R consecutive outputs along L, as LINE_R / 16 blocks of 16, for 64
+// columns (the (o, e) pairs, flattened, so any number of channels fills it):
+// four 16-column blocks, lane n of a block holding column 4 n + block, so that
+// its row of each is one 16-byte load (`vec`: E a multiple of 4 and aligned
+// buffers) or, without that, column 16 * block + n.  Each step multiplies four
+// input rows into every block of outputs that they reach; the taps of a step
+// come from a zero-padded FP64 copy in LDS, one read for eight products.
+// Sums are FP64 in a fixed order (deterministic; FP32 rounding only at the
+// output).
+//
+// Bound by HBM (8 bytes per voxel and pass) and the matrix units together:
+// k + 15 rows, rounded up to fours, are multiplied for 16 outputs.  On
+// 538 x 538 x 256 with 27 taps a pass takes 146 us (4.1 TB/s), about 110 of
+// which the products would take alone; the previous vector form (eight outputs
+// per lane, one tap test and one LDS tap read per four multiply-adds, each
+// input row read (k + 7) / 8 times) took 200 us.  16 outputs per wave read more
+// halo rows (168 us), 64 leave too few registers for four waves per SIMD;
+// stores that stay in the caches 156 us.
+// A row outside the band meets a zero tap, and zero times an infinity or a NaN
+// would spread it to its neighbours along L, so a wave that ends with a
+// non-finite sum forms its sums again tap by tap.
+constexpr int LINE_R = 32;       // outputs per wave along the axis
+constexpr int LINE_T = LINE_R / 16;
+constexpr int LINE_WAVES = 2;    // waves per work group (consecutive strips along L)
+constexpr int LINE_COLS = 64;    // columns per wave
+constexpr int LINE_MAX_K = 4096; // taps held in LDS (33 KB); longer images take k_convolve_beam
+constexpr int LINE_PAD = 20;     // zeros on either side of the taps
+constexpr int LINE_G = 2;        // steps whose rows are loaded together
 
-template <class V>
-__device__ inline void fma_into(double (&acc)[4], double w, const V& v);
-template <>
-__device__ inline void fma_into<float4>(double (&acc)[4], double w, const float4& v) {
-    acc[0] = fma(w, (double)v.x, acc[0]);
-    acc[1] = fma(w, (double)v.y, acc[1]);
-    acc[2] = fma(w, (double)v.z, acc[2]);
-    acc[3] = fma(w, (double)v.w, acc[3]);
-}
-template <>
-__device__ inline void fma_into<float>(double (&acc)[4], double w, const float& v) {
-    acc[0] = fma(w, (double)v, acc[0]);
-}
-__device__ inline float4 round_out(const double (&a)[4], float4*) {
-    return make_float4((float)a[0], (float)a[1], (float)a[2], (float)a[3]);
-}
-__device__ inline float round_out(const double (&a)[4], float*) { return (float)a[0]; }
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-template <class V>
-__global__ __launch_bounds__(64 * LINE_WAVES) void k_convolve_line(
-    const V* __restrict__ in, V* __restrict__ out, int L, int64_t E, const float* __restrict__ K,
-    int k) {
-    extern __shared__ double taps[];
-    for (int a = threadIdx.x; a < k; a += 64 * LINE_WAVES) taps[a] = (double)K[a];
+template <bool VEC>
+__global__ __launch_bounds__(64 * LINE_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void
+k_convolve_line(
+    const float* __restrict__ in, float* __restrict__ out, int L, int64_t E, int64_t cols,
+    const float* __restrict__ K, int k) {
+    extern __shared__ double taps[];  // taps[LINE_PAD + a]
+    for (int a = threadIdx.x; a < k + 2 * LINE_PAD; a += 64 * LINE_WAVES)
+        taps[a] = a >= LINE_PAD && a < k + LINE_PAD ? (double)K[a - LINE_PAD] : 0.0;
     __syncthreads();
-    const int64_t e = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    const int lane = threadIdx.x & 63, n = lane & 15, kk = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l0 = (blockIdx.y * LINE_WAVES + wave) * LINE_R;
-    if (e >= E || l0 >= L) return;
-    const V* src = in + (int64_t)blockIdx.z * L * E + e;
-    V* dst = out + (int64_t)blockIdx.z * L * E + e;
-    double acc[LINE_R][4];
+    if (l0 >= L) return;
+    // This lane's columns: their offsets from row 0 (in floats), -1 past the end.
+    int64_t at[VEC ? 1 : 4];
 #pragma unroll
-    for (int q = 0; q < LINE_R; ++q)
+    for (int j = 0; j < (VEC ? 1 : 4); ++j) {
+        const int64_t c = (int64_t)blockIdx.x * LINE_COLS + (VEC ? 4 * n : 16 * j + n);
+        const int64_t o = c / E;
+        at[j] = c < cols ? o * L * E + (c - o * E) : -1;
+    }
+    f64x4 acc[LINE_T][4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[q][c] = 0.0;
-    // Input row m0 + r feeds output l0 + q through tap a = q + k - 1 - r; rows
-    // outside [0, L) are zero and skipped.  Rows are taken LINE_G at a time, their
-    // loads issued together.
+    for (int q = 0; q < LINE_T; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[q][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    // Step s takes input rows m0 + 4 s + kk; row m0 + r feeds output l0 + q
+    // through tap q + k - 1 - r.  Block q of 16 outputs needs steps 4 q .. 4 q + S - 1.
     const int m0 = l0 + k / 2 - (k - 1);
-    const int r0 = max(0, -m0), r1 = min(LINE_R + k - 1, L - m0);
-    int r = r0;
-    for (; r + LINE_G <= r1; r += LINE_G) {
-        V v[LINE_G];
+    const int S = (k + 15 + 3) / 4;
+    const int steps = S + 4 * (LINE_T - 1);
+    auto load = [&](int s, float (&v)[4]) {
+        const int m = m0 + 4 * s + kk;
+        const bool ok = m >= 0 && m < L;
+        if (VEC) {
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (ok && at[0] >= 0) x = *reinterpret_cast<const float4*>(in + at[0] + (int64_t)m * E);
+            v[0] = x.x;
+            v[1] = x.y;
+            v[2] = x.z;
+            v[3] = x.w;
+        } else {
 #pragma unroll
-        for (int g = 0; g < LINE_G; ++g) v[g] = src[(int64_t)(m0 + r + g) * E];
+            for (int j = 0; j < 4; ++j)
+                v[j] = ok && at[VEC ? 0 : j] >= 0 ? in[at[VEC ? 0 : j] + (int64_t)m * E] : 0.0f;
+        }
+    };
+    const double* tap = taps + LINE_PAD + n - kk + k - 1;  // the lane's tap of step s: tap[-4 s]
+    float v[LINE_G][4];
+#pragma unroll
+    for (int g = 0; g < LINE_G; ++g) load(g, v[g]);
+    for (int s0 = 0; s0 < steps; s0 += LINE_G) {
+        float w[LINE_G][4];
+#pragma unroll
+        for (int g = 0; g < LINE_G; ++g)
+            if (s0 + LINE_G < steps) load(s0 + LINE_G + g, w[g]);
+#pragma unroll
+        for (int g = 0; g < LINE_G; ++g) {
+            const int s = s0 + g;
+#pragma unroll
+            for (int q = 0; q < LINE_T; ++q) {
+                const int sq = s - 4 * q;
+                if (sq < 0 || sq >= S) continue;  // uniform
+                const double a = tap[-4 * sq];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    acc[q][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)v[g][j], acc[q][j],
+                                                                     0, 0, 0);
+            }
+        }
 #pragma unroll
         for (int g = 0; g < LINE_G; ++g)
 #pragma unroll
-            for (int q = 0; q < LINE_R; ++q) {
-                const int a = q + k - 1 - (r + g);
-                if (a >= 0 && a < k) fma_into<V>(acc[q], taps[a], v[g]);  // uniform
+            for (int j = 0; j < 4; ++j) v[g][j] = w[g][j];
+    }
+    // Lane: outputs l0 + 16 q + 4 i + kk (i = 0..3) of its columns.
+    bool finite = true;
+#pragma unroll
+    for (int q = 0; q < LINE_T; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) finite = finite && __builtin_isfinite(acc[q][j][i]);
+    if (!__all(finite)) {
+#pragma unroll 1
+        for (int q = 0; q < LINE_T; ++q)
+#pragma unroll 1
+            for (int i = 0; i < 4; ++i) {
+                const int l = l0 + 16 * q + 4 * i + kk;
+                double sum[4] = {0.0, 0.0, 0.0, 0.0};
+                for (int a = min(k - 1, l + k / 2); a >= 0; --a) {
+                    const int m = l + k / 2 - a;
+                    if (m >= L) break;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int64_t c = VEC ? at[0] : at[VEC ? 0 : j];
+                        if (c >= 0)
+                            sum[j] = fma(taps[LINE_PAD + a],
+                                         (double)in[c + (VEC ? j : 0) + (int64_t)m * E], sum[j]);
+                    }
+                }
+#pragma unroll
+                for (int q2 = 0; q2 < LINE_T; ++q2)
+#pragma unroll
+                    for (int i2 = 0; i2 < 4; ++i2)
+                        if (q2 == q && i2 == i)
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) acc[q2][j][i2] = sum[j];
             }
     }
-    for (; r < r1; ++r) {
-        const V v = src[(int64_t)(m0 + r) * E];
 #pragma unroll
-        for (int q = 0; q < LINE_R; ++q) {
-            const int a = q + k - 1 - r;
-            if (a >= 0 && a < k) fma_into<V>(acc[q], taps[a], v);  // uniform
+    for (int q = 0; q < LINE_T; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int l = l0 + 16 * q + 4 * i + kk;
+            if (l >= L) continue;
+            if (VEC) {
+                if (at[0] >= 0)
+                    __builtin_nontemporal_store(
+                        f32x4{(float)acc[q][0][i], (float)acc[q][1][i], (float)acc[q][2][i],
+                              (float)acc[q][3][i]},
+                        reinterpret_cast<f32x4*>(out + at[0] + (int64_t)l * E));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (at[VEC ? 0 : j] >= 0)
+                        out[at[VEC ? 0 : j] + (int64_t)l * E] = (float)acc[q][j][i];
+            }
         }
-    }
-#pragma unroll
-    for (int q = 0; q < LINE_R; ++q)
-        if (l0 + q < L) dst[(int64_t)(l0 + q) * E] = round_out(acc[q], (V*)nullptr);
 }
 
-static hipError_t convolve_line(const float* in, float* out, int64_t O, int L, int64_t E_floats,
+static hipError_t convolve_line(const float* in, float* out, int64_t O, int L, int64_t E,
                                 const float* K, int k, hipStream_t s) {
-    const unsigned strips = (unsigned)((L + LINE_R * LINE_WAVES - 1) / (LINE_R * LINE_WAVES));
-    const size_t lds = sizeof(double) * (size_t)k;
-    const bool vec = E_floats % 4 == 0 &&
+    const int64_t cols = O * E;
+    const dim3 grid((unsigned)((cols + LINE_COLS - 1) / LINE_COLS),
+                    (unsigned)((L + LINE_R * LINE_WAVES - 1) / (LINE_R * LINE_WAVES)));
+    const size_t lds = sizeof(double) * (size_t)(k + 2 * LINE_PAD);
+    const bool vec = E % 4 == 0 &&
                      ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    if (vec) {
-        const int64_t E = E_floats / 4;
-        hipLaunchKernelGGL(k_convolve_line<float4>, dim3((unsigned)((E + 63) / 64), strips, (unsigned)O),
-                           dim3(64 * LINE_WAVES), lds, s, reinterpret_cast<const float4*>(in),
-                           reinterpret_cast<float4*>(out), L, E, K, k);
-    } else {
-        hipLaunchKernelGGL(k_convolve_line<float>, dim3((unsigned)((E_floats + 63) / 64), strips, (unsigned)O),
-                           dim3(64 * LINE_WAVES), lds, s, in, out, L, E_floats, K, k);
-    }
+    if (vec)
+        hipLaunchKernelGGL(k_convolve_line<true>, grid, dim3(64 * LINE_WAVES), lds, s, in, out, L, E,
+                           cols, K, k);
+    else
+        hipLaunchKernelGGL(k_convolve_line<false>, grid, dim3(64 * LINE_WAVES), lds, s, in, out, L,
+                           E, cols, K, k);
     return hipGetLastError();
 }
 
@@ -234,6 +496,20 @@ hipError_t convolve_beam(const float* in, float* out, int nx, int ny, int nc, co
         return convolve_line(in, out, 1, nx, (int64_t)ny * nc, K, kx, s);
     if (kx == 1 && ky <= LINE_MAX_K)  // along y: [nx][ny][nc]
         return convolve_line(in, out, nx, ny, nc, K, ky, s);
+    // k_convolve_image where it fills the chip: with fewer than a work group per
+    // CU its rows, one after another, are a chain that k_convolve_beam's small
+    // tiles do not have (90 x 81 x 45, 138 groups: 39 us against 29.5;
+    // 128 x 128 x 12, 96 groups: 57 against 40; 128 x 128 x 64, 384 groups: 60
+    // against 64.5; 282 x 282 x 128: 283 against 596), and where its tiles of
+    // 48 columns or more are not half empty (256 x 24 x 128: 66 against 62).
+    // Three outputs per lane against four by the columns they cover: three take
+    // 1.09 times as long per column.
+    const int64_t y3 = (ny + 47) / 48, y4 = (ny + 63) / 64;
+    const bool three = y3 * 48 * 12 < y4 * 64 * 11;
+    if (ny > 32 &&
+        ((nx + IMG_X - 1) / IMG_X) * (three ? y3 : y4) * ((nc + IMG_C - 1) / IMG_C) >= IMG_GROUPS)
+        return three ? convolve_image<3>(in, out, nx, ny, nc, K, kx, ky, s)
+                     : convolve_image<4>(in, out, nx, ny, nc, K, kx, ky, s);
     const int h = beam_block_rows(kx, ky), w = beam_block_cols(ky);
     const size_t lds = beam_lds_bytes(kx, ky);
     const unsigned tiles = (unsigned)(((nx + BT - 1) / BT) * ((ny + BT - 1) / BT));

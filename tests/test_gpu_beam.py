@@ -187,3 +187,82 @@ def test_one_dimensional_pass_unaligned_buffers():
     aligned_out = torch.empty_like(aligned_in)
     _lib.convolve_beam(aligned_in, aligned_out, *shape, taps, 1, 7)
     assert torch.equal(d_out.reshape(shape), aligned_out)
+
+
+def _direct(cube, K):
+    """The convolution and the sum of its terms' magnitudes, in FP64, tap by tap
+    (a term outside the map does not exist, so infinities stay in their reach)."""
+    nx, ny, _ = cube.shape
+    kx, ky = K.shape
+    out, mag = np.zeros(cube.shape), np.zeros(cube.shape)
+    with np.errstate(invalid="ignore"):
+        for a in range(kx):
+            for b in range(ky):
+                s, t = kx // 2 - a, ky // 2 - b
+                i0, i1, j0, j1 = max(0, -s), min(nx, nx - s), max(0, -t), min(ny, ny - t)
+                if i0 >= i1 or j0 >= j1:
+                    continue
+                term = K[a, b] * cube[i0 + s:i1 + s, j0 + t:j1 + t]
+                out[i0:i1, j0:j1] += term
+                mag[i0:i1, j0:j1] += np.abs(term)
+    return out, mag
+
+
+def _check(shape, K, special, ulps, offset=0):
+    """mi_convolve_beam against _direct within `ulps` FP32 half-ulps of the sum
+    of magnitudes, and infinities and NaN exactly where the direct sum has them."""
+    import torch
+
+    rng = np.random.default_rng(shape[0] + 31 * shape[1] + 7 * K.size)
+    cube = rng.normal(size=shape).astype(np.float32)
+    if special:
+        cube[shape[0] // 2, shape[1] // 3, 0] = np.inf
+        cube[shape[0] // 5, shape[1] - 1, -1] = np.nan
+        cube[0, 0, shape[2] // 2] = -np.inf
+    buf = torch.zeros(cube.size + offset, device="cuda")
+    buf[offset:] = torch.from_numpy(cube.ravel()).cuda()
+    out = torch.full((cube.size + offset,), 7.0, device="cuda")
+    K = K.astype(np.float32)
+    _lib.convolve_beam(buf[offset:], out[offset:], *shape, torch.from_numpy(K).cuda(), *K.shape)
+    gpu = out[offset:].cpu().numpy().reshape(shape).astype(float)
+    ref, mag = _direct(cube.astype(float), K.astype(float))
+    fine = np.isfinite(ref)
+    assert np.array_equal(fine, np.isfinite(gpu))
+    assert np.array_equal(gpu[~fine & ~np.isnan(ref)], ref[~fine & ~np.isnan(ref)])
+    assert np.array_equal(np.isnan(gpu), np.isnan(ref))
+    worst = np.max(np.abs(gpu - ref)[fine] - ulps * 2.0**-24 * mag[fine])
+    assert worst <= 0.0, worst
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("shape,k", [
+    ((132, 48, 128), (3, 3)), ((130, 47, 126), (5, 7)),     # three outputs per lane, one tile
+    ((131, 64, 120), (7, 5)), ((70, 65, 128), (3, 9)),      # four; a tile of one column
+    ((130, 96, 70), (1, 3)), ((130, 49, 128), (9, 1)),      # single rows and columns
+    ((129, 33, 128), (5, 131)), ((260, 40, 64), (3, 257)),  # image rows of two and three segments
+    ((21, 210, 256), (27, 27)),                             # an image larger than the map
+])
+def test_image_tiles(shape, k, special):
+    """The tiled image kernel at the edges of its tiles, segments and register
+    windows.  Each row segment of at most W = min(ky, 128) taps is an FP32 sum
+    (W roundings), the rest FP64, and the result is rounded once."""
+    rng = np.random.default_rng(k[0] * 1000 + k[1])
+    if 1 in k:  # keep it out of the one-dimensional pass: an explicit zero row or column
+        K = np.zeros((max(k[0], 3), max(k[1], 3)))
+        K[: k[0], : k[1]] = rng.random(k)
+    else:
+        K = rng.random(k)
+    _check(shape, K, special, min(K.shape[1], 128) + 2)
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("shape,k,axis", [
+    ((31, 3, 24), 1, 0), ((32, 5, 24), 3, 0), ((33, 4, 36), 17, 0), ((65, 2, 5), 27, 0),
+    ((5, 31, 16), 15, 1), ((3, 64, 100), 27, 1), ((70, 97, 4), 41, 1), ((3, 129, 7), 63, 1),
+])
+def test_line_tiles(shape, k, axis, special, offset):
+    """The one-dimensional pass at the edges of its 16-output blocks, strips and
+    64-column groups, aligned and not: an FP64 sum, rounded once."""
+    K = np.random.default_rng(k).random((k, 1) if axis == 0 else (1, k))
+    _check(shape, K, special, 1.001, offset)
