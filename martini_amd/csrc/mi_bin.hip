@@ -10,8 +10,19 @@
 // by a hash of the particle index (chunks spread over the tile).
 // Long segments are cut into work items of at most item_length() particles;
 // such cells get one partial tile per item.
+//
+// Launches: k_bin_init, k_emit (pairs, in particle order), one k_radix per
+// digit, k_cell_bounds, k_items (and k_build_items for many cells).  Every
+// kernel that places data by a running total (k_emit, k_radix) takes it from a
+// decoupled look-back: work groups are numbered by a ticket, publish their own
+// count in a 64-bit word (state and value together, so no other memory needs
+// ordering) and sum the words before theirs, back to the nearest one that holds
+// a total.  A group waits only for lower tickets, which run already and publish
+// before they wait.
 #include <hip/hip_runtime.h>
-#include <rocprim/device/device_radix_sort.hpp>
+
+#include <algorithm>
+#include <utility>
 
 #include "mi_device.h"
 #include "mi_internal.h"
@@ -41,14 +52,47 @@ Grid make_grid(const mi_cube_desc& d) {
     return g;
 }
 
-// Count and emit passes: EMIT_T threads per block, EMIT_ROUNDS particles per
-// thread.
-constexpr int EMIT_T = 256;
-constexpr int EMIT_ROUNDS = 4;
-constexpr int64_t EMIT_SPAN = (int64_t)EMIT_T * EMIT_ROUNDS;
+// Work group shapes of the emit and radix passes.
+struct GroupShape {
+    int threads, items;  // items per thread
+};
+constexpr bool same(const GroupShape& a, const GroupShape& b) {
+    return a.threads == b.threads && a.items == b.items;
+}
 
-__host__ __device__ inline int64_t emit_blocks(int64_t n) {
-    return n > 0 ? (n + EMIT_SPAN - 1) / EMIT_SPAN : 0;
+// Emit pass: `threads` threads per group, `items` particles per thread.  Large
+// groups on large inputs: a group's look-back waits for those before it, and
+// the waiting groups' reads delay each other (1e7 particles: 320 us with 1024
+// particles per group, 248 with 4096); small groups on small ones, so that they
+// spread over the CUs.
+constexpr GroupShape EMIT_SMALL{256, 1}, EMIT_MID{1024, 1}, EMIT_LARGE{1024, 4};
+
+static GroupShape emit_shape(int64_t n) {
+    return n >= 524288 ? EMIT_LARGE : n >= 65536 ? EMIT_MID : EMIT_SMALL;
+}
+static int64_t emit_groups(int64_t n) {
+    const GroupShape e = emit_shape(n);
+    const int64_t span = (int64_t)e.threads * e.items;
+    return n > 0 ? (n + span - 1) / span : 0;
+}
+
+// Radix passes: tiles of `threads` x `items` pairs.  Large tiles write longer
+// runs of equal digits and look back less (2.9e7 pairs, a pass: 240 us with tiles
+// of 2048, 196 with 4096, 180 with 8192; rocPRIM's took 212); small inputs take
+// small ones, so that they spread over the CUs.
+constexpr GroupShape RADIX_TILE_SMALL{256, 4}, RADIX_TILE_MID{1024, 4}, RADIX_TILE_LARGE{1024, 8};
+constexpr int64_t RADIX_MID = 131072, RADIX_LARGE = 1 << 20;
+constexpr int RADIX_BITS = 8;  // at most, per pass
+constexpr int RADIX_PASSES = (32 + RADIX_BITS - 1) / RADIX_BITS;
+
+static GroupShape radix_shape(int64_t n_pairs) {
+    return n_pairs >= RADIX_LARGE ? RADIX_TILE_LARGE
+           : n_pairs >= RADIX_MID ? RADIX_TILE_MID : RADIX_TILE_SMALL;
+}
+static int64_t radix_tiles(int64_t n_pairs) {
+    const GroupShape r = radix_shape(n_pairs);
+    const int64_t tile = (int64_t)r.threads * r.items;
+    return (n_pairs + tile - 1) / tile;
 }
 
 // Lowest key bit the coarse sort orders on: the top 16 bits of the key
@@ -57,6 +101,21 @@ __host__ __device__ inline int64_t emit_blocks(int64_t n) {
 static int coarse_begin_bit(const Grid& g) {
     const int b = g.cell_bits + KEY_LOCAL_BITS - 16;
     return b < 0 ? 0 : (b > 8 ? 8 : b);
+}
+
+// The passes over the sorted bits: as few as RADIX_BITS allows, of equal width.
+// In record order only the cell and the kernel group are sorted (two passes up
+// to 2^14 cells); the stable sort keeps the rest.
+struct RadixPlan {
+    int begin, passes, bits;
+};
+static RadixPlan radix_plan(const Grid& g, bool record_order) {
+    RadixPlan r;
+    r.begin = record_order ? KEY_LOCAL_BITS - 2 : coarse_begin_bit(g);
+    const int width = g.cell_bits + KEY_LOCAL_BITS - r.begin;
+    r.passes = (width + RADIX_BITS - 1) / RADIX_BITS;
+    r.bits = (width + r.passes - 1) / r.passes;
+    return r;
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -68,42 +127,36 @@ hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L) {
         off = align256(off + bytes);
         return at;
     };
-    size_t np = (size_t)(n_pairs > 0 ? n_pairs : 1);
-    const size_t nb2 = (size_t)emit_blocks(n) + 2;
-    size_t nc1 = (size_t)g.ncells + 1;
+    const size_t np = (size_t)(n_pairs > 0 ? n_pairs : 1);
+    const size_t nc = (size_t)g.ncells, nc1 = nc + 1;
     L->item_len = item_length(n_pairs);
     L->items_max = g.ncells + n_pairs / L->item_len + 1;
     L->multi_max = 2 * (n_pairs / L->item_len) + 1;
-    L->counts = take(4 * nb2);
-    L->offsets = take(4 * nb2);
+    // cleared by k_bin_init, from status on
+    L->status = take(sizeof(uint32_t) * ST_WORDS);
+    L->hist = take(sizeof(uint32_t) * RADIX_PASSES << RADIX_BITS);
+    L->cell_start = take(4 * nc);
+    L->cell_end = take(4 * nc);
+    L->emit_look = take(sizeof(unsigned long long) * (size_t)emit_groups(n));
+    size_t look = 0;
+    for (int order = 0; order < 2; ++order) {  // either gather's sort fits
+        const RadixPlan r = radix_plan(g, order != 0);
+        const size_t words = ((size_t)r.passes * (size_t)radix_tiles(n_pairs)) << r.bits;
+        look = words > look ? words : look;
+    }
+    L->radix_look = take(sizeof(unsigned long long) * look);
+    L->cleared = off;
     L->keys = take(4 * np);
     L->vals = take(4 * np);
     L->keys2 = take(4 * np);
     L->vals2 = take(4 * np);
-    L->cell_start = take(4 * (size_t)g.ncells);
-    L->cell_end = take(4 * (size_t)g.ncells);
     L->item_off = take(4 * nc1);
     L->multi_off = take(4 * nc1);
+    L->full_pos = take(4 * nc);
+    L->rest_pos = take(4 * nc);
     L->items = take(sizeof(Item) * (size_t)L->items_max);
-    L->item_keys = take(4 * (size_t)L->items_max);
-    L->item_keys2 = take(4 * (size_t)L->items_max);
-    L->item_idx = take(4 * (size_t)L->items_max);
-    L->item_order = take(4 * (size_t)L->items_max);
     L->partials = take(sizeof(float) * (size_t)L->multi_max * CELL_VOXELS);
     L->part_masks = take(sizeof(uint64_t) * (size_t)L->multi_max);
-    L->status = take(4 * 8);
-    // rocPRIM temporary storage: the larger of its two uses (the pair and the item sort).
-    size_t t1 = 0, t2 = 0;
-    uint32_t* nul = nullptr;
-    hipError_t e = rocprim::radix_sort_pairs(nullptr, t1, nul, nul, nul, nul, np, 0,
-                                             g.cell_bits + KEY_LOCAL_BITS, 0);
-    if (e != hipSuccess) return e;
-    e = rocprim::radix_sort_pairs(nullptr, t2, nul, nul, nul, nul, (size_t)L->items_max, 0,
-                                  ITEM_KEY_BITS, 0);
-    if (e != hipSuccess) return e;
-    const size_t tb = t1 > t2 ? t1 : t2;
-    L->temp_bytes = tb;
-    L->temp = take(tb);
     L->total = off;
     return hipSuccess;
 }
@@ -130,165 +183,326 @@ __device__ inline bool record_ok(const mi_particle& p, const Grid& g, const floa
     return end <= uw_n;
 }
 
-// Count and emit passes: block b takes particles b * EMIT_SPAN + i * EMIT_T + t
-// (rounds i = 0 .. EMIT_ROUNDS - 1, thread t), so the record loads of a round
-// are contiguous.  k_count writes each block's pair total, k_scan_blocks turns
-// them into block bases, and k_emit recounts its particles and scans them in
-// the block: particle k's pairs start at the sum of the counts before k, as
-// one global exclusive scan would place them, without a per-particle array.
+// Look-back words: state in the top bits, a count in the rest (of the group
+// alone, or of all groups up to it).
+constexpr unsigned long long LB_GROUP = 1ull << 62, LB_ALL = 2ull << 62;
+constexpr unsigned long long LB_STATE = 3ull << 62;
 
-// Exclusive block-wide scan (EMIT_T threads, all active); the block total in `total`.
-__device__ inline uint32_t block_excl_scan(uint32_t x, uint32_t* wsum, uint32_t& total) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t incl = (uint32_t)wave_scan_add((int)x);
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();
-    uint32_t base = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < EMIT_T / 64; ++i) {
-        const uint32_t v = wsum[i];
-        base += i < w ? v : 0u;
-        tot += v;
-    }
-    __syncthreads();  // wsum may be written again
-    total = tot;
-    return base + incl - x;
+// Pause between two looks at words that are not published yet (x 64 cycles):
+// the groups that wait would otherwise fill the fabric with their reads.
+constexpr int LOOK_SLEEP = 8;
+
+__device__ inline unsigned long long look_load(const unsigned long long* w) {
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void look_store(unsigned long long* w, unsigned long long v) {
+    __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(EMIT_T) void k_count(const mi_particle* __restrict__ P, int64_t n,
-                                                  Grid g, const float* __restrict__ uw,
-                                                  int64_t uw_n, uint32_t* __restrict__ block_tot,
-                                                  uint32_t* __restrict__ status) {
-    __shared__ uint32_t wsum[EMIT_T / 64];
-    const int64_t base = (int64_t)blockIdx.x * EMIT_SPAN + threadIdx.x;
-    uint32_t sum = 0;
-#pragma unroll
-    for (int i = 0; i < EMIT_ROUNDS; ++i) {
-        const int64_t k = base + (int64_t)i * EMIT_T;
-        if (k >= n) break;
-        const mi_particle p = P[k];
-        int a, b, c, d, e, f;
-        const uint32_t cells = cells_of(p, g, a, b, c, d, e, f);
-        sum += cells;
-        if (cells > 0 && !record_ok(p, g, uw, uw_n)) status[ST_BADREC] = 1u;  // same value from all
-    }
-    uint32_t total;
-    block_excl_scan(sum, wsum, total);
-    if (threadIdx.x == 0) block_tot[blockIdx.x] = total;
-}
-
-// Exclusive scan of the nb block totals in one work group (runs per thread,
-// then the run totals in LDS); base[nb], base[nb + 1] hold the 64-bit grand
-// total (low, high word), so a device count beyond 2^32 is still seen.
-constexpr int SCAN_T = 1024;
-
-__global__ __launch_bounds__(SCAN_T) void k_scan_blocks(const uint32_t* __restrict__ tot,
-                                                        int64_t nb, uint32_t* __restrict__ base) {
-    __shared__ unsigned long long s[SCAN_T];
-    const int t = threadIdx.x;
-    const int64_t per = (nb + SCAN_T - 1) / SCAN_T;
-    const int64_t b0 = min((int64_t)t * per, nb), b1 = min(b0 + per, nb);
-    unsigned long long run = 0;
-    for (int64_t b = b0; b < b1; ++b) run += tot[b];
-    s[t] = run;
-    __syncthreads();
-    for (int d = 1; d < SCAN_T; d <<= 1) {  // inclusive scan of the run totals
-        const unsigned long long v = t >= d ? s[t - d] : 0ull;
-        __syncthreads();
-        s[t] += v;
-        __syncthreads();
-    }
-    unsigned long long at = s[t] - run;
-    for (int64_t b = b0; b < b1; ++b) {
-        base[b] = (uint32_t)at;
-        at += tot[b];
-    }
-    if (t == SCAN_T - 1) {
-        base[nb] = (uint32_t)s[t];
-        base[nb + 1] = (uint32_t)(s[t] >> 32);
-    }
-}
-
-// Writes the (key, particle) pairs of each particle at its scanned offset.
-// With `mix` the low 8 key bits are a hash of the particle index: the FP32
-// gather's waves each own 4 tile rows, and a chunk of particles drawn from all
-// over the tile gives them even shares of the products, where a spatially
-// compact chunk loads one or two of them.  Without it they are zero and a
-// cell's pairs keep the record order (the MFMA form, whose records are laid
-// out in tile and pixel Z order).
-// Entries past the device total up to the capacity get key 0xffffffff so the
-// sort moves them to the end; a total above the capacity raises the overflow
-// flag and writes nothing.
-__global__ __launch_bounds__(EMIT_T) void k_emit(const mi_particle* __restrict__ P, int64_t n,
-                                                 int64_t cap, Grid g,
-                                                 const uint32_t* __restrict__ block_base,
-                                                 uint32_t* __restrict__ keys,
-                                                 uint32_t* __restrict__ vals,
-                                                 uint32_t* __restrict__ status, int mix) {
-    __shared__ uint32_t wsum[EMIT_T / 64];
-    const int64_t nb = emit_blocks(n);
-    const uint64_t total = (uint64_t)block_base[nb] | ((uint64_t)block_base[nb + 1] << 32);
-    const int64_t k0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k0 == 0) {
-        status[ST_PAIRS] = (uint32_t)total;
-        status[ST_OVERFLOW] = total > (uint64_t)cap ? 1u : 0u;
-    }
-    if (total > (uint64_t)cap) return;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t q = (int64_t)total + k0; q < cap; q += stride) {  // padding entries
-        keys[q] = 0xffffffffu;
-        vals[q] = 0u;
-    }
-    if ((int64_t)blockIdx.x >= nb) return;  // uniform
-    uint32_t run = block_base[blockIdx.x];
-    const int64_t base = (int64_t)blockIdx.x * EMIT_SPAN + threadIdx.x;
-#pragma unroll 1
-    for (int i = 0; i < EMIT_ROUNDS; ++i) {
-        const int64_t k = base + (int64_t)i * EMIT_T;
-        mi_particle p;
-        int tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1, cb0 = 0, cb1 = -1;
-        uint32_t cnt = 0;
-        if (k < n) {
-            p = P[k];
-            cnt = cells_of(p, g, tx0, tx1, ty0, ty1, cb0, cb1);
+// Sum of the counts of the groups before `group`, taken by one wave, 64 words
+// at a time.
+__device__ inline unsigned long long look_back(const unsigned long long* look, int64_t group) {
+    const int lane = threadIdx.x & 63;
+    unsigned long long base = 0;
+    for (int64_t j = group - 1; j >= 0; j -= 64) {
+        unsigned long long v;
+        uint64_t all, need;
+        while (true) {
+            v = j - lane >= 0 ? look_load(&look[j - lane]) : LB_ALL;
+            all = __ballot((v & LB_STATE) == LB_ALL);
+            need = all ? (all & (0ull - all)) * 2ull - 1ull : ~0ull;  // up to the nearest total
+            if ((__ballot((v & LB_STATE) != 0ull) & need) == need) break;
+            __builtin_amdgcn_s_sleep(LOOK_SLEEP);
         }
-        uint32_t round_total;
-        uint32_t at = run + block_excl_scan(cnt, wsum, round_total);
-        run += round_total;
-        if (cnt == 0) continue;
-        const uint32_t kg = kernel_group(kind_of(p.r_kind));
-        const uint32_t hash = ((uint32_t)k * 2654435761u) >> 24;
-        const uint32_t local = (kg << 8) | (mix ? hash : 0u);
-        for (int tx = tx0; tx <= tx1; ++tx) {
-            for (int ty = ty0; ty <= ty1; ++ty) {
-                for (int cb = cb0; cb <= cb1; ++cb) {
-                    uint32_t cell = (uint32_t)(((int64_t)tx * g.nty + ty) * g.ncb + cb);
-                    keys[at] = (cell << KEY_LOCAL_BITS) | local;
-                    vals[at] = (uint32_t)k;
-                    ++at;
-                }
+        unsigned long long x = (need >> lane) & 1ull ? v & ~LB_STATE : 0ull;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
+        base += x;
+        if (all) break;
+    }
+    return base;
+}
+
+// Writes the (key, particle) pairs of each particle, in particle order: group b
+// takes particles b * ROUNDS * T + i * T + t (rounds i, thread t), so the record
+// loads of a round are contiguous.  The records are read once: a
+// group holds its particles' cell ranges in registers, scans their counts and
+// takes its base from the look-back.  A particle of more than EMIT_WIDE cells is
+// written by its whole wave.  The digits of every radix pass are counted too
+// (hist), in EMIT_COPIES copies in LDS, a lane in eight to each: neighbouring
+// records share their cells, and adds to one address wait for each other.
+// With `mix` the low 8 key bits are a hash of the particle index:
+// the FP32 gather's waves each own 4 tile rows, and a chunk of particles drawn
+// from all over the tile gives them even shares of the products, where a
+// spatially compact chunk loads one or two of them.  Without it they are zero
+// and a cell's pairs keep the record order (the MFMA form, whose records are
+// laid out in tile and pixel Z order).  A total above the capacity raises the
+// overflow flag; nothing is written past the capacity, and the passes that
+// follow do nothing.
+constexpr uint32_t EMIT_WIDE = 8;
+constexpr int EMIT_COPIES = 8;
+
+template <int T, int ROUNDS>
+__global__ __launch_bounds__(T) void k_emit(
+    const mi_particle* __restrict__ P, int64_t n, int64_t cap, Grid g,
+    const float* __restrict__ uw, int64_t uw_n, unsigned long long* __restrict__ look,
+    uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, uint32_t* __restrict__ hist,
+    uint32_t* __restrict__ status, int mix, int begin, int passes, int bits) {
+    __shared__ uint32_t wsum[ROUNDS][T / 64];
+    extern __shared__ uint32_t lhist[];  // EMIT_COPIES x ((passes << bits) + 1)
+    __shared__ uint32_t s_group;
+    __shared__ unsigned long long s_base;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (t == 0)
+        s_group = __hip_atomic_fetch_add(&status[ST_TICKET], 1u, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t mask = (1u << bits) - 1u;
+    const int digits = passes << bits, copy = digits + 1;
+    for (int e = t; e < EMIT_COPIES * copy; e += T) lhist[e] = 0u;
+    __syncthreads();
+    const int64_t group = s_group;
+    const int64_t base_k = group * (T * ROUNDS) + t;
+    // tile and block ranges of the thread's particles, and their pair counts
+    uint32_t tx[ROUNDS], ty[ROUNDS], kg[ROUNDS], cnt[ROUNDS], at[ROUNDS];
+    int cb0[ROUNDS], cb1[ROUNDS];
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i) {
+        const int64_t k = base_k + (int64_t)i * T;
+        cnt[i] = 0u;
+        tx[i] = ty[i] = kg[i] = 0u;
+        cb0[i] = cb1[i] = 0;
+        if (k < n) {
+            const mi_particle p = P[k];
+            int tx0, tx1, ty0, ty1;
+            cnt[i] = cells_of(p, g, tx0, tx1, ty0, ty1, cb0[i], cb1[i]);
+            if (cnt[i] > 0u) {  // tile indices below 2^15
+                if (!record_ok(p, g, uw, uw_n)) status[ST_BADREC] = 1u;  // same value from all
+                tx[i] = (uint32_t)tx0 | (uint32_t)tx1 << 16;
+                ty[i] = (uint32_t)ty0 | (uint32_t)ty1 << 16;
+                kg[i] = kernel_group(kind_of(p.r_kind));
             }
         }
     }
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i) {
+        const uint32_t incl = (uint32_t)wave_scan_add((int)cnt[i]);
+        at[i] = incl - cnt[i];
+        if (lane == 63) wsum[i][wave] = incl;
+    }
+    __syncthreads();
+    uint32_t total = 0;
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i)
+#pragma unroll
+        for (int w = 0; w < T / 64; ++w) {
+            if (w == wave) at[i] += total;
+            total += wsum[i][w];
+        }
+    if (t == 0) look_store(&look[group], (group == 0 ? LB_ALL : LB_GROUP) | total);
+    if (wave == 0) {
+        const unsigned long long b = look_back(look, group);
+        if (lane == 0) {
+            s_base = b;
+            if (group > 0) look_store(&look[group], LB_ALL | (b + total));
+            if ((group + 1) * (T * ROUNDS) >= n) {
+                status[ST_PAIRS] = (uint32_t)(b + total);
+                status[ST_OVERFLOW] = b + total > (uint64_t)cap ? 1u : 0u;
+            }
+        }
+    }
+    __syncthreads();
+    const unsigned long long base = s_base;
+    if (base + total > (uint64_t)cap) return;  // uniform
+    uint32_t* mine = lhist + (lane & (EMIT_COPIES - 1)) * copy;
+    auto put = [&](uint32_t x, uint32_t y, uint32_t cb, uint32_t local, uint32_t k, size_t q) {
+        const uint32_t cell = (x * (uint32_t)g.nty + y) * (uint32_t)g.ncb + cb;
+        const uint32_t key = (cell << KEY_LOCAL_BITS) | local;
+        keys[q] = key;
+        vals[q] = k;
+        for (int p = 0; p < passes; ++p)
+            atomicAdd(&mine[(p << bits) + ((key >> (begin + p * bits)) & mask)], 1u);
+    };
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i) {
+        const uint32_t k = (uint32_t)(base_k + (int64_t)i * T);
+        const uint32_t local = (kg[i] << 8) | (mix ? (k * 2654435761u) >> 24 : 0u);
+        if (cnt[i] > 0u && cnt[i] <= EMIT_WIDE) {
+            size_t q = (size_t)base + at[i];
+            for (uint32_t x = tx[i] & 0xffffu; x <= tx[i] >> 16; ++x)
+                for (uint32_t y = ty[i] & 0xffffu; y <= ty[i] >> 16; ++y)
+                    for (int cb = cb0[i]; cb <= cb1[i]; ++cb) put(x, y, (uint32_t)cb, local, k, q++);
+        }
+        uint64_t wide = __ballot(cnt[i] > EMIT_WIDE);
+        while (wide) {
+            const int l = __builtin_ctzll(wide);
+            wide &= wide - 1ull;
+            auto of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); };
+            const uint32_t x0 = of(tx[i]) & 0xffffu, yy = of(ty[i]), y0 = yy & 0xffffu;
+            const uint32_t ny = (yy >> 16) - y0 + 1u, b0 = of((uint32_t)cb0[i]);
+            const uint32_t nb = of((uint32_t)cb1[i]) - b0 + 1u, n_cells = of(cnt[i]);
+            const uint32_t lk = of(k), ll = of(local);
+            const size_t q = (size_t)base + of(at[i]);
+            for (uint32_t e = lane; e < n_cells; e += 64) {
+                const uint32_t xy = e / nb, x = xy / ny;
+                put(x0 + x, y0 + (xy - x * ny), b0 + (e - xy * nb), ll, lk, q + e);
+            }
+        }
+    }
+    __syncthreads();
+    for (int e = t; e < digits; e += T) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (int c = 0; c < EMIT_COPIES; ++c) sum += lhist[c * copy + e];
+        if (sum) atomicAdd(&hist[e], sum);
+    }
 }
 
-// Zeroes the status words and the cell bounds (cells without particles keep
-// start = end = 0).
-__global__ void k_bin_init(uint32_t* __restrict__ status, uint32_t* __restrict__ start,
-                           uint32_t* __restrict__ end, int64_t ncells) {
-    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < 8) status[k] = 0u;
-    if (k < ncells) {
-        start[k] = 0u;
-        end[k] = 0u;
+// Pairs the emit pass produced, zero after an overflow.
+__device__ inline int64_t device_pairs(const uint32_t* __restrict__ status) {
+    return status[ST_OVERFLOW] ? 0 : (int64_t)status[ST_PAIRS];
+}
+
+// One stable radix pass over `bits` key bits from `shift` on.  A tile of
+// T * ITEMS pairs is ranked wave by wave (each wave a contiguous run, 64
+// pairs at a time, lanes of equal digit found by ballots), its digit counts are
+// published, digit d's place in the output is the look-back sum of the earlier
+// tiles' counts of d after all smaller digits (hist), and the tile goes out
+// through LDS in sorted order, so that equal digits are written side by side.
+template <int T, int ITEMS>
+__global__ __launch_bounds__(T) void k_radix(
+    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
+    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
+    const uint32_t* __restrict__ hist, unsigned long long* __restrict__ look,
+    uint32_t* __restrict__ ticket, const uint32_t* __restrict__ status, int shift, int bits) {
+    constexpr int WAVES = T / 64, TILE = T * ITEMS, RADIX = 1 << RADIX_BITS;
+    static_assert(T >= RADIX, "a thread per digit");
+    __shared__ uint32_t whist[WAVES][RADIX];
+    __shared__ uint32_t tbase[RADIX], gbase[RADIX];
+    __shared__ uint32_t wtot[2][WAVES];
+    __shared__ uint32_t skey[TILE], sval[TILE];
+    __shared__ uint32_t s_tile;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (t == 0)
+        s_tile = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int e = t; e < WAVES * RADIX; e += T) (&whist[0][0])[e] = 0u;
+    __syncthreads();
+    const int64_t tile = s_tile, np = device_pairs(status);
+    const int64_t begin = tile * TILE;
+    if (begin >= np) return;  // uniform
+    const int count = (int)min((int64_t)TILE, np - begin);
+    const uint32_t mask = (1u << bits) - 1u;
+
+    uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
+    const int first = wave * 64 * ITEMS + lane;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int e = first + i * 64;
+        key[i] = e < count ? keys[begin + e] : 0xffffffffu;
+        val[i] = e < count ? vals[begin + e] : 0u;
     }
+    volatile uint32_t* mine = whist[wave];  // read and written by this wave only, in order
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t d = (key[i] >> shift) & mask;
+        uint64_t peers = __ballot(first + i * 64 < count);
+        for (int b = 0; b < bits; ++b) {  // uniform
+            const bool one = (d >> b) & 1u;
+            const uint64_t m = __ballot(one);
+            peers &= one ? m : ~m;
+        }
+        const uint32_t before = (uint32_t)__builtin_popcountll(peers & ((1ull << lane) - 1ull));
+        const uint32_t old = mine[d];
+        rank[i] = old + before;
+        if (first + i * 64 < count && before == 0u)
+            mine[d] = old + (uint32_t)__builtin_popcountll(peers);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // thread d: this tile's count of digit d; the waves' offsets within it
+    uint32_t mycount = 0;
+    if (t < RADIX) {
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const uint32_t c = whist[w][t];
+            whist[w][t] = mycount;
+            mycount += c;
+        }
+    }
+    const int radix = 1 << bits;
+    unsigned long long* word = look + (tile << bits) + t;
+    if (t < radix) look_store(word, (tile == 0 ? LB_ALL : LB_GROUP) | mycount);
+    // exclusive scans over the digits: of the tile's counts and of all counts
+    const uint32_t all = t < radix ? hist[t] : 0u;
+    const uint32_t i0 = (uint32_t)wave_scan_add((int)mycount), i1 = (uint32_t)wave_scan_add((int)all);
+    if (lane == 63) {
+        wtot[0][wave] = i0;
+        wtot[1][wave] = i1;
+    }
+    __syncthreads();
+    uint32_t tb = i0 - mycount, gb = i1 - all;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+        if (w < wave) {
+            tb += wtot[0][w];
+            gb += wtot[1][w];
+        }
+    if (t < radix) {
+        // four earlier tiles at a time, nearest first
+        unsigned long long before = 0;
+        int64_t j = 1;
+        for (bool done = tile == 0; !done;) {
+            unsigned long long v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                v[i] = j + i <= tile ? look_load(word - ((j + i) << bits)) : LB_ALL;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (done || (v[i] & LB_STATE) == 0ull) break;  // not published yet: read again
+                before += v[i] & ~LB_STATE;
+                done = (v[i] & LB_STATE) == LB_ALL;
+                ++j;
+            }
+        }
+        if (tile > 0) look_store(word, LB_ALL | (before + mycount));
+        tbase[t] = tb;
+        gbase[t] = gb + (uint32_t)before - tb;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (first + i * 64 >= count) continue;
+        const uint32_t d = (key[i] >> shift) & mask;
+        const uint32_t at = tbase[d] + whist[wave][d] + rank[i];
+        skey[at] = key[i];
+        sval[at] = val[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int e = t + i * T;
+        if (e >= count) continue;
+        const uint32_t k = skey[e];
+        const size_t o = (size_t)(uint32_t)(gbase[(k >> shift) & mask] + (uint32_t)e);
+        keys_out[o] = k;
+        vals_out[o] = sval[e];
+    }
+}
+
+// Clears the status words, histograms, cell bounds (cells without particles
+// keep start = end = 0) and look-back words: `words` 16-byte words.
+__global__ void k_bin_init(uint4* __restrict__ at, int64_t words) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < words; k += stride)
+        at[k] = make_uint4(0u, 0u, 0u, 0u);
 }
 
 // Cell bounds from the sorted keys: thread t takes keys 4t .. 4t + 3 (one
 // 16-byte load when the run lies inside the array, the workspace keys being
 // 256-byte aligned) and the key on either side.
-__global__ void k_cell_bounds(const uint32_t* __restrict__ keys, int64_t np, int64_t ncells,
+__global__ void k_cell_bounds(const uint32_t* __restrict__ keys,
+                              const uint32_t* __restrict__ status, int64_t ncells,
                               uint32_t* __restrict__ start, uint32_t* __restrict__ end) {
+    const int64_t np = device_pairs(status);
     const int64_t q0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (q0 >= np) return;
     uint32_t c[6];  // cells of keys q0 - 1 .. q0 + 4 (0xffffffff outside the array)
@@ -306,101 +520,140 @@ __global__ void k_cell_bounds(const uint32_t* __restrict__ keys, int64_t np, int
     c[5] = q0 + 4 < np ? keys[q0 + 4] >> KEY_LOCAL_BITS : 0xffffffffu;
 #pragma unroll
     for (int i = 1; i <= 4; ++i) {
-        if ((int64_t)c[i] >= ncells) continue;  // padding (and past the end)
+        if ((int64_t)c[i] >= ncells) continue;  // past the end
         if (c[i] != c[i - 1]) start[c[i]] = (uint32_t)(q0 + i - 1);
         if (c[i] != c[i + 1]) end[c[i]] = (uint32_t)(q0 + i);
     }
 }
 
-// Work items per cell (ceil(len / item_len), none after an overflow) and
-// their exclusive scans, in one work group: thread t takes a contiguous run of
-// cells, the run totals are scanned in LDS, and the offsets written.
-// item_off[ncells] and multi_off[ncells] hold the totals (also status words).
+// Work items per cell (ceil(len / item_len), none after an overflow), in one
+// work group: thread t takes a contiguous run of cells, the run totals are
+// scanned, and the offsets written.  item_off[ncells] and multi_off[ncells]
+// hold the totals (also status words).
+//
+// The items are stored in their launch order, longest first: the gathers' work
+// groups, dispatched in order, then take the long items early and the short
+// ones fill the tail.  All items of item_len particles come first, in cell order
+// (full_pos: the first of each cell); then the cells' remainders, in buckets of
+// 32 particles by falling length (rest_pos).  Only the schedule depends on it:
+// every cell still sums its items in item order (their partial-tile slots), so
+// the cube is bitwise the same in any launch order, and the order within a
+// bucket may be left to the LDS atomics.
+constexpr int SCAN_T = 1024;
+constexpr int REST_BUCKETS = ITEM_MAX / 32;
+constexpr int64_t ITEMS_IN_PLACE = 128;  // cells up to which k_items writes the items itself
 
-__global__ __launch_bounds__(SCAN_T) void k_item_scan(const uint32_t* __restrict__ start,
-                                                      const uint32_t* __restrict__ end,
-                                                      int64_t ncells, int item_len,
-                                                      uint32_t* __restrict__ status,
-                                                      uint32_t* __restrict__ item_off,
-                                                      uint32_t* __restrict__ multi_off) {
-    __shared__ uint32_t si[SCAN_T], sm[SCAN_T];
-    const int t = threadIdx.x;
-    const int64_t per = (ncells + SCAN_T - 1) / SCAN_T;
-    const int64_t c0 = min((int64_t)t * per, ncells), c1 = min(c0 + per, ncells);
-    const bool overflow = status[ST_OVERFLOW] != 0u || status[ST_BADREC] != 0u;
-    const uint32_t L = (uint32_t)item_len;
-    auto items_of = [&](int64_t c) {
-        const uint32_t s0 = start[c], e0 = end[c];
-        return (overflow || e0 <= s0) ? 0u : (e0 - s0 + L - 1) / L;
-    };
-    uint32_t ai = 0, am = 0;
-    for (int64_t c = c0; c < c1; ++c) {
-        const uint32_t ni = items_of(c);
-        ai += ni;
-        am += ni > 1 ? ni : 0u;
-    }
-    si[t] = ai;
-    sm[t] = am;
-    __syncthreads();
-    for (int d = 1; d < SCAN_T; d <<= 1) {  // inclusive scan of the run totals
-        const uint32_t vi = t >= d ? si[t - d] : 0u, vm = t >= d ? sm[t - d] : 0u;
-        __syncthreads();
-        si[t] += vi;
-        sm[t] += vm;
-        __syncthreads();
-    }
-    uint32_t bi = si[t] - ai, bm = sm[t] - am;
-    for (int64_t c = c0; c < c1; ++c) {
-        const uint32_t ni = items_of(c);
-        item_off[c] = bi;
-        multi_off[c] = bm;
-        bi += ni;
-        bm += ni > 1 ? ni : 0u;
-    }
-    if (t == SCAN_T - 1) {
-        item_off[ncells] = si[t];
-        multi_off[ncells] = sm[t];
-        status[ST_ITEMS] = si[t];
-        status[ST_MULTI] = sm[t];
-    }
+struct CellItems {
+    uint32_t full, rest, all, multi;
+};
+
+__device__ inline CellItems cell_items(uint32_t len, uint32_t L) {
+    CellItems c;
+    c.full = len / L;
+    c.rest = len - c.full * L;
+    c.all = c.full + (c.rest ? 1u : 0u);
+    c.multi = c.all > 1u ? c.all : 0u;
+    return c;
 }
 
-// One work group per cell writes the cell's items; a cell cut into several
-// items gives each a partial-tile slot.
-__global__ __launch_bounds__(64) void k_build_items(const uint32_t* __restrict__ start,
-                                                    const uint32_t* __restrict__ end,
-                                                    int item_len,
-                                                    const uint32_t* __restrict__ item_off,
-                                                    const uint32_t* __restrict__ multi_off,
-                                                    Item* __restrict__ items) {
-    const uint32_t c = blockIdx.x;
-    const uint32_t base = item_off[c], ni = item_off[c + 1] - base;
-    if (ni == 0u) return;
-    const uint32_t s0 = start[c], e0 = end[c], L = (uint32_t)item_len;
-    for (uint32_t q = threadIdx.x; q < ni; q += blockDim.x) {
+// Writes cell c's items with the lanes of one wave.
+__device__ inline void write_items(uint32_t c, uint32_t s0, uint32_t e0, uint32_t L, uint32_t slot,
+                                   uint32_t full_at, uint32_t rest_at, Item* __restrict__ items) {
+    const CellItems n = cell_items(e0 - s0, L);
+    for (uint32_t q = threadIdx.x & 63; q < n.all; q += 64) {
         Item it;
         it.cell = (int32_t)c;
         it.begin = (int32_t)(s0 + q * L);
         it.end = (int32_t)min(e0, s0 + (q + 1) * L);
-        it.slot = ni > 1 ? (int32_t)(multi_off[c] + q) : -1;
-        items[base + q] = it;
+        it.slot = n.all > 1u ? (int32_t)(slot + q) : -1;
+        items[q < n.full ? full_at + q : rest_at] = it;
     }
 }
 
-// Launch order of the work items: longest first (ties in cell order), so that
-// the gathers' work groups, dispatched in order, take the long items early and
-// the short ones fill the tail.  The key is ITEM_MAX_LEN - length; slots past
-// the item count sort last.  Only the schedule changes: every cell still sums
-// its items in item order, so the cube is bitwise the same in any order.
-__global__ void k_item_keys(const Item* __restrict__ items, const uint32_t* __restrict__ status,
-                            int64_t items_max, uint32_t* __restrict__ keys,
-                            uint32_t* __restrict__ idx) {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= items_max) return;
-    const uint32_t n_items = status[ST_ITEMS];
-    keys[j] = (uint32_t)j < n_items ? (uint32_t)(ITEM_MAX - (items[j].end - items[j].begin))
-                                    : (1u << (ITEM_KEY_BITS - 1));
-    idx[j] = (uint32_t)j;
+__global__ __launch_bounds__(SCAN_T) void k_items(
+    const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, int64_t ncells,
+    int item_len, uint32_t* __restrict__ status, uint32_t* __restrict__ item_off,
+    uint32_t* __restrict__ multi_off, uint32_t* __restrict__ full_pos,
+    uint32_t* __restrict__ rest_pos, Item* __restrict__ items) {
+    constexpr int WAVES = SCAN_T / 64;
+    __shared__ uint32_t wtot[3][WAVES];
+    __shared__ uint32_t bucket[REST_BUCKETS];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t per = (ncells + SCAN_T - 1) / SCAN_T;
+    const int64_t c0 = min((int64_t)t * per, ncells), c1 = min(c0 + per, ncells);
+    const bool none = status[ST_OVERFLOW] != 0u || status[ST_BADREC] != 0u;
+    const uint32_t L = (uint32_t)item_len;
+    if (t < REST_BUCKETS) bucket[t] = 0u;
+    __syncthreads();
+    auto of = [&](int64_t c) { return cell_items(none ? 0u : end[c] - start[c], L); };
+    auto bucket_of = [](uint32_t rest) { return (uint32_t)REST_BUCKETS - 1u - (rest - 1u) / 32u; };
+    uint32_t sum[3] = {0u, 0u, 0u};  // items, partial tiles, full items
+    for (int64_t c = c0; c < c1; ++c) {
+        const CellItems n = of(c);
+        sum[0] += n.all;
+        sum[1] += n.multi;
+        sum[2] += n.full;
+        if (n.rest) atomicAdd(&bucket[bucket_of(n.rest)], 1u);
+    }
+    uint32_t at[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const uint32_t incl = (uint32_t)wave_scan_add((int)sum[k]);
+        at[k] = incl - sum[k];
+        if (lane == 63) wtot[k][wave] = incl;
+    }
+    __syncthreads();
+    uint32_t total[3] = {0u, 0u, 0u};
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            if (w == wave) at[k] += total[k];
+            total[k] += wtot[k][w];
+        }
+    if (wave == 0) {  // the buckets' first positions, after the full items
+        uint32_t run = total[2];
+#pragma unroll
+        for (int b = 0; b < REST_BUCKETS; b += 64) {
+            const uint32_t v = bucket[b + lane], incl = (uint32_t)wave_scan_add((int)v);
+            bucket[b + lane] = run + incl - v;
+            run += __builtin_amdgcn_readlane(incl, 63);
+        }
+    }
+    if (t == 0) {
+        item_off[ncells] = total[0];
+        multi_off[ncells] = total[1];
+        status[ST_ITEMS] = total[0];
+        status[ST_MULTI] = total[1];
+    }
+    __syncthreads();
+    for (int64_t c = c0; c < c1; ++c) {
+        const CellItems n = of(c);
+        item_off[c] = at[0];
+        multi_off[c] = at[1];
+        full_pos[c] = at[2];
+        rest_pos[c] = n.rest ? atomicAdd(&bucket[bucket_of(n.rest)], 1u) : 0u;
+        at[0] += n.all;
+        at[1] += n.multi;
+        at[2] += n.full;
+    }
+    if (ncells > ITEMS_IN_PLACE || none) return;  // uniform
+    __syncthreads();  // the positions above, read back from this work group's own writes
+    for (int64_t c = wave; c < ncells; c += WAVES)
+        write_items((uint32_t)c, start[c], end[c], L, multi_off[c], full_pos[c], rest_pos[c], items);
+}
+
+// One wave per cell writes the cell's items (cubes of more cells than k_items
+// handles by itself).
+__global__ __launch_bounds__(64) void k_build_items(
+    const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, int item_len,
+    const uint32_t* __restrict__ status, const uint32_t* __restrict__ multi_off,
+    const uint32_t* __restrict__ full_pos, const uint32_t* __restrict__ rest_pos,
+    Item* __restrict__ items) {
+    if (status[ST_OVERFLOW] != 0u || status[ST_BADREC] != 0u) return;
+    const uint32_t c = blockIdx.x;
+    write_items(c, start[c], end[c], (uint32_t)item_len, multi_off[c], full_pos[c], rest_pos[c],
+                items);
 }
 
 static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
@@ -408,61 +661,67 @@ static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t -
 hipError_t bin_particles(const mi_particle* d_p, int64_t n, int64_t n_pairs, const Grid& g,
                          const mi_cube_desc& d, char* ws, const Layout& L, bool record_order,
                          hipStream_t s) {
-    uint32_t* counts = (uint32_t*)(ws + L.counts);
-    uint32_t* offsets = (uint32_t*)(ws + L.offsets);
-    uint32_t* keys = (uint32_t*)(ws + L.keys);
-    uint32_t* vals = (uint32_t*)(ws + L.vals);
-    uint32_t* keys2 = (uint32_t*)(ws + L.keys2);
-    uint32_t* vals2 = (uint32_t*)(ws + L.vals2);
-    uint32_t* cstart = (uint32_t*)(ws + L.cell_start);
-    uint32_t* cend = (uint32_t*)(ws + L.cell_end);
-    uint32_t* ioff = (uint32_t*)(ws + L.item_off);
-    uint32_t* moff = (uint32_t*)(ws + L.multi_off);
-    Item* items = (Item*)(ws + L.items);
-    uint32_t* status = (uint32_t*)(ws + L.status);
-    void* temp = ws + L.temp;
-    size_t tb = L.temp_bytes;
+    auto words = [&](size_t at) { return (uint32_t*)(ws + at); };
+    uint32_t* status = words(L.status);
+    uint32_t* hist = words(L.hist);
+    auto* emit_look = (unsigned long long*)(ws + L.emit_look);
+    auto* radix_look = (unsigned long long*)(ws + L.radix_look);
     const int T = 256;
 
-    hipLaunchKernelGGL(k_bin_init, dim3(blocks_for(g.ncells > 8 ? g.ncells : 8, T)), dim3(T), 0, s,
-                       status, cstart, cend, g.ncells);
-    const int64_t nb = emit_blocks(n);
-    if (nb > 0)
-        hipLaunchKernelGGL(k_count, dim3((unsigned)nb), dim3(EMIT_T), 0, s, d_p, n, g, d.weights,
-                           d.weights_n, counts, status);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(SCAN_T), 0, s, counts, nb, offsets);
-    // the emit grid: one block per particle block, at least enough threads
-    // (up to 2^24) to fill any padding entries in a few strides
-    int64_t eb = nb;
-    const int64_t pad_blocks = (n_pairs + EMIT_T - 1) / EMIT_T;
-    if (eb < pad_blocks) eb = pad_blocks < 65536 ? pad_blocks : 65536;
-    if (eb < 1) eb = 1;
-    hipLaunchKernelGGL(k_emit, dim3((unsigned)eb), dim3(EMIT_T), 0, s, d_p, n, n_pairs, g, offsets,
-                       keys, vals, status, record_order ? 0 : 1);
-    if (n_pairs > 0) {
-        // In record order only the cell and the kernel group are sorted (two
-        // radix passes up to 2^14 cells); the stable sort keeps the rest.
-        const int begin_bit = record_order ? KEY_LOCAL_BITS - 2 : coarse_begin_bit(g);
-        hipError_t e = rocprim::radix_sort_pairs(temp, tb, keys, keys2, vals, vals2,
-                                                 (size_t)n_pairs, begin_bit,
-                                                 g.cell_bits + KEY_LOCAL_BITS, s);
-        if (e != hipSuccess) return e;
+    const int64_t clear = (int64_t)(L.cleared - L.status) / 16;
+    hipLaunchKernelGGL(k_bin_init, dim3((unsigned)std::min<int64_t>((clear + T - 1) / T, 2048)),
+                       dim3(T), 0, s, (uint4*)(ws + L.status), clear);
+    const RadixPlan r = radix_plan(g, record_order);
+    // the last pass ends in keys2 / vals2
+    uint32_t *k0 = words(L.keys), *v0 = words(L.vals), *k1 = words(L.keys2), *v1 = words(L.vals2);
+    if (r.passes % 2 == 0) {
+        std::swap(k0, k1);
+        std::swap(v0, v1);
+    }
+    const int64_t groups = emit_groups(n);
+    const GroupShape shape = emit_shape(n);
+    if (groups > 0) {
+        auto emit = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3((unsigned)shape.threads),
+                               sizeof(uint32_t) * EMIT_COPIES * ((r.passes << r.bits) + 1), s, d_p, n, n_pairs,
+                               g, d.weights, d.weights_n, emit_look, k0, v0, hist, status,
+                               record_order ? 0 : 1, r.begin, r.passes, r.bits);
+        };
+        if (same(shape, EMIT_SMALL))
+            emit(k_emit<EMIT_SMALL.threads, EMIT_SMALL.items>);
+        else if (same(shape, EMIT_MID))
+            emit(k_emit<EMIT_MID.threads, EMIT_MID.items>);
+        else
+            emit(k_emit<EMIT_LARGE.threads, EMIT_LARGE.items>);
+    }
+    const int64_t tiles = radix_tiles(n_pairs);
+    const GroupShape rs = radix_shape(n_pairs);
+    for (int p = 0; p < r.passes && tiles > 0; ++p) {
+        auto pass = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3((unsigned)rs.threads), 0, s, k0, v0, k1, v1,
+                               hist + (p << r.bits), radix_look + ((p * tiles) << r.bits),
+                               status + ST_TICKET + 1 + p, status, r.begin + p * r.bits, r.bits);
+        };
+        if (same(rs, RADIX_TILE_SMALL))
+            pass(k_radix<RADIX_TILE_SMALL.threads, RADIX_TILE_SMALL.items>);
+        else if (same(rs, RADIX_TILE_MID))
+            pass(k_radix<RADIX_TILE_MID.threads, RADIX_TILE_MID.items>);
+        else
+            pass(k_radix<RADIX_TILE_LARGE.threads, RADIX_TILE_LARGE.items>);
+        std::swap(k0, k1);
+        std::swap(v0, v1);
     }
     if (n_pairs > 0)
         hipLaunchKernelGGL(k_cell_bounds, dim3(blocks_for((n_pairs + 3) / 4, T)), dim3(T), 0, s,
-                           keys2, n_pairs, g.ncells, cstart, cend);
-    hipLaunchKernelGGL(k_item_scan, dim3(1), dim3(SCAN_T), 0, s, cstart, cend, g.ncells,
-                       L.item_len, status, ioff, moff);
-    hipLaunchKernelGGL(k_build_items, dim3((unsigned)g.ncells), dim3(64), 0, s, cstart, cend,
-                       L.item_len, ioff, moff, items);
-    uint32_t* ikeys = (uint32_t*)(ws + L.item_keys);
-    uint32_t* iidx = (uint32_t*)(ws + L.item_idx);
-    hipLaunchKernelGGL(k_item_keys, dim3(blocks_for(L.items_max, T)), dim3(T), 0, s, items, status,
-                       L.items_max, ikeys, iidx);
-    hipError_t e = rocprim::radix_sort_pairs(temp, tb, ikeys, (uint32_t*)(ws + L.item_keys2), iidx,
-                                             (uint32_t*)(ws + L.item_order), (size_t)L.items_max,
-                                             0, ITEM_KEY_BITS, s);
-    if (e != hipSuccess) return e;
+                           words(L.keys2), status, g.ncells, words(L.cell_start), words(L.cell_end));
+    hipLaunchKernelGGL(k_items, dim3(1), dim3(SCAN_T), 0, s, words(L.cell_start), words(L.cell_end),
+                       g.ncells, L.item_len, status, words(L.item_off), words(L.multi_off),
+                       words(L.full_pos), words(L.rest_pos), (Item*)(ws + L.items));
+    if (g.ncells > ITEMS_IN_PLACE)
+        hipLaunchKernelGGL(k_build_items, dim3((unsigned)g.ncells), dim3(64), 0, s,
+                           words(L.cell_start), words(L.cell_end), L.item_len, status,
+                           words(L.multi_off), words(L.full_pos), words(L.rest_pos),
+                           (Item*)(ws + L.items));
     return hipGetLastError();
 }
 

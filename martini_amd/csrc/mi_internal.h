@@ -42,19 +42,19 @@ __host__ __device__ inline uint32_t cells_of(const mi_particle& p, const Grid& g
 
 // Byte offsets of the workspace regions (each 256-byte aligned).
 struct Layout {
-    size_t counts, offsets;            // uint32[emit blocks + 2] each: block totals, bases
-    size_t keys, vals, keys2, vals2;   // uint32[n_pairs] each; vals2: particle index in cell order
+    // cleared at the start of every binning (status .. cleared)
+    size_t status;                     // uint32[ST_WORDS]
+    size_t hist;                       // uint32: digit counts of every radix pass
     size_t cell_start, cell_end;       // uint32[ncells] each
+    size_t emit_look, radix_look;      // uint64: look-back words of the emit groups and radix tiles
+    size_t cleared;                    // end of the region
+    size_t keys, vals, keys2, vals2;   // uint32[n_pairs] each; vals2: particle index in cell order
     size_t item_off, multi_off;        // uint32[ncells + 1] each: exclusive scans of the
                                        // items and the partial-tile slots per cell
-    size_t items;                      // int4[items_max], in cell order
-    size_t item_keys, item_keys2;      // uint32[items_max]: sort keys of the launch order
-    size_t item_idx, item_order;       // uint32[items_max]: item index; launch order
+    size_t full_pos, rest_pos;         // uint32[ncells] each: launch positions of a cell's items
+    size_t items;                      // int4[items_max], in launch order
     size_t partials;                   // float[multi_max * CELL_VOXELS]
     size_t part_masks;                 // uint64[multi_max]: the sub-tiles each partial holds
-    size_t status;                     // uint32[8]
-    size_t temp;                       // rocPRIM temporary storage
-    size_t temp_bytes;
     size_t total;
     int64_t items_max, multi_max;
     int item_len;                      // particles per work item
@@ -63,7 +63,9 @@ struct Layout {
 // status[0]: number of pairs the device produced; status[1]: overflow flag.
 // status[4]: a record with a footprint has an unknown kernel kind or table
 // weights beyond the descriptor's table (no work items are then made).
-enum { ST_PAIRS = 0, ST_OVERFLOW = 1, ST_ITEMS = 2, ST_MULTI = 3, ST_BADREC = 4 };
+// ST_TICKET on: group tickets of the emit pass and of each radix pass.
+enum { ST_PAIRS = 0, ST_OVERFLOW = 1, ST_ITEMS = 2, ST_MULTI = 3, ST_BADREC = 4, ST_TICKET = 8,
+       ST_WORDS = 16 };
 
 hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L);
 
