@@ -73,15 +73,25 @@ static_assert(GeoSquare::TY == TILE_Y && GeoWide::TY == TILE_Y, "one row length"
 __host__ __device__ inline bool wide_cells(int nc) { return nc >= 128; }
 // Particles per cell processed by one work item: longer cells are split and
 // their partial tiles summed in item order by a reduction pass.  The split
-// length depends only on the pair count (about ITEM_TARGET items, between
-// ITEM_MIN and ITEM_MAX particles each), so a given input always sums in the
-// same order.
-constexpr int ITEM_MIN = 256;
+// length depends only on the pair count, so a given input always sums in the
+// same order: about ITEM_TARGET items of at most ITEM_MAX particles, which
+// balances the CUs; below ITEM_WHOLE particles per item, instead, as many items
+// as run at once (ITEM_FILL: three work groups on each of 256 CUs) and no more,
+// since each split costs a partial tile.  13000 pairs, FP32, in items of 256
+// (52 of them): 159 us per insertion, of 32: 107; 1.7e5 pairs, MFMA: 154 us in
+// 768 items, 167 in 2048.  The partial tiles of ITEM_FILL items take at most
+// 101 MB of workspace, the cells of the largest grid beside them 84 MB.
+constexpr int ITEM_MIN = 32;
+constexpr int ITEM_WHOLE = 256;
 constexpr int ITEM_MAX = 4096;
 constexpr int ITEM_TARGET = 2048;
+constexpr int ITEM_FILL = 768;
+
 __host__ __device__ inline int item_length(int64_t n_pairs) {
-    int64_t len = (n_pairs / ITEM_TARGET + 31) / 32 * 32;
-    return (int)(len < ITEM_MIN ? ITEM_MIN : (len > ITEM_MAX ? ITEM_MAX : len));
+    const int64_t balanced = (n_pairs / ITEM_TARGET + 31) / 32 * 32;
+    if (balanced >= ITEM_WHOLE) return (int)(balanced > ITEM_MAX ? ITEM_MAX : balanced);
+    const int64_t filled = (n_pairs / ITEM_FILL + 31) / 32 * 32;
+    return (int)(filled < ITEM_MIN ? ITEM_MIN : (filled > ITEM_WHOLE ? ITEM_WHOLE : filled));
 }
 // Key layout: cell << KEY_LOCAL_BITS | kernel group << 8 | 8-bit local order
 // (zero, keeping the record order, or a hash of the particle index).
