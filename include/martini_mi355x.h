@@ -71,7 +71,7 @@ extern "C" {
 #define MI_SPECTRUM_TABLE 2  /* spectra evaluated by the caller, read from a device table */
 
 /* Insertion methods. */
-#define MI_METHOD_PLAIN_F32 0   /* FP32 VALU tile gather */
+#define MI_METHOD_PLAIN_F32 0   /* FP32 products (matrix cores, FP32 operands and sums) */
 #define MI_METHOD_MFMA_BF16X3 1 /* BF16 split-precision MFMA contraction */
 
 /*
@@ -184,12 +184,9 @@ int mi_insert_noalloc(const mi_particle* d_particles, int64_t n, int64_t n_pairs
  * callers that time or overlap them.  mi_bin sorts the particles into cells
  * inside the workspace; mi_gather then evaluates the contraction over those
  * cells with `method` and adds it to d_cube.  mi_bin's `method` names the
- * gather it prepares for: the MFMA form gets each cell's particles in record
- * order (records laid out by tile and pixel Z order make its 32-particle
- * chunks compact, and its skips are per chunk), the FP32 form an order by a
- * hash of the particle index (each chunk then spreads over the tile, which
- * balances its products over the waves).  Either order gives a correct gather
- * with either method.  The workspace must not be reused between the
+ * gather that follows; both take the same order, each cell's particles by
+ * kernel family and tile row (their 32-particle chunks are then compact, and
+ * products are skipped by tile row), and in record order within.  The workspace must not be reused between the
  * two calls.  Overflow of n_pairs is reported by mi_status (which
  * synchronises the stream); a gather after an overflowed bin leaves the cube
  * untouched.

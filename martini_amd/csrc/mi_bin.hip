@@ -3,11 +3,8 @@
 // Replaces the reference's per-pixel O(N) square mask
 // (martini/martini.py:271-274): every particle is listed once in each cell
 // its footprint and channel window touch, and the list is sorted by
-// (cell, kernel group, local order) with a stable radix sort, so that each
-// cell's particles form one contiguous, deterministic segment.  The MFMA form
-// keeps the record order within a cell (its records are laid out by tile and
-// pixel Z order, so its chunks are spatially compact); the FP32 form orders
-// by a hash of the particle index (chunks spread over the tile).
+// (cell, kernel group, tile row) with a stable radix sort, so that each cell's
+// particles form one contiguous, deterministic segment, spatially compact.
 // Long segments are cut into work items of at most item_length() particles;
 // such cells get one partial tile per item.
 //
@@ -84,6 +81,7 @@ constexpr GroupShape RADIX_TILE_SMALL{256, 4}, RADIX_TILE_MID{1024, 4}, RADIX_TI
 constexpr int64_t RADIX_MID = 131072, RADIX_LARGE = 1 << 20;
 constexpr int RADIX_BITS = 8;  // at most, per pass
 constexpr int RADIX_PASSES = (32 + RADIX_BITS - 1) / RADIX_BITS;
+constexpr int LOCAL_ROW_BITS = 4;  // of the local order, enough for a 16-row tile's row
 
 static GroupShape radix_shape(int64_t n_pairs) {
     return n_pairs >= RADIX_LARGE ? RADIX_TILE_LARGE
@@ -95,25 +93,18 @@ static int64_t radix_tiles(int64_t n_pairs) {
     return (n_pairs + tile - 1) / tile;
 }
 
-// Lowest key bit the coarse sort orders on: the top 16 bits of the key
-// (cell, kernel group and the high bits of the index hash) fit two 8-bit radix
-// passes.  Within equal sorted bits the stable sort keeps emit order.
-static int coarse_begin_bit(const Grid& g) {
-    const int b = g.cell_bits + KEY_LOCAL_BITS - 16;
-    return b < 0 ? 0 : (b > 8 ? 8 : b);
-}
-
-// The passes over the sorted bits: as few as RADIX_BITS allows, of equal width.
-// In record order only the cell and the kernel group are sorted (two passes up
-// to 2^14 cells); the stable sort keeps the rest.
+// The passes over the sorted bits, which are the cell and the kernel group and,
+// as far as the passes that these take have bits left, the top of the local
+// order; the stable sort keeps the record order in the rest.
 struct RadixPlan {
     int begin, passes, bits;
 };
-static RadixPlan radix_plan(const Grid& g, bool record_order) {
+static RadixPlan radix_plan(const Grid& g) {
     RadixPlan r;
-    r.begin = record_order ? KEY_LOCAL_BITS - 2 : coarse_begin_bit(g);
-    const int width = g.cell_bits + KEY_LOCAL_BITS - r.begin;
-    r.passes = (width + RADIX_BITS - 1) / RADIX_BITS;
+    const int need = g.cell_bits + KEY_LOCAL_BITS - 8;
+    r.passes = (need + RADIX_BITS - 1) / RADIX_BITS;
+    const int width = std::min(r.passes * RADIX_BITS, need + LOCAL_ROW_BITS);
+    r.begin = g.cell_bits + KEY_LOCAL_BITS - width;
     r.bits = (width + r.passes - 1) / r.passes;
     return r;
 }
@@ -138,13 +129,9 @@ hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L) {
     L->cell_start = take(4 * nc);
     L->cell_end = take(4 * nc);
     L->emit_look = take(sizeof(unsigned long long) * (size_t)emit_groups(n));
-    size_t look = 0;
-    for (int order = 0; order < 2; ++order) {  // either gather's sort fits
-        const RadixPlan r = radix_plan(g, order != 0);
-        const size_t words = ((size_t)r.passes * (size_t)radix_tiles(n_pairs)) << r.bits;
-        look = words > look ? words : look;
-    }
-    L->radix_look = take(sizeof(unsigned long long) * look);
+    const RadixPlan r = radix_plan(g);
+    L->radix_look = take(sizeof(unsigned long long) *
+                         (((size_t)r.passes * (size_t)radix_tiles(n_pairs)) << r.bits));
     L->cleared = off;
     L->keys = take(4 * np);
     L->vals = take(4 * np);
@@ -231,12 +218,10 @@ __device__ inline unsigned long long look_back(const unsigned long long* look, i
 // written by its whole wave.  The digits of every radix pass are counted too
 // (hist), in EMIT_COPIES copies in LDS, a lane in eight to each: neighbouring
 // records share their cells, and adds to one address wait for each other.
-// With `mix` the low 8 key bits are a hash of the particle index:
-// the FP32 gather's waves each own 4 tile rows, and a chunk of particles drawn
-// from all over the tile gives them even shares of the products, where a
-// spatially compact chunk loads one or two of them.  Without it they are zero
-// and a cell's pairs keep the record order (the MFMA form, whose records are
-// laid out in tile and pixel Z order).  A total above the capacity raises the
+// The low 8 key bits are the particle's tile row (LOCAL_ROW_BITS) and column in
+// the cell, clamped to the tile: particles of one row side by side make the
+// gather's 32-particle chunks compact, and its products are skipped by tile row.
+// A total above the capacity raises the
 // overflow flag; nothing is written past the capacity, and the passes that
 // follow do nothing.
 constexpr uint32_t EMIT_WIDE = 8;
@@ -247,7 +232,7 @@ __global__ __launch_bounds__(T) void k_emit(
     const mi_particle* __restrict__ P, int64_t n, int64_t cap, Grid g,
     const float* __restrict__ uw, int64_t uw_n, unsigned long long* __restrict__ look,
     uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, uint32_t* __restrict__ hist,
-    uint32_t* __restrict__ status, int mix, int begin, int passes, int bits) {
+    uint32_t* __restrict__ status, int begin, int passes, int bits) {
     __shared__ uint32_t wsum[ROUNDS][T / 64];
     extern __shared__ uint32_t lhist[];  // EMIT_COPIES x ((passes << bits) + 1)
     __shared__ uint32_t s_group;
@@ -264,13 +249,13 @@ __global__ __launch_bounds__(T) void k_emit(
     const int64_t base_k = group * (T * ROUNDS) + t;
     // tile and block ranges of the thread's particles, and their pair counts
     uint32_t tx[ROUNDS], ty[ROUNDS], kg[ROUNDS], cnt[ROUNDS], at[ROUNDS];
-    int cb0[ROUNDS], cb1[ROUNDS];
+    int cb0[ROUNDS], cb1[ROUNDS], px[ROUNDS], py[ROUNDS];
 #pragma unroll
     for (int i = 0; i < ROUNDS; ++i) {
         const int64_t k = base_k + (int64_t)i * T;
         cnt[i] = 0u;
         tx[i] = ty[i] = kg[i] = 0u;
-        cb0[i] = cb1[i] = 0;
+        cb0[i] = cb1[i] = px[i] = py[i] = 0;
         if (k < n) {
             const mi_particle p = P[k];
             int tx0, tx1, ty0, ty1;
@@ -280,6 +265,8 @@ __global__ __launch_bounds__(T) void k_emit(
                 tx[i] = (uint32_t)tx0 | (uint32_t)tx1 << 16;
                 ty[i] = (uint32_t)ty0 | (uint32_t)ty1 << 16;
                 kg[i] = kernel_group(kind_of(p.r_kind));
+                px[i] = p.ix;
+                py[i] = p.iy;
             }
         }
     }
@@ -314,9 +301,14 @@ __global__ __launch_bounds__(T) void k_emit(
     const unsigned long long base = s_base;
     if (base + total > (uint64_t)cap) return;  // uniform
     uint32_t* mine = lhist + (lane & (EMIT_COPIES - 1)) * copy;
-    auto put = [&](uint32_t x, uint32_t y, uint32_t cb, uint32_t local, uint32_t k, size_t q) {
+    auto put = [&](uint32_t x, uint32_t y, uint32_t cb, uint32_t kind, int ix, int iy, uint32_t k,
+                   size_t q) {
         const uint32_t cell = (x * (uint32_t)g.nty + y) * (uint32_t)g.ncb + cb;
-        const uint32_t key = (cell << KEY_LOCAL_BITS) | local;
+        const int row = min(max(ix - (int)(x << g.tx_shift), 0), (1 << g.tx_shift) - 1);
+        const int col = min(max(iy - (int)(y << g.ty_shift), 0), TILE_Y - 1);
+        const uint32_t key = (cell << KEY_LOCAL_BITS) | (kind << 8) |
+                             ((uint32_t)row << (8 - g.tx_shift)) |
+                             ((uint32_t)col << (4 - g.tx_shift));
         keys[q] = key;
         vals[q] = k;
         for (int p = 0; p < passes; ++p)
@@ -325,12 +317,12 @@ __global__ __launch_bounds__(T) void k_emit(
 #pragma unroll
     for (int i = 0; i < ROUNDS; ++i) {
         const uint32_t k = (uint32_t)(base_k + (int64_t)i * T);
-        const uint32_t local = (kg[i] << 8) | (mix ? (k * 2654435761u) >> 24 : 0u);
         if (cnt[i] > 0u && cnt[i] <= EMIT_WIDE) {
             size_t q = (size_t)base + at[i];
             for (uint32_t x = tx[i] & 0xffffu; x <= tx[i] >> 16; ++x)
                 for (uint32_t y = ty[i] & 0xffffu; y <= ty[i] >> 16; ++y)
-                    for (int cb = cb0[i]; cb <= cb1[i]; ++cb) put(x, y, (uint32_t)cb, local, k, q++);
+                    for (int cb = cb0[i]; cb <= cb1[i]; ++cb) 
+                        put(x, y, (uint32_t)cb, kg[i], px[i], py[i], k, q++);
         }
         uint64_t wide = __ballot(cnt[i] > EMIT_WIDE);
         while (wide) {
@@ -340,11 +332,12 @@ __global__ __launch_bounds__(T) void k_emit(
             const uint32_t x0 = of(tx[i]) & 0xffffu, yy = of(ty[i]), y0 = yy & 0xffffu;
             const uint32_t ny = (yy >> 16) - y0 + 1u, b0 = of((uint32_t)cb0[i]);
             const uint32_t nb = of((uint32_t)cb1[i]) - b0 + 1u, n_cells = of(cnt[i]);
-            const uint32_t lk = of(k), ll = of(local);
+            const uint32_t lk = of(k), lg = of(kg[i]);
+            const int lx = (int)of((uint32_t)px[i]), ly = (int)of((uint32_t)py[i]);
             const size_t q = (size_t)base + of(at[i]);
             for (uint32_t e = lane; e < n_cells; e += 64) {
                 const uint32_t xy = e / nb, x = xy / ny;
-                put(x0 + x, y0 + (xy - x * ny), b0 + (e - xy * nb), ll, lk, q + e);
+                put(x0 + x, y0 + (xy - x * ny), b0 + (e - xy * nb), lg, lx, ly, lk, q + e);
             }
         }
     }
@@ -659,8 +652,7 @@ __global__ __launch_bounds__(64) void k_build_items(
 static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 hipError_t bin_particles(const mi_particle* d_p, int64_t n, int64_t n_pairs, const Grid& g,
-                         const mi_cube_desc& d, char* ws, const Layout& L, bool record_order,
-                         hipStream_t s) {
+                         const mi_cube_desc& d, char* ws, const Layout& L, hipStream_t s) {
     auto words = [&](size_t at) { return (uint32_t*)(ws + at); };
     uint32_t* status = words(L.status);
     uint32_t* hist = words(L.hist);
@@ -671,7 +663,7 @@ hipError_t bin_particles(const mi_particle* d_p, int64_t n, int64_t n_pairs, con
     const int64_t clear = (int64_t)(L.cleared - L.status) / 16;
     hipLaunchKernelGGL(k_bin_init, dim3((unsigned)std::min<int64_t>((clear + T - 1) / T, 2048)),
                        dim3(T), 0, s, (uint4*)(ws + L.status), clear);
-    const RadixPlan r = radix_plan(g, record_order);
+    const RadixPlan r = radix_plan(g);
     // the last pass ends in keys2 / vals2
     uint32_t *k0 = words(L.keys), *v0 = words(L.vals), *k1 = words(L.keys2), *v1 = words(L.vals2);
     if (r.passes % 2 == 0) {
@@ -684,8 +676,8 @@ hipError_t bin_particles(const mi_particle* d_p, int64_t n, int64_t n_pairs, con
         auto emit = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3((unsigned)shape.threads),
                                sizeof(uint32_t) * EMIT_COPIES * ((r.passes << r.bits) + 1), s, d_p, n, n_pairs,
-                               g, d.weights, d.weights_n, emit_look, k0, v0, hist, status,
-                               record_order ? 0 : 1, r.begin, r.passes, r.bits);
+                               g, d.weights, d.weights_n, emit_look, k0, v0, hist, status, r.begin, r.passes,
+                               r.bits);
         };
         if (same(shape, EMIT_SMALL))
             emit(k_emit<EMIT_SMALL.threads, EMIT_SMALL.items>);

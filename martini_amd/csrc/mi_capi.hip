@@ -121,7 +121,7 @@ int mi_bin(const mi_particle* d_particles, int64_t n, int64_t n_pairs, const mi_
     int rc = prepare(d_particles, n, n_pairs, desc, d_workspace, workspace_bytes, &g, &L);
     if (rc) return rc;
     if (bin_particles(d_particles, n, n_pairs, g, *desc, (char*)d_workspace, L,
-                      method == MI_METHOD_MFMA_BF16X3, (hipStream_t)stream) != hipSuccess)
+                      (hipStream_t)stream) != hipSuccess)
         return MI_ERR_DEVICE;
     return MI_OK;
 }
@@ -137,8 +137,7 @@ int mi_gather(const mi_particle* d_particles, int64_t n, int64_t n_pairs,
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)d_workspace;
-    hipError_t e = method == MI_METHOD_PLAIN_F32 ? gather_plain(d_particles, g, *desc, ws, L, d_cube, s)
-                                                 : gather_mfma(d_particles, g, *desc, ws, L, d_cube, s);
+    hipError_t e = gather(d_particles, g, *desc, ws, L, method == MI_METHOD_MFMA_BF16X3, d_cube, s);
     if (e == hipErrorNotSupported) return MI_ERR_UNSUPPORTED;
     if (e != hipSuccess) return MI_ERR_DEVICE;
     if (reduce_partials(g, ws, L, d_cube, s) != hipSuccess) return MI_ERR_DEVICE;

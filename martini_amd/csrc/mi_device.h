@@ -93,8 +93,8 @@ __host__ __device__ inline int item_length(int64_t n_pairs) {
     const int64_t filled = (n_pairs / ITEM_FILL + 31) / 32 * 32;
     return (int)(filled < ITEM_MIN ? ITEM_MIN : (filled > ITEM_WHOLE ? ITEM_WHOLE : filled));
 }
-// Key layout: cell << KEY_LOCAL_BITS | kernel group << 8 | 8-bit local order
-// (zero, keeping the record order, or a hash of the particle index).
+// Key layout: cell << KEY_LOCAL_BITS | kernel group << 8 | 8-bit local order (tile
+// row and column).
 constexpr int KEY_LOCAL_BITS = 10;
 
 __host__ __device__ inline int kind_of(int32_t r_kind) { return r_kind & 15; }

@@ -1,21 +1,6 @@
-// Pixel-tile gather: the FP32 form of the insertion contraction
-//
-//   cube[i, j, c] += sum_p W[(i, j), p] * S[p, c]
-//
-// over one cell (16 x 16 pixels x 64 channels, or 8 x 16 x 128 for cubes of
-// 128 channels or more) per work item, replacing the
-// reference's per-pixel loop (martini/martini.py:243-283, :327-362).
-//
-// A work group of 256 threads takes the item's particles in chunks of 32:
-//   1. the chunk's records go to LDS with their footprints clipped to the tile;
-//   2. W[k][pixel] is evaluated once per (particle, footprint pixel) pair --
-//      pairs are enumerated over the chunk so every lane does useful
-//      transcendental work -- into a zeroed 32 x pixels LDS tile;
-//   3. S[k][channel] (line profile times amplitude) fills a 32 x channels LDS tile;
-//   4. each thread owns one tile row (16 pixels) x 4 channels and accumulates
-//      up to 64 FMAs per particle; a wave skips particles whose footprint
-//      misses its rows (4 or 2), and the 4-column groups the footprint misses.
-// Summation follows the sorted particle order: no atomics, deterministic.
+// What stands around the gather: the reduction of split cells' partial tiles,
+// the kernel weight tables, and the entry points that evaluate kernel
+// integrals and spectra by themselves.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -25,201 +10,6 @@
 #include "mi_tile.h"
 
 namespace mi {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// Three waves per SIMD (at most 168 VGPRs): three work groups share a CU.
-template <class G>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_gather_plain(
-    const mi_particle* __restrict__ P, const uint32_t* __restrict__ order,
-    const Item* __restrict__ items, const uint32_t* __restrict__ status, const float4* __restrict__ wtab, Grid g, mi_cube_desc d,
-    float* __restrict__ cube, float* __restrict__ partials, uint64_t* __restrict__ part_masks) {
-    if (status[ST_OVERFLOW]) return;
-    if (blockIdx.x >= status[ST_ITEMS]) return;
-    const Item it = items[blockIdx.x];  // longest items first
-    const CellPos cp = cell_pos(it.cell, g);
-    const int x0 = cp.x0, y0 = cp.y0, c0 = cp.c0;
-
-    __shared__ __attribute__((aligned(16))) float Wt[KC][G::PX];
-    // rows padded to CB + 4 floats: the S fill writes a column (32
-    // particles) per store, which then spreads over the LDS banks
-    __shared__ __attribute__((aligned(16))) float St[KC][G::CB + 4];
-    __shared__ ChunkState cs;
-    __shared__ float4 Tk[LTAB_N];  // the item's kernel table
-    __shared__ GaussTables gt;     // the chunk's Gaussian-kernel factors
-
-    const int t = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // wave-uniform
-    constexpr int CG = G::CB / 4;              // 4-channel groups of a block
-    constexpr int WROWS = G::TX / (NT / 64);   // tile rows per wave
-    static_assert(G::TX * CG == NT && WROWS * (NT / 64) == G::TX,
-                  "a thread per (tile row, 4-channel group)");
-    const int pg = t / CG;  // tile row (pixel offset along x)
-    const int cg = t % CG;  // 4-channel group
-    const int lane = t & 63;
-
-    for (int e = t; e < KC * G::PX / 4; e += NT)
-        reinterpret_cast<float4*>(&Wt[0][0])[e] = make_float4(0.f, 0.f, 0.f, 0.f);
-
-    float acc[TILE_Y][4];
-#pragma unroll
-    for (int jj = 0; jj < TILE_Y; ++jj)
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) acc[jj][cc] = 0.0f;
-
-    // Every wave holds the records of the next chunk and the sort indices of the
-    // one after.  A chunk is staged by the wave that had the fewest particles to
-    // multiply in the chunk before (it reaches the staging first); every wave
-    // picks it from the same counts.
-    const int tkind = stage_table(P, order, it.begin, wtab, Tk);
-    RecRegs next{};
-    uint32_t next_idx = 0;
-    if (lane < min(KC, it.end - it.begin)) next = load_record(P, order[it.begin + lane]);
-    if (lane < min(KC, it.end - it.begin - KC)) next_idx = order[it.begin + KC + lane];
-    int stager = 0;
-
-    for (int kb = it.begin; kb < it.end; kb += KC) {
-        const int nk = min(KC, it.end - kb);
-        if (wave == __builtin_amdgcn_readfirstlane(stager))
-            stage_chunk(next, lane < nk, x0, y0, c0, g, d, cs);
-        if (lane < min(KC, it.end - kb - KC)) next = load_record(P, next_idx);
-        if (lane < min(KC, it.end - kb - 2 * KC)) next_idx = order[kb + 2 * KC + lane];
-        __syncthreads();
-        // Particles whose footprint meets each wave's rows (wave-uniform masks);
-        // this wave keeps its own, and the least loaded wave stages the next chunk.
-        const int klo = cs.ilo[lane & (KC - 1)], khi = cs.ihi[lane & (KC - 1)];
-        const bool valid = lane < KC && klo <= khi;
-        uint32_t kmask = 0;
-        int fewest = KC + 1;
-#pragma unroll
-        for (int w2 = 0; w2 < NT / 64; ++w2) {
-            const int r0 = x0 + w2 * WROWS;
-            const uint32_t m = (uint32_t)__ballot(valid && khi >= r0 && klo <= r0 + WROWS - 1);
-            const int c = __builtin_popcount(m);
-            if (c < fewest) {
-                fewest = c;
-                stager = w2;
-            }
-            if (w2 == wave) kmask = m;
-        }
-        const bool hit = lane < KC && ((kmask >> lane) & 1u);
-        // Lane k: the 4-column groups of the tile that particle k's footprint
-        // covers (W is zero in the others).  Read here, before the next chunk's
-        // staging may overwrite the chunk state.
-        uint32_t qm = 0;
-        if (hit) {
-            const WalkRec& wk = cs.walk[lane];
-            const int j0 = (wk.ij >> 16) - y0;
-            qm = (2u << ((j0 + (wk.kw >> 8) - 1) >> 2)) - (1u << (j0 >> 2));
-        }
-        if (cs.gmask != 0u) {  // the same for every thread
-            fill_gauss_tables(cs, gt);
-            __syncthreads();
-        }
-        fill_weights(
-            cs, x0, y0, wtab, tkind, Tk, gt, d.weights, [&](int k, int px, float w) { Wt[k][px] = w; },
-            [&](int k, int p1, float w1, int p2, float w2) {
-                Wt[k][p1] = w1;
-                Wt[k][p2] = w2;
-            });
-        fill_spectra<G::CB>(cs, nk, c0, g.nc, d, [&](int k, int c1, float v1, int c2, float v2) {
-            St[k][c1] = v1;
-            St[k][c2] = v2;
-        });
-        __syncthreads();
-        if (kmask == 0u) continue;
-        while (kmask != 0u) {
-            const int k = __builtin_ctz(kmask);
-            kmask &= kmask - 1u;
-            const uint32_t qk = __builtin_amdgcn_readlane(qm, k);  // wave-uniform
-            const f32x4* wr = reinterpret_cast<const f32x4*>(&Wt[k][pg * TILE_Y]);
-            const f32x4 sv = *reinterpret_cast<const f32x4*>(&St[k][cg * 4]);
-            // all five LDS reads are issued together, ahead of the skips
-            f32x4 wq[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) wq[q] = wr[q];
-            asm volatile("" ::"v"(wq[0]), "v"(wq[1]), "v"(wq[2]), "v"(wq[3]), "v"(sv));
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (!((qk >> q) & 1u)) continue;
-                const f32x4 w = wq[q];
-                const float wv[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    acc[q * 4 + u][0] = fmaf(wv[u], sv.x, acc[q * 4 + u][0]);
-                    acc[q * 4 + u][1] = fmaf(wv[u], sv.y, acc[q * 4 + u][1]);
-                    acc[q * 4 + u][2] = fmaf(wv[u], sv.z, acc[q * 4 + u][2]);
-                    acc[q * 4 + u][3] = fmaf(wv[u], sv.w, acc[q * 4 + u][3]);
-                }
-            }
-        }
-        // Clear this wave's band of W (its rows' pixels, read only by this wave)
-        // for the next fill: BAND / 4 lanes per particle, 64 / (BAND / 4) particles
-        // per store.
-        constexpr int BAND = WROWS * TILE_Y;
-        static_assert(BAND % 4 == 0 && 64 % (BAND / 4) == 0, "whole float4 rows per store");
-#pragma unroll
-        for (int k = 0; k < KC; k += 64 / (BAND / 4))
-            *reinterpret_cast<float4*>(
-                &Wt[k + lane / (BAND / 4)][wave * BAND + (lane % (BAND / 4)) * 4]) =
-                make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-
-    // A thread's 16 pixels x 4 channels that are all zero (no particle reached
-    // them) are not written.  The four threads of a sub-tile (one tile row x 16
-    // channels) are neighbouring lanes; a partial tile's mask gets the sub-tiles
-    // with a nonzero value, and each wave stores the whole bytes of the mask
-    // that cover its rows (no two waves share a byte).
-    bool nz = false;
-#pragma unroll
-    for (int jj = 0; jj < TILE_Y; ++jj)
-        nz = nz || acc[jj][0] != 0.f || acc[jj][1] != 0.f || acc[jj][2] != 0.f ||
-             acc[jj][3] != 0.f;
-    const uint64_t any = __ballot(nz);
-    const bool quad = ((any >> (lane & ~3)) & 0xFu) != 0u;  // this sub-tile has a value
-    const int i = x0 + pg;
-    if (it.slot < 0) {
-        if (i < g.nx && nz) {
-#pragma unroll
-            for (int jj = 0; jj < TILE_Y; ++jj) {
-                const int j = y0 + jj;
-                if (j >= g.ny) continue;
-                float* dst = cube + ((size_t)i * g.ny + j) * g.nc;
-#pragma unroll
-                for (int cc = 0; cc < 4; ++cc) {
-                    const int c = c0 + cg * 4 + cc;
-                    if (c < g.nc) dst[c] += acc[jj][cc];
-                }
-            }
-        }
-    } else {
-        static_assert(SUB_CH == 16, "four float4 per sub-tile row");
-        if (quad) {
-            float* dst = partials + (size_t)it.slot * CELL_VOXELS + (cg & 3) * 4;
-#pragma unroll
-            for (int jj = 0; jj < TILE_Y; ++jj)
-                *reinterpret_cast<float4*>(dst + sub_offset(G::CB / SUB_CH, pg, cg >> 2, jj)) =
-                    make_float4(acc[jj][0], acc[jj][1], acc[jj][2], acc[jj][3]);
-        }
-        // The wave's 16 sub-tiles: lanes 4 q .. 4 q + 3 hold row
-        // wave * WROWS + 4 q / CG, block (4 q % CG) / 4.
-        constexpr int TXS = __builtin_ctz(G::TX);
-        static_assert((1 << TXS) == G::TX && CG % 4 == 0, "tile rows a power of two");
-        uint64_t mine = 0u, owned = 0u;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const uint64_t bit = 1ull << sub_bit(TXS, wave * WROWS + 4 * q / CG, (4 * q % CG) / 4);
-            owned |= bit;
-            if ((any >> (4 * q)) & 0xFu) mine |= bit;
-        }
-        if (lane == 0) {
-            unsigned char* mb = reinterpret_cast<unsigned char*>(part_masks + it.slot);
-#pragma unroll
-            for (int b = 0; b < 8; ++b)
-                if ((owned >> (8 * b)) & 0xFFu) mb[b] = (unsigned char)(mine >> (8 * b));
-        }
-    }
-}
 
 // Sums the partial tiles of each split cell in item order and adds them to
 // the cube.  Block (cell, part): 256 threads x 4 voxels cover four 1 KiB
@@ -339,25 +129,6 @@ __global__ void k_spectra(const mi_particle* __restrict__ P, int64_t n, mi_cube_
     int64_t p = e / nc;
     int c = (int)(e - p * nc);
     out[e] = channel_flux(P[p], c, d);
-}
-
-hipError_t gather_plain(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,
-                        const Layout& L, float* d_cube, hipStream_t s) {
-    if (L.items_max <= 0) return hipSuccess;
-    const float4* wtab = nullptr;
-    hipError_t e = weight_table(s, &wtab);
-    if (e != hipSuccess) return e;
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)L.items_max), dim3(NT), 0, s, d_p,
-                           (const uint32_t*)(ws + L.vals2), (const Item*)(ws + L.items),
-                           (const uint32_t*)(ws + L.status), wtab, g, d, d_cube, (float*)(ws + L.partials),
-                           (uint64_t*)(ws + L.part_masks));
-    };
-    if (g.wide)
-        launch(k_gather_plain<GeoWide>);
-    else
-        launch(k_gather_plain<GeoSquare>);
-    return hipGetLastError();
 }
 
 hipError_t reduce_partials(const Grid& g, char* ws, const Layout& L, float* d_cube,

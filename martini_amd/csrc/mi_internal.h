@@ -69,21 +69,14 @@ enum { ST_PAIRS = 0, ST_OVERFLOW = 1, ST_ITEMS = 2, ST_MULTI = 3, ST_BADREC = 4,
 
 hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L);
 
-// Binning: count, scan, emit, sort, cell bounds, items.  Asynchronous.
-// record_order: a cell's pairs keep the record order (the MFMA form: records
-// laid out in tile and pixel Z order make its chunks compact) and are sorted on
-// the cell and kernel group only; otherwise the keys end in a hash of the
-// particle index, which spreads each chunk over its tile, and are sorted on
-// the top 16 bits (two radix passes) when the key is longer.
+// Binning: emit, sort, cell bounds, items.  Asynchronous.
 hipError_t bin_particles(const mi_particle* d_p, int64_t n, int64_t n_pairs, const Grid& g,
-                         const mi_cube_desc& d, char* ws, const Layout& L, bool record_order,
-                         hipStream_t s);
+                         const mi_cube_desc& d, char* ws, const Layout& L, hipStream_t s);
 
-// Gather over work items (plain FP32 or MFMA), then the partial-tile reduction.
-hipError_t gather_plain(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,
-                        const Layout& L, float* d_cube, hipStream_t s);
-hipError_t gather_mfma(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,
-                       const Layout& L, float* d_cube, hipStream_t s);
+// Gather over work items (products in FP32, or in split BF16), then the
+// partial-tile reduction.
+hipError_t gather(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,
+                  const Layout& L, bool split_bf16, float* d_cube, hipStream_t s);
 hipError_t reduce_partials(const Grid& g, char* ws, const Layout& L, float* d_cube,
                            hipStream_t s);
 

@@ -1,28 +1,39 @@
-// Precision form of the insertion contraction on the matrix cores:
+// The insertion contraction on the matrix cores:
 //
 //   cube[(i, j), c] += sum_p W[(i, j), p] * S[p, c]
 //
 // per cell (16 x 16 pixels x 64 channels, or 8 x 16 x 128 for cubes of 128
 // channels or more) as a block-sparse product of a pixels x 32 W tile and a
-// 32 x channels S tile per chunk of 32 spatially sorted particles.  Both operands are split into BF16 pairs x = hi + lo
-// (|x - hi - lo| <= 2^-16 |x|) when they are written to LDS, and each
-// 16 x 16 x 32 block takes three v_mfma_f32_16x16x32_bf16 products -- hi*hi,
-// hi*lo, lo*hi -- accumulated in FP32 (the dropped lo*lo term is below 2^-16
-// of the product).
+// 32 x channels S tile per chunk of 32 particles, replacing the reference's
+// per-pixel loop (martini/martini.py:243-283, :327-362).  Two forms of the
+// products, the rest alike:
+//
+//   Float32    v_mfma_f32_16x16x4_f32: FP32 operands, products and sums.  A
+//              16 x 16 x 4 step is skipped when none of its four particles
+//              reaches the tile row or the channel block, so the cost follows the
+//              footprints also where a chunk is not compact;
+//   SplitBf16  both operands split into BF16 pairs x = hi + lo (|x - hi - lo| <=
+//              2^-16 |x|) when they are written to LDS, and three
+//              v_mfma_f32_16x16x32_bf16 products per 16 x 16 x 32 block -- hi*hi,
+//              hi*lo, lo*hi -- accumulated in FP32 (the dropped lo*lo term is below
+//              2^-16 of the product).
+//
+// Both are bound by the evaluation of W and S on the vector units; the FP32
+// products take about half of their time beside it.  On the vector units the
+// FP32 products (64 multiply-adds per particle, thread and tile row, all
+// channels) took most of that form's time: gather 643 us on 1e6 particles
+// (WendlandC2, 256 x 256 x 128), 4.42 ms on 3e6 of heterogeneous size
+// (1024 x 1024 x 64); on the matrix units 597 us and 3.59 ms with the same
+// records.
 //
 // Wave w owns four tile rows (M = the 16 pixels of a row) and four 16-channel
 // blocks (N): with 16 x 16-pixel x 64-channel cells the rows 4w..4w+3 and all
 // four blocks; with 8 x 16 x 128 cells rows 4 (w % 2) .. + 3 and blocks
 // 4 (w / 2) .. + 3, each pair of waves sharing its rows, which the second of
-// the two to finish reading them clears (an LDS counter per row group decides).  A (row, channel-block) product is
-// skipped when no footprint of the chunk touches the row or no spectral window
-// touches the block; the masks are wave-uniform, so the skips are scalar
-// branches.
-//
-// LDS operand tiles hold 32 BF16 values (64 bytes) per pixel or channel, k
-// contiguous, with the four 16-byte k-groups of a row permuted by bits 2..3 of
-// the row index: the 16 rows a 16-lane group reads for one k-group then fall
-// in 16 distinct 16-byte bank slots.
+// the two to finish reading them clears (an LDS counter per row group decides).
+// A (row, channel-block) product is skipped when no footprint of the chunk
+// touches the row or no spectral window touches the block; the masks are
+// wave-uniform, so the skips are scalar branches.
 //
 // Per chunk there are two barriers: staging -> (W, S fill) -> products, and a
 // third in chunks with Gaussian-kernel particles, whose row and column factors
@@ -36,6 +47,8 @@
 // Accumulation order is fixed: deterministic, no atomics.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mi_device.h"
 #include "mi_internal.h"
 #include "mi_tile.h"
@@ -47,84 +60,151 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
-constexpr int KROW = KC * 2;  // bytes per LDS operand row (32 BF16)
+// Operand tiles in LDS: OPK bytes per pixel (W) or channel (S) and chunk in
+// either form.
+constexpr int OPK = KC * 4;
 
-// Byte offset of element (row, k) in an operand tile:
-//   row * KROW + (((k >> 3) ^ (row >> 2)) & 3) * 16 + (k & 7) * 2,
-// written with the k terms folded into one constant per thread (k_bits(k)).
-__device__ inline int k_bits(int k) { return (((k >> 3) & 3) << 4) | ((k & 7) << 1); }
-__device__ inline int op_offset(int row, int kb) { return row * KROW + (((row << 2) & 48) ^ kb); }
+// BF16x3: a hi and a lo tile of 64 bytes per row, k contiguous, the four 16-byte
+// k-groups of a row permuted by bits 2..3 of the row index: the 16 rows a
+// 16-lane group reads for one k-group then fall in 16 distinct 16-byte bank slots.
+template <int ROWS>
+struct SplitTile {
+    static constexpr int KROW = KC * 2;
+    __attribute__((aligned(16))) char hi[ROWS * KROW];
+    __attribute__((aligned(16))) char lo[ROWS * KROW];
 
-// Writes x as a BF16 pair (round to nearest even) at (row, k) of the hi and lo tiles.
-__device__ inline void put_split(char* hi, char* lo, int row, int k, float x) {
-    const __bf16 h = (__bf16)x;
-    const __bf16 l = (__bf16)(x - (float)h);
-    const int o = op_offset(row, k_bits(k));
-    *reinterpret_cast<__bf16*>(hi + o) = h;
-    *reinterpret_cast<__bf16*>(lo + o) = l;
-}
+    // Byte offset of element (row, k):
+    //   row * KROW + (((k >> 3) ^ (row >> 2)) & 3) * 16 + (k & 7) * 2,
+    // written with the k terms folded into one constant per thread (k_bits(k)).
+    __device__ static int k_bits(int k) { return (((k >> 3) & 3) << 4) | ((k & 7) << 1); }
+    __device__ static int at(int row, int kb) { return row * KROW + (((row << 2) & 48) ^ kb); }
 
-// put_split of two values of column k, converted together (one packed
-// conversion each for the hi and the lo parts).
-__device__ inline void put_split2(char* hi, char* lo, int k, int row1, float x1, int row2,
-                                  float x2) {
-    const floatx2 x = {x1, x2};
-    const bf16x2 h = __builtin_convertvector(x, bf16x2);
-    const floatx2 hf = __builtin_convertvector(h, floatx2);
-    const bf16x2 l = __builtin_convertvector(floatx2{x1 - hf.x, x2 - hf.y}, bf16x2);
-    const int kb = k_bits(k);
-    const int o1 = op_offset(row1, kb), o2 = op_offset(row2, kb);
-    *reinterpret_cast<__bf16*>(hi + o1) = h.x;
-    *reinterpret_cast<__bf16*>(lo + o1) = l.x;
-    *reinterpret_cast<__bf16*>(hi + o2) = h.y;
-    *reinterpret_cast<__bf16*>(lo + o2) = l.y;
-}
+    // Writes x as a BF16 pair (round to nearest even).
+    __device__ void put(int row, int k, float x) {
+        const __bf16 h = (__bf16)x;
+        const __bf16 l = (__bf16)(x - (float)h);
+        const int o = at(row, k_bits(k));
+        *reinterpret_cast<__bf16*>(hi + o) = h;
+        *reinterpret_cast<__bf16*>(lo + o) = l;
+    }
+    // Two values of column k, converted together (one packed conversion each for
+    // the hi and the lo parts).
+    __device__ void put2(int k, int row1, float x1, int row2, float x2) {
+        const floatx2 x = {x1, x2};
+        const bf16x2 h = __builtin_convertvector(x, bf16x2);
+        const floatx2 hf = __builtin_convertvector(h, floatx2);
+        const bf16x2 l = __builtin_convertvector(floatx2{x1 - hf.x, x2 - hf.y}, bf16x2);
+        const int kb = k_bits(k);
+        const int o1 = at(row1, kb), o2 = at(row2, kb);
+        *reinterpret_cast<__bf16*>(hi + o1) = h.x;
+        *reinterpret_cast<__bf16*>(lo + o1) = l.x;
+        *reinterpret_cast<__bf16*>(hi + o2) = h.y;
+        *reinterpret_cast<__bf16*>(lo + o2) = l.y;
+    }
+    // put2 for the S fill, whose lanes l and l ^ 1 hold the same two rows of
+    // particles k and k ^ 1 (rows given as 16 * block + r: the block's 1 KiB step
+    // plus at(r)).  After one lane swap (DPP quad_perm [1, 0, 3, 2]) the even lane
+    // writes row1 and the odd lane row2, each as the pair (k even, k odd) --
+    // adjacent BF16 slots of one 4-byte word -- in both tiles: one paired 4-byte
+    // store per lane (the hi and lo tiles lie a fixed distance apart) instead of
+    // four 2-byte ones.  Every lane of the wave must call it.
+    __device__ void put_pairs(int k, int row1, float x1, int row2, float x2) {
+        constexpr int SWAP = 0xB1;  // quad_perm [1, 0, 3, 2]: lanes l and l ^ 1
+        const float y1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x1), SWAP, 0xF, 0xF, false));
+        const float y2 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x2), SWAP, 0xF, 0xF, false));
+        const bool even = (k & 1) == 0;
+        const int row = even ? row1 : row2;
+        const floatx2 x = even ? floatx2{x1, y1} : floatx2{y2, x2};  // particles k & ~1, k | 1
+        const bf16x2 h = __builtin_convertvector(x, bf16x2);
+        const floatx2 hf = __builtin_convertvector(h, floatx2);
+        const bf16x2 l = __builtin_convertvector(floatx2{x.x - hf.x, x.y - hf.y}, bf16x2);
+        const int o = (row >> 4) * (16 * KROW) + at(row & 15, k_bits(k & ~1));
+        *reinterpret_cast<bf16x2*>(hi + o) = h;
+        *reinterpret_cast<bf16x2*>(lo + o) = l;
+    }
+    // The 8 values of k-group kg of `row`, hi and lo.
+    struct Op {
+        bf16x8 h, l;
+    };
+    __device__ Op get(int row, int kg) const {
+        const int o = row * KROW + (((kg ^ (row >> 2)) & 3) << 4);
+        return Op{*reinterpret_cast<const bf16x8*>(hi + o), *reinterpret_cast<const bf16x8*>(lo + o)};
+    }
+    // Clears 16 rows from `row` on with one wave.
+    __device__ void clear16(int row, int lane) {
+        const int o = row * KROW + lane * 16;
+        *reinterpret_cast<uint4*>(hi + o) = make_uint4(0u, 0u, 0u, 0u);
+        *reinterpret_cast<uint4*>(lo + o) = make_uint4(0u, 0u, 0u, 0u);
+    }
+};
 
-// The 8 BF16 values of k-group kg of `row`.
-__device__ inline bf16x8 get8(const char* tile, int row, int kg) {
-    return *reinterpret_cast<const bf16x8*>(tile + row * KROW + (((kg ^ (row >> 2)) & 3) << 4));
-}
+// FP32: 128 bytes per row.  A 16 x 16 x 4 product takes one value per lane and
+// operand, lane group kg (of 16) the k-th of its four, so particle k is kept in
+// slot 8 (k % 4) + k / 4: lane group kg then reads its eight values of the chunk
+// with two 16-byte loads, and step s of the eight multiplies particles 4 s ..
+// 4 s + 3.  The eight 16-byte groups of a row are permuted by bits 1..3 of the
+// row index: the 16 rows that a 16-lane group reads together fall in distinct
+// bank slots (even and odd rows lie in different halves of the banks).
+template <int ROWS>
+struct FloatTile {
+    __attribute__((aligned(16))) char v[ROWS * OPK];
 
-// put_split2 for the S fill, whose lanes l and l ^ 1 hold the same two rows of
-// particles k and k ^ 1 (rows given as 16 * block + r: the block's 1 KiB step
-// plus op_offset(r)).  After one lane swap (DPP quad_perm [1, 0, 3, 2]) the
-// even lane writes row1 and the odd lane row2, each as the pair (k even, k odd)
-// -- adjacent BF16 slots of one 4-byte word -- in both tiles: one paired
-// 4-byte store per lane (the hi and lo tiles lie a fixed distance apart)
-// instead of four 2-byte ones.  Every lane of the wave must call it.
-__device__ inline void put_split2_pairs(char* hi, char* lo, int k, int row1, float x1, int row2,
-                                        float x2) {
-    constexpr int SWAP = 0xB1;  // quad_perm [1, 0, 3, 2]: lanes l and l ^ 1
-    const float y1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x1), SWAP, 0xF, 0xF, false));
-    const float y2 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x2), SWAP, 0xF, 0xF, false));
-    const bool even = (k & 1) == 0;
-    const int row = even ? row1 : row2;
-    const floatx2 x = even ? floatx2{x1, y1} : floatx2{y2, x2};  // particles k & ~1, k | 1
-    const bf16x2 h = __builtin_convertvector(x, bf16x2);
-    const floatx2 hf = __builtin_convertvector(h, floatx2);
-    const bf16x2 l = __builtin_convertvector(floatx2{x.x - hf.x, x.y - hf.y}, bf16x2);
-    const int o = (row >> 4) * (16 * KROW) + op_offset(row & 15, k_bits(k & ~1));
-    *reinterpret_cast<bf16x2*>(hi + o) = h;
-    *reinterpret_cast<bf16x2*>(lo + o) = l;
-}
+    __device__ static int k_bits(int k) { return ((k & 3) << 5) | ((k >> 2) << 2); }
+    __device__ static int at(int row, int kb) { return row * OPK + (((row << 3) & 0x70) ^ kb); }
+    __device__ void put(int row, int k, float x) {
+        *reinterpret_cast<float*>(v + at(row, k_bits(k))) = x;
+    }
+    __device__ void put2(int k, int row1, float x1, int row2, float x2) {
+        const int kb = k_bits(k);
+        *reinterpret_cast<float*>(v + at(row1, kb)) = x1;
+        *reinterpret_cast<float*>(v + at(row2, kb)) = x2;
+    }
+    __device__ void put_pairs(int k, int row1, float x1, int row2, float x2) {
+        put2(k, row1, x1, row2, x2);
+    }
+    struct Op {
+        floatx4 a, b;  // steps 0..3 and 4..7
+        __device__ float step(int s) const { return s < 4 ? a[s] : b[s - 4]; }
+    };
+    __device__ Op get(int row, int kg) const {
+        const int o = at(row, kg << 5);
+        return Op{*reinterpret_cast<const floatx4*>(v + o),
+                  *reinterpret_cast<const floatx4*>(v + (o ^ 16))};
+    }
+    __device__ void clear16(int row, int lane) {
+        const int o = row * OPK + lane * 16;
+        *reinterpret_cast<uint4*>(v + o) = make_uint4(0u, 0u, 0u, 0u);
+        *reinterpret_cast<uint4*>(v + o + 1024) = make_uint4(0u, 0u, 0u, 0u);
+    }
+};
+
+struct SplitBf16 {
+    template <int ROWS>
+    using Tile = SplitTile<ROWS>;
+};
+struct Float32 {
+    template <int ROWS>
+    using Tile = FloatTile<ROWS>;
+};
 
 // Three waves per SIMD: the 64 accumulators then live in VGPRs and three work
 // groups share a CU (LDS 48 KB each).
-template <class G>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_gather_mfma(
+template <class G, class F>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_gather(
     const mi_particle* __restrict__ P, const uint32_t* __restrict__ order,
-    const Item* __restrict__ items, const uint32_t* __restrict__ status, const float4* __restrict__ wtab, Grid g, mi_cube_desc d,
-    float* __restrict__ cube, float* __restrict__ partials, uint64_t* __restrict__ part_masks) {
+    const Item* __restrict__ items, const uint32_t* __restrict__ status,
+    const float4* __restrict__ wtab, Grid g, mi_cube_desc d, float* __restrict__ cube,
+    float* __restrict__ partials, uint64_t* __restrict__ part_masks) {
     if (status[ST_OVERFLOW]) return;
     if (blockIdx.x >= status[ST_ITEMS]) return;
     const Item it = items[blockIdx.x];  // longest items first
     const CellPos cp = cell_pos(it.cell, g);
     const int x0 = cp.x0, y0 = cp.y0, c0 = cp.c0;
 
-    __shared__ __attribute__((aligned(16))) char Ah[G::PX * KROW];  // W hi [pixel][k]
-    __shared__ __attribute__((aligned(16))) char Al[G::PX * KROW];  // W lo
-    __shared__ __attribute__((aligned(16))) char Bh[G::CB * KROW];  // S hi [channel][k]
-    __shared__ __attribute__((aligned(16))) char Bl[G::CB * KROW];  // S lo
+    using WTile = typename F::template Tile<G::PX>;
+    using STile = typename F::template Tile<G::CB>;
+    __shared__ WTile W;            // [pixel][k]
+    __shared__ STile S;            // [channel][k]
     __shared__ ChunkState cs;
     __shared__ float4 Tk[LTAB_N];  // the item's kernel table
     __shared__ GaussTables gt;     // the chunk's Gaussian-kernel factors
@@ -138,12 +218,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // wave-uniform
     const int lane = t & 63;
     const int m = lane & 15;   // A row / B column / D column of this lane
-    const int kg = lane >> 4;  // K group of 8 (A, B); D row group of 4
+    const int kg = lane >> 4;  // K group (A, B); D row group of 4
 
-    for (int e = t; e < G::PX * KROW / 16; e += NT) {
-        reinterpret_cast<uint4*>(Ah)[e] = make_uint4(0u, 0u, 0u, 0u);
-        reinterpret_cast<uint4*>(Al)[e] = make_uint4(0u, 0u, 0u, 0u);
-    }
+    static_assert(sizeof(WTile) == G::PX * OPK && TILE_Y == 16, "16 pixels per tile row");
+    for (int e = wave; e < G::TX; e += NT / 64) W.clear16(e * TILE_Y, lane);
     if (t < RG) done_rows[t] = 0u;
     const int rh = wave % RG, ch = wave / RG;  // this wave's row group and channel group
 
@@ -189,60 +267,76 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
             __syncthreads();
         }
         fill_weights(cs, x0, y0, wtab, tkind, Tk, gt, d.weights,
-                     [&](int k, int px, float w) { put_split(Ah, Al, px, k, w); },
-                     [&](int k, int p1, float w1, int p2, float w2) {
-                         put_split2(Ah, Al, k, p1, w1, p2, w2);
-                     });
+                     [&](int k, int px, float w) { W.put(px, k, w); },
+                     [&](int k, int p1, float w1, int p2, float w2) { W.put2(k, p1, w1, p2, w2); });
         fill_spectra<G::CB>(cs, nk, c0, g.nc, d,
-                     [&](int k, int c1, float s1, int c2, float s2) {
-                         put_split2_pairs(Bh, Bl, k, c1, s1, c2, s2);
-                     },
+                     [&](int k, int c1, float s1, int c2, float s2) { S.put_pairs(k, c1, s1, c2, s2); },
                      chanmask);
+        // FP32: the particles (bits) that reach each of this wave's rows and blocks
+        uint32_t prow[4] = {}, pblk[4] = {};
+        if constexpr (std::is_same_v<F, Float32>) {
+            const uint32_t cover = lane < KC ? cs.cover[lane] : 0u;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) prow[r] = (uint32_t)__ballot((cover >> (rh * 4 + r)) & 1u);
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb)
+                pblk[nb] = (uint32_t)__ballot((cover >> (16 + ch * 4 + nb)) & 1u);
+        }
         __syncthreads();
         if (rows != 0u) {
             // The wave's four tile rows held together: each S operand read serves all.
-            bf16x8 ah[4], al[4];
+            typename WTile::Op a[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                ah[r] = bf16x8{};
-                al[r] = bf16x8{};
+                a[r] = typename WTile::Op{};
                 if (!(rows & (1u << r)) || chans == 0u) continue;
-                const int row = (rh * 4 + r) * TILE_Y + m;
-                ah[r] = get8(Ah, row, kg);
-                al[r] = get8(Al, row, kg);
+                a[r] = W.get((rh * 4 + r) * TILE_Y + m, kg);
             }
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb) {
                 if (!(chans & (1u << nb))) continue;
-                const int col = (ch * 4 + nb) * 16 + m;
-                const bf16x8 bh = get8(Bh, col, kg), bl = get8(Bl, col, kg);
+                const typename STile::Op b = S.get((ch * 4 + nb) * 16 + m, kg);
+                if constexpr (std::is_same_v<F, Float32>) {
+                    // bit 4 s: one of the particles 4 s .. 4 s + 3 reaches this row and block
+                    uint32_t need[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (!(rows & (1u << r))) continue;
-                    floatx4 c = acc[r][nb];
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[r], bh, c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[r], bl, c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[r], bh, c, 0, 0, 0);
-                    acc[r][nb] = c;
+                    for (int r = 0; r < 4; ++r) {
+                        uint32_t q = prow[r] & pblk[nb];
+                        q |= q >> 1;
+                        need[r] = q | (q >> 2);
+                    }
+#pragma unroll
+                    for (int s = 0; s < KC / 4; ++s)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (need[r] & (1u << (4 * s)))
+                                acc[r][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                    a[r].step(s), b.step(s), acc[r][nb], 0, 0, 0);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if (!(rows & (1u << r))) continue;
+                        floatx4 c = acc[r][nb];
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r].h, b.h, c, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r].h, b.l, c, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r].l, b.h, c, 0, 0, 0);
+                        acc[r][nb] = c;
+                    }
                 }
             }
             // The last of the CGN waves sharing these rows to get here clears
-            // the rows' 1 KiB in both W tiles (one 16-byte store per lane
-            // each): the counter's update orders it after every such wave's
-            // reads of them (LDS requests of a wave are served in order; the
-            // release keeps the reads before the update).
+            // the rows' 2 KiB (two 16-byte stores per lane each): the counter's
+            // update orders it after every such wave's reads of them (LDS requests
+            // of a wave are served in order; the release keeps the reads before the
+            // update).
             uint32_t before = 0u;
             if (CGN > 1 && lane == 0)
                 before = __hip_atomic_fetch_add(&done_rows[rh], 1u, __ATOMIC_ACQ_REL,
                                                 __HIP_MEMORY_SCOPE_WORKGROUP);
             if (CGN == 1 || __builtin_amdgcn_readlane(before, 0) == CGN - 1) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (!(rows & (1u << r))) continue;
-                    const int zb = (rh * 4 + r) * TILE_Y * KROW + lane * 16;
-                    *reinterpret_cast<uint4*>(Ah + zb) = make_uint4(0u, 0u, 0u, 0u);
-                    *reinterpret_cast<uint4*>(Al + zb) = make_uint4(0u, 0u, 0u, 0u);
-                }
+                for (int r = 0; r < 4; ++r)
+                    if (rows & (1u << r)) W.clear16((rh * 4 + r) * TILE_Y, lane);
                 if (CGN > 1 && lane == 0) done_rows[rh] = 0u;
             }
         }
@@ -282,8 +376,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         reinterpret_cast<uint16_t*>(part_masks + it.slot)[wave] = (uint16_t)mine;
 }
 
-hipError_t gather_mfma(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,
-                       const Layout& L, float* d_cube, hipStream_t s) {
+hipError_t gather(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,
+                  const Layout& L, bool split_bf16, float* d_cube, hipStream_t s) {
     if (L.items_max <= 0) return hipSuccess;
     const float4* wtab = nullptr;
     hipError_t e = weight_table(s, &wtab);
@@ -291,13 +385,20 @@ hipError_t gather_mfma(const mi_particle* d_p, const Grid& g, const mi_cube_desc
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)L.items_max), dim3(NT), 0, s, d_p,
                            (const uint32_t*)(ws + L.vals2), (const Item*)(ws + L.items),
-                           (const uint32_t*)(ws + L.status), wtab, g, d, d_cube, (float*)(ws + L.partials),
-                           (uint64_t*)(ws + L.part_masks));
+                           (const uint32_t*)(ws + L.status), wtab, g, d, d_cube,
+                           (float*)(ws + L.partials), (uint64_t*)(ws + L.part_masks));
     };
-    if (g.wide)
-        launch(k_gather_mfma<GeoWide>);
-    else
-        launch(k_gather_mfma<GeoSquare>);
+    if (split_bf16) {
+        if (g.wide)
+            launch(k_gather<GeoWide, SplitBf16>);
+        else
+            launch(k_gather<GeoSquare, SplitBf16>);
+    } else {
+        if (g.wide)
+            launch(k_gather<GeoWide, Float32>);
+        else
+            launch(k_gather<GeoSquare, Float32>);
+    }
     return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-// Chunk staging shared by the FP32 and MFMA tile gathers: the cell-sorted
+// Chunk staging of the tile gather, shared by its two forms: the cell-sorted
 // particle records of a work item are taken 32 at a time, their footprints
 // clipped to the cell's tile, and W evaluated once per (particle, footprint
 // pixel) pair.
@@ -59,7 +59,8 @@ struct ChunkState {
     mi_particle p[KC];
     WalkRec walk[KC];
     GaussRec gr[KC];    // Gaussian kernel factors
-    int ilo[KC], ihi[KC];
+    uint32_t cover[KC]; // tile rows (low half) and 16-channel blocks (high half) a
+                        // particle reaches in the cell, zero without a footprint in it
     int off[KC + 1];    // exclusive scan of the per-particle pair counts
     // exclusive scan of the threads given to each particle's pairs (16-byte
     // aligned: fill_weights reads it eight entries at a time)
@@ -182,8 +183,7 @@ __device__ inline void stage_chunk(const RecRegs& r, bool valid, int x0, int y0,
     const int tincl = wave_scan_add((int)(((float)(cnt + per - 1) + 0.5f) * rper));
     if (lane < KC) {
         if (valid) cs.p[lane] = p;
-        cs.ilo[lane] = ilo;
-        cs.ihi[lane] = ihi;
+        cs.cover[lane] = rows | (chans << 16);
         const int width = max(jhi - jlo + 1, 1);
         cs.off[lane + 1] = incl;
         cs.toff[lane + 1] = tincl;
@@ -255,7 +255,7 @@ __device__ inline void fill_gauss_tables(const ChunkState& cs, GaussTables& gt) 
     const WalkRec w = cs.walk[k];
     const float bf = cs.gr[k].f.x;
     const int i0 = w.ij & 0xffff, j0 = w.ij >> 16;
-    const int rows = gk ? cs.ihi[k] - i0 + 1 : 0, cols = gk ? w.kw >> 8 : 0;
+    const int rows = gk ? __builtin_popcount(cs.cover[k] & 0xffffu) : 0, cols = gk ? w.kw >> 8 : 0;
     for (int r = slot; __any(r < rows); r += NT / KC)
         if (r < rows) gt.ex[k][r] = erf_span((float)(w.px - (double)(i0 + r)) * bf, bf);
     for (int c = slot; __any(c < cols); c += NT / KC)

@@ -1,0 +1,79 @@
+"""The gather's products against an FP64 sum, both forms, at the edges of its
+chunks (32 particles), pairs of chunks and tiles.
+
+Table kernels and table spectra give every (particle, pixel, channel) product
+freely chosen factors, so what is tested is the contraction alone: operand
+slots, the skips by row, block and group of four particles, and the clearing
+between chunks.  With whole-number factors (exact in BF16, sums below 2^24)
+both forms are exact; with real ones an FP32 sum of m terms of magnitude sum A
+is off by at most (m + 1) 2^-24 A."""
+
+import numpy as np
+import pytest
+
+from martini_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(n, shape, spread, seed, whole):
+    rng = np.random.default_rng(seed)
+    nx, ny, nc = shape
+    rec = np.zeros(n, _lib.PARTICLE_DTYPE)
+    rec["ix"] = nx // 2 + rng.integers(-spread, spread + 1, n)
+    rec["iy"] = ny // 2 + rng.integers(-spread, spread + 1, n)
+    r = rng.choice([0, 1, 3, 9], n, p=[0.3, 0.3, 0.3, 0.1])
+    rec["r_kind"] = (r << 8) | _lib.KERNEL_TABLE
+    rec["c_lo"] = rng.integers(0, nc, n)
+    rec["c_hi"] = np.minimum(rec["c_lo"] + rng.integers(0, 40, n), nc - 1)
+    rec["k0"] = np.arange(n)
+    rec["amp"] = 1.0
+    if whole:
+        spectra = rng.integers(-100, 101, (n, nc)).astype(np.float32)
+    else:
+        spectra = (rng.normal(size=(n, nc)) * 10.0 ** rng.uniform(-3, 3, (n, 1))).astype(np.float32)
+    want, mag, terms = np.zeros(shape), np.zeros(shape), np.zeros(shape)
+    offs, weights, at = np.zeros(n, np.uint32), [], 0
+    for k in range(n):
+        i0, i1 = max(rec["ix"][k] - r[k], 0), min(rec["ix"][k] + r[k], nx - 1)
+        j0, j1 = max(rec["iy"][k] - r[k], 0), min(rec["iy"][k] + r[k], ny - 1)
+        offs[k] = at
+        if i0 > i1 or j0 > j1:
+            continue
+        size = (i1 - i0 + 1, j1 - j0 + 1)
+        w = (rng.integers(-16, 17, size) if whole else rng.normal(size=size)).astype(np.float32)
+        weights.append(w.ravel())
+        at += w.size
+        c = slice(rec["c_lo"][k], rec["c_hi"][k] + 1)
+        term = w.astype(float)[:, :, None] * spectra[k, c].astype(float)
+        box = (slice(i0, i1 + 1), slice(j0, j1 + 1), c)
+        want[box] += term
+        mag[box] += np.abs(term)
+        terms[box] += 1
+    rec["h"] = offs.view(np.float32)
+    return rec, spectra, np.concatenate(weights), want, mag, terms
+
+
+@pytest.mark.parametrize("method,whole", [("plain", False), ("plain", True), ("mfma", True)])
+@pytest.mark.parametrize("shape,spread", [((16, 16, 64), 6), ((33, 47, 70), 15),
+                                          ((8, 16, 128), 5), ((21, 40, 200), 12)])
+@pytest.mark.parametrize("n", [1, 3, 31, 32, 33, 63, 64, 65, 97, 129, 1000])
+def test_products(method, whole, shape, spread, n):
+    import torch
+
+    rec, spectra, weights, want, mag, terms = _case(n, shape, spread, n + shape[2], whole)
+    d_s, d_w = torch.from_numpy(spectra).cuda(), torch.from_numpy(weights).cuda()
+    desc = _lib.make_desc(*shape, _lib.SPECTRUM_TABLE, spectra=d_s, spectra_ld=shape[2])
+    desc.weights, desc.weights_n = d_w.data_ptr(), weights.size
+    pairs = _lib.count_pairs(rec, desc)
+    d_rec = torch.from_numpy(rec.view(np.uint8)).cuda()
+    cube = torch.zeros(want.size, dtype=torch.float32, device="cuda")
+    ws = torch.full((_lib.workspace_bytes(desc, n, pairs),), 255, dtype=torch.uint8, device="cuda")
+    _lib.insert(d_rec, n, pairs, desc, cube, ws, method=method)
+    got = cube.cpu().numpy().reshape(shape).astype(float)
+    if whole:
+        assert np.array_equal(got, want)
+        return
+    assert np.all(got[terms == 0] == 0.0)
+    worst = np.max(np.abs(got - want) - (terms + 1) * 2.0**-24 * mag)
+    assert worst <= 0.0, worst
