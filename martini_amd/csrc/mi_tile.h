@@ -3,9 +3,9 @@
 // clipped to the cell's tile, and W evaluated once per (particle, footprint
 // pixel) pair.
 //
-// Staging is done by one wave with wave-wide DPP scans (no serial loop): the
+// Staging is done by one wave, two chunks at once, with DPP scans (no serial loop): the
 // gathers pick the wave with the least product work in the previous chunk.
-// Every wave loads the next chunk's records while the current one is
+// Every wave loads the next chunks' records while the current ones are
 // processed, so the global-memory latency is hidden behind the W/S/accumulate
 // work.
 #pragma once
@@ -32,9 +32,21 @@ constexpr int LTAB_N = WTAB_N + 1;
 // row stride of the particle's weights.
 struct __attribute__((aligned(16))) WalkRec {
     double px, py;  // particle position ix + fx, iy + fy (exact in FP64)
-    double fa;      // WFactors::a: 1/h^2, or 1/(h sig)^2 for the Gaussian
-    int32_t ij;     // first row | first column << 16 of the clipped footprint
-    int32_t kw;     // kernel kind | footprint width << 8
+    float fa;       // tabulated kernels: 1/h^2
+    float b;        // Gaussian: WFactors::b
+    // the footprint clipped to the tile: its corner (row | column << 4), width
+    // (<< 8) and rows (<< 16)
+    uint32_t box;
+    // tile rows (bits 0..15) and 16-channel blocks (16..23) reached, zero without
+    // a footprint in the cell; kernel kind << 24 | Gaussian table index << 28
+    uint32_t cover;
+
+    __device__ int row() const { return box & 15; }
+    __device__ int col() const { return (box >> 4) & 15; }
+    __device__ int width() const { return (box >> 8) & 31; }
+    __device__ int rows() const { return box >> 16; }
+    __device__ int kind() const { return (cover >> 24) & 15; }
+    __device__ int gidx() const { return cover >> 28; }
 };
 
 // Weight-table walk of an MI_KERNEL_TABLE particle: weights[base + i * stride + j]
@@ -47,25 +59,29 @@ __device__ inline TableWalk table_walk(const WalkRec& w) {
     return TableWalk{__double_as_longlong(w.px), __double_as_longlong(w.py)};
 }
 
-// What the Gaussian walk needs beyond the WalkRec: WFactors::b, t, n and e,
-// at the WalkRec's 32-byte stride.
-struct __attribute__((aligned(16))) GaussRec {
-    float4 f;  // b, t, n, 0
-    double e;
-    double unused;
+// What the Gaussian walk needs beyond the WalkRec: WFactors::a and e.
+struct GaussRec {
+    double a, e;
 };
 
+// What the S fill needs of a particle: mi_particle's spectral fields, the window
+// clipped to the cell (first channel | last << 16, an empty one 1 | 0).
+struct SpecRec {
+    uint32_t window;
+    int32_t k0;
+    float fu, s, amp;
+};
+
+// One chunk's state, small enough that two chunks', with the 16 x 16 x 64 cells'
+// operand tiles, leave room for three work groups on a CU.
 struct ChunkState {
-    mi_particle p[KC];
     WalkRec walk[KC];
     GaussRec gr[KC];    // Gaussian kernel factors
-    uint32_t cover[KC]; // tile rows (low half) and 16-channel blocks (high half) a
-                        // particle reaches in the cell, zero without a footprint in it
-    int off[KC + 1];    // exclusive scan of the per-particle pair counts
+    SpecRec p[KC];
     // exclusive scan of the threads given to each particle's pairs (16-byte
     // aligned: fill_weights reads it eight entries at a time)
-    __attribute__((aligned(16))) int toff[KC + 1];
-    int per;            // pairs per thread
+    __attribute__((aligned(16))) uint16_t toff[KC + 1];
+    uint16_t per;       // pairs per thread
     uint32_t rowmask;   // tile rows (x offsets) touched by any footprint of the chunk
     uint32_t chanmask;  // 16-channel sub-blocks of the cell touched by any window
     uint32_t gmask;     // particles of the Gaussian kernel with a footprint in the tile
@@ -97,13 +113,18 @@ __device__ inline uint32_t wave_scan(uint32_t x, Op op) {
     return x;
 }
 
-__device__ inline int wave_scan_add(int x) {
-    return (int)wave_scan((uint32_t)x, [](uint32_t a, uint32_t b) { return a + b; });
+// The same within each half of the wave: lanes 0..31 and 32..63.
+template <class Op>
+__device__ inline uint32_t half_scan(uint32_t x, Op op) {
+    x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false));
+    x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false));
+    x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false));
+    x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false));
+    return op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false));
 }
 
-__device__ inline uint32_t wave_or(uint32_t x) {
-    return __builtin_amdgcn_readlane(wave_scan(x, [](uint32_t a, uint32_t b) { return a | b; }),
-                                     63);
+__device__ inline int wave_scan_add(int x) {
+    return (int)wave_scan((uint32_t)x, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 // A particle record held in registers between its prefetch and its staging,
@@ -147,13 +168,17 @@ __device__ inline float pick4(const float (&v)[4], int i) {
     return i == 0 ? v0 : i == 1 ? v1 : i == 2 ? v2 : v3;
 }
 
-// Called by all 64 lanes of one wave: lane t < KC holds particle t of the chunk
-// in `r` (valid when t < nk).  Clips footprints to the tile, scans the pair
-// counts, ORs the row and channel-block masks across the wave and forms each
-// particle's weight factors.
-__device__ inline void stage_chunk(const RecRegs& r, bool valid, int x0, int y0, int c0,
-                                   const Grid& g, const mi_cube_desc& d, ChunkState& cs) {
-    const int lane = threadIdx.x & 63;
+// Called by all 64 lanes of one wave, for two chunks at once: lane t holds
+// particle t % KC of chunk t / KC in `r`.  Clips footprints to the tile, scans
+// the pair counts, ORs the row and channel-block masks across each half of the
+// wave and forms each particle's weight factors.  The staging is on every
+// chunk's critical path (the other waves wait for it), and one wave's
+// instructions for two chunks are those of one.
+__device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0, int c0,
+                                    const Grid& g, const mi_cube_desc& d, ChunkState (&both)[2]) {
+    static_assert(KC == 32, "half a wave per chunk");
+    const int half = (threadIdx.x >> 5) & 1, lane = threadIdx.x & (KC - 1);
+    ChunkState& cs = both[half];
     const mi_particle p = unpack_record(r);
     // Straight-line code with selects: every lane forms the clipped footprint,
     // lanes without a particle or a footprint in the tile end with cnt = 0.
@@ -168,59 +193,61 @@ __device__ inline void stage_chunk(const RecRegs& r, bool valid, int x0, int y0,
     const uint32_t rows = ok ? (2u << (ihi - x0)) - (1u << (ilo - x0)) : 0u;
     const int ca = max(p.c_lo, c0) - c0, cb = min(p.c_hi, c0 + (1 << g.cb_shift) - 1) - c0;
     const uint32_t chans = ok && ca <= cb ? (2u << (cb >> 4)) - (1u << (ca >> 4)) : 0u;
-    const int incl = wave_scan_add(cnt);
+    const auto add = [](uint32_t a, uint32_t b) { return a + b; };
+    const auto bit_or = [](uint32_t a, uint32_t b) { return a | b; };
+    const int incl = (int)half_scan((uint32_t)cnt, add);
     static_assert(TILE_MAX <= 16 && GeoWide::CB / 16 <= 16, "rows and channel blocks share one word");
-    const uint32_t masks = wave_or(rows | (chans << 16));  // one reduction for both
-    const uint32_t gauss = (uint32_t)__ballot(lane < KC && cnt > 0 &&
-                                              kind_of(p.r_kind) == MI_KERNEL_GAUSS);
+    const uint32_t masks = half_scan(rows | (chans << 16), bit_or);  // one reduction for both
+    const uint64_t gauss = __ballot(cnt > 0 && kind_of(p.r_kind) == MI_KERNEL_GAUSS);
     // Each particle's pairs go to ceil(cnt / per) threads of their own, per =
     // ceil(total / (NT - KC)): at most total / per + KC <= NT threads in all.
-    const int total = __builtin_amdgcn_readlane(incl, 63);
-    const int per = max(1, (total + (NT - KC) - 1) / (NT - KC));
+    const int total0 = __builtin_amdgcn_readlane(incl, KC - 1);
+    const int total1 = __builtin_amdgcn_readlane(incl, 2 * KC - 1);
+    const int per0 = max(1, (total0 + (NT - KC) - 1) / (NT - KC));
+    const int per1 = max(1, (total1 + (NT - KC) - 1) / (NT - KC));
+    const int per = half ? per1 : per0;
     // ceil(cnt / per) = floor((cnt + per - 1 + 1/2) / per): the quotient lies at
     // least 1/74 from an integer (per <= 37), far beyond the reciprocal's error
     const float rper = __builtin_amdgcn_rcpf((float)per);
-    const int tincl = wave_scan_add((int)(((float)(cnt + per - 1) + 0.5f) * rper));
-    if (lane < KC) {
-        if (valid) cs.p[lane] = p;
-        cs.cover[lane] = rows | (chans << 16);
-        const int width = max(jhi - jlo + 1, 1);
-        cs.off[lane + 1] = incl;
-        cs.toff[lane + 1] = tincl;
-        if (cnt > 0) {
-            const int kind = kind_of(p.r_kind);
-            WFactors f;
-            if (kind == MI_KERNEL_GAUSS) {  // the truncation and norm only for the Gaussian
-                const int gi = gidx_of(p.r_kind);
-                f = weight_factors(kind, p.h, pick4(d.gauss_t, gi), pick4(d.gauss_inv_norm, gi));
-            } else {
-                f = weight_factors(kind, p.h, 0.0f, 0.0f);
-            }
-            WalkRec w;
-            w.px = (double)p.ix + (double)p.fx;
-            w.py = (double)p.iy + (double)p.fy;
-            if (kind == MI_KERNEL_TABLE) {
-                // its weights are laid out over its cube-clipped footprint
-                const int64_t stride = fj_hi - fj_lo + 1;
-                w.px = __longlong_as_double((int64_t)table_offset(p) - (int64_t)fi_lo * stride - fj_lo);
-                w.py = __longlong_as_double(stride);
-            }
-            w.fa = f.a;
-            w.ij = ilo | (jlo << 16);
-            w.kw = kind | (width << 8);
-            cs.walk[lane] = w;
-            if (kind == MI_KERNEL_GAUSS) {
-                cs.gr[lane] = GaussRec{make_float4(f.b, f.t, f.n, 0.0f), f.e, 0.0};
-            }
+    const int tincl = (int)half_scan((uint32_t)(((float)(cnt + per - 1) + 0.5f) * rper), add);
+    const bool window = valid && ca <= cb;
+    cs.p[lane] = SpecRec{window ? (uint32_t)ca | (uint32_t)cb << 16 : 1u, p.k0, p.fu, p.s, p.amp};
+    const int width = max(jhi - jlo + 1, 1);
+    cs.toff[lane + 1] = (uint16_t)tincl;
+    const int kind = kind_of(p.r_kind), gi = gidx_of(p.r_kind);
+    WalkRec w;
+    w.px = (double)p.ix + (double)p.fx;
+    w.py = (double)p.iy + (double)p.fy;
+    w.box = 0u;
+    w.cover = 0u;
+    w.b = 0.0f;
+    WFactors f{0.0, 0.0, 0.0f, 0.0f, 0.0f};
+    if (ok) {
+        w.box = (uint32_t)(ilo - x0) | (uint32_t)(jlo - y0) << 4 | (uint32_t)width << 8 |
+                (uint32_t)(ihi - ilo + 1) << 16;
+        w.cover = rows | (chans << 16) | (uint32_t)kind << 24 | (uint32_t)gi << 28;
+        if (kind == MI_KERNEL_GAUSS) {  // the truncation only for the Gaussian
+            f = weight_factors(kind, p.h, pick4(d.gauss_t, gi), 0.0f);
+            cs.gr[lane] = GaussRec{f.a, f.e};
+            w.b = f.b;
+        } else {
+            f = weight_factors(kind, p.h, 0.0f, 0.0f);
+        }
+        if (kind == MI_KERNEL_TABLE) {
+            // its weights are laid out over its cube-clipped footprint
+            const int64_t stride = fj_hi - fj_lo + 1;
+            w.px = __longlong_as_double((int64_t)table_offset(p) - (int64_t)fi_lo * stride - fj_lo);
+            w.py = __longlong_as_double(stride);
         }
     }
-    if (lane == 0) {
-        cs.off[0] = 0;
+    w.fa = f.b;
+    cs.walk[lane] = w;
+    if (lane == KC - 1) {  // holds its half's reductions
         cs.toff[0] = 0;
-        cs.per = per;
+        cs.per = (uint16_t)per;
         cs.rowmask = masks & 0xffffu;
         cs.chanmask = masks >> 16;
-        cs.gmask = gauss;
+        cs.gmask = (uint32_t)(gauss >> (half * KC));
     }
 }
 
@@ -249,17 +276,16 @@ __device__ inline float table_weight_select(const float4* __restrict__ tab, floa
 // particle t % KC and rows (then columns) t / KC, t / KC + NT / KC, ... of its
 // clipped footprint.  Loops end once no lane of the wave has a row (column)
 // left.  The values are weight_at's: the same offsets and spans.
-__device__ inline void fill_gauss_tables(const ChunkState& cs, GaussTables& gt) {
+__device__ inline void fill_gauss_tables(const ChunkState& cs, int x0, int y0, GaussTables& gt) {
     const int k = threadIdx.x & (KC - 1), slot = threadIdx.x / KC;
     const bool gk = (cs.gmask >> k) & 1u;
     const WalkRec w = cs.walk[k];
-    const float bf = cs.gr[k].f.x;
-    const int i0 = w.ij & 0xffff, j0 = w.ij >> 16;
-    const int rows = gk ? __builtin_popcount(cs.cover[k] & 0xffffu) : 0, cols = gk ? w.kw >> 8 : 0;
+    const int i0 = x0 + w.row(), j0 = y0 + w.col();
+    const int rows = gk ? w.rows() : 0, cols = gk ? w.width() : 0;
     for (int r = slot; __any(r < rows); r += NT / KC)
-        if (r < rows) gt.ex[k][r] = erf_span((float)(w.px - (double)(i0 + r)) * bf, bf);
+        if (r < rows) gt.ex[k][r] = erf_span((float)(w.px - (double)(i0 + r)) * w.b, w.b);
     for (int c = slot; __any(c < cols); c += NT / KC)
-        if (c < cols) gt.ey[k][c] = erf_span((float)(w.py - (double)(j0 + c)) * bf, bf);
+        if (c < cols) gt.ey[k][c] = erf_span((float)(w.py - (double)(j0 + c)) * w.b, w.b);
 }
 
 // The Gaussian kernel's weight as weight_at computes it, its separable
@@ -286,7 +312,7 @@ template <class Store, class Store2>
 __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
                                     const float4* __restrict__ wtab, int tab_kind,
                                     const float4* __restrict__ tab, const GaussTables& gt,
-                                    const float* __restrict__ uw, Store store, Store2 store2) {
+                                    const mi_cube_desc& d, Store store, Store2 store2) {
     const int t = threadIdx.x;
     const bool active = t < cs.toff[KC];
     // k = the last particle with toff[k] <= t (toff is non-decreasing, and
@@ -296,28 +322,29 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
     int k = 0;
     if (active) {
         const int m = 8 * ((cs.toff[8] <= t) + (cs.toff[16] <= t) + (cs.toff[24] <= t));
-        const int4 u = *reinterpret_cast<const int4*>(cs.toff + m);
-        const int4 v = *reinterpret_cast<const int4*>(cs.toff + m + 4);
-        k = m + (u.y <= t) + (u.z <= t) + (u.w <= t) + (v.x <= t) + (v.y <= t) + (v.z <= t) +
-            (v.w <= t);
+        const uint4 u = *reinterpret_cast<const uint4*>(cs.toff + m);  // eight entries
+        const uint32_t v[4] = {u.x, u.y, u.z, u.w};
+        k = m - 1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            k += ((int)(v[i] & 0xffffu) <= t) + ((int)(v[i] >> 16) <= t);
     }
     const WalkRec w = cs.walk[k];
-    const int width = w.kw >> 8, kind = w.kw & 255;
+    const int width = max(w.width(), 1), kind = w.kind();
     const int l0 = (t - cs.toff[k]) * cs.per;
-    const int l1 = active ? min(l0 + cs.per, cs.off[k + 1] - cs.off[k]) : l0;
+    const int l1 = active ? min(l0 + cs.per, w.rows() * width) : l0;
     // l0 / width: (l0 + 1/2) / width lies at least 1/32 from an integer (l0 <
     // 256 pixels, width <= 16), far beyond the reciprocal's error
     int a = (int)(((float)l0 + 0.5f) * __builtin_amdgcn_rcpf((float)width));
     int b = l0 - a * width;
-    const int ti = (w.ij & 0xffff) - x0, tj = (w.ij >> 16) - y0;  // footprint corner in the tile
-    const double px = w.px - (double)x0, py = w.py - (double)y0;   // particle in tile coordinates
+    const int ti = w.row(), tj = w.col();  // footprint corner in the tile
 
     if (tab_kind >= 0 && __all(!active || kind == tab_kind)) {
         // The particle's offset from the footprint's first pixel in FP32 (one
         // rounding of the exact FP64 value); q^2 follows in FP32, a few ulps
         // from the FP64 form, far below the table's own error.
-        const float gx = (float)(px - (double)ti), gy = (float)(py - (double)tj);
-        const float fa = (float)w.fa;
+        const float gx = (float)(w.px - (double)(x0 + ti)), gy = (float)(w.py - (double)(y0 + tj));
+        const float fa = w.fa;
         // Pixel l of the footprint lies in row floor((l + 1/2) / width) (exact, as
         // for a above) and column l - row * width, all small integers formed in
         // FP32: no wrap tests, and the offsets from the particle need no
@@ -366,7 +393,7 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
         const TableWalk tw = table_walk(w);
         for (int l = l0; l < l1; ++l) {
             const int i = x0 + ti + a, j = y0 + tj + b;
-            store(k, (ti + a) * TILE_Y + tj + b, uw[tw.base + (int64_t)i * tw.stride + j]);
+            store(k, (ti + a) * TILE_Y + tj + b, d.weights[tw.base + (int64_t)i * tw.stride + j]);
             if (++b == width) {
                 b = 0;
                 ++a;
@@ -376,12 +403,13 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
     }
     if (kind == MI_KERNEL_GAUSS || !active) {
         // Gaussian particles: the separable factors come from the chunk's tables
-        const double fe = cs.gr[k].e;
-        const float4 gg = cs.gr[k].f;
+        const GaussRec gg = cs.gr[k];
+        const int gi = w.gidx();
+        const float gt_t = pick4(d.gauss_t, gi), gt_n = pick4(d.gauss_inv_norm, gi);
         for (int l = l0; l < l1; ++l) {
             const int i = x0 + ti + a, j = y0 + tj + b;
             store(k, (ti + a) * TILE_Y + tj + b,
-                  gauss_weight(w.px - (double)i, w.py - (double)j, w.fa, fe, gg.y, gg.z,
+                  gauss_weight(w.px - (double)i, w.py - (double)j, gg.a, gg.e, gt_t, gt_n,
                                gt.ex[k][a], gt.ey[k][b]));
             if (++b == width) {
                 b = 0;
@@ -390,7 +418,7 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
         }
         return;
     }
-    const WFactors f{w.fa, 0.0, (float)w.fa, 0.0f, 0.0f};
+    const WFactors f{(double)w.fa, 0.0, w.fa, 0.0f, 0.0f};
     for (int l = l0; l < l1; ++l) {
         const int i = x0 + ti + a, j = y0 + tj + b;
         store(k, (ti + a) * TILE_Y + tj + b,
@@ -420,15 +448,16 @@ __device__ inline void fill_spectra(const ChunkState& cs, int nk, int c0, int nc
     static_assert(PER_BLOCK == 2, "a thread stores its two channels of a block together");
     const int k = threadIdx.x & (KC - 1);
     const int cl0 = threadIdx.x / KC;
-    const mi_particle& p = cs.p[k];
-    const bool live = k < nk;
-    const int lo = live ? p.c_lo : 1, hi = live ? min(p.c_hi, nc - 1) : 0;
+    const SpecRec p = cs.p[k];
+    // the window within the cell, empty past the item's last particle
+    const int lo = k < nk ? (int)(p.window & 0xffffu) : 1;
+    const int hi = k < nk ? min((int)(p.window >> 16), nc - 1 - c0) : 0;
     const int k0 = p.k0;
     const float fu = p.fu, s = p.s, amp = p.amp;
     const int spectrum = d.spectrum;
     // Channel cl0 + o of the cell lies in the window [lo, hi] when
     // (unsigned)(o - w0) <= wl; an empty window takes an offset no o reaches.
-    const int w0 = lo <= hi ? lo - c0 - cl0 : (1 << 30);
+    const int w0 = lo <= hi ? lo - cl0 : (1 << 30);
     const uint32_t wl = lo <= hi ? (uint32_t)(hi - lo) : 0u;
     auto inside = [&](int o) { return (uint32_t)(o - w0) <= wl; };
     auto put = [&](int b, float v0, float v1) {
