@@ -51,7 +51,7 @@ struct Layout {
     size_t keys, vals, keys2, vals2;   // uint32[n_pairs] each; vals2: particle index in cell order
     size_t item_off, multi_off;        // uint32[ncells + 1] each: exclusive scans of the
                                        // items and the partial-tile slots per cell
-    size_t full_pos, rest_pos;         // uint32[ncells] each: launch positions of a cell's items
+    size_t item_pos;                   // uint32[ncells]: launch position of a cell's first item
     size_t items;                      // int4[items_max], in launch order
     size_t partials;                   // float[multi_max * CELL_VOXELS]
     size_t part_masks;                 // uint64[multi_max]: the sub-tiles each partial holds
@@ -109,10 +109,11 @@ hipError_t cube_to_fits(const void* cube, bool cube_f64, int nx, int ny, int nc,
 hipError_t convolve_beam(const float* in, float* out, int nx, int ny, int nc, const float* K,
                          int kx, int ky, hipStream_t s);
 
-// One work item: particles [begin, end) of the sorted pair list belonging to
-// one cell; slot >= 0 names its partial tile, -1 means it writes the cube.
+// One work item: the q-th of a cell's n, which takes the cell's chunks q, q + n,
+// ... of the sorted pair list; slot >= 0 names its partial tile, -1 means it
+// writes the cube.
 struct Item {
-    int32_t cell, begin, end, slot;
+    int32_t cell, q, n, slot;
 };
 
 }  // namespace mi

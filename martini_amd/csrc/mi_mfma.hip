@@ -195,12 +195,15 @@ struct Float32 {
 template <class G, class F>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_gather(
     const mi_particle* __restrict__ P, const uint32_t* __restrict__ order,
-    const Item* __restrict__ items, const uint32_t* __restrict__ status,
+    const Item* __restrict__ items, const uint32_t* __restrict__ cell_start,
+    const uint32_t* __restrict__ cell_end, const uint32_t* __restrict__ status,
     const float4* __restrict__ wtab, Grid g, mi_cube_desc d, float* __restrict__ cube,
     float* __restrict__ partials, uint64_t* __restrict__ part_masks) {
     if (status[ST_OVERFLOW]) return;
     if (blockIdx.x >= status[ST_ITEMS]) return;
     const Item it = items[blockIdx.x];  // longest items first
+    const int begin = (int)cell_start[it.cell] + it.q * KC, end = (int)cell_end[it.cell];
+    const int step = it.n * KC;  // from one of the item's chunks to the next
     const CellPos cp = cell_pos(it.cell, g);
     const int x0 = cp.x0, y0 = cp.y0, c0 = cp.c0;
 
@@ -238,22 +241,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     // the two after.  Two chunks are staged together by the wave that had the
     // fewest (row, block) products in the chunk before (it reaches the staging
     // first); every wave picks it from the same row and channel-block masks.
-    const int tkind = stage_table(P, order, it.begin, wtab, Tk);
-    constexpr int KC2 = 2 * KC;
+    const int tkind = stage_table(P, order, begin, wtab, Tk);
+    const int at = (lane / KC) * step + (lane & (KC - 1));  // of the lane's particle from a chunk pair on
     RecRegs next{};
     uint32_t next_idx = 0;
-    if (lane < it.end - it.begin) next = load_record(P, order[it.begin + lane]);
-    if (lane < it.end - it.begin - KC2) next_idx = order[it.begin + KC2 + lane];
+    if (at < end - begin) next = load_record(P, order[begin + at]);
+    if (at + 2 * step < end - begin) next_idx = order[begin + 2 * step + at];
     int stager = 0;
 
-    for (int kb = it.begin; kb < it.end; kb += KC) {
-        const int half = ((kb - it.begin) / KC) & 1;
+    for (int kb = begin, half = 0; kb < end; kb += step, half ^= 1) {
         if (half == 0) {
-            if (wave == stager) stage_chunks(next, lane < it.end - kb, x0, y0, c0, g, d, both);
-            if (lane < it.end - kb - KC2) next = load_record(P, next_idx);
-            if (lane < it.end - kb - 2 * KC2) next_idx = order[kb + 2 * KC2 + lane];
+            const int left = end - kb;
+            if (wave == stager) stage_chunks(next, at < left, x0, y0, c0, g, d, both);
+            if (at + 2 * step < left) next = load_record(P, next_idx);
+            if (at + 4 * step < left) next_idx = order[kb + 4 * step + at];
         }
-        const int nk = min(KC, it.end - kb);
+        const int nk = min(KC, end - kb);
         const ChunkState& cs = both[half];
         __syncthreads();
         const uint32_t rowmask = __builtin_amdgcn_readfirstlane(cs.rowmask);
@@ -393,7 +396,8 @@ hipError_t gather(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, 
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)L.items_max), dim3(NT), 0, s, d_p,
                            (const uint32_t*)(ws + L.vals2), (const Item*)(ws + L.items),
-                           (const uint32_t*)(ws + L.status), wtab, g, d, d_cube,
+                           (const uint32_t*)(ws + L.cell_start),
+                           (const uint32_t*)(ws + L.cell_end), (const uint32_t*)(ws + L.status), wtab, g, d, d_cube,
                            (float*)(ws + L.partials), (uint64_t*)(ws + L.part_masks));
     };
     if (split_bf16) {
