@@ -112,18 +112,24 @@ def record_permutation(n: int, device):
     return torch.argsort(_mix32(_mix32(k) ^ 0x6D617274))
 
 
+def _room(d_rec, per_record: int) -> bool:
+    """Whether the records' device has `per_record` bytes a record free, and 1 GiB."""
+    import torch
+
+    if d_rec.device.type != "cuda":
+        return True
+    free, _ = torch.cuda.mem_get_info(d_rec.device)
+    free += torch.cuda.memory_reserved(d_rec.device) - torch.cuda.memory_allocated(d_rec.device)
+    n = d_rec.numel() // _lib.PARTICLE_DTYPE.itemsize
+    return free >= n * per_record + (1 << 30)
+
+
 def shuffle_records(d_rec):
     """Records (uint8 tensor of n * 48 bytes) in the fixed pseudo-random order
     of ``record_permutation``, gathered on the records' device.
 
-    The FP32 gather's coarse sort keeps a cell's particles in record order
-    within each bucket of its index hash, and takes them 32 at a time.
-    Records that arrive spatially ordered (as ordered snapshots do) would give
-    spatially compact chunks, which load one or two of the gather's four
-    waves; shuffled records give chunks spread over the tile whatever the input
-    order.  A structured reordering (a golden-ratio or other Weyl sweep) would
-    interact with the multiplicative index hash.  The inserted cube depends on
-    the order only through the FP32 summation order.
+    No gather wants this order any more (``layout_records``); it stands for
+    programs that call it, and for measuring records in random order.
 
     The shuffle needs, for a moment, a second copy of the records and the
     permutation with its sort space (taken as 32 bytes per record); when the
@@ -134,11 +140,8 @@ def shuffle_records(d_rec):
     n = d_rec.numel() // _lib.PARTICLE_DTYPE.itemsize
     if n <= 1:
         return d_rec
-    if d_rec.device.type == "cuda":
-        free, _ = torch.cuda.mem_get_info(d_rec.device)
-        free += torch.cuda.memory_reserved(d_rec.device) - torch.cuda.memory_allocated(d_rec.device)
-        if free < n * (_lib.PARTICLE_DTYPE.itemsize + 32) + (1 << 30):
-            return d_rec
+    if not _room(d_rec, _lib.PARTICLE_DTYPE.itemsize + 32):
+        return d_rec
     idx = record_permutation(n, d_rec.device)
     words = d_rec.view(torch.int32).view(n, _lib.PARTICLE_DTYPE.itemsize // 4)
     return words.index_select(0, idx).view(-1).view(torch.uint8)
@@ -161,10 +164,11 @@ def spatial_records(d_rec, nc=None):
     """Records (uint8 tensor of n * 48 bytes) sorted by the binning's pixel tile
     (``cell_tile(nc)``) of their pixel (ix, iy), tiles in its cell order
     (x-major), and by the pixel's Z order inside the tile (x and y bits
-    interleaved, x on the even bits).  The MFMA form's binning keeps the
-    record order within each cell, so its 32-particle chunks are then compact
-    patches of the tile, and a chunk reads neighbouring records, whole cache
-    lines instead of one 48-byte record per line.  Equal keys keep the given order (a stable sort),
+    interleaved, x on the even bits).  The binning orders each cell by tile
+    row and keeps the record order within, so that a chunk's 32 particles are a
+    compact patch of the tile and mostly neighbours in memory: whole cache lines
+    are read instead of one 48-byte record per line.  Equal keys keep the given
+    order (a stable sort),
     so the layout is the same on every device."""
     import torch
 
@@ -183,14 +187,22 @@ def spatial_records(d_rec, nc=None):
     return words.index_select(0, idx).view(-1).view(torch.uint8)
 
 
+# HBM that spatial_records needs for a moment, per record: the reordered copy,
+# the keys and their terms, and the sort's output and scratch.
+SPATIAL_BYTES = _lib.PARTICLE_DTYPE.itemsize + 96
+
+
 def layout_records(d_rec, method="plain", nc=None):
-    """The records' HBM layout for a gather method: shuffled for the FP32 form
-    (``shuffle_records``: its chunks should spread over the tile), in cell and
-    pixel Z order for the MFMA form (``spatial_records``: its chunks are
-    compact, and neighbouring reads then share cache lines).  The inserted cube
-    depends on the layout only through the FP32 summation order."""
-    if _lib.METHODS[method] == _lib.METHOD_PLAIN_F32:
-        return shuffle_records(d_rec)
+    """The records' HBM layout for a gather (``spatial_records``, for either
+    form: chunks are compact, products are skipped by tile row, and neighbouring
+    reads share cache lines).  The FP32 form keeps the given order when the device
+    has not the memory for the sort (``SPATIAL_BYTES`` a record and 1 GiB).  The
+    inserted cube depends on the layout only through the FP32 summation order,
+    and the speed by a few per cent, since the binning orders each cell's
+    particles too (heterogeneous 3e6 particles, FP32: 4.02 ms in random order,
+    3.74 laid out)."""
+    if _lib.METHODS[method] == _lib.METHOD_PLAIN_F32 and not _room(d_rec, SPATIAL_BYTES):
+        return d_rec
     return spatial_records(d_rec, nc)
 
 
