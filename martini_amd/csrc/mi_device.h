@@ -41,9 +41,10 @@ static_assert(GeoSquare::PX * GeoSquare::CB == CELL_VOXELS &&
 // either shape.  A partial tile stores them one after another, each 1 KiB
 // ([row][channel block][pixel][SUB_CH]).  Bit sub_bit(row, block) of its mask
 // is set where the item wrote that sub-tile; the others hold nothing of this
-// call and are read as zero.  The bits follow the MFMA gather's waves: wave
-// w = row / 4 + (TX / 4) * (block / 4) owns bits 16 w .. 16 w + 15 (4 (row % 4)
-// + block % 4), so each wave stores its own 16 bits.
+// call and are read as zero.  The bits follow the gather's waves: with RG = TX / 4
+// row groups and CG = 4 / RG channel groups, wave w = row % RG + RG * (block % CG)
+// owns bits 16 w .. 16 w + 15 (4 (row / RG) + block / CG), so each wave stores its
+// own 16 bits.
 constexpr int SUB_CH = 16;
 static_assert(GeoSquare::TX * (GeoSquare::CB / SUB_CH) == 64 &&
                   GeoWide::TX * (GeoWide::CB / SUB_CH) == 64,
@@ -52,7 +53,9 @@ __host__ __device__ constexpr int sub_offset(int cb_blocks, int row, int block, 
     return ((row * cb_blocks + block) * 16 + pixel) * 16;
 }
 __host__ __device__ constexpr int sub_bit(int tx_shift, int row, int block) {
-    return 16 * ((row >> 2) + ((1 << tx_shift) >> 2) * (block >> 2)) + (row & 3) * 4 + (block & 3);
+    const int rg_shift = tx_shift - 2, cg_shift = 4 - tx_shift;
+    const int wave = (row & ((1 << rg_shift) - 1)) | (block & ((1 << cg_shift) - 1)) << rg_shift;
+    return 16 * wave + (row >> rg_shift) * 4 + (block >> cg_shift);
 }
 constexpr bool sub_bits_distinct(int tx_shift, int rows, int blocks) {
     uint64_t seen = 0u;
