@@ -82,12 +82,15 @@ __host__ __device__ inline bool wide_cells(int nc) { return nc >= 128; }
 // as run at once (ITEM_FILL: three work groups on each of 256 CUs) and no more,
 // since each split costs a partial tile.  13000 pairs, FP32, in items of 256
 // (52 of them): 159 us per insertion, of 32: 107; 1.7e5 pairs, MFMA: 154 us in
-// 768 items, 167 in 2048.  The partial tiles of ITEM_FILL items take at most
+// 768 items, 167 in 2048.  ITEM_TARGET also bounds the FP32 error, which grows with
+// the longest run summed before the FP64 reduction: 1.4e6 particles, 512 x 512 x
+// 256, FP32, relative to FP64: 6.0e-7 with 2048 items, 5.2e-7 with 2304, 3.6e-7
+// with 3072; 1e6 particles, FP32: 556, 557 and 573 us per insertion.  The partial tiles of ITEM_FILL items take at most
 // 101 MB of workspace, the cells of the largest grid beside them 84 MB.
 constexpr int ITEM_MIN = 32;
 constexpr int ITEM_WHOLE = 256;
 constexpr int ITEM_MAX = 4096;
-constexpr int ITEM_TARGET = 2048;
+constexpr int ITEM_TARGET = 2304;
 constexpr int ITEM_FILL = 768;
 
 __host__ __device__ inline int item_length(int64_t n_pairs) {
