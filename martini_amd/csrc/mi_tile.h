@@ -25,15 +25,18 @@ constexpr int NT = 256;   // threads per work group
 // after them, which the branch-free walk reads for q >= 1.
 constexpr int LTAB_N = WTAB_N + 1;
 
-// What the W walk needs of a particle, read with two 16-byte loads whenever
-// a thread moves on to the next particle.
-// For MI_KERNEL_TABLE particles px and py hold instead, as int64 bits
-// (table_walk), the index of pixel (0, 0) in the caller's weight table and the
-// row stride of the particle's weights.
+// What the W walk needs of a particle, read with two 16-byte loads by every
+// thread that takes some of its pixels.  px, py hold
+//   the particle's position ix + fx, iy + fy (exact in FP64) for the Gaussian kernel;
+//   its offsets from the footprint's first pixel in FP32 (tile_offset; one
+//   rounding of the exact value) for the other closed forms, whose position is
+//   in the chunk's GaussRec slot;
+//   as int64 bits (table_walk) the index of pixel (0, 0) in the caller's weight
+//   table and the row stride of the particle's weights for MI_KERNEL_TABLE.
 struct __attribute__((aligned(16))) WalkRec {
-    double px, py;  // particle position ix + fx, iy + fy (exact in FP64)
-    float fa;       // tabulated kernels: 1/h^2
-    float b;        // Gaussian: WFactors::b
+    double px, py;
+    float f;         // WFactors::b
+    uint32_t first;  // the first of the threads that share its pixels
     // the footprint clipped to the tile: its corner (row | column << 4), width
     // (<< 8) and rows (<< 16)
     uint32_t box;
@@ -49,6 +52,13 @@ struct __attribute__((aligned(16))) WalkRec {
     __device__ int gidx() const { return cover >> 28; }
 };
 
+__device__ inline double pack_offset(float gx, float gy) {
+    return __hiloint2double(__float_as_int(gy), __float_as_int(gx));
+}
+__device__ inline float2 tile_offset(const WalkRec& w) {
+    return make_float2(__int_as_float(__double2loint(w.px)), __int_as_float(__double2hiint(w.px)));
+}
+
 // Weight-table walk of an MI_KERNEL_TABLE particle: weights[base + i * stride + j]
 // is its weight at pixel (i, j).
 struct TableWalk {
@@ -59,7 +69,8 @@ __device__ inline TableWalk table_walk(const WalkRec& w) {
     return TableWalk{__double_as_longlong(w.px), __double_as_longlong(w.py)};
 }
 
-// What the Gaussian walk needs beyond the WalkRec: WFactors::a and e.
+// What the Gaussian walk needs beyond the WalkRec: WFactors::a and e.  For the
+// other closed forms: the particle's position.
 struct GaussRec {
     double a, e;
 };
@@ -78,10 +89,11 @@ struct ChunkState {
     WalkRec walk[KC];
     GaussRec gr[KC];    // Gaussian kernel factors
     SpecRec p[KC];
-    // exclusive scan of the threads given to each particle's pairs (16-byte
-    // aligned: fill_weights reads it eight entries at a time)
-    __attribute__((aligned(16))) uint16_t toff[KC + 1];
-    uint16_t per;       // pairs per thread
+    // Bit t: thread t + 1 is the first of a particle; and, a byte per wave, how
+    // many of the bits belong to the waves before.
+    __attribute__((aligned(16))) uint32_t starts[NT / 32];
+    uint32_t started;
+    uint32_t per;       // pairs per thread
     uint32_t rowmask;   // tile rows (x offsets) touched by any footprint of the chunk
     uint32_t chanmask;  // 16-channel sub-blocks of the cell touched by any window
     uint32_t gmask;     // particles of the Gaussian kernel with a footprint in the tile
@@ -199,8 +211,10 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
     static_assert(TILE_MAX <= 16 && GeoWide::CB / 16 <= 16, "rows and channel blocks share one word");
     const uint32_t masks = half_scan(rows | (chans << 16), bit_or);  // one reduction for both
     const uint64_t gauss = __ballot(cnt > 0 && kind_of(p.r_kind) == MI_KERNEL_GAUSS);
-    // Each particle's pairs go to ceil(cnt / per) threads of their own, per =
-    // ceil(total / (NT - KC)): at most total / per + KC <= NT threads in all.
+    // Each particle's pairs go to max(1, ceil(cnt / per)) threads of their own, per
+    // = ceil(total / (NT - KC)): at most total / per + KC <= NT threads in all.  No
+    // two particles share a first thread, so a thread finds its particle by counting
+    // the first threads up to itself (one bit each).
     const int total0 = __builtin_amdgcn_readlane(incl, KC - 1);
     const int total1 = __builtin_amdgcn_readlane(incl, 2 * KC - 1);
     const int per0 = max(1, (total0 + (NT - KC) - 1) / (NT - KC));
@@ -209,18 +223,30 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
     // ceil(cnt / per) = floor((cnt + per - 1 + 1/2) / per): the quotient lies at
     // least 1/74 from an integer (per <= 37), far beyond the reciprocal's error
     const float rper = __builtin_amdgcn_rcpf((float)per);
-    const int tincl = (int)half_scan((uint32_t)(((float)(cnt + per - 1) + 0.5f) * rper), add);
+    const int threads = max((int)(((float)(cnt + per - 1) + 0.5f) * rper), 1);
+    const int first = (int)half_scan((uint32_t)threads, add) - threads;
+    if (lane < NT / 32) cs.starts[lane] = 0u;
+    if (lane > 0)
+        __hip_atomic_fetch_or(&cs.starts[(first - 1) >> 5], 1u << ((first - 1) & 31),
+                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    uint32_t started = 0u;
+    static_assert(NT / 64 == 4 && KC <= 255, "a byte per wave");
+#pragma unroll
+    for (int v = 1; v < NT / 64; ++v) {
+        const uint64_t b = __ballot(lane > 0 && first <= 64 * v);
+        started |= (uint32_t)__builtin_popcount((uint32_t)(b >> (half * KC))) << (8 * v);
+    }
     const bool window = valid && ca <= cb;
     cs.p[lane] = SpecRec{window ? (uint32_t)ca | (uint32_t)cb << 16 : 1u, p.k0, p.fu, p.s, p.amp};
     const int width = max(jhi - jlo + 1, 1);
-    cs.toff[lane + 1] = (uint16_t)tincl;
     const int kind = kind_of(p.r_kind), gi = gidx_of(p.r_kind);
     WalkRec w;
-    w.px = (double)p.ix + (double)p.fx;
-    w.py = (double)p.iy + (double)p.fy;
+    const double px = (double)p.ix + (double)p.fx, py = (double)p.iy + (double)p.fy;
+    w.px = px;
+    w.py = py;
+    w.first = (uint32_t)first;
     w.box = 0u;
     w.cover = 0u;
-    w.b = 0.0f;
     WFactors f{0.0, 0.0, 0.0f, 0.0f, 0.0f};
     if (ok) {
         w.box = (uint32_t)(ilo - x0) | (uint32_t)(jlo - y0) << 4 | (uint32_t)width << 8 |
@@ -229,9 +255,10 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
         if (kind == MI_KERNEL_GAUSS) {  // the truncation only for the Gaussian
             f = weight_factors(kind, p.h, pick4(d.gauss_t, gi), 0.0f);
             cs.gr[lane] = GaussRec{f.a, f.e};
-            w.b = f.b;
         } else {
             f = weight_factors(kind, p.h, 0.0f, 0.0f);
+            cs.gr[lane] = GaussRec{px, py};
+            w.px = pack_offset((float)(px - (double)ilo), (float)(py - (double)jlo));
         }
         if (kind == MI_KERNEL_TABLE) {
             // its weights are laid out over its cube-clipped footprint
@@ -240,11 +267,11 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
             w.py = __longlong_as_double(stride);
         }
     }
-    w.fa = f.b;
+    w.f = f.b;
     cs.walk[lane] = w;
     if (lane == KC - 1) {  // holds its half's reductions
-        cs.toff[0] = 0;
-        cs.per = (uint16_t)per;
+        cs.started = started;
+        cs.per = (uint32_t)per;
         cs.rowmask = masks & 0xffffu;
         cs.chanmask = masks >> 16;
         cs.gmask = (uint32_t)(gauss >> (half * KC));
@@ -283,9 +310,9 @@ __device__ inline void fill_gauss_tables(const ChunkState& cs, int x0, int y0, G
     const int i0 = x0 + w.row(), j0 = y0 + w.col();
     const int rows = gk ? w.rows() : 0, cols = gk ? w.width() : 0;
     for (int r = slot; __any(r < rows); r += NT / KC)
-        if (r < rows) gt.ex[k][r] = erf_span((float)(w.px - (double)(i0 + r)) * w.b, w.b);
+        if (r < rows) gt.ex[k][r] = erf_span((float)(w.px - (double)(i0 + r)) * w.f, w.f);
     for (int c = slot; __any(c < cols); c += NT / KC)
-        if (c < cols) gt.ey[k][c] = erf_span((float)(w.py - (double)(j0 + c)) * w.b, w.b);
+        if (c < cols) gt.ey[k][c] = erf_span((float)(w.py - (double)(j0 + c)) * w.f, w.f);
 }
 
 // The Gaussian kernel's weight as weight_at computes it, its separable
@@ -303,9 +330,12 @@ __device__ inline float gauss_weight(double dx, double dy, double fa, double fe,
 // Evaluates W for every (particle, pixel) pair of the chunk and hands each
 // value to store(k, pixel-in-tile, w), or two of them to
 // store2(k, pixel1, w1, pixel2, w2).  Particle k's pairs (pixel row l / width,
-// column l % width of its clipped footprint, l < cnt) are split over threads
-// toff[k] .. toff[k+1] - 1, `per` consecutive pairs each, so a thread stays on
-// one particle: one search of the thread scan, then a walk over its pixels.  When every
+// column l % width of its clipped footprint, l < cnt) are split over the threads
+// from its first one on, `per` consecutive pairs each, so a thread stays on one
+// particle.  It finds the particle by counting start bits: a search of the
+// threads' scan (three dependent LDS reads and 30 instructions, for 3 or 4 pixels)
+// cost 1 to 2% of an insertion (1e7 particles, split BF16: 5.04 -> 4.97 ms; 1e6,
+// FP32: 556 -> 547 us).  When every
 // particle of the wave's pairs uses the item's LDS table, the walk is
 // branch-free and takes two pixels per step, whose evaluations overlap.
 template <class Store, class Store2>
@@ -314,37 +344,23 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
                                     const float4* __restrict__ tab, const GaussTables& gt,
                                     const mi_cube_desc& d, Store store, Store2 store2) {
     const int t = threadIdx.x;
-    const bool active = t < cs.toff[KC];
-    // k = the last particle with toff[k] <= t (toff is non-decreasing, and
-    // particles without pairs share their successor's offset), in two rounds of
-    // LDS reads: the eighth it lies in, then the entries of that eighth.
-    static_assert(KC == 32, "the two-round search covers 32 particles");
-    int k = 0;
-    if (active) {
-        const int m = 8 * ((cs.toff[8] <= t) + (cs.toff[16] <= t) + (cs.toff[24] <= t));
-        const uint4 u = *reinterpret_cast<const uint4*>(cs.toff + m);  // eight entries
-        const uint32_t v[4] = {u.x, u.y, u.z, u.w};
-        k = m - 1;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            k += ((int)(v[i] & 0xffffu) <= t) + ((int)(v[i] >> 16) <= t);
-    }
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint2 starts = *reinterpret_cast<const uint2*>(cs.starts + 2 * wave);
+    const uint32_t before = (cs.started >> (8 * wave)) & 255u;
+    const int k = (int)__builtin_amdgcn_mbcnt_hi(starts.y, __builtin_amdgcn_mbcnt_lo(starts.x, before));
+    const int per = (int)cs.per;
     const WalkRec w = cs.walk[k];
     const int width = max(w.width(), 1), kind = w.kind();
-    const int l0 = (t - cs.toff[k]) * cs.per;
-    const int l1 = active ? min(l0 + cs.per, w.rows() * width) : l0;
-    // l0 / width: (l0 + 1/2) / width lies at least 1/32 from an integer (l0 <
-    // 256 pixels, width <= 16), far beyond the reciprocal's error
-    int a = (int)(((float)l0 + 0.5f) * __builtin_amdgcn_rcpf((float)width));
-    int b = l0 - a * width;
+    const int l0 = (t - (int)w.first) * per;
+    const int l1 = min(l0 + per, w.rows() * w.width());
+    const bool active = l0 < l1;
     const int ti = w.row(), tj = w.col();  // footprint corner in the tile
 
     if (tab_kind >= 0 && __all(!active || kind == tab_kind)) {
-        // The particle's offset from the footprint's first pixel in FP32 (one
-        // rounding of the exact FP64 value); q^2 follows in FP32, a few ulps
-        // from the FP64 form, far below the table's own error.
-        const float gx = (float)(w.px - (double)(x0 + ti)), gy = (float)(w.py - (double)(y0 + tj));
-        const float fa = w.fa;
+        // q^2 in FP32 from the offset, a few ulps from the FP64 form, far below the
+        // table's own error.
+        const float gx = tile_offset(w).x, gy = tile_offset(w).y;
+        const float fa = w.f;
         // Pixel l of the footprint lies in row floor((l + 1/2) / width) (exact, as
         // for a above) and column l - row * width, all small integers formed in
         // FP32: no wrap tests, and the offsets from the particle need no
@@ -388,6 +404,10 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
         return;
     }
 
+    // l0 / width: (l0 + 1/2) / width lies at least 1/32 from an integer (l0 <
+    // 256 pixels, width <= 16), far beyond the reciprocal's error
+    int a = (int)(((float)l0 + 0.5f) * __builtin_amdgcn_rcpf((float)width));
+    int b = l0 - a * width;
     if (kind == MI_KERNEL_TABLE) {
         // the caller's weights (binning checked that they lie inside the table)
         const TableWalk tw = table_walk(w);
@@ -418,11 +438,12 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
         }
         return;
     }
-    const WFactors f{(double)w.fa, 0.0, w.fa, 0.0f, 0.0f};
+    const WFactors f{(double)w.f, 0.0, w.f, 0.0f, 0.0f};
+    const GaussRec at = cs.gr[k];
     for (int l = l0; l < l1; ++l) {
         const int i = x0 + ti + a, j = y0 + tj + b;
         store(k, (ti + a) * TILE_Y + tj + b,
-              weight_at(kind, w.px - (double)i, w.py - (double)j, f, wtab, tab_kind, tab));
+              weight_at(kind, at.a - (double)i, at.e - (double)j, f, wtab, tab_kind, tab));
         if (++b == width) {
             b = 0;
             ++a;
