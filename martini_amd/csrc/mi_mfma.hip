@@ -35,16 +35,17 @@
 // on average on the 1e6 particles below): dealt out one by one they are shared by
 // the waves, where four adjacent ones were one wave's work that the others
 // waited for (1e6 particles, FP32: insertion 627 -> 559 us; the split form,
-// whose products are cheap, stays as it was).  The wave that stages the next
-// chunks runs ahead of the others on its SIMD (1e7 particles, split BF16: 5.07 ->
+// whose products are cheap, stays as it was).  The waves that stage the next
+// chunks run ahead of the others on their SIMD (1e7 particles, split BF16: 5.07 ->
 // 5.05 ms; 3e6 heterogeneous ones, FP32: 3.56 -> 3.54 ms).
 // A (row, channel-block) product is skipped when no footprint of the chunk
 // touches the row or no spectral window touches the block; the masks are
 // wave-uniform, so the skips are scalar branches.
 //
-// Two chunks are staged at a time, one per half of a wave: the staging is on
-// every chunk's critical path, and staging one at a time left half its lanes
-// idle (1e7 particles, 512 x 512 x 256, split BF16: gather 4.47 -> 4.32 ms).
+// Chunks are staged one per half of a wave, four at a time by two waves: the
+// staging is on every chunk's critical path, and half its lanes were idle with one
+// at a time (1e7 particles, 512 x 512 x 256, split BF16: gather 4.47 -> 4.32 ms;
+// four at a time: see STAGED).
 // Per chunk there are two barriers: (staging) -> W, S fill -> products, and a
 // third in chunks with Gaussian-kernel particles, whose row and column factors
 // are tabulated before the W fill.  Each wave clears the W rows it used right
@@ -197,11 +198,20 @@ struct Float32 {
     using Tile = FloatTile<ROWS>;
 };
 
+// Chunks staged at a time, two by each of STAGED / 2 waves at once: the other waves
+// wait for the staging, and with two chunks by one wave they did so twice as
+// often (1e7 particles, 512 x 512 x 256, split BF16: 4.99 -> 4.83 ms; 3e6
+// heterogeneous ones, FP32: 3.53 -> 3.47).  Eight by all four would leave LDS for
+// two work groups on a CU only.
+constexpr int STAGED = 4;
+static_assert(STAGED % 2 == 0 && STAGED <= NT / 32 && (STAGED & (STAGED - 1)) == 0,
+              "whole waves, and a power of two");
+
 // Bits 0, n, 2 n and 3 n.
 constexpr uint32_t every(int n) { return 1u | 1u << n | 1u << 2 * n | 1u << 3 * n; }
 
 // Three waves per SIMD: the 64 accumulators then live in VGPRs and three work
-// groups share a CU (LDS 48 KB each).
+// groups share a CU (LDS 49 and 53 KB each).
 template <class G, class F>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_gather(
     const mi_particle* __restrict__ P, const uint32_t* __restrict__ order,
@@ -221,9 +231,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     using STile = typename F::template Tile<G::CB>;
     __shared__ WTile W;            // [pixel][k]
     __shared__ STile S;            // [channel][k]
-    __shared__ ChunkState both[2]; // two chunks, staged together
+    __shared__ ChunkState staged[STAGED];  // chunks staged together
     __shared__ float4 Tk[LTAB_N];  // the item's kernel table
-    __shared__ GaussTables gt;     // the chunk's Gaussian-kernel factors
+    // The chunk's Gaussian-kernel factors.  The square cells' lie in the S tile, for
+    // which such a chunk waits once more: three work groups share the LDS then.
+    constexpr bool GT_IN_S = G::PX > G::CB;
+    __shared__ __attribute__((aligned(16))) char gt_own[GT_IN_S ? 16 : sizeof(GaussTables)];
+    static_assert(sizeof(GaussTables) <= sizeof(STile), "the factors fit the S tile");
+    GaussTables& gt = *reinterpret_cast<GaussTables*>(GT_IN_S ? reinterpret_cast<char*>(&S) : gt_own);
     // Waves: RG groups of four tile rows x CGN groups of four 16-channel blocks,
     // rows rh, rh + RG, ... and blocks ch, ch + CGN, ...
     constexpr int RG = G::TX / 4, CGN = G::CB / 64;
@@ -249,46 +264,33 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) acc[r][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    // Every wave holds the records of the next two chunks and the sort indices of
-    // the two after.  Two chunks are staged together by the wave that had the
-    // fewest (row, block) products in the chunk before (it reaches the staging
-    // first); every wave picks it from the same row and channel-block masks.
+    // STAGED chunks are staged at a time, two by each of two waves, which hold the
+    // records of their two of the next STAGED and the sort indices of those after.
     const int tkind = stage_table(P, order, begin, wtab, Tk);
-    const int at = (lane / KC) * step + (lane & (KC - 1));  // of the lane's particle from a chunk pair on
+    // Odd work groups stage with their last waves: every SIMD has its share.
+    const int pair = (wave + (int)blockIdx.x * 2) & (NT / 64 - 1);
+    const int at = (2 * pair + lane / KC) * step + (lane & (KC - 1));  // the lane's particle
+    const bool stages = 2 * pair < STAGED;
     RecRegs next{};
     uint32_t next_idx = 0;
-    if (at < end - begin) next = load_record(P, order[begin + at]);
-    if (at + 2 * step < end - begin) next_idx = order[begin + 2 * step + at];
-    int stager = 0;
+    if (stages && at < end - begin) next = load_record(P, order[begin + at]);
+    if (stages && at + STAGED * step < end - begin) next_idx = order[begin + STAGED * step + at];
 
-    for (int kb = begin, half = 0; kb < end; kb += step, half ^= 1) {
-        if (half == 0) {
-            const int left = end - kb;
-            if (wave == stager) {  // the other waves wait for it: first on its SIMD
-                __builtin_amdgcn_s_setprio(3);
-                stage_chunks(next, at < left, x0, y0, c0, g, d, both);
-                __builtin_amdgcn_s_setprio(0);
-            }
-            if (at + 2 * step < left) next = load_record(P, next_idx);
-            if (at + 4 * step < left) next_idx = order[kb + 4 * step + at];
+    for (int kb = begin, slot = 0; kb < end; kb += step, slot = (slot + 1) & (STAGED - 1)) {
+        const int left = end - kb;
+        if (slot == 0 && stages && 2 * pair * step < left) {
+            __builtin_amdgcn_s_setprio(3);  // the other waves wait for it: first on its SIMD
+            stage_chunks(next, at < left, x0, y0, c0, g, d, staged + 2 * pair);
+            __builtin_amdgcn_s_setprio(0);
+            if (at + STAGED * step < left) next = load_record(P, next_idx);
+            if (at + 2 * STAGED * step < left) next_idx = order[kb + 2 * STAGED * step + at];
         }
-        const int nk = min(KC, end - kb);
-        const ChunkState& cs = both[half];
+        const ChunkState& cs = staged[slot];
         __syncthreads();
-        const uint32_t rowmask = __builtin_amdgcn_readfirstlane(cs.rowmask);
-        const uint32_t chanmask = __builtin_amdgcn_readfirstlane(cs.chanmask);
+        const uint32_t rowmask = __builtin_amdgcn_readfirstlane(cs.rowmask());
+        const uint32_t chanmask = __builtin_amdgcn_readfirstlane(cs.chanmask());
         const uint32_t rows = (rowmask >> rh) & ROW_BITS;
         const uint32_t chans = (chanmask >> ch) & BLK_BITS;
-        int fewest = 17;
-#pragma unroll
-        for (int w2 = 0; w2 < NT / 64; ++w2) {
-            const int c = __builtin_popcount((rowmask >> (w2 % RG)) & ROW_BITS) *
-                          __builtin_popcount((chanmask >> (w2 / RG)) & BLK_BITS);
-            if (c < fewest) {
-                fewest = c;
-                stager = w2;
-            }
-        }
         if (cs.gmask != 0u) {  // the same for every thread
             fill_gauss_tables(cs, x0, y0, gt);
             __syncthreads();
@@ -296,7 +298,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         fill_weights(cs, x0, y0, wtab, tkind, Tk, gt, d,
                      [&](int k, int px, float w) { W.put(px, k, w); },
                      [&](int k, int p1, float w1, int p2, float w2) { W.put2(k, p1, w1, p2, w2); });
-        fill_spectra<G::CB>(cs, nk, c0, g.nc, d,
+        if (GT_IN_S && cs.gmask != 0u) __syncthreads();
+        fill_spectra<G::CB>(cs, c0, d,
                      [&](int k, int c1, float s1, int c2, float s2) { S.put_pairs(k, c1, s1, c2, s2); },
                      chanmask);
         // FP32: the particles (bits) that reach each of this wave's rows and blocks

@@ -3,11 +3,10 @@
 // clipped to the cell's tile, and W evaluated once per (particle, footprint
 // pixel) pair.
 //
-// Staging is done by one wave, two chunks at once, with DPP scans (no serial loop): the
-// gathers pick the wave with the least product work in the previous chunk.
-// Every wave loads the next chunks' records while the current ones are
-// processed, so the global-memory latency is hidden behind the W/S/accumulate
-// work.
+// A wave stages two chunks at once, with DPP scans (no serial loop), while its
+// work group waits; it loads the records of the next two while the current ones
+// are processed, so the global-memory latency is hidden behind the
+// W/S/accumulate work.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -36,7 +35,10 @@ constexpr int LTAB_N = WTAB_N + 1;
 struct __attribute__((aligned(16))) WalkRec {
     double px, py;
     float f;         // WFactors::b
-    uint32_t first;  // the first of the threads that share its pixels
+    // the first of the threads that share its pixels; and, << 16, its spectral window
+    // clipped to the cell and the cube: first channel | channels past it << 8,
+    // NO_WINDOW when empty
+    uint32_t first_win;
     // the footprint clipped to the tile: its corner (row | column << 4), width
     // (<< 8) and rows (<< 16)
     uint32_t box;
@@ -44,6 +46,9 @@ struct __attribute__((aligned(16))) WalkRec {
     // a footprint in the cell; kernel kind << 24 | Gaussian table index << 28
     uint32_t cover;
 
+    __device__ int first() const { return first_win & 255u; }
+    __device__ int win_lo() const { return (first_win >> 16) & 255u; }
+    __device__ uint32_t win_past() const { return first_win >> 24; }
     __device__ int row() const { return box & 15; }
     __device__ int col() const { return (box >> 4) & 15; }
     __device__ int width() const { return (box >> 8) & 31; }
@@ -75,16 +80,17 @@ struct GaussRec {
     double a, e;
 };
 
-// What the S fill needs of a particle: mi_particle's spectral fields, the window
-// clipped to the cell (first channel | last << 16, an empty one 1 | 0).
-struct SpecRec {
-    uint32_t window;
+constexpr uint32_t NO_WINDOW = 255u;  // no channel of a cell lies there
+
+// What the S fill needs of a particle beside its window: mi_particle's fields.
+struct __attribute__((aligned(16))) SpecRec {
     int32_t k0;
     float fu, s, amp;
 };
 
-// One chunk's state, small enough that two chunks', with the 16 x 16 x 64 cells'
-// operand tiles, leave room for three work groups on a CU.
+// One chunk's state, small enough that four chunks', with the 16 x 16 x 64 cells'
+// operand tiles, leave room for three work groups on a CU (2096 bytes; 192 more
+// in all would not).
 struct ChunkState {
     WalkRec walk[KC];
     GaussRec gr[KC];    // Gaussian kernel factors
@@ -93,10 +99,15 @@ struct ChunkState {
     // many of the bits belong to the waves before.
     __attribute__((aligned(16))) uint32_t starts[NT / 32];
     uint32_t started;
-    uint32_t per;       // pairs per thread
-    uint32_t rowmask;   // tile rows (x offsets) touched by any footprint of the chunk
-    uint32_t chanmask;  // 16-channel sub-blocks of the cell touched by any window
+    // tile rows (x offsets; bits 0..15) touched by any footprint of the chunk and
+    // 16-channel blocks of the cell (16..23) touched by any window; pairs per
+    // thread << 24
+    uint32_t cover_per;
     uint32_t gmask;     // particles of the Gaussian kernel with a footprint in the tile
+
+    __device__ uint32_t rowmask() const { return cover_per & 0xffffu; }
+    __device__ uint32_t chanmask() const { return (cover_per >> 16) & 255u; }
+    __device__ int per() const { return (int)(cover_per >> 24); }
 };
 
 // The separable factors of the Gaussian kernel's pixel weight for the chunk's
@@ -187,7 +198,7 @@ __device__ inline float pick4(const float (&v)[4], int i) {
 // chunk's critical path (the other waves wait for it), and one wave's
 // instructions for two chunks are those of one.
 __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0, int c0,
-                                    const Grid& g, const mi_cube_desc& d, ChunkState (&both)[2]) {
+                                    const Grid& g, const mi_cube_desc& d, ChunkState* both) {
     static_assert(KC == 32, "half a wave per chunk");
     const int half = (threadIdx.x >> 5) & 1, lane = threadIdx.x & (KC - 1);
     ChunkState& cs = both[half];
@@ -236,15 +247,16 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
         const uint64_t b = __ballot(lane > 0 && first <= 64 * v);
         started |= (uint32_t)__builtin_popcount((uint32_t)(b >> (half * KC))) << (8 * v);
     }
-    const bool window = valid && ca <= cb;
-    cs.p[lane] = SpecRec{window ? (uint32_t)ca | (uint32_t)cb << 16 : 1u, p.k0, p.fu, p.s, p.amp};
+    const int cl = min(cb, g.nc - 1 - c0);
+    const uint32_t window = valid && ca <= cl ? (uint32_t)ca | (uint32_t)(cl - ca) << 8 : NO_WINDOW;
+    cs.p[lane] = SpecRec{p.k0, p.fu, p.s, p.amp};
     const int width = max(jhi - jlo + 1, 1);
     const int kind = kind_of(p.r_kind), gi = gidx_of(p.r_kind);
     WalkRec w;
     const double px = (double)p.ix + (double)p.fx, py = (double)p.iy + (double)p.fy;
     w.px = px;
     w.py = py;
-    w.first = (uint32_t)first;
+    w.first_win = (uint32_t)first | window << 16;
     w.box = 0u;
     w.cover = 0u;
     WFactors f{0.0, 0.0, 0.0f, 0.0f, 0.0f};
@@ -271,9 +283,7 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
     cs.walk[lane] = w;
     if (lane == KC - 1) {  // holds its half's reductions
         cs.started = started;
-        cs.per = (uint32_t)per;
-        cs.rowmask = masks & 0xffffu;
-        cs.chanmask = masks >> 16;
+        cs.cover_per = masks | (uint32_t)per << 24;
         cs.gmask = (uint32_t)(gauss >> (half * KC));
     }
 }
@@ -348,10 +358,10 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
     const uint2 starts = *reinterpret_cast<const uint2*>(cs.starts + 2 * wave);
     const uint32_t before = (cs.started >> (8 * wave)) & 255u;
     const int k = (int)__builtin_amdgcn_mbcnt_hi(starts.y, __builtin_amdgcn_mbcnt_lo(starts.x, before));
-    const int per = (int)cs.per;
+    const int per = cs.per();
     const WalkRec w = cs.walk[k];
     const int width = max(w.width(), 1), kind = w.kind();
-    const int l0 = (t - (int)w.first) * per;
+    const int l0 = (t - w.first()) * per;
     const int l1 = min(l0 + per, w.rows() * w.width());
     const bool active = l0 < l1;
     const int ti = w.row(), tj = w.col();  // footprint corner in the tile
@@ -453,8 +463,7 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
 
 // Evaluates S for the chunk's KC particles x CB channels of the cell and
 // hands the values to store2(k, channel1, s1, channel2, s2), two channels of
-// one particle at a time; particles k >= nk and channels beyond the cube give
-// 0.  Thread t takes particle t % KC and the channels t / KC + 8 i, so its
+// one particle at a time; channels outside its window give 0.  Thread t takes particle t % KC and the channels t / KC + 8 i, so its
 // record fields are read once.  Only the 16-channel blocks set in `blocks`
 // (wave-uniform) are evaluated; the others are left untouched.  The values
 // are line_flux's (for narrow spans the same series with its polynomial
@@ -462,24 +471,20 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
 // test is one unsigned compare and a select, the wide-channel erfc path one
 // branch per block) so that the evaluations of a thread overlap.
 template <int CB, class Store2>
-__device__ inline void fill_spectra(const ChunkState& cs, int nk, int c0, int nc,
-                                    const mi_cube_desc& d, Store2 store2,
+__device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_desc& d,
+                                    Store2 store2,
                                     uint32_t blocks = (1u << (CB / 16)) - 1u) {
     constexpr int PER_BLOCK = 16 / (NT / KC);  // a thread's channels in one 16-channel block
     static_assert(PER_BLOCK == 2, "a thread stores its two channels of a block together");
     const int k = threadIdx.x & (KC - 1);
     const int cl0 = threadIdx.x / KC;
     const SpecRec p = cs.p[k];
-    // the window within the cell, empty past the item's last particle
-    const int lo = k < nk ? (int)(p.window & 0xffffu) : 1;
-    const int hi = k < nk ? min((int)(p.window >> 16), nc - 1 - c0) : 0;
     const int k0 = p.k0;
     const float fu = p.fu, s = p.s, amp = p.amp;
     const int spectrum = d.spectrum;
-    // Channel cl0 + o of the cell lies in the window [lo, hi] when
-    // (unsigned)(o - w0) <= wl; an empty window takes an offset no o reaches.
-    const int w0 = lo <= hi ? lo - cl0 : (1 << 30);
-    const uint32_t wl = lo <= hi ? (uint32_t)(hi - lo) : 0u;
+    // Channel cl0 + o of the cell lies in the window when (unsigned)(o - w0) <= wl.
+    const int w0 = cs.walk[k].win_lo() - cl0;
+    const uint32_t wl = cs.walk[k].win_past();
     auto inside = [&](int o) { return (uint32_t)(o - w0) <= wl; };
     auto put = [&](int b, float v0, float v1) {
         constexpr int STEP = NT / KC;

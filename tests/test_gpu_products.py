@@ -77,3 +77,43 @@ def test_products(method, whole, shape, spread, n):
     assert np.all(got[terms == 0] == 0.0)
     worst = np.max(np.abs(got - want) - (terms + 1) * 2.0**-24 * mag)
     assert worst <= 0.0, worst
+
+
+@pytest.mark.parametrize("method", ["plain", "mfma"])
+@pytest.mark.parametrize("shape", [(16, 16, 64), (8, 16, 128)])
+@pytest.mark.parametrize("n", [24577, 50001, 74015, 99000, 124033, 172800, 600001])
+def test_long_items(method, shape, n):
+    """One cell whose work items hold 2 to 9 chunks, over the edges of the chunks
+    staged together: one pixel and one of 64 spectra per particle, whole numbers, so
+    the cube is exact (sums below 2^24)."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    nx, ny, nc = shape
+    rows = 64
+    spectra = rng.integers(-8, 9, (rows, nc)).astype(np.float32)
+    lo = rng.integers(0, nc, rows)
+    hi = np.minimum(lo + rng.integers(0, 40, rows), nc - 1)
+    rec = np.zeros(n, _lib.PARTICLE_DTYPE)
+    rec["ix"], rec["iy"] = rng.integers(0, nx, n), rng.integers(0, ny, n)
+    rec["r_kind"] = _lib.KERNEL_TABLE
+    rec["h"] = np.arange(n, dtype=np.uint32).view(np.float32)
+    rec["k0"] = rng.integers(0, rows, n)
+    rec["c_lo"], rec["c_hi"] = lo[rec["k0"]], hi[rec["k0"]]
+    rec["amp"] = 1.0
+    weights = rng.integers(-4, 5, n).astype(np.float32)
+    sums = np.zeros((nx * ny, rows))
+    np.add.at(sums, (rec["ix"] * ny + rec["iy"], rec["k0"]), weights)
+    c = np.arange(nc)
+    inside = (c >= lo[:, None]) & (c <= hi[:, None])
+    want = (sums @ (spectra * inside)).reshape(shape)
+    d_s, d_w = torch.from_numpy(spectra).cuda(), torch.from_numpy(weights).cuda()
+    desc = _lib.make_desc(*shape, _lib.SPECTRUM_TABLE, spectra=d_s, spectra_ld=nc)
+    desc.weights, desc.weights_n = d_w.data_ptr(), n
+    pairs = _lib.count_pairs(rec, desc)
+    assert pairs == n
+    d_rec = torch.from_numpy(rec.view(np.uint8)).cuda()
+    cube = torch.zeros(want.size, dtype=torch.float32, device="cuda")
+    ws = torch.full((_lib.workspace_bytes(desc, n, pairs),), 255, dtype=torch.uint8, device="cuda")
+    _lib.insert(d_rec, n, pairs, desc, cube, ws, method=method)
+    assert np.array_equal(cube.cpu().numpy().reshape(shape), want)
