@@ -74,6 +74,7 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 // Operand tiles in LDS: OPK bytes per pixel (W) or channel (S) and chunk in
 // either form.
 constexpr int OPK = KC * 4;
+constexpr unsigned AND_XOR = 0x6a;  // v_bitop3_b32: (a & b) ^ c
 
 // BF16x3: a hi and a lo tile of 64 bytes per row, k contiguous, the four 16-byte
 // k-groups of a row permuted by bits 2..3 of the row index: the 16 rows a
@@ -90,23 +91,29 @@ struct SplitTile {
     __device__ static int k_bits(int k) { return (((k >> 3) & 3) << 4) | ((k & 7) << 1); }
     __device__ static int at(int row, int kb) { return row * KROW + (((row << 2) & 48) ^ kb); }
 
-    // Writes x as a BF16 pair (round to nearest even).
-    __device__ void put(int row, int k, float x) {
+    // at(row, kb) from q = SCALE * row: two instructions.
+    static constexpr int SCALE = 4;
+    __device__ static int at_scaled(int q, int kb) {
+        return (q << 4) | (int)__builtin_amdgcn_bitop3_b32((unsigned)q, 48u, (unsigned)kb, AND_XOR);
+    }
+
+    // Writes x as a BF16 pair (round to nearest even) at row q / SCALE.
+    __device__ void put(int q, int k, float x) {
         const __bf16 h = (__bf16)x;
         const __bf16 l = (__bf16)(x - (float)h);
-        const int o = at(row, k_bits(k));
+        const int o = at_scaled(q, k_bits(k));
         *reinterpret_cast<__bf16*>(hi + o) = h;
         *reinterpret_cast<__bf16*>(lo + o) = l;
     }
     // Two values of column k, converted together (one packed conversion each for
-    // the hi and the lo parts).
-    __device__ void put2(int k, int row1, float x1, int row2, float x2) {
+    // the hi and the lo parts) at rows q1 / SCALE and q2 / SCALE.
+    __device__ void put2(int k, int q1, float x1, int q2, float x2) {
         const floatx2 x = {x1, x2};
         const bf16x2 h = __builtin_convertvector(x, bf16x2);
         const floatx2 hf = __builtin_convertvector(h, floatx2);
         const bf16x2 l = __builtin_convertvector(floatx2{x1 - hf.x, x2 - hf.y}, bf16x2);
         const int kb = k_bits(k);
-        const int o1 = at(row1, kb), o2 = at(row2, kb);
+        const int o1 = at_scaled(q1, kb), o2 = at_scaled(q2, kb);
         *reinterpret_cast<__bf16*>(hi + o1) = h.x;
         *reinterpret_cast<__bf16*>(lo + o1) = l.x;
         *reinterpret_cast<__bf16*>(hi + o2) = h.y;
@@ -162,16 +169,22 @@ struct FloatTile {
 
     __device__ static int k_bits(int k) { return ((k & 3) << 5) | ((k >> 2) << 2); }
     __device__ static int at(int row, int kb) { return row * OPK + (((row << 3) & 0x70) ^ kb); }
-    __device__ void put(int row, int k, float x) {
-        *reinterpret_cast<float*>(v + at(row, k_bits(k))) = x;
+    static constexpr int SCALE = 8;
+    __device__ static int at_scaled(int q, int kb) {
+        return (q << 4) | (int)__builtin_amdgcn_bitop3_b32((unsigned)q, 0x70u, (unsigned)kb, AND_XOR);
     }
-    __device__ void put2(int k, int row1, float x1, int row2, float x2) {
+    __device__ void put(int q, int k, float x) {
+        *reinterpret_cast<float*>(v + at_scaled(q, k_bits(k))) = x;
+    }
+    __device__ void put2(int k, int q1, float x1, int q2, float x2) {
+        const int kb = k_bits(k);
+        *reinterpret_cast<float*>(v + at_scaled(q1, kb)) = x1;
+        *reinterpret_cast<float*>(v + at_scaled(q2, kb)) = x2;
+    }
+    __device__ void put_pairs(int k, int row1, float x1, int row2, float x2) {
         const int kb = k_bits(k);
         *reinterpret_cast<float*>(v + at(row1, kb)) = x1;
         *reinterpret_cast<float*>(v + at(row2, kb)) = x2;
-    }
-    __device__ void put_pairs(int k, int row1, float x1, int row2, float x2) {
-        put2(k, row1, x1, row2, x2);
     }
     struct Op {
         floatx4 a, b;  // steps 0..3 and 4..7
@@ -295,9 +308,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
             fill_gauss_tables(cs, x0, y0, gt);
             __syncthreads();
         }
-        fill_weights(cs, x0, y0, wtab, tkind, Tk, gt, d,
-                     [&](int k, int px, float w) { W.put(px, k, w); },
-                     [&](int k, int p1, float w1, int p2, float w2) { W.put2(k, p1, w1, p2, w2); });
+        fill_weights<WTile::SCALE>(cs, x0, y0, wtab, tkind, Tk, gt, d,
+                     [&](int k, int q, float w) { W.put(q, k, w); },
+                     [&](int k, int q1, float w1, int q2, float w2) { W.put2(k, q1, w1, q2, w2); });
         if (GT_IN_S && cs.gmask != 0u) __syncthreads();
         fill_spectra<G::CB>(cs, c0, d,
                      [&](int k, int c1, float s1, int c2, float s2) { S.put_pairs(k, c1, s1, c2, s2); },

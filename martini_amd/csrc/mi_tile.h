@@ -27,14 +27,14 @@ constexpr int LTAB_N = WTAB_N + 1;
 // What the W walk needs of a particle, read with two 16-byte loads by every
 // thread that takes some of its pixels.  px, py hold
 //   the particle's position ix + fx, iy + fy (exact in FP64) for the Gaussian kernel;
-//   its offsets from the footprint's first pixel in FP32 (tile_offset; one
-//   rounding of the exact value) for the other closed forms, whose position is
-//   in the chunk's GaussRec slot;
+//   for the other closed forms its offsets from the footprint's first pixel in
+//   FP32 (tile_offset), for the tabulated ones in table intervals (f a pixel), and
+//   1/h^2 (inv_h2); their position is in the chunk's GaussRec slot;
 //   as int64 bits (table_walk) the index of pixel (0, 0) in the caller's weight
 //   table and the row stride of the particle's weights for MI_KERNEL_TABLE.
 struct __attribute__((aligned(16))) WalkRec {
     double px, py;
-    float f;         // WFactors::b
+    float f;         // Gaussian: WFactors::b; tabulated kernels: WTAB_N / h
     // the first of the threads that share its pixels; and, << 16, its spectral window
     // clipped to the cell and the cube: first channel | channels past it << 8,
     // NO_WINDOW when empty
@@ -57,12 +57,13 @@ struct __attribute__((aligned(16))) WalkRec {
     __device__ int gidx() const { return cover >> 28; }
 };
 
-__device__ inline double pack_offset(float gx, float gy) {
-    return __hiloint2double(__float_as_int(gy), __float_as_int(gx));
+__device__ inline double pack2(float lo, float hi) {
+    return __hiloint2double(__float_as_int(hi), __float_as_int(lo));
 }
 __device__ inline float2 tile_offset(const WalkRec& w) {
     return make_float2(__int_as_float(__double2loint(w.px)), __int_as_float(__double2hiint(w.px)));
 }
+__device__ inline float inv_h2(const WalkRec& w) { return __int_as_float(__double2loint(w.py)); }
 
 // Weight-table walk of an MI_KERNEL_TABLE particle: weights[base + i * stride + j]
 // is its weight at pixel (i, j).
@@ -249,9 +250,9 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
     }
     const int cl = min(cb, g.nc - 1 - c0);
     const uint32_t window = valid && ca <= cl ? (uint32_t)ca | (uint32_t)(cl - ca) << 8 : NO_WINDOW;
-    cs.p[lane] = SpecRec{p.k0, p.fu, p.s, p.amp};
     const int width = max(jhi - jlo + 1, 1);
     const int kind = kind_of(p.r_kind), gi = gidx_of(p.r_kind);
+    cs.p[lane] = SpecRec{p.k0, p.fu, p.s, p.amp};
     WalkRec w;
     const double px = (double)p.ix + (double)p.fx, py = (double)p.iy + (double)p.fy;
     w.px = px;
@@ -268,9 +269,16 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
             f = weight_factors(kind, p.h, pick4(d.gauss_t, gi), 0.0f);
             cs.gr[lane] = GaussRec{f.a, f.e};
         } else {
-            f = weight_factors(kind, p.h, 0.0f, 0.0f);
             cs.gr[lane] = GaussRec{px, py};
-            w.px = pack_offset((float)(px - (double)ilo), (float)(py - (double)jlo));
+            f = weight_factors(kind, p.h, 0.0f, 0.0f);  // b = 1/h^2
+            float scale = 1.0f;
+            if (kind <= MI_KERNEL_QUARTIC) {  // WTAB_N / h, one Newton step past the hardware's 1/h
+                const float rh = __builtin_amdgcn_rcpf(p.h);
+                scale = (float)WTAB_N * fmaf(rh, fmaf(-p.h, rh, 1.0f), rh);
+            }
+            w.px = pack2((float)((px - (double)ilo) * scale), (float)((py - (double)jlo) * scale));
+            w.py = pack2(f.b, 0.0f);
+            f.b = scale;
         }
         if (kind == MI_KERNEL_TABLE) {
             // its weights are laid out over its cube-clipped footprint
@@ -288,23 +296,23 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
     }
 }
 
-// The weight of a tabulated kernel at q^2 = dr^2 / h^2, as weight_at computes
-// it, without branches: fb = 1/h^2, tab the kernel's table with its zero
-// entry at LTAB_N - 1, CUBIC whether the seam term of the cubic spline
-// applies.  The table position is clamped to that zero entry, so q >= 1 reads
+// The weight of a tabulated kernel as weight_at computes it but without
+// branches: fb = 1/h^2, x2 = (q WTAB_N)^2 for q = dr / h, tab the
+// kernel's table with its zero entry at LTAB_N - 1, CUBIC whether the seam term of
+// the cubic spline applies.  The table position is clamped to that zero entry, so q >= 1 reads
 // it (and the seam term is zero beyond q = 1/2): no mask, and the row is read
 // for every pixel (no branch around the LDS load).
 template <bool CUBIC>
-__device__ inline float table_weight_select(const float4* __restrict__ tab, float q2, float fb) {
-    const float q = __builtin_amdgcn_sqrtf(q2);
-    const float x = fminf(q * (float)WTAB_N, (float)WTAB_N);
+__device__ inline float table_weight_select(const float4* __restrict__ tab, float x2, float fb) {
+    const float x = fminf(__builtin_amdgcn_sqrtf(x2), (float)WTAB_N);
     const int i = (int)x;
     const float t = __builtin_amdgcn_fractf(x);
     const float4 c = tab[i];
     float w = fmaf(fmaf(fmaf(c.w, t, c.z), t, c.y), t, c.x);
     if (CUBIC) {  // R2 sqrt(1 - R2) / (8 * 1.5969), R2 = 4 q^2, zero for R2 >= 1
-        w = fmaf(q2 * (float)(4.0 / (8.0 * 1.59689476201133)),
-                 __builtin_amdgcn_sqrtf(fmaxf(fmaf(-4.0f, q2, 1.0f), 0.0f)), w);
+        constexpr double N2 = (double)WTAB_N * WTAB_N;
+        w = fmaf(x2 * (float)(4.0 / (8.0 * 1.59689476201133 * N2)),
+                 __builtin_amdgcn_sqrtf(fmaxf(fmaf((float)(-4.0 / N2), x2, 1.0f), 0.0f)), w);
     }
     return w * fb;
 }
@@ -338,8 +346,8 @@ __device__ inline float gauss_weight(double dx, double dy, double fa, double fe,
 }
 
 // Evaluates W for every (particle, pixel) pair of the chunk and hands each
-// value to store(k, pixel-in-tile, w), or two of them to
-// store2(k, pixel1, w1, pixel2, w2).  Particle k's pairs (pixel row l / width,
+// value to store(k, PXS * pixel-in-tile, w), or two of them to
+// store2(k, PXS * pixel1, w1, PXS * pixel2, w2).  Particle k's pairs (pixel row l / width,
 // column l % width of its clipped footprint, l < cnt) are split over the threads
 // from its first one on, `per` consecutive pairs each, so a thread stays on one
 // particle.  It finds the particle by counting start bits: a search of the
@@ -348,7 +356,7 @@ __device__ inline float gauss_weight(double dx, double dy, double fa, double fe,
 // FP32: 556 -> 547 us).  When every
 // particle of the wave's pairs uses the item's LDS table, the walk is
 // branch-free and takes two pixels per step, whose evaluations overlap.
-template <class Store, class Store2>
+template <int PXS, class Store, class Store2>
 __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
                                     const float4* __restrict__ wtab, int tab_kind,
                                     const float4* __restrict__ tab, const GaussTables& gt,
@@ -367,30 +375,29 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
     const int ti = w.row(), tj = w.col();  // footprint corner in the tile
 
     if (tab_kind >= 0 && __all(!active || kind == tab_kind)) {
-        // q^2 in FP32 from the offset, a few ulps from the FP64 form, far below the
-        // table's own error.
+        // x^2 in FP32 from the offset in table intervals, a few ulps from the FP64
+        // form, far below the table's own error.  (Offsets in pixels cost two more
+        // products a pixel: 3e6 heterogeneous particles, FP32, 3.45 -> 3.41 ms with
+        // the shorter addresses of put and put2.)
         const float gx = tile_offset(w).x, gy = tile_offset(w).y;
-        const float fa = w.f;
+        const float f = w.f, fb = inv_h2(w);
         // Pixel l of the footprint lies in row floor((l + 1/2) / width) (exact, as
         // for a above) and column l - row * width, all small integers formed in
         // FP32: no wrap tests, and the offsets from the particle need no
         // conversion.  Its index in the tile is row * TILE_Y + column + corner.
         const float rw = __builtin_amdgcn_rcpf((float)width), wf = (float)width;
-        const float hrw = 0.5f * rw, corner4 = (float)(4 * (ti * TILE_Y + tj));
+        const float hrw = 0.5f * rw, corner = (float)(PXS * (ti * TILE_Y + tj));
         auto at = [&](float lf, float& af, float& bf) {
             af = floorf(fmaf(lf, rw, hrw));  // (l + 1/2) / width, one rounding
             bf = fmaf(-af, wf, lf);
         };
         auto px_of = [&](float af, float bf) {
-            const int q = (int)fmaf(af, (float)(4 * TILE_Y), fmaf(bf, 4.0f, corner4));  // 4 * index
-            __builtin_assume((q & 3) == 0);
-            return q >> 2;
+            return (int)fmaf(af, (float)(PXS * TILE_Y), fmaf(bf, (float)PXS, corner));
         };
         auto walk = [&](auto cubic) {
             auto eval = [&](float af, float bf) {
-                const float dx = gx - af, dy = gy - bf;
-                return table_weight_select<decltype(cubic)::value>(tab, fmaf(dx, dx, dy * dy) * fa,
-                                                                   fa);
+                const float dx = fmaf(-af, f, gx), dy = fmaf(-bf, f, gy);
+                return table_weight_select<decltype(cubic)::value>(tab, fmaf(dx, dx, dy * dy), fb);
             };
             float lf = (float)l0;
             const float lend = (float)l1;
@@ -423,7 +430,7 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
         const TableWalk tw = table_walk(w);
         for (int l = l0; l < l1; ++l) {
             const int i = x0 + ti + a, j = y0 + tj + b;
-            store(k, (ti + a) * TILE_Y + tj + b, d.weights[tw.base + (int64_t)i * tw.stride + j]);
+            store(k, PXS * ((ti + a) * TILE_Y + tj + b), d.weights[tw.base + (int64_t)i * tw.stride + j]);
             if (++b == width) {
                 b = 0;
                 ++a;
@@ -438,7 +445,7 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
         const float gt_t = pick4(d.gauss_t, gi), gt_n = pick4(d.gauss_inv_norm, gi);
         for (int l = l0; l < l1; ++l) {
             const int i = x0 + ti + a, j = y0 + tj + b;
-            store(k, (ti + a) * TILE_Y + tj + b,
+            store(k, PXS * ((ti + a) * TILE_Y + tj + b),
                   gauss_weight(w.px - (double)i, w.py - (double)j, gg.a, gg.e, gt_t, gt_n,
                                gt.ex[k][a], gt.ey[k][b]));
             if (++b == width) {
@@ -448,11 +455,12 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
         }
         return;
     }
-    const WFactors f{(double)w.f, 0.0, w.f, 0.0f, 0.0f};
+    const float fb = inv_h2(w);
+    const WFactors f{(double)fb, 0.0, fb, 0.0f, 0.0f};
     const GaussRec at = cs.gr[k];
     for (int l = l0; l < l1; ++l) {
         const int i = x0 + ti + a, j = y0 + tj + b;
-        store(k, (ti + a) * TILE_Y + tj + b,
+        store(k, PXS * ((ti + a) * TILE_Y + tj + b),
               weight_at(kind, at.a - (double)i, at.e - (double)j, f, wtab, tab_kind, tab));
         if (++b == width) {
             b = 0;
