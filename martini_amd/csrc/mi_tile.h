@@ -553,8 +553,8 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
             for (int i = 0; i < PER_BLOCK; ++i) {
                 const int o = (NT / KC) * (b * PER_BLOCK + i);
                 if (!inside(o)) continue;
-                const float m = s * (((float)(kc - o) + fu) - 0.5f);  // kc - o = k0 - channel
-                v[i] = 0.5f * amp * erf_diff(m - 0.5f * s, m + 0.5f * s);
+                const float j = (float)(kc - o);  // k0 - channel; each edge to its own precision
+                v[i] = 0.5f * amp * erf_diff(s * ((j - 1.0f) + fu), s * (j + fu));
             }
         }
         put(b, v[0], v[1]);
