@@ -119,26 +119,26 @@ struct SplitTile {
         *reinterpret_cast<__bf16*>(hi + o2) = h.y;
         *reinterpret_cast<__bf16*>(lo + o2) = l.y;
     }
-    // put2 for the S fill, whose lanes l and l ^ 1 hold the same two rows of
-    // particles k and k ^ 1 (rows given as 16 * block + r: the block's 1 KiB step
-    // plus at(r)).  After one lane swap (DPP quad_perm [1, 0, 3, 2]) the even lane
-    // writes row1 and the odd lane row2, each as the pair (k even, k odd) --
+    // put2 for the S fill, whose lanes l and l ^ 1 hold the rows r and r + 8 of a
+    // block of 16 of particles k and k ^ 1 (a block is 1 KiB, an offset in the
+    // store: eight addresses kept in registers made the FP32 form spill, 1e6 particles
+    // 526 -> 504 us).  After one lane swap (DPP quad_perm [1, 0, 3, 2]) the even lane
+    // writes row r and the odd lane row r + 8, each as the pair (k even, k odd) --
     // adjacent BF16 slots of one 4-byte word -- in both tiles: one paired 4-byte
     // store per lane (the hi and lo tiles lie a fixed distance apart) instead of
     // four 2-byte ones.  Every lane of the wave must call it.
-    __device__ void put_pairs(int k, int row1, float x1, int row2, float x2) {
+    __device__ void put_pairs(int k, int block, int r, float x1, float x2) {
         constexpr int SWAP = 0xB1;  // quad_perm [1, 0, 3, 2]: lanes l and l ^ 1
         const float y1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x1), SWAP, 0xF, 0xF, false));
         const float y2 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x2), SWAP, 0xF, 0xF, false));
         const bool even = (k & 1) == 0;
-        const int row = even ? row1 : row2;
         const floatx2 x = even ? floatx2{x1, y1} : floatx2{y2, x2};  // particles k & ~1, k | 1
         const bf16x2 h = __builtin_convertvector(x, bf16x2);
         const floatx2 hf = __builtin_convertvector(h, floatx2);
         const bf16x2 l = __builtin_convertvector(floatx2{x.x - hf.x, x.y - hf.y}, bf16x2);
-        const int o = (row >> 4) * (16 * KROW) + at(row & 15, k_bits(k & ~1));
-        *reinterpret_cast<bf16x2*>(hi + o) = h;
-        *reinterpret_cast<bf16x2*>(lo + o) = l;
+        char* to = hi + at(even ? r : r + 8, k_bits(k & ~1)) + block * (16 * KROW);
+        *reinterpret_cast<bf16x2*>(to) = h;
+        *reinterpret_cast<bf16x2*>(to + ROWS * KROW) = l;
     }
     // The 8 values of k-group kg of `row`, hi and lo.
     struct Op {
@@ -181,10 +181,10 @@ struct FloatTile {
         *reinterpret_cast<float*>(v + at_scaled(q1, kb)) = x1;
         *reinterpret_cast<float*>(v + at_scaled(q2, kb)) = x2;
     }
-    __device__ void put_pairs(int k, int row1, float x1, int row2, float x2) {
+    __device__ void put_pairs(int k, int block, int r, float x1, float x2) {
         const int kb = k_bits(k);
-        *reinterpret_cast<float*>(v + at(row1, kb)) = x1;
-        *reinterpret_cast<float*>(v + at(row2, kb)) = x2;
+        *reinterpret_cast<float*>(v + at(r, kb) + block * (16 * OPK)) = x1;
+        *reinterpret_cast<float*>(v + at(r + 8, kb) + block * (16 * OPK)) = x2;
     }
     struct Op {
         floatx4 a, b;  // steps 0..3 and 4..7
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                      [&](int k, int q1, float w1, int q2, float w2) { W.put2(k, q1, w1, q2, w2); });
         if (GT_IN_S && cs.gmask != 0u) __syncthreads();
         fill_spectra<G::CB>(cs, c0, d,
-                     [&](int k, int c1, float s1, int c2, float s2) { S.put_pairs(k, c1, s1, c2, s2); },
+                     [&](int k, int b, int r, float s1, float s2) { S.put_pairs(k, b, r, s1, s2); },
                      chanmask);
         // FP32: the particles (bits) that reach each of this wave's rows and blocks
         uint32_t prow[4] = {}, pblk[4] = {};

@@ -470,8 +470,8 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
 }
 
 // Evaluates S for the chunk's KC particles x CB channels of the cell and
-// hands the values to store2(k, channel1, s1, channel2, s2), two channels of
-// one particle at a time; channels outside its window give 0.  Thread t takes particle t % KC and the channels t / KC + 8 i, so its
+// hands the values to store2(k, block, r, s1, s2), the channels r and r + 8 of
+// the 16-channel block of one particle at a time; channels outside its window give 0.  Thread t takes particle t % KC and the channels t / KC + 8 i, so its
 // record fields are read once.  Only the 16-channel blocks set in `blocks`
 // (wave-uniform) are evaluated; the others are left untouched.  The values
 // are line_flux's (for narrow spans the same series with its polynomial
@@ -495,9 +495,8 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
     const uint32_t wl = cs.walk[k].win_past();
     auto inside = [&](int o) { return (uint32_t)(o - w0) <= wl; };
     auto put = [&](int b, float v0, float v1) {
-        constexpr int STEP = NT / KC;
-        const int o0 = STEP * (b * PER_BLOCK), o1 = o0 + STEP;
-        store2(k, cl0 + o0, inside(o0) ? v0 : 0.0f, cl0 + o1, inside(o1) ? v1 : 0.0f);
+        const int o0 = 16 * b, o1 = o0 + NT / KC;
+        store2(k, b, cl0, inside(o0) ? v0 : 0.0f, inside(o1) ? v1 : 0.0f);
     };
     if (spectrum == MI_SPECTRUM_TABLE) {  // uniform: the caller's spectra
 #pragma unroll
@@ -507,8 +506,7 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
             // (channel c0 + cl0 + o is inside the window when inside(o))
             const float* row = d.spectra + ((int64_t)k0 * d.spectra_ld + c0 + cl0);
             const int o0 = (NT / KC) * (b * PER_BLOCK), o1 = o0 + NT / KC;
-            store2(k, cl0 + o0, inside(o0) ? amp * row[o0] : 0.0f, cl0 + o1,
-                   inside(o1) ? amp * row[o1] : 0.0f);
+            store2(k, b, cl0, inside(o0) ? amp * row[o0] : 0.0f, inside(o1) ? amp * row[o1] : 0.0f);
         }
         return;
     }
