@@ -469,6 +469,66 @@ __device__ inline void fill_weights(const ChunkState& cs, int x0, int y0,
     }
 }
 
+constexpr double LOG2E = 1.4426950408889634074;
+constexpr float SQRT_LOG2E = 1.20112240878645110f;
+
+// The flux of a Gaussian line of unit width in a channel of span D about m,
+//   amp / 2 (erf(m + D/2) - erf(m - D/2))
+//     = amp D / sqrt(pi) sum_k D^2k / (4^k (2k + 1)!) d^2k/dm^2k exp(-m^2)
+//     = exp(-m^2) sum_j e_j m^2j,
+// the sum over k to K (span_series' terms for K = 3); the e_j are formed once per
+// particle.  SCALED: as exp2(-n^2) times a polynomial in n^2 of n = m sqrt(log2 e),
+// a product less per channel and n's factor rounded once for all channels.  The first term left out is D^(2K+2) / (4^(K+1) (K+1)! (2K+3)) of the
+// peak at most: 1e-9 for K = 3, D = 1/2 and 2e-8 for K = 7, D = 3/2.
+template <int K, bool SCALED>
+struct LineSeries {
+    float e[K + 1];
+
+    // 1 / sqrt(pi) in FP32 is off by 5e-8, the same for every line: the coefficients
+    // take that back (1 - 5e-8 is within 1e-8 of an FP32 number).
+    static constexpr float ROOT = 0.564189583547756287f;
+    // c[k][j]: of D^2k m^2j (the Hermite polynomials' coefficients)
+    struct Table {
+        float c[K + 1][K + 1];
+    };
+    static constexpr Table table() {
+        Table t{};
+        // 1 / (2 j)!, its scale included, and (-1)^i / (4^i i!)
+        double inv_2j[K + 1] = {}, inv_i[K + 1] = {};
+        double a = 0.564189583547756287 / (double)ROOT, b = 1.0;
+        for (int j = 0; j <= K; ++j) {
+            inv_2j[j] = a;
+            inv_i[j] = b;
+            a /= (2 * j + 1) * (2 * j + 2) * (SCALED ? LOG2E : 1.0);
+            b /= -4.0 * (j + 1);
+        }
+        for (int k = 0; k <= K; ++k)
+            for (int j = 0; j <= k; ++j) t.c[k][j] = (float)(inv_i[k - j] * inv_2j[j] / (2 * k + 1));
+        return t;
+    }
+    __device__ LineSeries(float s, float amp) {
+        constexpr Table T = table();
+        const float D2 = s * s;
+        float f = amp * ROOT * s;
+#pragma unroll
+        for (int j = 0; j <= K; ++j) {
+            float c = T.c[K][j];
+#pragma unroll
+            for (int k = K - 1; k >= j; --k) c = fmaf(c, D2, T.c[k][j]);
+            e[j] = f * c;
+            f *= D2;
+        }
+    }
+    // at n (SCALED) or m
+    __device__ float operator()(float n) const {
+        const float n2 = n * n;
+        float p = e[K];
+#pragma unroll
+        for (int j = K - 1; j >= 0; --j) p = fmaf(p, n2, e[j]);
+        return __builtin_amdgcn_exp2f(SCALED ? -n2 : n2 * (float)-LOG2E) * p;
+    }
+};
+
 // Evaluates S for the chunk's KC particles x CB channels of the cell and
 // hands the values to store2(k, block, r, s1, s2), the channels r and r + 8 of
 // the 16-channel block of one particle at a time; channels outside its window give 0.  Thread t takes particle t % KC and the channels t / KC + 8 i, so its
@@ -516,40 +576,41 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
             if ((blocks >> b) & 1u) put(b, amp, amp);
         return;
     }
-    // Narrow spans: span_series with its D-dependent factors folded once per
-    // particle (D = s), 0.5 amp (erf(m + D/2) - erf(m - D/2)) =
-    // exp(-m^2) (e0 + e1 m^2 + e2 m^4 + e3 m^6); the same polynomial expanded.
-    const float D2 = s * s, K = amp * 0.564189583547756287f * s;  // amp D / sqrt(pi)
-    const float e0 = K * (1.0f + D2 * (-1.0f / 12.0f + D2 * (1.0f / 160.0f - D2 * (1.0f / 2688.0f))));
-    const float e1 = K * D2 * (1.0f / 6.0f + D2 * (-1.0f / 40.0f + D2 * (1.0f / 448.0f)));
-    const float e2 = K * D2 * D2 * (1.0f / 120.0f - D2 * (1.0f / 672.0f));
-    const float e3 = K * D2 * D2 * D2 * (1.0f / 5040.0f);
     // Channel c = c0 + cl0 + 8 j of this thread sits at k0 - c + fu - 1/2 =
     // A - 8 j from the line centre (in channels), A formed once; subtracting
     // the small integer 8 j from A is exact in the in-window range.
     const int kc = k0 - c0 - cl0;
     const float A = (float)kc + (fu - 0.5f);
-    // exp(-m^2) as exp2(-n^2) with n = m sqrt(log2 e): n = sn (A - 8 j), and the
-    // polynomial in m^2 = n^2 / log2 e with its coefficients scaled once.
-    constexpr float LOG2E = 1.44269504088896341f;
-    const float sn = s * 1.20112240878645110f;  // sqrt(log2 e)
-    const float g1 = e1 * (1.0f / LOG2E), g2 = e2 * (1.0f / (LOG2E * LOG2E)),
-                g3 = e3 * (1.0f / (LOG2E * LOG2E * LOG2E));
-    auto narrow = [&](int o) {
-        const float n = sn * (A - (float)o), n2 = n * n;
-        return __builtin_amdgcn_exp2f(-n2) * fmaf(fmaf(fmaf(g3, n2, g2), n2, g1), n2, e0);
-    };
+    // exp(-m^2) as exp2(-n^2) with n = m sqrt(log2 e): n = sn (A - 8 j).
+    const float sn = s * SQRT_LOG2E;
+    auto narrow = [&](const LineSeries<3, true>& line, int o) { return line(sn * (A - (float)o)); };
     if (!__any(s > 0.5f)) {
+        const LineSeries<3, true> line(s, amp);
 #pragma unroll
         for (int b = 0; b < CB / 16; ++b)
             if ((blocks >> b) & 1u)  // uniform
-                put(b, narrow(16 * b), narrow(16 * b + NT / KC));
+                put(b, narrow(line, 16 * b), narrow(line, 16 * b + NT / KC));
         return;
     }
-    // Wide channels: the line spans a few channels, and the erfc differences are
+    if (!__any(s > 1.5f)) {
+        // A longer series, a seventh of the erf difference's work per channel; the
+        // offsets each to their own precision (3e5 particles, s = 0.8, split BF16: 232
+        // -> 220 us per insertion; 3e6 of which half have s = 6 and go on: 3.05 -> 3.09 ms).
+        const LineSeries<7, false> line(s, amp);
+        const float kf = (float)kc, fh = fu - 0.5f;
+#pragma unroll 1
+        for (uint32_t left = blocks; left != 0u; left &= left - 1u) {
+            const int b = __builtin_ctz(left);
+            const float j = kf - (float)(16 * b);
+            put(b, line(s * (j + fh)), line(s * (j - (float)(NT / KC) + fh)));
+        }
+        return;
+    }
+    // Wider channels: the line spans a few channels, and the erfc differences are
     // taken only inside its window.  A loop of its own: unrolled into the narrow lines'
     // code it made the kernel too long for the instruction cache (1e7 particles,
     // narrow lines: 4.78 -> 4.67 ms; 3e6 with wide ones 3.05 -> 3.06).
+    const LineSeries<3, true> line(s, amp);
 #pragma unroll 1
     for (uint32_t left = blocks; left != 0u; left &= left - 1u) {
         const int b = __builtin_ctz(left);
@@ -557,7 +618,7 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
 #pragma unroll
         for (int i = 0; i < PER_BLOCK; ++i) {
             const int o = 16 * b + i * (NT / KC);
-            v[i] = narrow(o);
+            v[i] = narrow(line, o);
             if (s > 0.5f && inside(o)) {
                 const float j = (float)(kc - o);  // k0 - channel; each edge to its own precision
                 v[i] = 0.5f * amp * erf_diff(s * ((j - 1.0f) + fu), s * (j + fu));
