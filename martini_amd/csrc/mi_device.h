@@ -39,7 +39,7 @@ static_assert(GeoSquare::PX * GeoSquare::CB == CELL_VOXELS &&
               "both cell shapes hold the same number of voxels");
 // A cell's sub-tiles: one tile row (16 pixels) x SUB_CH channels each, 64 in
 // either shape.  A partial tile stores them one after another, each 1 KiB
-// ([row][channel block][pixel][SUB_CH]).  Bit sub_bit(row, block) of its mask
+// ([row][channel block][SUB_CH][pixel]).  Bit sub_bit(row, block) of its mask
 // is set where the item wrote that sub-tile; the others hold nothing of this
 // call and are read as zero.  The bits follow the gather's waves: with RG = TX / 4
 // row groups and CG = 4 / RG channel groups, wave w = row % RG + RG * (block % CG)
@@ -49,8 +49,8 @@ constexpr int SUB_CH = 16;
 static_assert(GeoSquare::TX * (GeoSquare::CB / SUB_CH) == 64 &&
                   GeoWide::TX * (GeoWide::CB / SUB_CH) == 64,
               "one 64-bit sub-tile mask per partial tile");
-__host__ __device__ constexpr int sub_offset(int cb_blocks, int row, int block, int pixel) {
-    return ((row * cb_blocks + block) * 16 + pixel) * 16;
+__host__ __device__ constexpr int sub_offset(int cb_blocks, int row, int block) {
+    return (row * cb_blocks + block) * (16 * SUB_CH);
 }
 __host__ __device__ constexpr int sub_bit(int tx_shift, int row, int block) {
     const int rg_shift = tx_shift - 2, cg_shift = 4 - tx_shift;

@@ -37,12 +37,12 @@ __global__ __launch_bounds__(NT) void k_reduce(const uint32_t* __restrict__ item
     const float4* base = reinterpret_cast<const float4*>(partials) + (size_t)multi_off[cell] * tile;
     const uint64_t* mk = part_masks + multi_off[cell];
     const int v4 = part * NT + threadIdx.x;  // float4 index within the tile
-    // v4 = (sub-tile * TILE_Y + pixel) * 4 + float4 within the 16 channels
+    // v4 = (sub-tile * SUB_CH + channel) * 4 + float4 within the 16 pixels
     static_assert(TILE_Y == 16 && SUB_CH == 16 && NT % 64 == 0, "one sub-tile per wave");
     const int sub = v4 >> 6;  // row * blocks + block, the same in a wave
     const int nblk = (1 << g.cb_shift) / SUB_CH;
-    const int prow = sub / nblk, jl = (v4 >> 2) & 15;
-    const int cl = (sub - prow * nblk) * SUB_CH + (v4 & 3) * 4;
+    const int prow = sub / nblk, jl = (v4 & 3) * 4;
+    const int cl = (sub - prow * nblk) * SUB_CH + ((v4 >> 2) & 15);
     const int bit = sub_bit(g.tx_shift, prow, sub - prow * nblk);
     const float4* src = base + v4;
     const uint32_t lane = threadIdx.x & 63;
@@ -74,12 +74,15 @@ __global__ __launch_bounds__(NT) void k_reduce(const uint32_t* __restrict__ item
     }
     if (!seen) return;
     const CellPos cp = cell_pos(cell, g);
-    const int i = cp.x0 + prow, j = cp.y0 + jl;
-    if (i >= g.nx || j >= g.ny) return;
-    float* dst = cube + ((size_t)i * g.ny + j) * g.nc + cp.c0 + cl;
+    const int i = cp.x0 + prow, j = cp.y0 + jl, c = cp.c0 + cl;
+    if (i >= g.nx || c >= g.nc) return;
+    float* dst = cube + ((size_t)i * g.ny + j) * g.nc + c;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-        if (cp.c0 + cl + u < g.nc) dst[u] = (float)((double)dst[u] + s0[u]);
+        if (j + u < g.ny) {
+            float& v = dst[(size_t)u * g.nc];
+            v = (float)((double)v + s0[u]);
+        }
 }
 
 // The weight tables are constant data (the FP64 closed forms of the four

@@ -388,35 +388,43 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     // D layout of a 16x16 block: lane holds rows 4*kg..4*kg+3 (pixels j) of column m
     // (channel).  Blocks that are all zero (no product reached them) are not
     // written; a partial tile's mask records the blocks that were.
-    uint32_t mine = 0u;  // bit 4 r + nb: block (r, nb) written
+    auto any = [](const floatx4& v) {
+        return __ballot(v[0] != 0.f || v[1] != 0.f || v[2] != 0.f || v[3] != 0.f) != 0u;
+    };
+    constexpr int BLOCKS = G::CB / SUB_CH;
+    if (it.slot >= 0) {
+        // a lane's four pixels are next to one another in a partial tile: one store each
+        floatx4* tile = reinterpret_cast<floatx4*>(partials + (size_t)it.slot * CELL_VOXELS +
+                                                   sub_offset(BLOCKS, rh, ch)) + m * 4 + kg;
+        uint32_t mine = 0u;  // bit 4 r + nb: block (r, nb) written
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb)
+                if (any(acc[r][nb])) {
+                    mine |= 1u << (4 * r + nb);
+                    tile[sub_offset(BLOCKS, RG * r, CGN * nb) / 4] = acc[r][nb];
+                }
+        static_assert(NT / 64 == 4, "four 16-bit parts per mask");
+        if (lane == 0)  // this wave's part: bits 16 * wave + 4 r + nb
+            reinterpret_cast<uint16_t*>(part_masks + it.slot)[wave] = (uint16_t)mine;
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int prow = rh + RG * r;  // tile row
-        const int i = x0 + prow;
+        const int i = x0 + rh + RG * r;
+        if (i >= g.nx) break;
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) {
-            const floatx4 v4 = acc[r][nb];
-            if (__ballot(v4[0] != 0.f || v4[1] != 0.f || v4[2] != 0.f || v4[3] != 0.f) == 0u)
-                continue;
-            mine |= 1u << (4 * r + nb);
+            if (!any(acc[r][nb])) continue;
+            const int c = c0 + (ch + CGN * nb) * 16 + m;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int jl = kg * 4 + q;
-                const int cl = (ch + CGN * nb) * 16 + m;
-                const float v = acc[r][nb][q];
-                if (it.slot < 0) {
-                    const int j = y0 + jl, c = c0 + cl;
-                    if (i < g.nx && j < g.ny && c < g.nc) cube[((size_t)i * g.ny + j) * g.nc + c] += v;
-                } else {
-                    partials[(size_t)it.slot * CELL_VOXELS +
-                             sub_offset(G::CB / SUB_CH, prow, ch + CGN * nb, jl) + m] = v;
-                }
+                const int j = y0 + kg * 4 + q;
+                if (j < g.ny && c < g.nc) cube[((size_t)i * g.ny + j) * g.nc + c] += acc[r][nb][q];
             }
         }
     }
-    static_assert(NT / 64 == 4, "four 16-bit parts per mask");
-    if (it.slot >= 0 && lane == 0)  // this wave's part: bits 16 * wave + 4 r + nb
-        reinterpret_cast<uint16_t*>(part_masks + it.slot)[wave] = (uint16_t)mine;
 }
 
 hipError_t gather(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,
