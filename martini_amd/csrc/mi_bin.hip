@@ -123,6 +123,7 @@ hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L) {
     L->item_len = item_length(n_pairs);
     L->items_max = g.ncells + n_pairs / L->item_len + 1;
     L->multi_max = 2 * (n_pairs / L->item_len) + 1;
+    L->split_max = std::min<int64_t>(g.ncells, n_pairs / L->item_len);
     // cleared by k_bin_init, from status on
     L->status = take(sizeof(uint32_t) * ST_WORDS);
     L->hist = take(sizeof(uint32_t) * RADIX_PASSES << RADIX_BITS);
@@ -140,6 +141,7 @@ hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L) {
     L->item_off = take(4 * nc1);
     L->multi_off = take(4 * nc1);
     L->item_pos = take(4 * nc);
+    L->split_cells = take(4 * (size_t)L->split_max);
     L->items = take(sizeof(Item) * (size_t)L->items_max);
     L->partials = take(sizeof(float) * (size_t)L->multi_max * CELL_VOXELS);
     L->part_masks = take(sizeof(uint64_t) * (size_t)L->multi_max);
@@ -561,9 +563,10 @@ __device__ inline void write_items(uint32_t c, uint32_t n, uint32_t slot, uint32
 __global__ __launch_bounds__(SCAN_T) void k_items(
     const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, int64_t ncells,
     int item_len, uint32_t* __restrict__ status, uint32_t* __restrict__ item_off,
-    uint32_t* __restrict__ multi_off, uint32_t* __restrict__ item_pos, Item* __restrict__ items) {
+    uint32_t* __restrict__ multi_off, uint32_t* __restrict__ item_pos,
+    uint32_t* __restrict__ split_cells, Item* __restrict__ items) {
     constexpr int WAVES = SCAN_T / 64;
-    __shared__ uint32_t wtot[2][WAVES];
+    __shared__ uint32_t wtot[3][WAVES];
     __shared__ uint32_t bucket[ITEM_BUCKETS];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t per = (ncells + SCAN_T - 1) / SCAN_T;
@@ -573,24 +576,25 @@ __global__ __launch_bounds__(SCAN_T) void k_items(
     if (t < ITEM_BUCKETS) bucket[t] = 0u;
     __syncthreads();
     auto of = [&](int64_t c) { return cell_items(none ? 0u : end[c] - start[c], L); };
-    uint32_t sum[2] = {0u, 0u};  // items, partial tiles
+    uint32_t sum[3] = {0u, 0u, 0u};  // items, partial tiles, split cells
     for (int64_t c = c0; c < c1; ++c) {
         const CellItems n = of(c);
         sum[0] += n.items;
         sum[1] += n.items > 1u ? n.items : 0u;
+        sum[2] += n.items > 1u;
         if (n.items) atomicAdd(&bucket[n.bucket], n.items);
     }
-    uint32_t at[2];
+    uint32_t at[3];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < 3; ++k) {
         const uint32_t incl = (uint32_t)wave_scan_add((int)sum[k]);
         at[k] = incl - sum[k];
         if (lane == 63) wtot[k][wave] = incl;
     }
     __syncthreads();
-    uint32_t total[2] = {0u, 0u};
+    uint32_t total[3] = {0u, 0u, 0u};
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < 3; ++k)
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
             if (w == wave) at[k] += total[k];
@@ -610,6 +614,7 @@ __global__ __launch_bounds__(SCAN_T) void k_items(
         multi_off[ncells] = total[1];
         status[ST_ITEMS] = total[0];
         status[ST_MULTI] = total[1];
+        status[ST_SPLIT] = total[2];
     }
     __syncthreads();
     for (int64_t c = c0; c < c1; ++c) {
@@ -619,6 +624,7 @@ __global__ __launch_bounds__(SCAN_T) void k_items(
         item_pos[c] = n.items ? atomicAdd(&bucket[n.bucket], n.items) : 0u;
         at[0] += n.items;
         at[1] += n.items > 1u ? n.items : 0u;
+        if (n.items > 1u) split_cells[at[2]++] = (uint32_t)c;
     }
     if (ncells > ITEMS_IN_PLACE) return;  // uniform
     __syncthreads();  // the positions above, read back from this work group's own writes
@@ -695,7 +701,7 @@ hipError_t bin_particles(const mi_particle* d_p, int64_t n, int64_t n_pairs, con
                            words(L.keys2), status, g.ncells, words(L.cell_start), words(L.cell_end));
     hipLaunchKernelGGL(k_items, dim3(1), dim3(SCAN_T), 0, s, words(L.cell_start), words(L.cell_end),
                        g.ncells, L.item_len, status, words(L.item_off), words(L.multi_off),
-                       words(L.item_pos), (Item*)(ws + L.items));
+                       words(L.item_pos), words(L.split_cells), (Item*)(ws + L.items));
     if (g.ncells > ITEMS_IN_PLACE)
         hipLaunchKernelGGL(k_build_items, dim3((unsigned)g.ncells), dim3(64), 0, s,
                            words(L.item_off), words(L.multi_off), words(L.item_pos),

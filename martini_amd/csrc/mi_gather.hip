@@ -3,6 +3,7 @@
 // integrals and spectra by themselves.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "mi_device.h"
@@ -11,78 +12,111 @@
 
 namespace mi {
 
-// Sums the partial tiles of each split cell in item order, in FP64 (their sum
-// then costs one rounding: 1.3e-7 -> 0.8e-7 of error on 1e4 particles in 400
-// items), and adds them to the cube.  Block (cell, part): 256 threads x 4 voxels cover four 1 KiB
-// sub-tiles of the CELL_VOXELS = 16384-voxel tile, one per wave.  A wave reads
-// the masks of 64 items at a time, one per lane, and then only the sub-tiles
-// that their items wrote, RED_DEEP loads in flight (1e6 particles, MFMA: 28 us;
-// 39 with the masks read item by item, 31 with four loads in flight);
-// voxels no item wrote keep the cube's value.
-constexpr int RED_PARTS = CELL_VOXELS / (NT * 4);
+// Sums the partial tiles of the split cells in FP64 (their sum then costs one
+// rounding: 1.3e-7 -> 0.8e-7 of error on 1e4 particles in 400 items), and adds
+// them to the cube.  A wave takes a 1 KiB sub-tile of a cell at a time: it reads
+// the masks of 64 items, one per lane, and then only the sub-tiles that those items
+// wrote, RED_DEEP loads in flight (1e6 particles, MFMA: 39 us with the masks read
+// item by item, 31 with four loads in flight).
+//
+// Where cells are split RED_SHARED times or more on average, too few sub-tiles are
+// left for the chip and each is a long chain of loads: the waves of a work group
+// then share one, every fourth item each (1e6 particles, 72 cells in 32 items: 38
+// -> 21 us; 1e4: 9.2 -> 6.8).  With fewer items the sharing's barrier costs more than
+// the loads (3e5 particles, 11 a cell: 20 us, shared 26).  The sub-tiles of the listed
+// split cells go round RED_GROUPS work groups: work groups for every cell of the
+// cube were mostly for empty ones (1e7 particles: 95 -> 87 us; 3e5 on 512 x 512 x
+// 256: 55 -> 38).
+// Voxels no item wrote keep the cube's value; the order of a sum depends on the
+// input alone.
 constexpr int RED_DEEP = 8;
+constexpr int RED_GROUPS = 8192;
+constexpr int RED_SHARED = 16;
+constexpr int RED_SUBS = CELL_VOXELS / (16 * SUB_CH);  // sub-tiles of a cell
 
 __global__ __launch_bounds__(NT) void k_reduce(const uint32_t* __restrict__ item_off,
                                                const uint32_t* __restrict__ multi_off,
+                                               const uint32_t* __restrict__ split_cells,
                                                const uint32_t* __restrict__ status, Grid g,
                                                const float* __restrict__ partials,
                                                const uint64_t* __restrict__ part_masks,
                                                float* __restrict__ cube) {
     if (status[ST_OVERFLOW]) return;
-    const int cell = blockIdx.x / RED_PARTS;
-    const int part = blockIdx.x - cell * RED_PARTS;
-    const uint32_t ni = item_off[cell + 1] - item_off[cell];
-    if (ni <= 1) return;
-    const size_t tile = (size_t)CELL_VOXELS / 4;  // float4 per partial tile
-    const float4* base = reinterpret_cast<const float4*>(partials) + (size_t)multi_off[cell] * tile;
-    const uint64_t* mk = part_masks + multi_off[cell];
-    const int v4 = part * NT + threadIdx.x;  // float4 index within the tile
-    // v4 = (sub-tile * SUB_CH + channel) * 4 + float4 within the 16 pixels
-    static_assert(TILE_Y == 16 && SUB_CH == 16 && NT % 64 == 0, "one sub-tile per wave");
-    const int sub = v4 >> 6;  // row * blocks + block, the same in a wave
-    const int nblk = (1 << g.cb_shift) / SUB_CH;
-    const int prow = sub / nblk, jl = (v4 & 3) * 4;
-    const int cl = (sub - prow * nblk) * SUB_CH + ((v4 >> 2) & 15);
-    const int bit = sub_bit(g.tx_shift, prow, sub - prow * nblk);
-    const float4* src = base + v4;
+    constexpr int SHARES = NT / 64;
+    // two, in turn: a wave may be one sub-tile ahead of the wave that sums
+    __shared__ double sums[2][SHARES - 1][4][64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63;
-    double s0[4] = {0.0, 0.0, 0.0, 0.0};
-    uint64_t seen = 0u;
-    for (uint32_t q0 = 0; q0 < ni; q0 += 64) {
-        uint64_t set = __ballot(q0 + lane < ni && ((mk[q0 + lane] >> bit) & 1u));
-        seen |= set;
-        const float4* p = src + q0 * tile;
-        while (set) {
-            float4 v[RED_DEEP];
-            int n = 0;
+    const size_t tile = (size_t)CELL_VOXELS / 4;  // float4 per partial tile
+    const int nblk = (1 << g.cb_shift) / SUB_CH;
+    const uint32_t n = status[ST_SPLIT] * RED_SUBS;
+    const bool shared = status[ST_MULTI] >= RED_SHARED * status[ST_SPLIT];
+    const uint64_t every = shared ? 0x1111111111111111ull << wave : ~0ull;
+    const uint32_t stride = shared ? gridDim.x : gridDim.x * SHARES;
+    int turn = 0;
+    for (uint32_t e = shared ? blockIdx.x : blockIdx.x * SHARES + wave; e < n; e += stride) {
+        const int cell = (int)split_cells[e / RED_SUBS];
+        const int sub = (int)(e % RED_SUBS);  // row * blocks + block
+        const uint32_t ni = item_off[cell + 1] - item_off[cell], first = multi_off[cell];
+        // float4 `lane` of the sub-tile: channel lane / 4, four pixels from 4 (lane % 4) on
+        static_assert(TILE_Y == 16 && SUB_CH == 16, "64 float4 a sub-tile");
+        const float4* src =
+            reinterpret_cast<const float4*>(partials) + (size_t)first * tile + sub * 64 + lane;
+        const uint64_t* mk = part_masks + first;
+        const int prow = sub / nblk, blk = sub - prow * nblk;
+        const int bit = sub_bit(g.tx_shift, prow, blk);
+        double s0[4] = {0.0, 0.0, 0.0, 0.0};
+        uint64_t seen = 0u;
+        for (uint32_t q0 = 0; q0 < ni; q0 += 64) {
+            const uint64_t all = __ballot(q0 + lane < ni && ((mk[q0 + lane] >> bit) & 1u));
+            seen |= all;
+            uint64_t set = all & every;
+            const float4* p = src + q0 * tile;
+            while (set) {
+                float4 v[RED_DEEP];
+                int m = 0;
 #pragma unroll
-            for (int k = 0; k < RED_DEEP; ++k) {
-                if (!set) break;  // uniform
-                v[k] = p[(size_t)__builtin_ctzll(set) * tile];
-                set &= set - 1u;
-                n = k + 1;
-            }
+                for (int k = 0; k < RED_DEEP; ++k) {
+                    if (!set) break;  // uniform
+                    v[k] = p[(size_t)__builtin_ctzll(set) * tile];
+                    set &= set - 1u;
+                    m = k + 1;
+                }
 #pragma unroll
-            for (int k = 0; k < RED_DEEP; ++k) {
-                if (k >= n) break;
-                s0[0] += (double)v[k].x;
-                s0[1] += (double)v[k].y;
-                s0[2] += (double)v[k].z;
-                s0[3] += (double)v[k].w;
+                for (int k = 0; k < RED_DEEP; ++k) {
+                    if (k >= m) break;
+                    s0[0] += (double)v[k].x;
+                    s0[1] += (double)v[k].y;
+                    s0[2] += (double)v[k].z;
+                    s0[3] += (double)v[k].w;
+                }
             }
         }
+        if (!seen) continue;  // the same for the waves that share a sub-tile
+        if (shared) {
+            double(&buf)[SHARES - 1][4][64] = sums[turn];
+            turn ^= 1;
+            if (wave > 0) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) buf[wave - 1][u][lane] = s0[u];
+            }
+            __syncthreads();
+            if (wave > 0) continue;
+#pragma unroll
+            for (int w = 0; w < SHARES - 1; ++w)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) s0[u] += buf[w][u][lane];
+        }
+        const CellPos cp = cell_pos(cell, g);
+        const int i = cp.x0 + prow, j = cp.y0 + (lane & 3) * 4, c = cp.c0 + blk * SUB_CH + (lane >> 2);
+        float* dst = cube + ((size_t)i * g.ny + j) * g.nc + c;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i < g.nx && c < g.nc && j + u < g.ny) {
+                float& v = dst[(size_t)u * g.nc];
+                v = (float)((double)v + s0[u]);
+            }
     }
-    if (!seen) return;
-    const CellPos cp = cell_pos(cell, g);
-    const int i = cp.x0 + prow, j = cp.y0 + jl, c = cp.c0 + cl;
-    if (i >= g.nx || c >= g.nc) return;
-    float* dst = cube + ((size_t)i * g.ny + j) * g.nc + c;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-        if (j + u < g.ny) {
-            float& v = dst[(size_t)u * g.nc];
-            v = (float)((double)v + s0[u]);
-        }
 }
 
 // The weight tables are constant data (the FP64 closed forms of the four
@@ -136,8 +170,10 @@ __global__ void k_spectra(const mi_particle* __restrict__ P, int64_t n, mi_cube_
 
 hipError_t reduce_partials(const Grid& g, char* ws, const Layout& L, float* d_cube,
                            hipStream_t s) {
-    hipLaunchKernelGGL(k_reduce, dim3((unsigned)(g.ncells * RED_PARTS)), dim3(NT), 0, s,
-                       (const uint32_t*)(ws + L.item_off), (const uint32_t*)(ws + L.multi_off),
+    if (L.split_max <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_reduce, dim3((unsigned)std::min<int64_t>(L.split_max * RED_SUBS, RED_GROUPS)),
+                       dim3(NT), 0, s, (const uint32_t*)(ws + L.item_off),
+                       (const uint32_t*)(ws + L.multi_off), (const uint32_t*)(ws + L.split_cells),
                        (const uint32_t*)(ws + L.status), g, (const float*)(ws + L.partials),
                        (const uint64_t*)(ws + L.part_masks), d_cube);
     return hipGetLastError();

@@ -52,19 +52,21 @@ struct Layout {
     size_t item_off, multi_off;        // uint32[ncells + 1] each: exclusive scans of the
                                        // items and the partial-tile slots per cell
     size_t item_pos;                   // uint32[ncells]: launch position of a cell's first item
+    size_t split_cells;                // uint32[split_max]: the cells of more than one item
     size_t items;                      // int4[items_max], in launch order
     size_t partials;                   // float[multi_max * CELL_VOXELS]
     size_t part_masks;                 // uint64[multi_max]: the sub-tiles each partial holds
     size_t total;
-    int64_t items_max, multi_max;
+    int64_t items_max, multi_max, split_max;
     int item_len;                      // particles per work item
 };
 
 // status[0]: number of pairs the device produced; status[1]: overflow flag.
 // status[4]: a record with a footprint has an unknown kernel kind or table
 // weights beyond the descriptor's table (no work items are then made).
+// ST_SPLIT: number of cells with more than one item.
 // ST_TICKET on: group tickets of the emit pass and of each radix pass.
-enum { ST_PAIRS = 0, ST_OVERFLOW = 1, ST_ITEMS = 2, ST_MULTI = 3, ST_BADREC = 4, ST_TICKET = 8,
+enum { ST_PAIRS = 0, ST_OVERFLOW = 1, ST_ITEMS = 2, ST_MULTI = 3, ST_BADREC = 4, ST_SPLIT = 5, ST_TICKET = 8,
        ST_WORDS = 16 };
 
 hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L);
