@@ -46,7 +46,7 @@ constexpr int IMG_X = 4;          // output rows (waves) per work group
 constexpr int IMG_T = 64 * IMG_X;
 constexpr int IMG_C = 16;         // channels per work group
 constexpr int IMG_MAX_W = 128;    // image columns per segment
-constexpr int IMG_GROUPS = 256;   // work groups from which this kernel is taken
+constexpr int IMG_MIN = 1000;      // k_convolve_beam's work groups from which this kernel is taken
 
 // LDS slots of 64 bytes (one pixel's 16 channels) in a row buffer of px pixels.
 // The pixel groups of a wave lie R pixels apart: with an even R one spare slot
@@ -496,25 +496,24 @@ hipError_t convolve_beam(const float* in, float* out, int nx, int ny, int nc, co
         return convolve_line(in, out, 1, nx, (int64_t)ny * nc, K, kx, s);
     if (kx == 1 && ky <= LINE_MAX_K)  // along y: [nx][ny][nc]
         return convolve_line(in, out, nx, ny, nc, K, ky, s);
-    // k_convolve_image where it fills the chip: with fewer than a work group per
-    // CU its rows, one after another, are a chain that k_convolve_beam's small
-    // tiles do not have (90 x 81 x 45, 138 groups: 39 us against 29.5;
-    // 128 x 128 x 12, 96 groups: 57 against 40; 128 x 128 x 64, 384 groups: 60
-    // against 64.5; 282 x 282 x 128: 283 against 596), and where its tiles of
-    // 48 columns or more are not half empty (256 x 24 x 128: 66 against 62).
-    // Three outputs per lane against four by the columns they cover: three take
+    const int64_t tiles = (int64_t)((nx + BT - 1) / BT) * ((ny + BT - 1) / BT), cq = (nc + 3) / 4;
+    // k_convolve_image where there is work for it: its rows, one after another, are a
+    // chain of some 60 us (27 x 27 taps) however few its work groups are, while
+    // k_convolve_beam's time goes with the number of its small tiles (720 of them, 256
+    // x 70 x 36: 65 us against 49; 768, 256 x 87 x 30: 58 against 50; 960, 89 x
+    // 65 x 128: 65 against 62; 1024, 128 x 128 x 64: 60 against 64.5; 2560, 256 x
+    // 68 x 128: 87 against 130; 10368, 282 x 282 x 128: 283 against 596); and where
+    // its tiles of 48 columns or more are not half empty (256 x 24 x 128: 66 against
+    // 62).  Three outputs per lane against four by the columns they cover: three take
     // 1.09 times as long per column.
     const int64_t y3 = (ny + 47) / 48, y4 = (ny + 63) / 64;
     const bool three = y3 * 48 * 12 < y4 * 64 * 11;
-    if (ny > 32 &&
-        ((nx + IMG_X - 1) / IMG_X) * (three ? y3 : y4) * ((nc + IMG_C - 1) / IMG_C) >= IMG_GROUPS)
+    if (ny > 32 && tiles * cq >= IMG_MIN)
         return three ? convolve_image<3>(in, out, nx, ny, nc, K, kx, ky, s)
                      : convolve_image<4>(in, out, nx, ny, nc, K, kx, ky, s);
     const int h = beam_block_rows(kx, ky), w = beam_block_cols(ky);
     const size_t lds = beam_lds_bytes(kx, ky);
-    const unsigned tiles = (unsigned)(((nx + BT - 1) / BT) * ((ny + BT - 1) / BT));
-    const unsigned cq = (unsigned)((nc + 3) / 4);
-    hipLaunchKernelGGL(k_convolve_beam, dim3(tiles, cq), dim3(256), lds, s, in, out, nx, ny, nc, K,
+    hipLaunchKernelGGL(k_convolve_beam, dim3((unsigned)tiles, (unsigned)cq), dim3(256), lds, s, in, out, nx, ny, nc, K,
                        kx, ky, h, w);
     return hipGetLastError();
 }

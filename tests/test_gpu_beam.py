@@ -256,6 +256,20 @@ def test_image_tiles(shape, k, special):
 
 
 @pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("shape,k", [
+    ((170, 48, 128), (3, 3)), ((180, 47, 126), (5, 7)),     # three outputs per lane, one tile
+    ((170, 64, 120), (7, 5)), ((180, 65, 110), (3, 9)),     # four; a tile of few columns
+    ((150, 96, 70), (1, 3)), ((170, 49, 128), (9, 1)),
+    ((170, 33, 128), (5, 131)), ((340, 40, 64), (3, 257)),
+    ((128, 128, 62), (5, 3)), ((128, 125, 60), (5, 3)),     # 1024 and 960 of the small tiles
+])
+def test_image_tiles_from_1000(shape, k, special):
+    """The same on cubes of at least 1000 of the small tiles, which the tiled image
+    kernel takes, and about that number."""
+    test_image_tiles(shape, k, special)
+
+
+@pytest.mark.parametrize("special", [False, True])
 @pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("shape,k,axis", [
     ((31, 3, 24), 1, 0), ((32, 5, 24), 3, 0), ((33, 4, 36), 17, 0), ((65, 2, 5), 27, 0),
