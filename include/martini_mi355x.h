@@ -133,6 +133,22 @@ int mi_abi_version(void);
 const char* mi_strerror(int code);
 
 /*
+ * Host FP64 setup to records (host pointers, no device access): one pass over
+ * n particles with pixel coordinates x, y, mask half-widths r, kernel sizes h
+ * (pixels), kernel codes (MI_KERNEL_* | Gaussian table index << 4; not
+ * MI_KERNEL_TABLE), line-of-sight velocities v (km/s), line widths sigma (km/s;
+ * sigma[k * sigma_step], step 0 or 1; unused for the Dirac line) and amplitudes,
+ * for nc channels of edges[0..nc] (m/s) and the uniform step de.  The same FP64
+ * operations in the same order as a NumPy evaluation, so the same bytes.
+ * MI_ERR_LIMIT: a particle in the cube with a pixel coordinate beyond 2^21.
+ */
+int mi_pack_records(int64_t n, const double* x, const double* y, const double* r,
+                    const double* h, const int32_t* kernel, const double* v,
+                    const double* sigma, int64_t sigma_step, const double* amp,
+                    const double* edges, double de, int32_t nx, int32_t ny, int32_t nc,
+                    int32_t spectrum, mi_particle* out);
+
+/*
  * Number of (particle, cell) pairs the binning of these particles produces:
  * a cell is an 8 x 16 pixel tile times a 128-channel block when the cube has
  * 128 channels or more (nc >= 128), else a 16 x 16 tile times a 64-channel

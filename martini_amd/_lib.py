@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(_HERE, "libmartini_mi355x.so")
 
 MI_OK = 0
 MI_ERR_WORKSPACE = -2
+MI_ERR_LIMIT = -5
 
 KERNEL_CUBIC, KERNEL_WC2, KERNEL_WC6, KERNEL_QUARTIC, KERNEL_GAUSS, KERNEL_DIRAC = range(6)
 KERNEL_TABLE = 6  # a kernel without a device form: weights evaluated by the host
@@ -101,6 +102,9 @@ def lib() -> ctypes.CDLL:
     L.mi_strerror.argtypes = [ctypes.c_int]
     L.mi_count_pairs_host.restype = i64
     L.mi_count_pairs_host.argtypes = [vp, i64, ctypes.POINTER(CubeDesc)]
+    L.mi_pack_records.restype = ctypes.c_int
+    L.mi_pack_records.argtypes = [i64, vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, ctypes.c_double,
+                                  ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, vp]
     L.mi_insert_workspace_size.restype = ctypes.c_int
     L.mi_insert_workspace_size.argtypes = [ctypes.POINTER(CubeDesc), i64, i64,
                                            ctypes.POINTER(ctypes.c_size_t)]
@@ -172,6 +176,30 @@ def make_desc(nx, ny, nc, spectrum, gauss_table=(), spectra=None, spectra_ld=0) 
         d.gauss_t[k] = float(t)
         d.gauss_inv_norm[k] = float(1.0 / norm)
     return d
+
+
+def pack_records(x, y, r, h, kernel, v, sigma, amp, edges, de, shape, spectrum):
+    """Records from host FP64 arrays (mi_pack_records), or None when a particle
+    in the cube lies beyond 2^21 pixels; sigma a scalar or one per particle."""
+    def f64(a):
+        return np.ascontiguousarray(a, np.float64)
+
+    arrays = [f64(a) for a in (x, y, r, h)] + [np.ascontiguousarray(kernel, np.int32), f64(v),
+                                              f64(sigma).reshape(-1)]
+    n = arrays[0].size
+    step = int(arrays[6].size > 1)
+    arrays += [f64(amp), f64(edges)]
+    if any(a.shape != (n,) for a in arrays[:6] + arrays[7:8]) or arrays[6].size not in (1, n) \
+            or arrays[8].size != shape[2] + 1:
+        raise ValueError("pack_records: arrays of different lengths")
+    out = np.empty(n, PARTICLE_DTYPE)
+    p = [ctypes.c_void_p(a.ctypes.data) for a in arrays]
+    rc = lib().mi_pack_records(n, *p[:7], step, *p[7:], float(de), *(int(m) for m in shape),
+                               int(spectrum), ctypes.c_void_p(out.ctypes.data))
+    if rc == MI_ERR_LIMIT:
+        return None
+    check(rc, "mi_pack_records")
+    return out
 
 
 def count_pairs(records: np.ndarray, desc: CubeDesc) -> int:

@@ -39,6 +39,11 @@ def channel_grid(datacube):
     return e, e[0], (e[-1] - e[0]) / nc
 
 
+def amplitude(mHI, dist_mpc, de, out_scale):
+    return (np.asarray(mHI, float) * np.asarray(dist_mpc, float) ** -2.0
+            / (abs(de) / 1e3) / MHI_TO_JY * out_scale)
+
+
 def spectral_fields(vlos_kms, sigma_kms, mHI, dist_mpc, datacube, spectrum_kind,
                     out_scale=1.0):
     """k0, fu, s, amp, c_lo, c_hi per particle."""
@@ -52,8 +57,7 @@ def spectral_fields(vlos_kms, sigma_kms, mHI, dist_mpc, datacube, spectrum_kind,
     uu = np.where(finite, u, 0.0)
     k0 = np.floor(uu)
     fu = uu - k0
-    amp = (np.asarray(mHI, float) * np.asarray(dist_mpc, float) ** -2.0
-           / (abs(de) / 1e3) / MHI_TO_JY * out_scale)
+    amp = amplitude(mHI, dist_mpc, de, out_scale)
     if spectrum_kind == _lib.SPECTRUM_GAUSS:
         sig = np.broadcast_to(np.asarray(sigma_kms, float), (n,)) * 1e3
         with np.errstate(divide="ignore"):
@@ -164,22 +168,30 @@ def table_weights(sph_kernel, kernels, which, kinds, x, y, ix, iy, fx, fy, rr, h
     return offsets, out
 
 
-def kernel_fields(sph_kernel, pixcoords, nx, ny):
-    """ix, iy, fx, fy, h, r_kind per particle, the Gaussian (t, norm) table and
-    the host-evaluated weights of kernels without a device form (None when
-    there are none); for those particles h holds their table offset's bits."""
+def kernel_codes(sph_kernel):
+    """The concrete kernels, each particle's, their device kinds and indices into
+    the Gaussian (t, norm) table, and that table."""
     kernels, which = sph_kernel._device_kernels()
-    kinds = np.array([device_kind(K) for K in kernels], np.int64)[which]
+    kinds = np.array([device_kind(K) for K in kernels], np.int64)
     gauss = []
-    gidx_of_kernel = np.zeros(len(kernels), np.int64)
+    gidx = np.zeros(len(kernels), np.int64)
     for ik, K in enumerate(kernels):
         if K._mi_kind == _lib.KERNEL_GAUSS:
             key = (float(K.truncate), float(K.norm))
             if key not in gauss:
                 gauss.append(key)
-            gidx_of_kernel[ik] = gauss.index(key)
+            gidx[ik] = gauss.index(key)
     if len(gauss) > 4:
         raise ValueError("at most 4 distinct Gaussian truncations per insertion")
+    return kernels, which, kinds, gidx, gauss
+
+
+def kernel_fields(sph_kernel, pixcoords, nx, ny):
+    """ix, iy, fx, fy, h, r_kind per particle, the Gaussian (t, norm) table and
+    the host-evaluated weights of kernels without a device form (None when
+    there are none); for those particles h holds their table offset's bits."""
+    kernels, which, kind_of_kernel, gidx_of_kernel, gauss = kernel_codes(sph_kernel)
+    kinds = kind_of_kernel[which]
     gidx = gidx_of_kernel[which]
     h_px = np.asarray(sph_kernel.sm_lengths, float)
     h_eff = h_px * np.asarray(sph_kernel._rescale, float)
@@ -261,6 +273,37 @@ def table_fields(spectral_model, source, datacube, out_scale=1.0):
             c_hi.astype(np.int64), np.ascontiguousarray(S, np.float32))
 
 
+def _native_records(source, sph_kernel, spectral_model, datacube, out_scale):
+    """(records, Gaussian table) by ``_lib.pack_records``, which computes what
+    ``kernel_fields``, ``spectral_fields`` and ``make_records`` do with one pass
+    over the particles instead of some eighty (1e5 particles: 4.5 -> 2.2 ms);
+    None when a kernel or the spectrum has no device form, or the library is not
+    there."""
+    if spectral_model._mi_kind == _lib.SPECTRUM_TABLE:
+        return None
+    _, which, kinds, gidx, gauss = kernel_codes(sph_kernel)
+    if np.any(kinds == _lib.KERNEL_TABLE):
+        return None
+    try:
+        _lib.lib()
+    except ImportError:
+        return None
+    nx, ny, nc = datacube._array.shape[:3]
+    x, y = source.pixcoords[0], source.pixcoords[1]
+    sc = source.skycoords
+    e, _, de = channel_grid(datacube)
+    h = np.asarray(sph_kernel.sm_lengths, float) * np.asarray(sph_kernel._rescale, float)
+    rec = _lib.pack_records(x, y, sph_kernel.sm_ranges, h, (gidx << 4 | kinds)[which],
+                            sc.radial_velocity,
+                            spectral_model._sigma_kms(source)
+                            if spectral_model._mi_kind == _lib.SPECTRUM_GAUSS else 0.0,
+                            amplitude(source.mHI_g, sc.distance, de, out_scale), e, de,
+                            (nx, ny, nc), spectral_model._mi_kind)
+    if rec is None:
+        raise ValueError("pixel coordinates beyond 2^21 cannot be represented")
+    return rec, gauss
+
+
 def pack_particles(source, sph_kernel, spectral_model, datacube, out_scale=1.0):
     """Records and cube descriptor for an initialised (and pruned) source.
     For a table spectrum the descriptor carries the host table as
@@ -268,6 +311,10 @@ def pack_particles(source, sph_kernel, spectral_model, datacube, out_scale=1.0):
     pixel weights as ``host_weights``; the inserter uploads them and points
     the descriptor at them."""
     nx, ny, nc = datacube._array.shape[:3]
+    native = _native_records(source, sph_kernel, spectral_model, datacube, out_scale)
+    if native is not None:
+        rec, gauss = native
+        return rec, _lib.make_desc(nx, ny, nc, spectral_model._mi_kind, gauss, spectra_ld=0)
     ix, iy, fx, fy, h, r_kind, gauss, ktable = kernel_fields(sph_kernel, source.pixcoords, nx, ny)
     sc = source.skycoords
     table = None

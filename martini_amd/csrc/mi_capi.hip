@@ -3,6 +3,8 @@
 // stage sequence bin -> gather -> reduce.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+#include <limits>
 #include <mutex>
 
 #include "../../include/martini_mi355x.h"
@@ -74,6 +76,97 @@ const char* mi_strerror(int code) {
                "(MI_SCRATCH_BYTES)";
     }
     return "unknown error";
+}
+
+int mi_pack_records(int64_t n, const double* x, const double* y, const double* r,
+                    const double* h, const int32_t* kernel, const double* v, const double* sigma,
+                    int64_t sigma_step, const double* amp, const double* edges, double de,
+                    int32_t nx, int32_t ny, int32_t nc, int32_t spectrum, mi_particle* out) {
+#pragma clang fp contract(off)
+    if (n < 0 || nx <= 0 || ny <= 0 || nc <= 0 || !edges ||
+        (n > 0 && (!x || !y || !r || !h || !kernel || !v || !amp || !out)))
+        return MI_ERR_ARGUMENT;
+    if (spectrum != MI_SPECTRUM_GAUSS && spectrum != MI_SPECTRUM_DIRAC) return MI_ERR_UNSUPPORTED;
+    if (spectrum == MI_SPECTRUM_GAUSS && n > 0 && !sigma) return MI_ERR_ARGUMENT;
+    // floor and ceil by a conversion (a call each otherwise); larger values are whole.
+    // A zero's sign is lost: t - floor(t) + 0.0 is +0.0 then as well.
+    auto floor_of = [](double t) {
+        if (!(std::fabs(t) < 0x1p52)) return t;
+        const double w = (double)(int64_t)t;
+        return w > t ? w - 1.0 : w;
+    };
+    auto ceil_of = [&](double t) { return -floor_of(-t); };
+    // as NumPy converts: INT64_MIN for NaN and what does not fit
+    auto whole = [](double t) {
+        return t >= -0x1p63 && t < 0x1p63 ? (int64_t)t : std::numeric_limits<int64_t>::min();
+    };
+    // as np.clip: NaN stays
+    auto clip = [](double t, double lo, double hi) { return t < lo ? lo : t > hi ? hi : t; };
+    const double e0 = edges[0], width = std::fabs(de), last_x = nx - 1.0, last_y = ny - 1.0;
+    const double chans = nc, sqrt2 = std::sqrt(2.0);
+    constexpr double FINITE = std::numeric_limits<double>::max();
+    for (int64_t k = 0; k < n; ++k) {
+        mi_particle& p = out[k];
+        const double xk = x[k], yk = y[k], rk = r[k];
+        const bool alive = std::fabs(xk) <= FINITE && std::fabs(yk) <= FINITE && rk >= 0.0 &&
+                           xk + rk >= 0.0 && yk + rk >= 0.0 && xk - rk <= last_x && yk - rk <= last_y;
+        const double xs = alive ? xk : 0.0, ys = alive ? yk : 0.0;
+        if (std::fabs(xs) >= 0x1p21 || std::fabs(ys) >= 0x1p21) return MI_ERR_LIMIT;
+        double ix = floor_of(xs), iy = floor_of(ys), fx = xs - ix + 0.0, fy = ys - iy + 0.0;
+        double rr = alive ? (rk < 0x1p22 ? rk : 0x1p22) : -1.0;
+        if (kind_of(kernel[k]) == MI_KERNEL_DIRAC) {
+            // the one pixel with |x - i| < 0.5 (strict) that the mask also admits
+            ix = floor_of(xs + 0.5);
+            iy = floor_of(ys + 0.5);
+            const double ax = std::fabs(xs - ix), ay = std::fabs(ys - iy);
+            const bool ok = ax < 0.5 && ay < 0.5 && ax <= rr && ay <= rr && ix >= 0.0 &&
+                            ix <= last_x && iy >= 0.0 && iy <= last_y && alive;
+            fx = fy = 0.0;
+            rr = ok ? 0.0 : -1.0;
+        }
+        p.ix = (int32_t)ix;
+        p.iy = (int32_t)iy;
+        p.fx = (float)fx;
+        p.fy = (float)fy;
+        p.h = (float)h[k];
+        p.r_kind = (int32_t)((uint32_t)(int32_t)rr << 8 | (uint32_t)kernel[k]);
+
+        const double vk = v[k] * 1e3, u = (vk - e0) / de;
+        const bool finite = std::fabs(u) <= FINITE;
+        const double uu = finite ? u : 0.0, k0 = floor_of(uu);
+        double s = 0.0, lo, hi;
+        if (spectrum == MI_SPECTRUM_GAUSS) {
+            s = width / (sqrt2 * (sigma[k * sigma_step] * 1e3));
+            const double half = 4.0 / s;
+            lo = floor_of(uu - 1.0 - half) + 1.0;
+            hi = ceil_of(uu + half) - 1.0;
+        } else {
+            lo = std::numeric_limits<double>::infinity();
+            hi = -lo;
+            for (int d = -1; d <= 1; ++d) {
+                const double at = k0 + d;
+                if (!finite || at < 0.0 || at > chans - 1.0) continue;
+                const double a = edges[(int64_t)at], b = edges[(int64_t)at + 1];
+                if (vk < (a < b ? a : b) || vk > (a < b ? b : a)) continue;
+                lo = at < lo ? at : lo;
+                hi = at > hi ? at : hi;
+            }
+        }
+        lo = clip(finite ? lo : chans, 0.0, chans);
+        hi = clip(finite ? hi : -1.0, -1.0, chans - 1.0);
+        if (lo > hi) {
+            lo = 1.0;
+            hi = 0.0;
+        }
+        p.c_lo = (int32_t)whole(lo);
+        p.c_hi = (int32_t)whole(hi);
+        const int64_t kw = whole(k0);
+        p.k0 = (int32_t)(kw < -(1 << 30) ? -(1 << 30) : kw > 1 << 30 ? 1 << 30 : kw);
+        p.fu = (float)(uu - k0 + 0.0);
+        p.s = (float)s;
+        p.amp = (float)amp[k];
+    }
+    return MI_OK;
 }
 
 int64_t mi_count_pairs_host(const mi_particle* h_particles, int64_t n, const mi_cube_desc* desc) {

@@ -106,13 +106,18 @@ class _BaseMartini:
         was_empty = not np.any(dc._array)
         d_cube = default_inserter().insert(rec, desc, method=method)
         added = d_cube.cpu().numpy().astype(np.float64).reshape(dc._array.shape[:3])
-        if dc._array_unit == "Jy/pix2":
-            dc._array = dc._array / px2
+        if was_empty and dc._array_unit == "Jy/pix2" and dc._array.dtype == np.float64:
+            # 0 / px2 + added, without the two passes over the host cube
+            dc._array = added[..., None] if dc.stokes_axis else added
             dc._array_unit = "Jy/arcsec2"
-        if dc.stokes_axis:
-            dc._array[..., 0] += added
         else:
-            dc._array += added
+            if dc._array_unit == "Jy/pix2":
+                dc._array = dc._array / px2
+                dc._array_unit = "Jy/arcsec2"
+            if dc.stokes_axis:
+                dc._array[..., 0] += added
+            else:
+                dc._array += added
         # The device cube equals the host cube while this array object holds
         # exactly the insertion (FP32 values widened to FP64); convolve_beam
         # then starts from it.  The methods of this class replace the array
