@@ -77,25 +77,37 @@ __host__ __device__ inline bool wide_cells(int nc) { return nc >= 128; }
 // Particles per cell processed by one work item: longer cells are split and
 // their partial tiles summed in item order by a reduction pass.  The split
 // length depends only on the pair count, so a given input always sums in the
-// same order: about ITEM_TARGET items of at most ITEM_MAX particles, which
-// balances the CUs; below ITEM_WHOLE particles per item, instead, as many items
-// as run at once (ITEM_FILL: three work groups on each of 256 CUs) and no more,
+// same order: about 2304 items (three rounds of ITEM_FILL) of at most ITEM_MAX
+// particles, which balances the CUs, or 2048 below 2^20 pairs, whose partial tiles
+// the static scratch of mi_insert_noalloc may have to hold (1e6 particles: 473 us
+// with 2248 items, 480 with 2000); below ITEM_WHOLE particles per item, instead, as
+// many items as run at once (ITEM_FILL: three work groups on each of 256 CUs) and no more,
 // since each split costs a partial tile.  13000 pairs, FP32, in items of 256
 // (52 of them): 159 us per insertion, of 32: 107; 1.7e5 pairs, MFMA: 154 us in
-// 768 items, 167 in 2048.  ITEM_TARGET also bounds the FP32 error, which grows with
-// the longest run summed before the FP64 reduction: 1.4e6 particles, 512 x 512 x
-// 256, FP32, relative to FP64: 6.0e-7 with 2048 items, 5.2e-7 with 2304, 3.6e-7
-// with 3072; 1e6 particles, FP32: 556, 557 and 573 us per insertion.  The partial tiles of ITEM_FILL items take at most
-// 101 MB of workspace, the cells of the largest grid beside them 84 MB.
+// 768 items, 167 in 2048.  The FP32 error grows with the longest run that is summed
+// before the FP64 reduction, so that past ITEM_EVEN particles the length grows half
+// as fast as the pair count (1.5e6 particles, 512 x 512 x 256, FP32, relative to
+// FP64: 3.2e-7 with 2304 items throughout, 2.1e-7 so; the times are the same within
+// 0.5%; 3072 items throughout: 2% more on 1e6 particles).  The partial tiles of
+// ITEM_FILL items take at most 101 MB of workspace, the cells of the largest grid
+// beside them 84 MB.
 constexpr int ITEM_MIN = 32;
 constexpr int ITEM_WHOLE = 256;
 constexpr int ITEM_MAX = 4096;
-constexpr int ITEM_TARGET = 2304;
+constexpr int ITEM_EVEN = 896;
 constexpr int ITEM_FILL = 768;
 
+__host__ __device__ inline int item_target(int64_t n_pairs) {
+    return n_pairs < (1 << 20) ? 2048 : 3 * ITEM_FILL;
+}
+
 __host__ __device__ inline int item_length(int64_t n_pairs) {
-    const int64_t balanced = (n_pairs / ITEM_TARGET + 31) / 32 * 32;
-    if (balanced >= ITEM_WHOLE) return (int)(balanced > ITEM_MAX ? ITEM_MAX : balanced);
+    const int64_t balanced = (n_pairs / item_target(n_pairs) + 31) / 32 * 32;
+    if (balanced >= ITEM_WHOLE) {
+        const int64_t len =
+            balanced <= ITEM_EVEN ? balanced : (ITEM_EVEN + (balanced - ITEM_EVEN) / 2 + 31) / 32 * 32;
+        return (int)(len > ITEM_MAX ? ITEM_MAX : len);
+    }
     const int64_t filled = (n_pairs / ITEM_FILL + 31) / 32 * 32;
     return (int)(filled < ITEM_MIN ? ITEM_MIN : (filled > ITEM_WHOLE ? ITEM_WHOLE : filled));
 }

@@ -484,8 +484,11 @@ template <int K, bool SCALED>
 struct LineSeries {
     float e[K + 1];
 
-    // 1 / sqrt(pi) in FP32 is off by 5e-8, the same for every line: the coefficients
-    // take that back (1 - 5e-8 is within 1e-8 of an FP32 number).
+    // 1 / sqrt(pi) in FP32 is 5e-8 too large, for every line alike.  The longer series'
+    // coefficients take that back (1 - 5e-8 is within 1e-8 of an FP32 number).  The
+    // narrow lines' do not: the FP32 sums of such lines, many small tails among them,
+    // come out about 1e-7 low on sparse cubes (1.6e5 particles, 512 x 512 x 256: 1.3e-7
+    // of error with it, 1.7e-7 without).
     static constexpr float ROOT = 0.564189583547756287f;
     // c[k][j]: of D^2k m^2j (the Hermite polynomials' coefficients)
     struct Table {
@@ -495,7 +498,7 @@ struct LineSeries {
         Table t{};
         // 1 / (2 j)!, its scale included, and (-1)^i / (4^i i!)
         double inv_2j[K + 1] = {}, inv_i[K + 1] = {};
-        double a = 0.564189583547756287 / (double)ROOT, b = 1.0;
+        double a = SCALED ? 1.0 : 0.564189583547756287 / (double)ROOT, b = 1.0;
         for (int j = 0; j <= K; ++j) {
             inv_2j[j] = a;
             inv_i[j] = b;
@@ -576,14 +579,16 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
             if ((blocks >> b) & 1u) put(b, amp, amp);
         return;
     }
-    // Channel c = c0 + cl0 + 8 j of this thread sits at k0 - c + fu - 1/2 =
-    // A - 8 j from the line centre (in channels), A formed once; subtracting
-    // the small integer 8 j from A is exact in the in-window range.
+    // Channel c = c0 + cl0 + o of this thread sits at k0 - c + fu - 1/2 = (kf - o) + fh
+    // from the line centre (in channels): the first difference is exact, so that each
+    // offset is rounded to its own precision (formed from the cell's first channel
+    // it was off by up to 4e-6 channels: 1.2e4 particles, 256 x 256 x 128, FP32,
+    // relative to FP64: 1.7e-7, 0.7e-7 so).
     const int kc = k0 - c0 - cl0;
-    const float A = (float)kc + (fu - 0.5f);
-    // exp(-m^2) as exp2(-n^2) with n = m sqrt(log2 e): n = sn (A - 8 j).
+    const float kf = (float)kc, fh = fu - 0.5f;
+    // exp(-m^2) as exp2(-n^2) with n = m sqrt(log2 e).
     const float sn = s * SQRT_LOG2E;
-    auto narrow = [&](const LineSeries<3, true>& line, int o) { return line(sn * (A - (float)o)); };
+    auto narrow = [&](const LineSeries<3, true>& line, int o) { return line(sn * ((kf - (float)o) + fh)); };
     if (!__any(s > 0.5f)) {
         const LineSeries<3, true> line(s, amp);
 #pragma unroll
@@ -593,11 +598,9 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
         return;
     }
     if (!__any(s > 1.5f)) {
-        // A longer series, a seventh of the erf difference's work per channel; the
-        // offsets each to their own precision (3e5 particles, s = 0.8, split BF16: 232
+        // A longer series, a seventh of the erf difference's work per channel (3e5 particles, s = 0.8, split BF16: 232
         // -> 220 us per insertion; 3e6 of which half have s = 6 and go on: 3.05 -> 3.09 ms).
         const LineSeries<7, false> line(s, amp);
-        const float kf = (float)kc, fh = fu - 0.5f;
 #pragma unroll 1
         for (uint32_t left = blocks; left != 0u; left &= left - 1u) {
             const int b = __builtin_ctz(left);
