@@ -18,13 +18,16 @@
 //              hi*lo, lo*hi -- accumulated in FP32 (the dropped lo*lo term is below
 //              2^-16 of the product).
 //
-// Both are bound by the evaluation of W and S on the vector units; the FP32
-// products take about half of their time beside it.  On the vector units the
+// Both are bound by the evaluation of W and S on the vector units (70% busy on 1e7
+// particles, 512 x 512 x 256, split BF16: gather 3.83 ms; without the W fill 1.1 ms
+// less, without the S fill 0.7, without the products 0.6); the FP32 products take
+// about a quarter of the matrix units' time beside it (26% on 3e6 of heterogeneous
+// size, 1024 x 1024 x 64: 2.8 ms).  On the vector units the
 // FP32 products (64 multiply-adds per particle, thread and tile row, all
 // channels) took most of that form's time: gather 643 us on 1e6 particles
 // (WendlandC2, 256 x 256 x 128), 4.42 ms on 3e6 of heterogeneous size
-// (1024 x 1024 x 64); on the matrix units 597 us and 3.59 ms with the same
-// records.
+// (1024 x 1024 x 64); on the matrix units 597 us and 3.59 ms at first, 360 us and
+// 2.8 ms with what is described below.
 //
 // Wave w owns four tile rows (M = the 16 pixels of a row) and four 16-channel
 // blocks (N): with 16 x 16-pixel x 64-channel cells the rows w, w + 4, .. and
@@ -46,9 +49,9 @@
 // staging is on every chunk's critical path, and half its lanes were idle with one
 // at a time (1e7 particles, 512 x 512 x 256, split BF16: gather 4.47 -> 4.32 ms;
 // four at a time: see STAGED).
-// Per chunk there are two barriers: (staging) -> W, S fill -> products, and a
-// third in chunks with Gaussian-kernel particles, whose row and column factors
-// are tabulated before the W fill.  Each wave clears the W rows it used right
+// Per chunk there are two barriers: (staging) -> W, S fill -> products, and one more
+// (two with the square cells) in chunks with Gaussian-kernel particles, whose row
+// and column factors are tabulated before the W fill.  Each wave clears the W rows it used right
 // after reading them, so the next fill finds them zero; every fill rewrites
 // the S blocks that the products will read.
 // At the end of an item, accumulator blocks that are all zero are not
