@@ -118,4 +118,18 @@ struct Item {
     int32_t cell, q, n, slot;
 };
 
+// A work item's chunks of `chunk` pairs: a walk over the sorted pair list from
+// `begin`, the item's first chunk, to `end`, its cell's end, a step being the
+// chunks of the cell's other items.  It counts the pairs left, not the
+// position: a step is up to a 128th of the cell's pairs, and a position past the
+// end of a cell that ends within a step of 2^31 would not be an int any more.
+struct ItemWalk {
+    int end, step, left;
+    __host__ __device__ ItemWalk(uint32_t cell_start, uint32_t cell_end, const Item& it, int chunk)
+        : end((int)cell_end), step(it.n * chunk), left((int)(cell_end - cell_start) - it.q * chunk) {}
+    __host__ __device__ bool more() const { return left > 0; }
+    __host__ __device__ int at() const { return end - left; }  // while more()
+    __host__ __device__ void next() { left -= step; }
+};
+
 }  // namespace mi

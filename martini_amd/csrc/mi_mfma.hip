@@ -238,8 +238,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     if (status[ST_OVERFLOW]) return;
     if (blockIdx.x >= status[ST_ITEMS]) return;
     const Item it = items[blockIdx.x];  // longest items first
-    const int begin = (int)cell_start[it.cell] + it.q * KC, end = (int)cell_end[it.cell];
-    const int step = it.n * KC;  // from one of the item's chunks to the next
+    ItemWalk chunks(cell_start[it.cell], cell_end[it.cell], it, KC);
+    const int begin = chunks.at(), step = chunks.step;
     const CellPos cp = cell_pos(it.cell, g);
     const int x0 = cp.x0, y0 = cp.y0, c0 = cp.c0;
 
@@ -289,17 +289,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const bool stages = 2 * pair < STAGED;
     RecRegs next{};
     uint32_t next_idx = 0;
-    if (stages && at < end - begin) next = load_record(P, order[begin + at]);
-    if (stages && at + STAGED * step < end - begin) next_idx = order[begin + STAGED * step + at];
+    if (stages && at < chunks.left) next = load_record(P, order[begin + at]);
+    if (stages && at + STAGED * step < chunks.left) next_idx = order[begin + STAGED * step + at];
 
-    for (int kb = begin, slot = 0; kb < end; kb += step, slot = (slot + 1) & (STAGED - 1)) {
-        const int left = end - kb;
+    for (int slot = 0; chunks.more(); chunks.next(), slot = (slot + 1) & (STAGED - 1)) {
+        const int left = chunks.left;
         if (slot == 0 && stages && 2 * pair * step < left) {
             __builtin_amdgcn_s_setprio(3);  // the other waves wait for it: first on its SIMD
             stage_chunks(next, at < left, x0, y0, c0, g, d, staged + 2 * pair);
             __builtin_amdgcn_s_setprio(0);
             if (at + STAGED * step < left) next = load_record(P, next_idx);
-            if (at + 2 * STAGED * step < left) next_idx = order[kb + 2 * STAGED * step + at];
+            if (at + 2 * STAGED * step < left) next_idx = order[chunks.at() + 2 * STAGED * step + at];
         }
         const ChunkState& cs = staged[slot];
         __syncthreads();
