@@ -286,15 +286,23 @@ __global__ __launch_bounds__(T) void k_emit(
             if (w == wave) at[i] += total;
             total += wsum[i][w];
         }
-    if (t == 0) look_store(&look[group], (group == 0 ? LB_ALL : LB_GROUP) | total);
     if (wave == 0) {
+        // The total again without wrapping: 4096 particles of up to 2^21 cells make up
+        // to 2^33 pairs.  (In 64 bits by every thread, above, 1e7 particles took 160 us
+        // more.)
+        static_assert(ROUNDS * (T / 64) <= 64, "a lane per sum");
+        PairSum sum(lane < ROUNDS * (T / 64) ? (&wsum[0][0])[lane] : 0u);
+        sum.upper = __builtin_amdgcn_readlane(wave_scan_add((int)sum.upper), 63);
+        sum.lower = __builtin_amdgcn_readlane(wave_scan_add((int)sum.lower), 63);
+        const unsigned long long all = sum.total();
+        if (lane == 0) look_store(&look[group], (group == 0 ? LB_ALL : LB_GROUP) | all);
         const unsigned long long b = look_back(look, group);
         if (lane == 0) {
-            s_base = b;
-            if (group > 0) look_store(&look[group], LB_ALL | (b + total));
+            s_base = b + (all - total);  // past any capacity where `total` has wrapped
+            if (group > 0) look_store(&look[group], LB_ALL | (b + all));
             if ((group + 1) * (T * ROUNDS) >= n) {
-                status[ST_PAIRS] = (uint32_t)(b + total);
-                status[ST_OVERFLOW] = b + total > (uint64_t)cap ? 1u : 0u;
+                status[ST_PAIRS] = (uint32_t)(b + all);
+                status[ST_OVERFLOW] = b + all > (uint64_t)cap ? 1u : 0u;
             }
         }
     }

@@ -39,6 +39,15 @@ __host__ __device__ inline uint32_t cells_of(const mi_particle& p, const Grid& g
     return (uint32_t)((tx1 - tx0 + 1) * (ty1 - ty0 + 1) * (cb1 - cb0 + 1));
 }
 
+// A sum of pair counts in two 32-bit parts, of the counts' upper and lower 16 bits
+// (64 counts of up to 2^27 each do not fit 32 bits together).
+struct PairSum {
+    uint32_t upper, lower;
+    __host__ __device__ explicit PairSum(uint32_t count = 0u) : upper(count >> 16), lower(count & 0xffffu) {}
+    __host__ __device__ unsigned long long total() const {
+        return ((unsigned long long)upper << 16) + lower;
+    }
+};
 
 // Byte offsets of the workspace regions (each 256-byte aligned).
 struct Layout {

@@ -25,7 +25,19 @@ static long walk(long start, long end, int q, int n) {
     return seen;
 }
 
+// Total of `n` counts of `each` pairs, as a wave sums them (32 bits a part).
+static unsigned long long total(int n, uint32_t each) {
+    PairSum sum;
+    for (int k = 0; k < n; ++k) {
+        const PairSum one(each);
+        sum.upper += one.upper;
+        sum.lower += one.lower;
+    }
+    return sum.total();
+}
+
 int main(int argc, char** argv) {
+    if (argc == 2) return printf("%llu %llu\n", total(16, atol(argv[1])), total(64, atol(argv[1]))), 0;
     const long start = atol(argv[1]), end = atol(argv[2]);
     const int n = (int)((end - start + ITEM_MAX - 1) / ITEM_MAX);
     long chunks = 0;
@@ -41,9 +53,9 @@ int main(int argc, char** argv) {
 
 
 @pytest.fixture(scope="module")
-def walk_items(tmp_path_factory):
-    d = tmp_path_factory.mktemp("walk")
-    src, exe = d / "walk.hip", d / "walk"
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp("index")
+    src, exe = d / "index.hip", d / "index"
     src.write_text(PROGRAM)
     subprocess.run([build_native.HIPCC, "--offload-host-only", "-O1", "-std=c++17",
                     "-I", build_native.CSRC, str(src), "-o", str(exe)], check=True)
@@ -56,7 +68,42 @@ def walk_items(tmp_path_factory):
     (2**31 - 100, 2**31 - 1), (2**31 - 1000000, 2**31 - 1), (2**30, 2**31 - 7),
     (5, 6), (0, 32), (7, 4103), (7, 4104), (1000, 50000),
 ])
-def test_items_visit_each_chunk_of_their_cell_once(walk_items, start, end):
-    r = subprocess.run([str(walk_items), str(start), str(end)], capture_output=True, text=True,
+def test_items_visit_each_chunk_of_their_cell_once(program, start, end):
+    r = subprocess.run([str(program), str(start), str(end)], capture_output=True, text=True,
                        timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+@pytest.mark.parametrize("each", [0, 1, 64, 64 * 4096, 2**26 - 1, 2**26, 64 * (2**21 - 1)])
+def test_group_pair_totals_do_not_wrap(program, each):
+    """A wave's 64 particles make up to 64 (2^21 - 1) pairs; groups of 16 waves, and of 16 in 4 rounds."""
+    r = subprocess.run([str(program), str(each)], capture_output=True, text=True, check=True)
+    assert [int(v) for v in r.stdout.split()] == [16 * each, 64 * each]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [4096, 2**19, 2**19 + 4096])
+def test_an_undercounted_capacity_is_refused(n):
+    """Particles that each cover a whole 16384 x 16384 map, 2^20 cells: from 2^19
+    particles on, a group of 4096 makes 2^32 pairs.  Nothing is written past the
+    workspace and the overflow is reported."""
+    import numpy as np
+    import torch
+
+    from martini_amd import _lib
+
+    desc = _lib.make_desc(16384, 16384, 64, _lib.SPECTRUM_GAUSS)
+    rec = np.zeros(n, _lib.PARTICLE_DTYPE)
+    rec["ix"] = rec["iy"] = 8192
+    rec["h"], rec["r_kind"] = 20000.0, (16384 << 8) | _lib.KERNEL_CUBIC
+    rec["c_hi"], rec["s"], rec["amp"] = 63, 0.1, 1.0
+    assert _lib.count_pairs(rec[:2], desc) == 2 << 20
+    for cap in (0, 1000):
+        need = _lib.workspace_bytes(desc, n, cap)
+        whole = torch.full((need + (1 << 20),), 0xA5, dtype=torch.uint8, device="cuda")
+        ws = whole[:need]
+        d = torch.from_numpy(rec.view(np.uint8)).cuda()
+        _lib.bin(d, n, cap, desc, ws)
+        pairs, overflow, items, _ = _lib.status(desc, n, cap, ws)
+        assert (pairs, overflow, items) == ((n << 20) & 0xFFFFFFFF, 1, 0)
+        assert bool((whole[need:] == 0xA5).all())
