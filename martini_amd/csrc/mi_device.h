@@ -11,6 +11,7 @@
 // neither cancels.
 #pragma once
 
+#include <float.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -492,6 +493,15 @@ __device__ inline float table_flux(int lo, int hi, int row, float amp, int c,
                                    const float* __restrict__ tab, int64_t ld) {
     if (c < lo || c > hi) return 0.0f;
     return amp * tab[(int64_t)row * ld + c];
+}
+
+// Whether a line has no finite spectrum.  The FP32 gather leaves such a particle,
+// and values of the caller's table that are not finite, out of its products, where
+// they would meet the zero weights of pixels outside the footprint, and adds them by
+// themselves (add_not_finite).
+__device__ inline bool not_finite(float x) { return !(fabsf(x) <= FLT_MAX); }
+__device__ inline bool odd_line(float s, float fu, float amp) {
+    return not_finite(amp) || __builtin_isunordered(s, fu);
 }
 
 __device__ inline float channel_flux(const mi_particle& p, int c, const mi_cube_desc& d) {

@@ -223,6 +223,44 @@ constexpr int STAGED = 4;
 static_assert(STAGED % 2 == 0 && STAGED <= NT / 32 && (STAGED & (STAGED - 1)) == 0,
               "whole waves, and a power of two");
 
+// What an item's chunks left out of the products because it is not finite
+// (odd_line, values of the caller's table), each over its own footprint and
+// channels: one particle after another, for the lane's voxels at rows i0 + RG r,
+// columns j0 + q and channels ch0 + 16 CGN nb.  Rare, and kept short rather than fast.
+template <int RG, int CGN, class Add>
+__device__ inline void add_not_finite(const mi_particle* __restrict__ P,
+                                      const uint32_t* __restrict__ order, ItemWalk chunks,
+                                      const Grid& g, const mi_cube_desc& d,
+                                      const float4* __restrict__ wtab, int i0, int j0, int ch0,
+                                      Add add) {
+    const bool table = d.spectrum == MI_SPECTRUM_TABLE;
+#pragma unroll 1
+    for (; chunks.more(); chunks.next())
+#pragma unroll 1
+        for (int k = 0; k < min(KC, chunks.left); ++k) {
+            const mi_particle p = P[order[chunks.at() + k]];
+            if (!table && !odd_line(p.s, p.fu, p.amp)) continue;
+            const int kind = kind_of(p.r_kind), gi = gidx_of(p.r_kind);
+            int i_lo, i_hi, j_lo, j_hi;
+            if (!footprint(p, g.nx, g.ny, i_lo, i_hi, j_lo, j_hi)) continue;
+#pragma unroll 1
+            for (int e = 0; e < 64; ++e) {
+                const int r = e >> 4, nb = (e >> 2) & 3, q = e & 3;
+                const int i = i0 + RG * r, j = j0 + q, c = ch0 + 16 * CGN * nb;
+                if (i < i_lo || i > i_hi || j < j_lo || j > j_hi || c < p.c_lo || c > p.c_hi || c >= g.nc)
+                    continue;
+                const float s = channel_flux(p, c, d);
+                if (table && !not_finite(s)) continue;
+                const float w = kind == MI_KERNEL_TABLE
+                                    ? d.weights[table_offset(p) + (int64_t)(i - i_lo) * (j_hi - j_lo + 1) + j - j_lo]
+                                    : pixel_weight(kind, (double)(p.ix - i) + (double)p.fx,
+                                                   (double)(p.iy - j) + (double)p.fy, p.h, d.gauss_t[gi],
+                                                   d.gauss_inv_norm[gi], wtab);
+                add(r, nb, q, w * s);
+            }
+        }
+}
+
 // Bits 0, n, 2 n and 3 n.
 constexpr uint32_t every(int n) { return 1u | 1u << n | 1u << 2 * n | 1u << 3 * n; }
 
@@ -292,20 +330,27 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     if (stages && at < chunks.left) next = load_record(P, order[begin + at]);
     if (stages && at + STAGED * step < chunks.left) next_idx = order[begin + STAGED * step + at];
 
+    // The split form takes infinities and NaN like any value: they reach all columns of
+    // the tile rows and blocks that their chunk reaches.  (Left out there too, their
+    // addresses spilled to more scalar registers: 1e7 particles 4590 -> 4675 us.)
+    constexpr bool LEAVE_ODD = std::is_same_v<F, Float32>;
+    bool odd = false;        // a line was left out (the same for every thread)
+    bool odd_value = false;  // this thread left out a value of the caller's table
     for (int slot = 0; chunks.more(); chunks.next(), slot = (slot + 1) & (STAGED - 1)) {
         const int left = chunks.left;
         if (slot == 0 && stages && 2 * pair * step < left) {
             __builtin_amdgcn_s_setprio(3);  // the other waves wait for it: first on its SIMD
-            stage_chunks(next, at < left, x0, y0, c0, g, d, staged + 2 * pair);
+            stage_chunks<LEAVE_ODD>(next, at < left, x0, y0, c0, g, d, staged + 2 * pair);
             __builtin_amdgcn_s_setprio(0);
             if (at + STAGED * step < left) next = load_record(P, next_idx);
             if (at + 2 * STAGED * step < left) next_idx = order[chunks.at() + 2 * STAGED * step + at];
         }
         const ChunkState& cs = staged[slot];
         __syncthreads();
-        const uint32_t rowmask = __builtin_amdgcn_readfirstlane(cs.rowmask());
-        const uint32_t chanmask = __builtin_amdgcn_readfirstlane(cs.chanmask());
-        const uint32_t rows = (rowmask >> rh) & ROW_BITS;
+        const uint32_t cover = __builtin_amdgcn_readfirstlane(cs.cover_per);
+        const uint32_t chanmask = ChunkState::chanmask(cover);
+        odd = odd || (LEAVE_ODD && ChunkState::odd(cover));
+        const uint32_t rows = (ChunkState::rowmask(cover) >> rh) & ROW_BITS;
         const uint32_t chans = (chanmask >> ch) & BLK_BITS;
         if (cs.gmask != 0u) {  // the same for every thread
             fill_gauss_tables(cs, x0, y0, gt);
@@ -315,18 +360,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                      [&](int k, int q, float w) { W.put(q, k, w); },
                      [&](int k, int q1, float w1, int q2, float w2) { W.put2(k, q1, w1, q2, w2); });
         if (GT_IN_S && cs.gmask != 0u) __syncthreads();
-        fill_spectra<G::CB>(cs, c0, d,
+        odd_value |= fill_spectra<G::CB, LEAVE_ODD>(cs, c0, d,
                      [&](int k, int b, int r, float s1, float s2) { S.put_pairs(k, b, r, s1, s2); },
                      chanmask);
         // FP32: the particles (bits) that reach each of this wave's rows and blocks
         uint32_t prow[4] = {}, pblk[4] = {};
         if constexpr (std::is_same_v<F, Float32>) {
-            const uint32_t cover = lane < KC ? cs.walk[lane].cover : 0u;
+            const uint32_t mine = lane < KC ? cs.walk[lane].cover : 0u;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) prow[r] = (uint32_t)__ballot((cover >> (rh + RG * r)) & 1u);
+            for (int r = 0; r < 4; ++r) prow[r] = (uint32_t)__ballot((mine >> (rh + RG * r)) & 1u);
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb)
-                pblk[nb] = (uint32_t)__ballot((cover >> (16 + ch + CGN * nb)) & 1u);
+                pblk[nb] = (uint32_t)__ballot((mine >> (16 + ch + CGN * nb)) & 1u);
         }
         __syncthreads();
         if (rows != 0u) {
@@ -394,23 +439,44 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     auto any = [](const floatx4& v) {
         return __ballot(v[0] != 0.f || v[1] != 0.f || v[2] != 0.f || v[3] != 0.f) != 0u;
     };
+    if (LEAVE_ODD && d.spectrum == MI_SPECTRUM_TABLE) {  // uniform
+        __syncthreads();  // S is no longer read
+        uint32_t* seen = reinterpret_cast<uint32_t*>(&S);
+        const bool some = __any(odd_value);
+        if (lane == 0) seen[wave] = some;
+        __syncthreads();
+        odd = (seen[0] | seen[1] | seen[2] | seen[3]) != 0u;
+    }
     constexpr int BLOCKS = G::CB / SUB_CH;
+    float* part = partials + (size_t)it.slot * CELL_VOXELS + sub_offset(BLOCKS, rh, ch);
+    // Adds to this lane's voxel (row rh + RG r, column 4 kg + q; channel m of block
+    // ch + CGN nb) in the cube or the partial tile.
+    auto add = [&](int r, int nb, int q, float v) {
+        if (it.slot >= 0)
+            part[sub_offset(BLOCKS, RG * r, CGN * nb) + m * 16 + kg * 4 + q] += v;
+        else
+            cube[((size_t)(x0 + rh + RG * r) * g.ny + y0 + kg * 4 + q) * g.nc + c0 + (ch + CGN * nb) * 16 + m] += v;
+    };
+    auto add_odd = [&]() {
+        ItemWalk again(cell_start[it.cell], cell_end[it.cell], it, KC);
+        add_not_finite<RG, CGN>(P, order, again, g, d, wtab, x0 + rh, y0 + kg * 4, c0 + ch * 16 + m, add);
+    };
     if (it.slot >= 0) {
         // a lane's four pixels are next to one another in a partial tile: one store each
-        floatx4* tile = reinterpret_cast<floatx4*>(partials + (size_t)it.slot * CELL_VOXELS +
-                                                   sub_offset(BLOCKS, rh, ch)) + m * 4 + kg;
+        floatx4* tile = reinterpret_cast<floatx4*>(part) + m * 4 + kg;
         uint32_t mine = 0u;  // bit 4 r + nb: block (r, nb) written
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb)
-                if (any(acc[r][nb])) {
+                if ((LEAVE_ODD && odd) || any(acc[r][nb])) {
                     mine |= 1u << (4 * r + nb);
                     tile[sub_offset(BLOCKS, RG * r, CGN * nb) / 4] = acc[r][nb];
                 }
         static_assert(NT / 64 == 4, "four 16-bit parts per mask");
         if (lane == 0)  // this wave's part: bits 16 * wave + 4 r + nb
             reinterpret_cast<uint16_t*>(part_masks + it.slot)[wave] = (uint16_t)mine;
+        if (LEAVE_ODD && odd) add_odd();
         return;
     }
 #pragma unroll
@@ -428,6 +494,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
             }
         }
     }
+    if (LEAVE_ODD && odd) add_odd();
 }
 
 hipError_t gather(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,

@@ -102,13 +102,14 @@ struct ChunkState {
     uint32_t started;
     // tile rows (x offsets; bits 0..15) touched by any footprint of the chunk and
     // 16-channel blocks of the cell (16..23) touched by any window; pairs per
-    // thread << 24
+    // thread << 24; whether a line is left out (odd_line) << 31
     uint32_t cover_per;
     uint32_t gmask;     // particles of the Gaussian kernel with a footprint in the tile
 
-    __device__ uint32_t rowmask() const { return cover_per & 0xffffu; }
-    __device__ uint32_t chanmask() const { return (cover_per >> 16) & 255u; }
-    __device__ int per() const { return (int)(cover_per >> 24); }
+    __device__ static uint32_t rowmask(uint32_t cover_per) { return cover_per & 0xffffu; }
+    __device__ static uint32_t chanmask(uint32_t cover_per) { return (cover_per >> 16) & 255u; }
+    __device__ static bool odd(uint32_t cover_per) { return cover_per >> 31; }
+    __device__ int per() const { return (int)((cover_per >> 24) & 127u); }
 };
 
 // The separable factors of the Gaussian kernel's pixel weight for the chunk's
@@ -197,7 +198,9 @@ __device__ inline float pick4(const float (&v)[4], int i) {
 // the pair counts, ORs the row and channel-block masks across each half of the
 // wave and forms each particle's weight factors.  The staging is on every
 // chunk's critical path (the other waves wait for it), and one wave's
-// instructions for two chunks are those of one.
+// instructions for two chunks are those of one.  LEAVE_ODD: lines that are not
+// finite (odd_line) get no window and are only marked in cover_per.
+template <bool LEAVE_ODD>
 __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0, int c0,
                                     const Grid& g, const mi_cube_desc& d, ChunkState* both) {
     static_assert(KC == 32, "half a wave per chunk");
@@ -220,8 +223,9 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
     const auto add = [](uint32_t a, uint32_t b) { return a + b; };
     const auto bit_or = [](uint32_t a, uint32_t b) { return a | b; };
     const int incl = (int)half_scan((uint32_t)cnt, add);
-    static_assert(TILE_MAX <= 16 && GeoWide::CB / 16 <= 16, "rows and channel blocks share one word");
-    const uint32_t masks = half_scan(rows | (chans << 16), bit_or);  // one reduction for both
+    static_assert(TILE_MAX <= 16 && GeoWide::CB / 16 <= 8, "rows and channel blocks share one word");
+    const bool odd = LEAVE_ODD && valid && d.spectrum != MI_SPECTRUM_TABLE && odd_line(p.s, p.fu, p.amp);
+    const uint32_t masks = half_scan(rows | (chans << 16) | (uint32_t)odd << 31, bit_or);  // one reduction for all
     const uint64_t gauss = __ballot(cnt > 0 && kind_of(p.r_kind) == MI_KERNEL_GAUSS);
     // Each particle's pairs go to max(1, ceil(cnt / per)) threads of their own, per
     // = ceil(total / (NT - KC)): at most total / per + KC <= NT threads in all.  No
@@ -249,7 +253,7 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
         started |= (uint32_t)__builtin_popcount((uint32_t)(b >> (half * KC))) << (8 * v);
     }
     const int cl = min(cb, g.nc - 1 - c0);
-    const uint32_t window = valid && ca <= cl ? (uint32_t)ca | (uint32_t)(cl - ca) << 8 : NO_WINDOW;
+    const uint32_t window = valid && !odd && ca <= cl ? (uint32_t)ca | (uint32_t)(cl - ca) << 8 : NO_WINDOW;
     const int width = max(jhi - jlo + 1, 1);
     const int kind = kind_of(p.r_kind), gi = gidx_of(p.r_kind);
     cs.p[lane] = SpecRec{p.k0, p.fu, p.s, p.amp};
@@ -536,13 +540,14 @@ struct LineSeries {
 // hands the values to store2(k, block, r, s1, s2), the channels r and r + 8 of
 // the 16-channel block of one particle at a time; channels outside its window give 0.  Thread t takes particle t % KC and the channels t / KC + 8 i, so its
 // record fields are read once.  Only the 16-channel blocks set in `blocks`
-// (wave-uniform) are evaluated; the others are left untouched.  The values
+// (wave-uniform) are evaluated; the others are left untouched.  LEAVE_ODD: returns
+// whether the thread left out a value of the caller's table that is not finite.  The values
 // are line_flux's (for narrow spans the same series with its polynomial
 // expanded, to FP32 rounding), computed as straight-line code (the window
 // test is one unsigned compare and a select) so that the evaluations of a thread
 // overlap.
-template <int CB, class Store2>
-__device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_desc& d,
+template <int CB, bool LEAVE_ODD, class Store2>
+__device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_desc& d,
                                     Store2 store2,
                                     uint32_t blocks = (1u << (CB / 16)) - 1u) {
     constexpr int PER_BLOCK = 16 / (NT / KC);  // a thread's channels in one 16-channel block
@@ -562,6 +567,7 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
         store2(k, b, cl0, inside(o0) ? v0 : 0.0f, inside(o1) ? v1 : 0.0f);
     };
     if (spectrum == MI_SPECTRUM_TABLE) {  // uniform: the caller's spectra
+        bool odd = false;
 #pragma unroll
         for (int b = 0; b < CB / 16; ++b) {
             if (!((blocks >> b) & 1u)) continue;
@@ -569,15 +575,18 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
             // (channel c0 + cl0 + o is inside the window when inside(o))
             const float* row = d.spectra + ((int64_t)k0 * d.spectra_ld + c0 + cl0);
             const int o0 = (NT / KC) * (b * PER_BLOCK), o1 = o0 + NT / KC;
-            store2(k, b, cl0, inside(o0) ? amp * row[o0] : 0.0f, inside(o1) ? amp * row[o1] : 0.0f);
+            const float v0 = inside(o0) ? amp * row[o0] : 0.0f, v1 = inside(o1) ? amp * row[o1] : 0.0f;
+            const bool odd0 = LEAVE_ODD && not_finite(v0), odd1 = LEAVE_ODD && not_finite(v1);
+            odd = odd || odd0 || odd1;
+            store2(k, b, cl0, odd0 ? 0.0f : v0, odd1 ? 0.0f : v1);
         }
-        return;
+        return odd;
     }
     if (spectrum == MI_SPECTRUM_DIRAC) {  // uniform: the whole amplitude in the window
 #pragma unroll
         for (int b = 0; b < CB / 16; ++b)
             if ((blocks >> b) & 1u) put(b, amp, amp);
-        return;
+        return false;
     }
     // Channel c = c0 + cl0 + o of this thread sits at k0 - c + fu - 1/2 = (kf - o) + fh
     // from the line centre (in channels): the first difference is exact, so that each
@@ -595,7 +604,7 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
         for (int b = 0; b < CB / 16; ++b)
             if ((blocks >> b) & 1u)  // uniform
                 put(b, narrow(line, 16 * b), narrow(line, 16 * b + NT / KC));
-        return;
+        return false;
     }
     if (!__any(s > 1.5f)) {
         // A longer series, a seventh of the erf difference's work per channel (3e5 particles, s = 0.8, split BF16: 232
@@ -607,7 +616,7 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
             const float j = kf - (float)(16 * b);
             put(b, line(s * (j + fh)), line(s * (j - (float)(NT / KC) + fh)));
         }
-        return;
+        return false;
     }
     // Wider channels: the line spans a few channels, and the erfc differences are
     // taken only inside its window.  A loop of its own: unrolled into the narrow lines'
@@ -629,6 +638,7 @@ __device__ inline void fill_spectra(const ChunkState& cs, int c0, const mi_cube_
         }
         put(b, v[0], v[1]);
     }
+    return false;
 }
 
 // Copies the table of the kernel kind of the item's first particle (when it
