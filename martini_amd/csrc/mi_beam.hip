@@ -337,7 +337,11 @@ constexpr int LINE_G = 2;        // steps whose rows are loaded together
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-template <bool VEC>
+// LONG leaves out the steps whose rows all lie outside the cube: for an image longer
+// than the cube, most of them (4001 taps along 256 rows of 256 x 128: 1623 us with them,
+// 131 without).  For a shorter one the loop's plain start costs less (27 taps, 538 x
+// 538 x 256: two passes 281 us, 318 with LONG).
+template <bool VEC, bool LONG>
 __global__ __launch_bounds__(64 * LINE_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void
 k_convolve_line(
     const float* __restrict__ in, float* __restrict__ out, int L, int64_t E, int64_t cols,
@@ -365,9 +369,10 @@ k_convolve_line(
         for (int j = 0; j < 4; ++j) acc[q][j] = f64x4{0.0, 0.0, 0.0, 0.0};
     // Step s takes input rows m0 + 4 s + kk; row m0 + r feeds output l0 + q
     // through tap q + k - 1 - r.  Block q of 16 outputs needs steps 4 q .. 4 q + S - 1.
-    const int m0 = l0 + k / 2 - (k - 1);
     const int S = (k + 15 + 3) / 4;
-    const int steps = S + 4 * (LINE_T - 1);
+    const LineSteps steps(l0, L, k, S + 4 * (LINE_T - 1));
+    const int m0 = steps.m0, first = LONG ? steps.first : 0;
+    const int last = LONG ? steps.last : S + 4 * (LINE_T - 1);
     auto load = [&](int s, float (&v)[4]) {
         const int m = m0 + 4 * s + kk;
         const bool ok = m >= 0 && m < L;
@@ -387,12 +392,12 @@ k_convolve_line(
     const double* tap = taps + LINE_PAD + n - kk + k - 1;  // the lane's tap of step s: tap[-4 s]
     float v[LINE_G][4];
 #pragma unroll
-    for (int g = 0; g < LINE_G; ++g) load(g, v[g]);
-    for (int s0 = 0; s0 < steps; s0 += LINE_G) {
+    for (int g = 0; g < LINE_G; ++g) load(first + g, v[g]);
+    for (int s0 = first; s0 < last; s0 += LINE_G) {
         float w[LINE_G][4];
 #pragma unroll
         for (int g = 0; g < LINE_G; ++g)
-            if (s0 + LINE_G < steps) load(s0 + LINE_G + g, w[g]);
+            if (s0 + LINE_G < last) load(s0 + LINE_G + g, w[g]);
 #pragma unroll
         for (int g = 0; g < LINE_G; ++g) {
             const int s = s0 + g;
@@ -476,12 +481,13 @@ static hipError_t convolve_line(const float* in, float* out, int64_t O, int L, i
     const size_t lds = sizeof(double) * (size_t)(k + 2 * LINE_PAD);
     const bool vec = E % 4 == 0 &&
                      ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    if (vec)
-        hipLaunchKernelGGL(k_convolve_line<true>, grid, dim3(64 * LINE_WAVES), lds, s, in, out, L, E,
-                           cols, K, k);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * LINE_WAVES), lds, s, in, out, L, E, cols, K, k);
+    };
+    if (k > L)
+        launch(vec ? k_convolve_line<true, true> : k_convolve_line<false, true>);
     else
-        hipLaunchKernelGGL(k_convolve_line<false>, grid, dim3(64 * LINE_WAVES), lds, s, in, out, L,
-                           E, cols, K, k);
+        launch(vec ? k_convolve_line<true, false> : k_convolve_line<false, false>);
     return hipGetLastError();
 }
 

@@ -120,6 +120,19 @@ hipError_t cube_to_fits(const void* cube, bool cube_f64, int nx, int ny, int nc,
 hipError_t convolve_beam(const float* in, float* out, int nx, int ny, int nc, const float* K,
                          int kx, int ky, hipStream_t s);
 
+// A one-dimensional beam pass over L rows takes its input rows four a step, from
+// m0 on (row m feeds output l through tap l + k/2 - m): the steps of the outputs from
+// l0 on, `steps` without a border, of which those from `first` up to `last` meet a row of
+// the cube.
+struct LineSteps {
+    int m0, first, last;
+    __host__ __device__ LineSteps(int l0, int L, int k, int steps) : m0(l0 + k / 2 - (k - 1)) {
+        first = m0 < 0 ? -m0 / 4 : 0;
+        last = L > m0 ? (L - m0 + 3) / 4 : 0;
+        if (last > steps) last = steps;
+    }
+};
+
 // One work item: the q-th of a cell's n, which takes the cell's chunks q, q + n,
 // ... of the sorted pair list; slot >= 0 names its partial tile, -1 means it
 // writes the cube.

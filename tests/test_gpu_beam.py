@@ -280,3 +280,13 @@ def test_line_tiles(shape, k, axis, special, offset):
     64-column groups, aligned and not: an FP64 sum, rounded once."""
     K = np.random.default_rng(k).random((k, 1) if axis == 0 else (1, k))
     _check(shape, K, special, 1.001, offset)
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("shape,k,axis", [
+    ((31, 3, 24), 101, 0), ((33, 2, 5), 401, 0), ((64, 2, 8), 4001, 0), ((1, 40, 12), 201, 0),
+    ((5, 31, 16), 101, 1), ((2, 97, 7), 1001, 1), ((70, 1, 4), 63, 1), ((3, 33, 4), 67, 1),
+])
+def test_lines_longer_than_the_cube(shape, k, axis, special):
+    """Images that reach past both ends of the cube."""
+    test_line_tiles(shape, k, axis, special, 0)

@@ -1,6 +1,6 @@
 """Index arithmetic at the limits that the library accepts (pair counts below
-2^31, cubes of up to 2^21 cells), on the CPU: the functions that the kernels
-use, compiled for the host."""
+2^31, cubes of up to 2^21 cells) and of loops whose ends matter, on the CPU: the
+functions that the kernels use, compiled for the host."""
 
 import subprocess
 
@@ -36,7 +36,32 @@ static unsigned long long total(int n, uint32_t each) {
     return sum.total();
 }
 
+// Whether the steps of a beam pass take every row of the cube that feeds an output
+// of [l0, l0 + 32), and at most two steps more than those rows need.
+static bool line_steps(int l0, int L, int k) {
+    const int S = (k + 15 + 3) / 4, all = S + 4;
+    const LineSteps s(l0, L, k, all);
+    int lowest = L, highest = -1;
+    for (int l = l0; l < l0 + 32 && l < L; ++l)
+        for (int a = 0; a < k; ++a) {
+            const int m = l + k / 2 - a;
+            if (m < 0 || m >= L) continue;
+            lowest = m < lowest ? m : lowest;
+            highest = m > highest ? m : highest;
+        }
+    return s.first >= 0 && s.last <= all && s.m0 + 4 * s.first <= lowest &&
+           s.m0 + 4 * s.last > highest && s.last - s.first <= (highest - lowest) / 4 + 10 &&
+           s.last - s.first <= L / 4 + 2;
+}
+
 int main(int argc, char** argv) {
+    if (argc == 3 && argv[1][0] == 'L') {
+        const int L = atoi(argv[2]);
+        for (int k = 1; k < 4096; k = k < 130 ? k + 2 : k * 3 / 2 | 1)
+            for (int l0 = 0; l0 < L; l0 += 32)
+                if (!line_steps(l0, L, k)) return printf("%d taps, output %d\n", k, l0), 1;
+        return 0;
+    }
     if (argc == 2) return printf("%llu %llu\n", total(16, atol(argv[1])), total(64, atol(argv[1]))), 0;
     const long start = atol(argv[1]), end = atol(argv[2]);
     const int n = (int)((end - start + ITEM_MAX - 1) / ITEM_MAX);
@@ -79,6 +104,12 @@ def test_group_pair_totals_do_not_wrap(program, each):
     """A wave's 64 particles make up to 64 (2^21 - 1) pairs; groups of 16 waves, and of 16 in 4 rounds."""
     r = subprocess.run([str(program), str(each)], capture_output=True, text=True, check=True)
     assert [int(v) for v in r.stdout.split()] == [16 * each, 64 * each]
+
+
+@pytest.mark.parametrize("length", [1, 2, 3, 4, 5, 15, 16, 31, 32, 33, 64, 65, 97, 300])
+def test_beam_steps_reach_the_cube(program, length):
+    r = subprocess.run([str(program), "L", str(length)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
 
 
 @pytest.mark.gpu
