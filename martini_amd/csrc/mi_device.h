@@ -259,10 +259,13 @@ __host__ __device__ inline double w_quartic(double dx, double dy, double h) {
 }
 
 // erf and erfc of |x|, neither the other's complement where it is the smaller:
-// up to 0.85, erf = x P(x^2); beyond, erfc = exp(-x^2) Q(t), t = 1 / (1 + 0.4 x).
-// P and Q are least-maximum fits of the relative error (6e-9 and 1.2e-8; in FP32
-// 4e-8 and 8e-8 rms), x^2 and its logarithm to base 2 are carried to twice FP32's
-// precision.
+// up to 0.85, erf = x (C + P(x^2)), C = 2 / sqrt(pi) in FP32 and P's constant term what
+// that leaves (5.4e-8 of it; without it every erf was that much low); beyond, erfc =
+// exp(-x^2) Q(t), t = 1 / (1 + 0.4 x).  P and Q are least-maximum fits of the relative
+// error.  With their coefficients as rounded to FP32 they are within 1.6e-8 and, up
+// to x = 9.2, where erfc leaves FP32's normal range, 2.8e-8 (6.3e-7 at x = 12);
+// evaluated in FP32 2.6e-8 rms, 8e-8 at most, and 9e-8 rms, 4e-7 at most.  x^2 and its
+// logarithm to base 2 are carried to twice FP32's precision.
 struct ErfParts {
     float e, c;
 };
@@ -271,12 +274,12 @@ __device__ inline ErfParts erf_parts(float x) {
     x = fabsf(x);
     x = x > 12.0f ? 12.0f : x;  // erfc is 0 in FP32 there; NaN stays
     const float z = x * x, zl = fmaf(x, x, -z);
-    float p = -6.31512725e-4f;
-    p = fmaf(p, z, 5.05109457e-3f);
-    p = fmaf(p, z, -2.68025473e-2f);
-    p = fmaf(p, z, 1.12827174e-1f);
-    p = fmaf(p, z, -3.76125724e-1f);
-    p = fmaf(p, z, 1.12837911f);
+    float p = -6.31269882e-4f;
+    p = fmaf(p, z, 5.05065126e-3f);
+    p = fmaf(p, z, -2.68022642e-2f);
+    p = fmaf(p, z, 1.1282710e-1f);
+    p = fmaf(p, z, -3.76125723e-1f);
+    p = fmaf(p, z, 5.36047793e-8f);
     const float t = __builtin_amdgcn_rcpf(fmaf(0.4f, x, 1.0f));
     float q = 2.81441752e-2f;
     q = fmaf(q, t, -2.18506634e-1f);
@@ -292,7 +295,7 @@ __device__ inline ErfParts erf_parts(float x) {
     const float y = z * L, yl = fmaf(z, LL, fmaf(z, L, -y));
     float g = __builtin_amdgcn_exp2f(-y);
     g = fmaf(-g, fmaf(yl, 0.693147181f, zl), g);
-    const float e = x * p, c = g * q;
+    const float e = fmaf(x, 1.12837911f, x * p), c = g * q;
     return x < 0.85f ? ErfParts{e, 1.0f - e} : ErfParts{1.0f - c, c};
 }
 

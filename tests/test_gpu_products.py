@@ -173,3 +173,21 @@ def test_lines(method, shape, widths):
     assert np.all(got[~inside] == 0.0)
     worst = np.max(np.where(inside, np.abs(got - want) / tol, 0.0))
     assert worst <= 1.0, worst
+
+
+def test_line_centres_have_no_bias():
+    """The channel that holds a line's centre, both edges within 0.85 of it: over many
+    lines the mean relative error is that of the fit of erf, below 1.6e-8, and five
+    standard errors of roundings of at most 2^-22 each."""
+    from scipy.special import erf
+
+    n, nc = 1 << 16, 8
+    rng = np.random.default_rng(0)
+    rec = np.zeros(n, _lib.PARTICLE_DTYPE)
+    rec["s"], rec["fu"] = rng.uniform(0.55, 0.84, n), rng.uniform(0, 1, n)
+    rec["k0"], rec["c_hi"], rec["amp"] = 4, nc - 1, rng.uniform(0.5, 2.0, n)
+    got = _lib.spectra(rec, _lib.make_desc(1, 1, nc, _lib.SPECTRUM_GAUSS))[:, 4].astype(float)
+    s, fu, amp = (rec[k].astype(float) for k in ("s", "fu", "amp"))
+    want = 0.5 * amp * (erf(s * fu) + erf(s * (1.0 - fu)))
+    bias = np.mean(got / want - 1.0)
+    assert abs(bias) <= 1.6e-8 + 5 * 2.0**-22 / np.sqrt(n), bias
