@@ -482,8 +482,10 @@ constexpr float SQRT_LOG2E = 1.20112240878645110f;
 //     = exp(-m^2) sum_j e_j m^2j,
 // the sum over k to K (span_series' terms for K = 3); the e_j are formed once per
 // particle.  SCALED: as exp2(-n^2) times a polynomial in n^2 of n = m sqrt(log2 e),
-// a product less per channel and n's factor rounded once for all channels.  The first term left out is D^(2K+2) / (4^(K+1) (K+1)! (2K+3)) of the
-// peak at most: 1e-9 for K = 3, D = 1/2 and 2e-8 for K = 7, D = 3/2.
+// a product less per channel and n's factor rounded once for all channels.  The first
+// term left out is D^(2K+2) / (4^(K+1) (K+1)! (2K+3)) of the peak at most: 7e-8 for
+// K = 3, D = 1/2 (1.2e-9 at 0.3) and 8e-10 for K = 8, D = 3/2.  In the line's last
+// channels, at 1e-7 of the peak and less, it is 2.3e-4 and 1.3e-6 of the value.
 template <int K, bool SCALED>
 struct LineSeries {
     float e[K + 1];
@@ -526,13 +528,25 @@ struct LineSeries {
             f *= D2;
         }
     }
-    // at n (SCALED) or m
-    __device__ float operator()(float n) const {
-        const float n2 = n * n;
+    __device__ float polynomial(float x) const {
         float p = e[K];
 #pragma unroll
-        for (int j = K - 1; j >= 0; --j) p = fmaf(p, n2, e[j]);
-        return __builtin_amdgcn_exp2f(SCALED ? -n2 : n2 * (float)-LOG2E) * p;
+        for (int j = K - 1; j >= 0; --j) p = fmaf(p, x, e[j]);
+        return p;
+    }
+    // at n (SCALED)
+    __device__ float operator()(float n) const {
+        const float n2 = n * n;
+        return __builtin_amdgcn_exp2f(-n2) * polynomial(n2);
+    }
+    // at m = s d (not SCALED), m^2 and its logarithm to base 2 carried to twice FP32's
+    // precision: they reach 22 there, and a rounding of 2^-24 of that is 1.3e-6 of the value.
+    __device__ float at(float s, float d) const {
+        const float m = s * d, ml = fmaf(s, d, -m);
+        const float m2 = m * m, m2l = fmaf(m + m, ml, fmaf(m, m, -m2));
+        const float y = m2 * (float)LOG2E, yl = fmaf(m2, (float)LOG2E, -y);
+        const float g = __builtin_amdgcn_exp2f(-y);
+        return fmaf(-g, fmaf(yl, 0.693147181f, m2l), g) * polynomial(m2);
     }
 };
 
@@ -542,10 +556,10 @@ struct LineSeries {
 // record fields are read once.  Only the 16-channel blocks set in `blocks`
 // (wave-uniform) are evaluated; the others are left untouched.  LEAVE_ODD: returns
 // whether the thread left out a value of the caller's table that is not finite.  The values
-// are line_flux's (for narrow spans the same series with its polynomial
-// expanded, to FP32 rounding), computed as straight-line code (the window
-// test is one unsigned compare and a select) so that the evaluations of a thread
-// overlap.
+// are line_flux's to FP32 rounding (channels up to half a line width by the same series
+// with its polynomial expanded, up to 3/2 by a longer one in place of an erf difference),
+// computed as straight-line code (the window test is one unsigned compare and a
+// select) so that the evaluations of a thread overlap.
 template <int CB, bool LEAVE_ODD, class Store2>
 __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_desc& d,
                                     Store2 store2,
@@ -607,14 +621,16 @@ __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_
         return false;
     }
     if (!__any(s > 1.5f)) {
-        // A longer series, a seventh of the erf difference's work per channel (3e5 particles, s = 0.8, split BF16: 232
-        // -> 220 us per insertion; 3e6 of which half have s = 6 and go on: 3.05 -> 3.09 ms).
-        const LineSeries<7, false> line(s, amp);
+        // A longer series, a third of the erf difference's work per channel (1e6 particles,
+        // s = 0.62, split BF16: 382 -> 338 us per insertion; 3e5, s = 0.81: 216 -> 206).  With
+        // seven terms and a plain exponent it took 325 and 203 us, and the last channels
+        // at s = 3/2 were off by up to 1e-5 of their value (erf differences: 2.5e-6, now 3e-6).
+        const LineSeries<8, false> line(s, amp);
 #pragma unroll 1
         for (uint32_t left = blocks; left != 0u; left &= left - 1u) {
             const int b = __builtin_ctz(left);
             const float j = kf - (float)(16 * b);
-            put(b, line(s * (j + fh)), line(s * (j - (float)(NT / KC) + fh)));
+            put(b, line.at(s, j + fh), line.at(s, j - (float)(NT / KC) + fh));
         }
         return false;
     }

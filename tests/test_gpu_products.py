@@ -191,3 +191,49 @@ def test_line_centres_have_no_bias():
     want = 0.5 * amp * (erf(s * fu) + erf(s * (1.0 - fu)))
     bias = np.mean(got / want - 1.0)
     assert abs(bias) <= 1.6e-8 + 5 * 2.0**-22 / np.sqrt(n), bias
+
+
+@pytest.mark.parametrize("method", ["plain", "mfma"])
+@pytest.mark.parametrize("shape", [(16, 16, 64), (8, 16, 128)])
+@pytest.mark.parametrize("widths", [(1.0, 1.4999), (0.2, 1.4999), (0.5001, 1.4999), (1.4, 1.6)])
+def test_lines_of_the_longer_series(method, shape, widths):
+    """Channels of up to 3/2, where a wave whose lines are all that narrow takes a
+    series, and chunks with lines on both sides of it."""
+    test_lines(method, shape, widths)
+
+
+def test_last_channels_of_wide_lines():
+    """The last channels of lines of 1.45 to 1.5 per channel, at 1e-7 of the peak: over
+    many their mean relative error is at most the first term that a series to D^16 leaves
+    out and five standard errors of a rounding of the exponent (up to 21, two roundings of
+    2^-24 of it, twice that in the square) and eight more."""
+    import torch
+    from scipy.special import erfc, eval_hermite, factorial
+
+    shape = (64, 64, 64)
+    n, nc = 4096, shape[2]
+    rng = np.random.default_rng(1)
+    rec = np.zeros(n, _lib.PARTICLE_DTYPE)
+    rec["ix"], rec["iy"] = np.arange(n) // 64, np.arange(n) % 64
+    rec["r_kind"], rec["amp"], rec["h"] = _lib.KERNEL_DIRAC, 1.0, 1.0
+    rec["s"], rec["fu"] = rng.uniform(1.45, 1.4999, n), rng.uniform(0, 1, n)
+    rec["k0"], rec["c_lo"], rec["c_hi"] = 32, 20, 44
+    desc = _lib.make_desc(*shape, _lib.SPECTRUM_GAUSS)
+    pairs = _lib.count_pairs(rec, desc)
+    d_rec = torch.from_numpy(rec.view(np.uint8)).cuda()
+    cube = torch.zeros(n * nc, dtype=torch.float32, device="cuda")
+    ws = torch.zeros(_lib.workspace_bytes(desc, n, pairs), dtype=torch.uint8, device="cuda")
+    _lib.insert(d_rec, n, pairs, desc, cube, ws, method="plain")
+    got = cube.cpu().numpy().reshape(n, nc).astype(float)
+    s = rec["s"].astype(float)[:, None]
+    b = s * (32 - np.arange(nc) + rec["fu"].astype(float)[:, None])
+    m = np.abs(b - 0.5 * s)
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = 0.5 * (erfc(m - 0.5 * s) - erfc(m + 0.5 * s))
+    last = (m > 4.2) & (m < 4.5)
+    S, M = np.broadcast_to(s, m.shape)[last], m[last]
+    left_out = (S / np.sqrt(np.pi) * np.exp(-M**2) * S**18 * np.abs(eval_hermite(18, M))
+                / (4.0**9 * factorial(19)))
+    rel = got[last] / want[last] - 1.0
+    bound = np.mean(left_out / want[last]) + 5 * (4 * 21 + 8) * 2.0**-24 / np.sqrt(rel.size)
+    assert rel.size > 1000 and abs(rel.mean()) <= bound, (rel.mean(), bound)
