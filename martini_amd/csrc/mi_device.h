@@ -320,7 +320,8 @@ __device__ inline float span_series(float m, float D) {
     p = p * m2 + 720.0f;
     p = p * m2 - 120.0f;                                   // H6-type polynomial
     float q = (16.0f * m2 - 48.0f) * m2 + 12.0f;            // H4-type polynomial
-    float poly = 1.0f + D2 * ((4.0f * m2 - 2.0f) * (1.0f / 24.0f) +
+    // 2 / sqrt(pi) in FP32 is 5.2e-8 too large; the leading 1 takes that back
+    float poly = 0.99999994f + D2 * ((4.0f * m2 - 2.0f) * (1.0f / 24.0f) +
                               D2 * (q * (1.0f / 1920.0f) + D2 * p * (1.0f / 322560.0f)));
     return 1.12837916709551257f * __expf(-m2) * D * poly;
 }

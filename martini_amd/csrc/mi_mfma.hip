@@ -59,6 +59,15 @@
 // cell's partial tile receives only the 1 KiB sub-tiles written, with a mask
 // (16 bits per wave) that tells the reduction which to read.
 // Accumulation order is fixed: deterministic, no atomics.
+//
+// FP32 sums: a chunk's 32 terms are a chain of multiply-adds of its own, the chunks'
+// sums a chain of additions.  In one chain over all terms the many tails of far
+// channels and pixels were lost against the bright voxels one by one, each sum 5e-8
+// to 2e-7 low on sparse cubes (1.6e5 particles, 512 x 512 x 256, error against FP64:
+// 1.4e-7 so, 5.2e-8 now; 1.5e6: 2.0e-7, 5.5e-8; heterogeneous 1e6, 512 x 512 x 64:
+// 5.6e-8, 4.3e-8), for 2 to 3% of the form's time.  The tile rows are taken one by one
+// for it: with a row's operands and one sum held instead of four rows' nothing spills.
+// The split form keeps one chain (the additions took 5% of 1e7 particles there).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -281,6 +290,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const CellPos cp = cell_pos(it.cell, g);
     const int x0 = cp.x0, y0 = cp.y0, c0 = cp.c0;
 
+    constexpr bool FP32 = std::is_same_v<F, Float32>;
     using WTile = typename F::template Tile<G::PX>;
     using STile = typename F::template Tile<G::CB>;
     __shared__ WTile W;            // [pixel][k]
@@ -330,17 +340,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     if (stages && at < chunks.left) next = load_record(P, order[begin + at]);
     if (stages && at + STAGED * step < chunks.left) next_idx = order[begin + STAGED * step + at];
 
-    // The split form takes infinities and NaN like any value: they reach all columns of
-    // the tile rows and blocks that their chunk reaches.  (Left out there too, their
-    // addresses spilled to more scalar registers: 1e7 particles 4590 -> 4675 us.)
-    constexpr bool LEAVE_ODD = std::is_same_v<F, Float32>;
+    // What is not finite is left out and added at the end.  The split form takes it like
+    // any value: it reaches all columns of the tile rows and blocks that its chunk
+    // reaches.  (Left out there too, more scalar registers spilled: 1e7 particles 4590 ->
+    // 4675 us.)
     bool odd = false;        // a line was left out (the same for every thread)
     bool odd_value = false;  // this thread left out a value of the caller's table
     for (int slot = 0; chunks.more(); chunks.next(), slot = (slot + 1) & (STAGED - 1)) {
         const int left = chunks.left;
         if (slot == 0 && stages && 2 * pair * step < left) {
             __builtin_amdgcn_s_setprio(3);  // the other waves wait for it: first on its SIMD
-            stage_chunks<LEAVE_ODD>(next, at < left, x0, y0, c0, g, d, staged + 2 * pair);
+            stage_chunks<FP32>(next, at < left, x0, y0, c0, g, d, staged + 2 * pair);
             __builtin_amdgcn_s_setprio(0);
             if (at + STAGED * step < left) next = load_record(P, next_idx);
             if (at + 2 * STAGED * step < left) next_idx = order[chunks.at() + 2 * STAGED * step + at];
@@ -349,7 +359,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         __syncthreads();
         const uint32_t cover = __builtin_amdgcn_readfirstlane(cs.cover_per);
         const uint32_t chanmask = ChunkState::chanmask(cover);
-        odd = odd || (LEAVE_ODD && ChunkState::odd(cover));
+        odd = odd || (FP32 && ChunkState::odd(cover));
         const uint32_t rows = (ChunkState::rowmask(cover) >> rh) & ROW_BITS;
         const uint32_t chans = (chanmask >> ch) & BLK_BITS;
         if (cs.gmask != 0u) {  // the same for every thread
@@ -360,12 +370,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                      [&](int k, int q, float w) { W.put(q, k, w); },
                      [&](int k, int q1, float w1, int q2, float w2) { W.put2(k, q1, w1, q2, w2); });
         if (GT_IN_S && cs.gmask != 0u) __syncthreads();
-        odd_value |= fill_spectra<G::CB, LEAVE_ODD>(cs, c0, d,
+        odd_value |= fill_spectra<G::CB, FP32>(cs, c0, d,
                      [&](int k, int b, int r, float s1, float s2) { S.put_pairs(k, b, r, s1, s2); },
                      chanmask);
         // FP32: the particles (bits) that reach each of this wave's rows and blocks
         uint32_t prow[4] = {}, pblk[4] = {};
-        if constexpr (std::is_same_v<F, Float32>) {
+        if constexpr (FP32) {
             const uint32_t mine = lane < KC ? cs.walk[lane].cover : 0u;
 #pragma unroll
             for (int r = 0; r < 4; ++r) prow[r] = (uint32_t)__ballot((mine >> (rh + RG * r)) & 1u);
@@ -375,35 +385,43 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         }
         __syncthreads();
         if (rows != 0u) {
-            // The wave's four tile rows held together: each S operand read serves all.
-            typename WTile::Op a[4];
+            if constexpr (FP32) {
+                // The chunk's sum by itself, then added: terms far below a voxel's value
+                // (a chunk's tails) would be rounded away one by one against it, all in one
+                // direction (see FP32 sums above).
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                a[r] = typename WTile::Op{};
-                if (!(rows & (1u << (RG * r))) || chans == 0u) continue;
-                a[r] = W.get((rh + RG * r) * TILE_Y + m, kg);
-            }
+                for (int r = 0; r < 4; ++r) {
+                    if (!(rows & (1u << (RG * r))) || chans == 0u) continue;
+                    const typename WTile::Op a = W.get((rh + RG * r) * TILE_Y + m, kg);
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                if (!(chans & (1u << (CGN * nb)))) continue;
-                const typename STile::Op b = S.get((ch + CGN * nb) * 16 + m, kg);
-                if constexpr (std::is_same_v<F, Float32>) {
-                    // bit 4 s: one of the particles 4 s .. 4 s + 3 reaches this row and block
-                    uint32_t need[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
+                    for (int nb = 0; nb < 4; ++nb) {
                         uint32_t q = prow[r] & pblk[nb];
+                        if (q == 0u) continue;
+                        const typename STile::Op b = S.get((ch + CGN * nb) * 16 + m, kg);
+                        // bit 4 s: one of the particles 4 s .. 4 s + 3 reaches this row and block
                         q |= q >> 1;
-                        need[r] = q | (q >> 2);
+                        const uint32_t need = q | (q >> 2);
+                        floatx4 sum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int s = 0; s < KC / 4; ++s)
+                            if (need & (1u << (4 * s)))
+                                sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a.step(s), b.step(s), sum, 0, 0, 0);
+                        acc[r][nb] += sum;
                     }
+                }
+            } else {
+                // The wave's four tile rows held together: each S operand read serves all.
+                typename WTile::Op a[4];
 #pragma unroll
-                    for (int s = 0; s < KC / 4; ++s)
+                for (int r = 0; r < 4; ++r) {
+                    a[r] = typename WTile::Op{};
+                    if (!(rows & (1u << (RG * r))) || chans == 0u) continue;
+                    a[r] = W.get((rh + RG * r) * TILE_Y + m, kg);
+                }
 #pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            if (need[r] & (1u << (4 * s)))
-                                acc[r][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                    a[r].step(s), b.step(s), acc[r][nb], 0, 0, 0);
-                } else {
+                for (int nb = 0; nb < 4; ++nb) {
+                    if (!(chans & (1u << (CGN * nb)))) continue;
+                    const typename STile::Op b = S.get((ch + CGN * nb) * 16 + m, kg);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         if (!(rows & (1u << (RG * r)))) continue;
@@ -439,7 +457,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     auto any = [](const floatx4& v) {
         return __ballot(v[0] != 0.f || v[1] != 0.f || v[2] != 0.f || v[3] != 0.f) != 0u;
     };
-    if (LEAVE_ODD && d.spectrum == MI_SPECTRUM_TABLE) {  // uniform
+    if (FP32 && d.spectrum == MI_SPECTRUM_TABLE) {  // uniform
         __syncthreads();  // S is no longer read
         uint32_t* seen = reinterpret_cast<uint32_t*>(&S);
         const bool some = __any(odd_value);
@@ -469,14 +487,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb)
-                if ((LEAVE_ODD && odd) || any(acc[r][nb])) {
+                if ((FP32 && odd) || any(acc[r][nb])) {
                     mine |= 1u << (4 * r + nb);
                     tile[sub_offset(BLOCKS, RG * r, CGN * nb) / 4] = acc[r][nb];
                 }
         static_assert(NT / 64 == 4, "four 16-bit parts per mask");
         if (lane == 0)  // this wave's part: bits 16 * wave + 4 r + nb
             reinterpret_cast<uint16_t*>(part_masks + it.slot)[wave] = (uint16_t)mine;
-        if (LEAVE_ODD && odd) add_odd();
+        if (FP32 && odd) add_odd();
         return;
     }
 #pragma unroll
@@ -494,7 +512,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
             }
         }
     }
-    if (LEAVE_ODD && odd) add_odd();
+    if (FP32 && odd) add_odd();
 }
 
 hipError_t gather(const mi_particle* d_p, const Grid& g, const mi_cube_desc& d, char* ws,

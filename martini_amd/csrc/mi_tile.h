@@ -198,9 +198,9 @@ __device__ inline float pick4(const float (&v)[4], int i) {
 // the pair counts, ORs the row and channel-block masks across each half of the
 // wave and forms each particle's weight factors.  The staging is on every
 // chunk's critical path (the other waves wait for it), and one wave's
-// instructions for two chunks are those of one.  LEAVE_ODD: lines that are not
+// instructions for two chunks are those of one.  In the FP32 form lines that are not
 // finite (odd_line) get no window and are only marked in cover_per.
-template <bool LEAVE_ODD>
+template <bool FP32>
 __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0, int c0,
                                     const Grid& g, const mi_cube_desc& d, ChunkState* both) {
     static_assert(KC == 32, "half a wave per chunk");
@@ -224,7 +224,7 @@ __device__ inline void stage_chunks(const RecRegs& r, bool valid, int x0, int y0
     const auto bit_or = [](uint32_t a, uint32_t b) { return a | b; };
     const int incl = (int)half_scan((uint32_t)cnt, add);
     static_assert(TILE_MAX <= 16 && GeoWide::CB / 16 <= 8, "rows and channel blocks share one word");
-    const bool odd = LEAVE_ODD && valid && d.spectrum != MI_SPECTRUM_TABLE && odd_line(p.s, p.fu, p.amp);
+    const bool odd = FP32 && valid && d.spectrum != MI_SPECTRUM_TABLE && odd_line(p.s, p.fu, p.amp);
     const uint32_t masks = half_scan(rows | (chans << 16) | (uint32_t)odd << 31, bit_or);  // one reduction for all
     const uint64_t gauss = __ballot(cnt > 0 && kind_of(p.r_kind) == MI_KERNEL_GAUSS);
     // Each particle's pairs go to max(1, ceil(cnt / per)) threads of their own, per
@@ -486,15 +486,16 @@ constexpr float SQRT_LOG2E = 1.20112240878645110f;
 // term left out is D^(2K+2) / (4^(K+1) (K+1)! (2K+3)) of the peak at most: 7e-8 for
 // K = 3, D = 1/2 (1.2e-9 at 0.3) and 8e-10 for K = 8, D = 3/2.  In the line's last
 // channels, at 1e-7 of the peak and less, it is 2.3e-4 and 1.3e-6 of the value.
-template <int K, bool SCALED>
+template <int K, bool SCALED, bool EXACT>
 struct LineSeries {
     float e[K + 1];
 
-    // 1 / sqrt(pi) in FP32 is 5e-8 too large, for every line alike.  The longer series'
-    // coefficients take that back (1 - 5e-8 is within 1e-8 of an FP32 number).  The
-    // narrow lines' do not: the FP32 sums of such lines, many small tails among them,
-    // come out about 1e-7 low on sparse cubes (1.6e5 particles, 512 x 512 x 256: 1.3e-7
-    // of error with it, 1.7e-7 without).
+    // 1 / sqrt(pi) in FP32 is 5e-8 too large, for every line alike.  EXACT: the
+    // coefficients take that back (1 - 5e-8 is within 1e-8 of an FP32 number).  The split
+    // form's narrow lines keep it, as they had it before the series: its chains over all
+    // of an item's chunks come out low by as much or more on the longest (error against
+    // FP64 of 1e7 particles, 512 x 512 x 256: 1.3e-7, 1.5e-7 without it; 1.5e6: 2.67e-7,
+    // 2.75e-7; 1.6e5, sparse: 4.43e-7 either way; 1e6, 256 x 256 x 128: 1.43e-7, 1.31e-7).
     static constexpr float ROOT = 0.564189583547756287f;
     // c[k][j]: of D^2k m^2j (the Hermite polynomials' coefficients)
     struct Table {
@@ -504,7 +505,7 @@ struct LineSeries {
         Table t{};
         // 1 / (2 j)!, its scale included, and (-1)^i / (4^i i!)
         double inv_2j[K + 1] = {}, inv_i[K + 1] = {};
-        double a = SCALED ? 1.0 : 0.564189583547756287 / (double)ROOT, b = 1.0;
+        double a = EXACT ? 0.564189583547756287 / (double)ROOT : 1.0, b = 1.0;
         for (int j = 0; j <= K; ++j) {
             inv_2j[j] = a;
             inv_i[j] = b;
@@ -554,13 +555,13 @@ struct LineSeries {
 // hands the values to store2(k, block, r, s1, s2), the channels r and r + 8 of
 // the 16-channel block of one particle at a time; channels outside its window give 0.  Thread t takes particle t % KC and the channels t / KC + 8 i, so its
 // record fields are read once.  Only the 16-channel blocks set in `blocks`
-// (wave-uniform) are evaluated; the others are left untouched.  LEAVE_ODD: returns
-// whether the thread left out a value of the caller's table that is not finite.  The values
+// (wave-uniform) are evaluated; the others are left untouched.  In the FP32 form,
+// returns whether the thread left out a value of the caller's table that is not finite.  The values
 // are line_flux's to FP32 rounding (channels up to half a line width by the same series
 // with its polynomial expanded, up to 3/2 by a longer one in place of an erf difference),
 // computed as straight-line code (the window test is one unsigned compare and a
 // select) so that the evaluations of a thread overlap.
-template <int CB, bool LEAVE_ODD, class Store2>
+template <int CB, bool FP32, class Store2>
 __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_desc& d,
                                     Store2 store2,
                                     uint32_t blocks = (1u << (CB / 16)) - 1u) {
@@ -590,7 +591,7 @@ __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_
             const float* row = d.spectra + ((int64_t)k0 * d.spectra_ld + c0 + cl0);
             const int o0 = (NT / KC) * (b * PER_BLOCK), o1 = o0 + NT / KC;
             const float v0 = inside(o0) ? amp * row[o0] : 0.0f, v1 = inside(o1) ? amp * row[o1] : 0.0f;
-            const bool odd0 = LEAVE_ODD && not_finite(v0), odd1 = LEAVE_ODD && not_finite(v1);
+            const bool odd0 = FP32 && not_finite(v0), odd1 = FP32 && not_finite(v1);
             odd = odd || odd0 || odd1;
             store2(k, b, cl0, odd0 ? 0.0f : v0, odd1 ? 0.0f : v1);
         }
@@ -611,9 +612,10 @@ __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_
     const float kf = (float)kc, fh = fu - 0.5f;
     // exp(-m^2) as exp2(-n^2) with n = m sqrt(log2 e).
     const float sn = s * SQRT_LOG2E;
-    auto narrow = [&](const LineSeries<3, true>& line, int o) { return line(sn * ((kf - (float)o) + fh)); };
+    using Narrow = LineSeries<3, true, FP32>;
+    auto narrow = [&](const Narrow& line, int o) { return line(sn * ((kf - (float)o) + fh)); };
     if (!__any(s > 0.5f)) {
-        const LineSeries<3, true> line(s, amp);
+        const Narrow line(s, amp);
 #pragma unroll
         for (int b = 0; b < CB / 16; ++b)
             if ((blocks >> b) & 1u)  // uniform
@@ -625,7 +627,7 @@ __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_
         // s = 0.62, split BF16: 382 -> 338 us per insertion; 3e5, s = 0.81: 216 -> 206).  With
         // seven terms and a plain exponent it took 325 and 203 us, and the last channels
         // at s = 3/2 were off by up to 1e-5 of their value (erf differences: 2.5e-6, now 3e-6).
-        const LineSeries<8, false> line(s, amp);
+        const LineSeries<8, false, true> line(s, amp);
 #pragma unroll 1
         for (uint32_t left = blocks; left != 0u; left &= left - 1u) {
             const int b = __builtin_ctz(left);
@@ -638,7 +640,7 @@ __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_
     // taken only inside its window.  A loop of its own: unrolled into the narrow lines'
     // code it made the kernel too long for the instruction cache (1e7 particles,
     // narrow lines: 4.78 -> 4.67 ms; 3e6 with wide ones 3.05 -> 3.06).
-    const LineSeries<3, true> line(s, amp);
+    const Narrow line(s, amp);
 #pragma unroll 1
     for (uint32_t left = blocks; left != 0u; left &= left - 1u) {
         const int b = __builtin_ctz(left);
