@@ -122,8 +122,8 @@ hipError_t layout_for(const Grid& g, int64_t n, int64_t n_pairs, Layout* L) {
     const size_t nc = (size_t)g.ncells, nc1 = nc + 1;
     L->item_len = item_length(n_pairs);
     L->items_max = g.ncells + n_pairs / L->item_len + 1;
-    L->multi_max = 2 * (n_pairs / L->item_len) + 1;
-    L->split_max = std::min<int64_t>(g.ncells, n_pairs / L->item_len);
+    L->split_max = split_cells_max(n_pairs, L->item_len, g.ncells);
+    L->multi_max = partial_tiles_max(n_pairs, L->item_len, g.ncells);
     // cleared by k_bin_init, from status on
     L->status = take(sizeof(uint32_t) * ST_WORDS);
     L->hist = take(sizeof(uint32_t) * RADIX_PASSES << RADIX_BITS);

@@ -70,6 +70,17 @@ struct Layout {
     int item_len;                      // particles per work item
 };
 
+// At most so many cells hold more than item_len of n_pairs pairs; and their items,
+// ceil(length / item_len) = 1 + (length - 1) / item_len each, are at most so many.
+inline int64_t split_cells_max(int64_t n_pairs, int item_len, int64_t ncells) {
+    const int64_t most = n_pairs / (item_len + 1);
+    return ncells < most ? ncells : most;
+}
+inline int64_t partial_tiles_max(int64_t n_pairs, int item_len, int64_t ncells) {
+    const int64_t cells = split_cells_max(n_pairs, item_len, ncells);
+    return cells + (n_pairs - cells) / item_len;
+}
+
 // status[0]: number of pairs the device produced; status[1]: overflow flag.
 // status[4]: a record with a footprint has an unknown kernel kind or table
 // weights beyond the descriptor's table (no work items are then made).

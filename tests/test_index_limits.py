@@ -54,7 +54,28 @@ static bool line_steps(int l0, int L, int k) {
            s.last - s.first <= L / 4 + 2;
 }
 
+// The most partial tiles that `pairs` pairs in `cells` cells can need: k cells of one
+// pair more than an item, the rest of the pairs in whole items of the last of them.
+static long worst_tiles(long pairs, long cells, int len) {
+    long most = 0;
+    for (long k = 1; k <= cells && k * (len + 1) <= pairs; ++k) {
+        const long rest = pairs - (k - 1) * (len + 1);
+        const long tiles = 2 * (k - 1) + (rest + len - 1) / len;
+        most = tiles > most ? tiles : most;
+    }
+    return most;
+}
+
 int main(int argc, char** argv) {
+    if (argc == 3 && argv[1][0] == 'T') {
+        const long cells = atol(argv[2]);
+        for (long pairs = 0; pairs < 40000000; pairs = pairs * 21 / 20 + 1) {
+            const int len = item_length(pairs);
+            const long most = worst_tiles(pairs, cells, len), room = partial_tiles_max(pairs, len, cells);
+            if (room < most || room > most + 1) return printf("%ld pairs: %ld, room %ld\n", pairs, most, room), 1;
+        }
+        return 0;
+    }
     if (argc == 3 && argv[1][0] == 'L') {
         const int L = atoi(argv[2]);
         for (int k = 1; k < 4096; k = k < 130 ? k + 2 : k * 3 / 2 | 1)
@@ -104,6 +125,13 @@ def test_group_pair_totals_do_not_wrap(program, each):
     """A wave's 64 particles make up to 64 (2^21 - 1) pairs; groups of 16 waves, and of 16 in 4 rounds."""
     r = subprocess.run([str(program), str(each)], capture_output=True, text=True, check=True)
     assert [int(v) for v in r.stdout.split()] == [16 * each, 64 * each]
+
+
+@pytest.mark.parametrize("cells", [1, 2, 7, 100, 512, 4096, 100000])
+def test_room_for_partial_tiles(program, cells):
+    """What the worst split of the pairs over the cells needs, and one more at most."""
+    r = subprocess.run([str(program), "T", str(cells)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
 
 
 @pytest.mark.parametrize("length", [1, 2, 3, 4, 5, 15, 16, 31, 32, 33, 64, 65, 97, 300])
