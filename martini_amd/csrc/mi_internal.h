@@ -126,6 +126,19 @@ hipError_t prepare_particles(const double* xyz, const double* vxyz, const double
 
 // Beam convolution of a cube (mi_beam.hip).
 size_t beam_lds_bytes(int kx, int ky);
+// Rows y of a tile per work group.  Work groups aimed at, at most while a group can
+// take more rows: four 33 KB tiles on each of the 256 CUs, so that a small cube still
+// fills them and a large one leaves a group rows to overlap (301 x 257 x 131 FP32: 54
+// us with 8 rows per group, 34 with the 4 of this rule; 512 x 512 x 256 FP64 253 us with
+// 8 rows, 246 with 16).  Rounded down, narrow tiles made twice as many groups, each
+// for a row (3 x 2000 x 5 FP32: 28 to 31 us, 25 with 8 rows per group, 22 so; 64 x 1025
+// x 64 FP64: 41, 64, 21).
+constexpr int64_t FITS_GROUPS = 1024;
+constexpr int FITS_MAX_ROWS = 16;
+inline int fits_rows(int64_t tiles, int ny) {
+    const int64_t rows = (tiles * ny + FITS_GROUPS - 1) / FITS_GROUPS;
+    return (int)(rows < FITS_MAX_ROWS ? rows : FITS_MAX_ROWS);
+}
 hipError_t cube_to_fits(const void* cube, bool cube_f64, int nx, int ny, int nc, int padx,
                         int pady, bool f64, void* out, double* range, hipStream_t s);
 hipError_t convolve_beam(const float* in, float* out, int nx, int ny, int nc, const float* K,

@@ -20,7 +20,6 @@
 // groups' atomics go to one cache line, about 11 ns each).
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <type_traits>
 
 #include "../../include/martini_mi355x.h"
@@ -29,12 +28,6 @@
 namespace mi {
 
 constexpr int FT = 64;  // tile edge (x and channel)
-// Work groups aimed at: four 33 KB tiles on each of the 256 CUs, so that a
-// small cube still fills them and a large one leaves a group rows to overlap
-// (301 x 257 x 131 FP32: 54 us with 8 rows per group, 35 with the 3 of this
-// rule; 512 x 512 x 256 FP64 253 us with 8 rows, 246 with 16).
-constexpr int64_t FITS_GROUPS = 1024;
-constexpr int FITS_MAX_ROWS = 16;  // rows y per work group
 
 // Unsigned image of a floating value whose integer order is the numeric order.
 __device__ inline uint32_t order_of(float f) {
@@ -179,7 +172,7 @@ template <typename In, typename Out>
 static void launch_to_fits(const In* cube, int nx, int ny, int nc, int padx, int pady, void* out,
                            unsigned long long* range, hipStream_t s) {
     const int64_t tiles = (int64_t)((nx + FT - 1) / FT) * ((nc + FT - 1) / FT);
-    const int rows = (int)std::clamp<int64_t>(tiles * ny / FITS_GROUPS, 1, FITS_MAX_ROWS);
+    const int rows = fits_rows(tiles, ny);
     const dim3 grid((unsigned)tiles, (unsigned)((ny + rows - 1) / rows));
     constexpr int L = 16 / sizeof(In), S = 16 / sizeof(Out);
     const bool la = nc % L == 0 && (reinterpret_cast<uintptr_t>(cube) & 15) == 0;

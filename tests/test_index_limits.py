@@ -67,6 +67,17 @@ static long worst_tiles(long pairs, long cells, int len) {
 }
 
 int main(int argc, char** argv) {
+    if (argc == 3 && argv[1][0] == 'F') {
+        const long tiles = atol(argv[2]);
+        for (int ny = 1; ny <= 32767; ++ny) {
+            const int rows = fits_rows(tiles, ny);
+            const long groups = tiles * ((ny + rows - 1) / rows);
+            if (rows < 1 || rows > FITS_MAX_ROWS) return printf("%d rows\n", rows), 1;
+            // one more for each tile's remainder
+            if (rows < FITS_MAX_ROWS && groups > FITS_GROUPS + tiles) return printf("%d: %ld groups\n", ny, groups), 1;
+        }
+        return 0;
+    }
     if (argc == 3 && argv[1][0] == 'T') {
         const long cells = atol(argv[2]);
         for (long pairs = 0; pairs < 40000000; pairs = pairs * 21 / 20 + 1) {
@@ -125,6 +136,12 @@ def test_group_pair_totals_do_not_wrap(program, each):
     """A wave's 64 particles make up to 64 (2^21 - 1) pairs; groups of 16 waves, and of 16 in 4 rounds."""
     r = subprocess.run([str(program), str(each)], capture_output=True, text=True, check=True)
     assert [int(v) for v in r.stdout.split()] == [16 * each, 64 * each]
+
+
+@pytest.mark.parametrize("tiles", [1, 2, 3, 10, 100, 1000])
+def test_fits_work_groups(program, tiles):
+    r = subprocess.run([str(program), "F", str(tiles)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
 
 
 @pytest.mark.parametrize("cells", [1, 2, 7, 100, 512, 4096, 100000])
