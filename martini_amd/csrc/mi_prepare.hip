@@ -86,12 +86,19 @@ __device__ Setup setup_particle(int64_t i, const double* __restrict__ xyz,
     // products are ratios of linear forms in it: no inverse trigonometry, and
     // no rounding of a right ascension near 360 degrees.
     double X = pos[0], Y = pos[1], Z = pos[2];
-    if (!(dist < INFINITY)) {  // the direction that atan2 gives infinite components
-        X = isinf(X) ? copysign(1.0, X) : X - X;
-        Y = isinf(Y) ? copysign(1.0, Y) : Y - Y;
-        Z = isinf(Z) ? copysign(1.0, Z) : Z - Z;
-    } else if (dist == 0.0) {  // the observer: right ascension and declination zero
-        X = 1.0;
+    if (!(dist < INFINITY) || dist < 0x1p-500) {
+        if (isinf(X) || isinf(Y) || isinf(Z)) {  // the direction that atan2 gives them
+            X = isinf(X) ? copysign(1.0, X) : X - X;
+            Y = isinf(Y) ? copysign(1.0, Y) : Y - Y;
+            const double across = sqrt(X * X + Y * Y);
+            Z = isinf(Z) ? copysign(across > 0.0 ? across : 1.0, Z) : Z - Z;
+        } else {  // components whose squares leave the range still have one
+            const double k = dist < 1.0 ? 0x1p600 : 0x1p-600;
+            X *= k;
+            Y *= k;
+            Z *= k;
+        }
+        if (X == 0.0 && Y == 0.0 && Z == 0.0) X = 1.0;  // the observer: both angles zero
     }
     const double across = Y * c.cos_a0 - X * c.sin_a0;  // cos dec sin(ra - a0)
     const double along = X * c.cos_a0 + Y * c.sin_a0;   // cos dec cos(ra - a0)

@@ -183,3 +183,39 @@ def test_prepare_directions_match_host():
         assert drec.size == hrec.size
         for f in ("ix", "iy", "c_lo", "c_hi"):
             assert np.array_equal(drec[f], hrec[f]), (f, drec[f], hrec[f])
+
+
+def test_prepare_directions_out_of_range_match_host():
+    """The same for positions whose squares overflow or underflow, and with
+    several infinite components."""
+    inf, D, c = np.inf, 3000.0, np.sqrt(0.5)  # kpc
+    xyz = np.array([[1e200, 1e197, 0], [1e160, -1e157, 2e157], [-1e200, 1, 1], [1e200, 1e200, 0],
+                    [-D, 1e-190, 0], [-D, 0, -1e-200], [inf, 1, inf], [inf, inf, inf],
+                    [inf, 1, 1e200], [1, inf, -inf], [1, 2, 3],
+                    # and one in the middle of each map below
+                    [0.5 * D - D, 0.5 * D, c * D], [c * D - D, 0, c * D]], float)
+    w = dataclasses.replace(synthetic.WORKLOADS["disc1e4_64px"], n=len(xyz))
+    n = len(xyz)
+    from martini_amd import DataCube, SPHSource, _pack
+
+    for ra, dec in ((0.0, 0.0), (45.0, 45.0), (0.0, 45.0)):
+        kw = dict(n_px_x=65, n_px_y=64, n_channels=16, px_size=16.0, channel_width=8.0,
+                  spectral_centre=w.vsys, ra=ra, dec=dec)
+        src = SPHSource(distance=w.distance, h=0.7, T_g=np.full(n, 1e4), mHI_g=np.full(n, 1e4),
+                        xyz_g=xyz, vxyz_g=np.zeros((n, 3)), hsm_g=np.full(n, 0.5))
+        with np.errstate(all="ignore"):
+            m = Martini(source=src, datacube=DataCube(**kw), sph_kernel=CubicSplineKernel(),
+                        spectral_model=GaussianSpectrum(sigma="thermal"), quiet=True)
+            hrec, _ = _pack.pack_particles(m.source, m.sph_kernel, m.spectral_model, m.datacube)
+        obs, _ = observation(distance=w.distance, datacube=DataCube(**kw),
+                             sph_kernel=CubicSplineKernel(),
+                             spectral_model=GaussianSpectrum(sigma="thermal"))
+        out, counts = prepare(DeviceSource(xyz, np.zeros((n, 3)), np.full(n, 1e4), np.full(n, 0.5),
+                                           np.full(n, 1e4)), obs)
+        drec = out[: int(counts.cpu()[0]) * 48].cpu().numpy().view(_lib.PARTICLE_DTYPE)
+        assert drec.size == hrec.size > 0
+        for i, f in (("ix", "fx"), ("iy", "fy")):  # a position may lie on a pixel's edge
+            at = [r[i] + r[f].astype(float) for r in (drec, hrec)]
+            assert np.allclose(*at, rtol=1e-9, atol=1e-6), (i, at)
+        for f in ("c_lo", "c_hi"):
+            assert np.array_equal(drec[f], hrec[f]), (f, drec[f], hrec[f])
