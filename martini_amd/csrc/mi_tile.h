@@ -547,7 +547,8 @@ struct LineSeries {
         const float m2 = m * m, m2l = fmaf(m + m, ml, fmaf(m, m, -m2));
         const float y = m2 * (float)LOG2E, yl = fmaf(m2, (float)LOG2E, -y);
         const float g = __builtin_amdgcn_exp2f(-y);
-        return fmaf(-g, fmaf(yl, 0.693147181f, m2l), g) * polynomial(m2);
+        // g is zero long before the polynomial overflows: its argument ends there
+        return fmaf(-g, fmaf(yl, 0.693147181f, m2l), g) * polynomial(fminf(m2, 256.0f));
     }
 };
 

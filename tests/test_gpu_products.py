@@ -330,3 +330,34 @@ def test_narrow_lines_have_no_bias():
         got = cube.cpu().numpy().reshape(n, shape[2])[use, 62:67].astype(float)
         bias = np.mean(got / want[use] - 1.0)
         assert abs(bias) <= bound, (bias, bound)
+
+
+@pytest.mark.parametrize("method", ["plain", "mfma"])
+@pytest.mark.parametrize("widths", [(0.05, 0.5), (0.5001, 1.4999), (1.5001, 30.0)])
+def test_windows_over_all_channels(method, widths):
+    """Windows that take in every channel, thousands from the line: zero there, and
+    1e-6 of the amplitude right elsewhere."""
+    import torch
+    from scipy.special import erf
+
+    shape = (8, 8, 4096)
+    n, nc = 64, shape[2]
+    rng = np.random.default_rng(2)
+    rec = np.zeros(n, _lib.PARTICLE_DTYPE)
+    rec["ix"], rec["iy"] = np.arange(n) // 8, np.arange(n) % 8
+    rec["r_kind"], rec["amp"], rec["h"] = _lib.KERNEL_DIRAC, 100.0, 1.0
+    rec["s"], rec["fu"] = np.exp(rng.uniform(*np.log(widths), n)), rng.uniform(0, 1, n)
+    rec["k0"], rec["c_hi"] = rng.choice([0, 5, 2000, nc - 1], n), nc - 1
+    desc = _lib.make_desc(*shape, _lib.SPECTRUM_GAUSS)
+    pairs = _lib.count_pairs(rec, desc)
+    d_rec = torch.from_numpy(rec.view(np.uint8)).cuda()
+    cube = torch.zeros(n * nc, dtype=torch.float32, device="cuda")
+    ws = torch.zeros(_lib.workspace_bytes(desc, n, pairs), dtype=torch.uint8, device="cuda")
+    _lib.insert(d_rec, n, pairs, desc, cube, ws, method=method)
+    got = cube.cpu().numpy().reshape(n, nc).astype(float)
+    b = rec["s"].astype(float)[:, None] * (rec["k0"][:, None] - np.arange(nc) + rec["fu"].astype(float)[:, None])
+    a = b - rec["s"].astype(float)[:, None]
+    want = 50.0 * (erf(b) - erf(a))
+    assert np.all(np.isfinite(got))
+    assert np.max(np.abs(got - want)) <= 100.0 * (1e-6 if method == "plain" else 2.0**-16)
+    assert np.all(got[(a > 20.0) | (b < -20.0)] == 0.0)
