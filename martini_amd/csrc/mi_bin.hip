@@ -9,13 +9,10 @@
 // such cells get one partial tile per item.
 //
 // Launches: k_bin_init, k_emit (pairs, in particle order), one k_radix per
-// digit, k_cell_bounds, k_items (and k_build_items for many cells).  Every
-// kernel that places data by a running total (k_emit, k_radix) takes it from a
-// decoupled look-back: work groups are numbered by a ticket, publish their own
-// count in a 64-bit word (state and value together, so no other memory needs
-// ordering) and sum the words before theirs, back to the nearest one that holds
-// a total.  A group waits only for lower tickets, which run already and publish
-// before they wait.
+// digit, k_cell_bounds, k_items (and k_build_items for many cells).  The kernels
+// that place data by a running total (k_emit, k_radix) take it from a decoupled
+// look-back (mi_lookback.h); the radix passes are those of Adinets and Merrill,
+// "Onesweep: A Faster Least Significant Digit Radix Sort for GPUs", 2022.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,6 +20,7 @@
 
 #include "mi_device.h"
 #include "mi_internal.h"
+#include "mi_lookback.h"
 #include "mi_tile.h"
 
 namespace mi {
@@ -169,46 +167,6 @@ __device__ inline bool record_ok(const mi_particle& p, const Grid& g, const floa
     if (!footprint(p, g.nx, g.ny, i_lo, i_hi, j_lo, j_hi)) return true;
     const int64_t end = (int64_t)table_offset(p) + (int64_t)(i_hi - i_lo + 1) * (j_hi - j_lo + 1);
     return end <= uw_n;
-}
-
-// Look-back words: state in the top bits, a count in the rest (of the group
-// alone, or of all groups up to it).
-constexpr unsigned long long LB_GROUP = 1ull << 62, LB_ALL = 2ull << 62;
-constexpr unsigned long long LB_STATE = 3ull << 62;
-
-// Pause between two looks at words that are not published yet (x 64 cycles):
-// the groups that wait would otherwise fill the fabric with their reads.
-constexpr int LOOK_SLEEP = 8;
-
-__device__ inline unsigned long long look_load(const unsigned long long* w) {
-    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void look_store(unsigned long long* w, unsigned long long v) {
-    __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Sum of the counts of the groups before `group`, taken by one wave, 64 words
-// at a time.
-__device__ inline unsigned long long look_back(const unsigned long long* look, int64_t group) {
-    const int lane = threadIdx.x & 63;
-    unsigned long long base = 0;
-    for (int64_t j = group - 1; j >= 0; j -= 64) {
-        unsigned long long v;
-        uint64_t all, need;
-        while (true) {
-            v = j - lane >= 0 ? look_load(&look[j - lane]) : LB_ALL;
-            all = __ballot((v & LB_STATE) == LB_ALL);
-            need = all ? (all & (0ull - all)) * 2ull - 1ull : ~0ull;  // up to the nearest total
-            if ((__ballot((v & LB_STATE) != 0ull) & need) == need) break;
-            __builtin_amdgcn_s_sleep(LOOK_SLEEP);
-        }
-        unsigned long long x = (need >> lane) & 1ull ? v & ~LB_STATE : 0ull;
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
-        base += x;
-        if (all) break;
-    }
-    return base;
 }
 
 // Writes the (key, particle) pairs of each particle, in particle order: group b

@@ -22,6 +22,7 @@
 #include "../../include/martini_mi355x.h"
 #include "mi_device.h"
 #include "mi_internal.h"
+#include "mi_lookback.h"
 
 namespace mi {
 
@@ -241,11 +242,6 @@ constexpr int PREP_SPAN = PREP_T * PREP_R;
 
 __host__ __device__ inline int64_t prep_groups(int64_t n) { return (n + PREP_SPAN - 1) / PREP_SPAN; }
 
-// A group's look-back word: state in the top bits, records kept in the low 32
-// (of the group alone, or of all groups up to it).
-constexpr unsigned long long LB_GROUP = 1ull << 62, LB_ALL = 2ull << 62;
-constexpr unsigned long long LB_STATE = 3ull << 62;
-
 // What a group adds to the totals (besides its records).
 struct PrepSums {
     unsigned long long pairs, px, flags;
@@ -273,9 +269,6 @@ __device__ inline unsigned long long wave_sum(unsigned long long v) {
 // (1.9 TB/s), and the whole call with its counters read back 482 -> 117 us.
 // Groups of 256 particles make it 127 us, of 1024 117 us; held to 128 registers
 // (four waves per SIMD instead of three) it spills and takes 130 us.
-// Groups are numbered by a ticket, so every group that a look-back waits for
-// holds a lower ticket: it is running or done, and publishes its own count
-// before it waits for anything.
 __global__ __launch_bounds__(PREP_T) void k_prepare(
     const double* __restrict__ xyz, const double* __restrict__ vxyz,
     const double* __restrict__ mHI, const double* __restrict__ hsm, const double* __restrict__ T,
@@ -319,39 +312,17 @@ __global__ __launch_bounds__(PREP_T) void k_prepare(
             for (int q = 0; q < 3; ++q) recs[at * 3 + q] = words[q];
         }
     }
-    if (t == 0)
-        __hip_atomic_store(&look[group], (group == 0 ? LB_ALL : LB_GROUP) | kept, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+    if (t == 0) look_store(&look[group], (group == 0 ? LB_ALL : LB_GROUP) | kept);
     pairs = wave_sum(pairs);
     px = wave_sum(px);
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) flags |= __shfl_xor(flags, d, 64);
     if (lane == 0) wsum[wave] = PrepSums{pairs, px, flags};
     if (wave == 0) {
-        // records kept by the groups before this one: 64 words at a time, back
-        // to the nearest group that already knows its total
-        uint32_t base = 0;
-        for (int64_t j = group - 1; j >= 0; j -= 64) {
-            unsigned long long v;
-            uint64_t all, need;
-            do {
-                v = j - lane >= 0 ? __hip_atomic_load(&look[j - lane], __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT)
-                                  : LB_ALL;
-                all = __ballot((v & LB_STATE) == LB_ALL);
-                need = all ? (all & (0ull - all)) * 2ull - 1ull : ~0ull;  // up to the nearest total
-            } while ((__ballot((v & LB_STATE) != 0ull) & need) != need);
-            uint32_t x = (need >> lane) & 1ull ? (uint32_t)v : 0u;
-#pragma unroll
-            for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
-            base += x;
-            if (all) break;
-        }
+        const uint32_t base = (uint32_t)look_back(look, group);  // records kept before this group's
         if (lane == 0) {
             s_base = base;
-            if (group > 0)
-                __hip_atomic_store(&look[group], LB_ALL | (base + kept), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+            if (group > 0) look_store(&look[group], LB_ALL | (base + kept));
             if (group == prep_groups(n) - 1) counts[0] = (unsigned long long)base + kept;
         }
     }
