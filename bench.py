@@ -39,7 +39,7 @@ PEAK_TFLOPS = {"plain": 157.3, "mfma": 2500.0}  # MI355X dense FP32 / BF16 (publ
 PEAK_HBM_GBS = 8000.0  # MI355X HBM3E
 PRODUCTS = {"plain": 1, "mfma": 3}  # products per logical multiply-add (bf16x3 spends 3)
 DTYPE = {"plain": "fp32", "mfma": "bf16x3"}
-BOUND = {"plain": "valu_fp32", "mfma": "mfma"}
+BOUND = {"plain": "mfma_fp32", "mfma": "mfma"}  # the unit that `peak` is of
 GATHER_KERNEL = {"plain": "k_gather<Float32>", "mfma": "k_gather<SplitBf16>"}
 TRAFFIC_FILE = "profiles/hbm_traffic_gather.md"
 METRIC = "particle-voxel updates/s; p50/p99 cube latency; MFMA vs FP32 at 1e-5 rel err"

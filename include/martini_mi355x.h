@@ -160,7 +160,14 @@ int64_t mi_count_pairs_host(const mi_particle* h_particles, int64_t n,
 
 /* Workspace bytes for mi_insert with n particles producing n_pairs pairs.
  * Every entry point that takes d_workspace requires it 256-byte aligned (as
- * hipMalloc returns it) and refuses it otherwise with MI_ERR_ARGUMENT. */
+ * hipMalloc returns it) and refuses it otherwise with MI_ERR_ARGUMENT.
+ * Up to 20 bytes per pair and 24 per cell, and the partial tiles (64 KiB) of cells split
+ * over work items, as many as n_pairs pairs on these cells can need.  Small inputs are
+ * split finely to fill the chip, so these dominate there, and the size does not grow with
+ * n_pairs throughout: 93 MiB for 24500 pairs and 49 for 25500 on 512 x 512 x 256 (13
+ * each in items of 256 particles, which took up to 1.5 times as long), 195 MiB for
+ * 1.5e6 on 256 x 256 x 128 (289).  A workspace kept for several inputs takes the
+ * largest of their sizes. */
 int mi_insert_workspace_size(const mi_cube_desc* desc, int64_t n, int64_t n_pairs,
                              size_t* bytes);
 

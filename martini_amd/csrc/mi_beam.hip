@@ -508,7 +508,8 @@ hipError_t convolve_beam(const float* in, float* out, int nx, int ny, int nc, co
     // k_convolve_beam's time goes with the number of its small tiles (720 of them, 256
     // x 70 x 36: 65 us against 49; 768, 256 x 87 x 30: 58 against 50; 960, 89 x
     // 65 x 128: 65 against 62; 1024, 128 x 128 x 64: 60 against 64.5; 2560, 256 x
-    // 68 x 128: 87 against 130; 10368, 282 x 282 x 128: 283 against 596); and where
+    // 68 x 128: 87 against 130; 10368, 282 x 282 x 128: 283 against 596; images of 3 x 3
+    // to 15 x 15 on nine shapes from 1000 tiles on: 0.33 to 1.01 of its time); and where
     // its tiles of 48 columns or more are not half empty (256 x 24 x 128: 66 against
     // 62).  Three outputs per lane against four by the columns they cover: three take
     // 1.09 times as long per column.

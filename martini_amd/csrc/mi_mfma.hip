@@ -19,15 +19,15 @@
 //              2^-16 of the product).
 //
 // Both are bound by the evaluation of W and S on the vector units (70% busy on 1e7
-// particles, 512 x 512 x 256, split BF16: gather 3.83 ms; without the W fill 1.1 ms
+// particles, 512 x 512 x 256, split BF16: gather 3.89 ms; without the W fill 1.1 ms
 // less, without the S fill 0.7, without the products 0.6); the FP32 products take
 // about a quarter of the matrix units' time beside it (26% on 3e6 of heterogeneous
-// size, 1024 x 1024 x 64: 2.8 ms).  On the vector units the
+// size, 1024 x 1024 x 64: 2.77 ms).  On the vector units the
 // FP32 products (64 multiply-adds per particle, thread and tile row, all
 // channels) took most of that form's time: gather 643 us on 1e6 particles
 // (WendlandC2, 256 x 256 x 128), 4.42 ms on 3e6 of heterogeneous size
-// (1024 x 1024 x 64); on the matrix units 597 us and 3.59 ms at first, 360 us and
-// 2.8 ms with what is described below.
+// (1024 x 1024 x 64); on the matrix units 597 us and 3.59 ms at first, 367 us and
+// 2.75 ms with what is described below.
 //
 // Wave w owns four tile rows (M = the 16 pixels of a row) and four 16-channel
 // blocks (N): with 16 x 16-pixel x 64-channel cells the rows w, w + 4, .. and
@@ -65,9 +65,11 @@
 // channels and pixels were lost against the bright voxels one by one, each sum 5e-8
 // to 2e-7 low on sparse cubes (1.6e5 particles, 512 x 512 x 256, error against FP64:
 // 1.4e-7 so, 5.2e-8 now; 1.5e6: 2.0e-7, 5.5e-8; heterogeneous 1e6, 512 x 512 x 64:
-// 5.6e-8, 4.3e-8), for 2 to 3% of the form's time.  The tile rows are taken one by one
-// for it: with a row's operands and one sum held instead of four rows' nothing spills.
-// The split form keeps one chain (the additions took 5% of 1e7 particles there).
+// 5.6e-8, 4.3e-8), for 1 to 5% of the form's time (1e7 particles, 512 x 512 x 256:
+// insertion 6.66 -> 6.97 ms; 1e6, 256 x 256 x 128: 475 -> 480 us).  The tile rows are
+// taken one by one for it: with a row's operands and one sum held instead of four
+// rows' nothing spills.  The split form keeps one chain (the additions took 5% of
+// 1e7 particles there).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Nothing in ``martini_amd`` imports, links or runs
 anything under this folder; only ``tests/``, ``__graft_entry__.smoke()`` and the
-``cpu_baseline`` leg of ``bench.py`` use it, and only as the checker.
+``cpu_baseline`` leg of ``bench.py`` use it, and only to check results and to time it.
 
 Contents
 --------
