@@ -628,12 +628,14 @@ __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_
         // s = 0.62, split BF16: 382 -> 338 us per insertion; 3e5, s = 0.81: 216 -> 206).  With
         // seven terms and a plain exponent it took 325 and 203 us, and the last channels
         // at s = 3/2 were off by up to 1e-5 of their value (erf differences: 2.5e-6, now 3e-6).
-        const LineSeries<8, false, true> line(s, amp);
+        // The amplitude last: in the coefficients, which grow with s^16 and are far larger
+        // than the flux beside the line, it left FP32's range from 1e36 on.
+        const LineSeries<8, false, true> line(s, 1.0f);
 #pragma unroll 1
         for (uint32_t left = blocks; left != 0u; left &= left - 1u) {
             const int b = __builtin_ctz(left);
             const float j = kf - (float)(16 * b);
-            put(b, line.at(s, j + fh), line.at(s, j - (float)(NT / KC) + fh));
+            put(b, amp * line.at(s, j + fh), amp * line.at(s, j - (float)(NT / KC) + fh));
         }
         return false;
     }

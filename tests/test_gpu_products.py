@@ -361,3 +361,38 @@ def test_windows_over_all_channels(method, widths):
     assert np.all(np.isfinite(got))
     assert np.max(np.abs(got - want)) <= 100.0 * (1e-6 if method == "plain" else 2.0**-16)
     assert np.all(got[(a > 20.0) | (b < -20.0)] == 0.0)
+
+
+@pytest.mark.parametrize("method", ["plain", "mfma"])
+@pytest.mark.parametrize("shape", [(16, 16, 64), (8, 16, 128)])
+@pytest.mark.parametrize("widths", [(0.2, 0.5), (0.5001, 1.0), (1.4, 1.4999), (2.0, 8.0)])
+def test_bright_lines(method, shape, widths):
+    """Lines of the largest amplitudes, a particle a pixel: 2^k times the cube of
+    amplitudes near 1, bit for bit where that is far from FP32's smallest numbers (a power
+    of two changes no rounding there; a split value's second part is 2^-17 of it)."""
+    import torch
+
+    nx, ny, nc = shape
+    n = nx * ny
+    rng = np.random.default_rng(nc)
+    rec = np.zeros(n, _lib.PARTICLE_DTYPE)
+    rec["ix"], rec["iy"] = np.arange(n) // ny, np.arange(n) % ny
+    rec["r_kind"], rec["h"] = _lib.KERNEL_DIRAC, 1.0
+    rec["s"], rec["fu"], rec["k0"] = rng.uniform(*widths, n), rng.uniform(0, 1, n), rng.integers(0, nc, n)
+    half = np.ceil(4.0 / rec["s"]).astype(int) + 1
+    rec["c_lo"], rec["c_hi"] = np.maximum(rec["k0"] - half, 0), np.minimum(rec["k0"] + half, nc - 1)
+    amp = rng.uniform(0.5, 1.0, n).astype(np.float32)
+    desc = _lib.make_desc(*shape, _lib.SPECTRUM_GAUSS)
+    pairs = _lib.count_pairs(rec, desc)
+    cubes = []
+    for k in (0, 127):
+        rec["amp"] = amp * np.float32(2.0**k)
+        d_rec = torch.from_numpy(rec.view(np.uint8)).cuda()
+        cube = torch.zeros(n * nc, dtype=torch.float32, device="cuda")
+        ws = torch.empty(_lib.workspace_bytes(desc, n, pairs), dtype=torch.uint8, device="cuda")
+        _lib.insert(d_rec, n, pairs, desc, cube, ws, method=method)
+        cubes.append(cube.cpu().numpy().astype(float))
+    assert np.all(np.isfinite(cubes[1])) and np.max(cubes[0]) > 0.1
+    normal = cubes[0] > 2.0**-100
+    assert np.array_equal(cubes[1][normal], cubes[0][normal] * 2.0**127)
+    assert np.all(cubes[1][~normal] <= 2.0**27)
