@@ -625,7 +625,7 @@ __device__ inline bool fill_spectra(const ChunkState& cs, int c0, const mi_cube_
     }
     if (!__any(s > 1.5f)) {
         // A longer series, a third of the erf difference's work per channel (1e6 particles,
-        // s = 0.62, split BF16: 382 -> 338 us per insertion; 3e5, s = 0.81: 216 -> 206).  With
+        // s = 0.62, split BF16: 382 -> 341 us per insertion; 3e5, s = 0.81: 216 -> 206).  With
         // seven terms and a plain exponent it took 325 and 203 us, and the last channels
         // at s = 3/2 were off by up to 1e-5 of their value (erf differences: 2.5e-6, now 3e-6).
         // The amplitude last: in the coefficients, which grow with s^16 and are far larger
